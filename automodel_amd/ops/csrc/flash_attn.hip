@@ -1,311 +1,288 @@
-// Flash attention fwd+bwd (CDNA4, gfx950) — BSHD + packed varlen (THD),
-// causal, GQA, head dims {64, 96, 128, 192, 256} and split-dim MLA (qk 192 /
-// v 128). Deterministic backward (no atomics).
+// Flash attention forward (CDNA4, gfx950): BSHD and packed varlen (THD), causal, GQA,
+// head dims {64, 96, 128, 192, 256} and split dims (qk 192 / v 128), optional sinks.
 //
-// MI355X-native replacement for the reference's TE DotProductAttention /
-// flash-attn backends (te_attention.py:352 arbitrary
-// dims, distributed/thd_utils.py:85 THD varlen). Structure follows the CDNA4
-// guide's fused-attention recipe (cdna_hip_programming.md Appendix B):
-//   * swapped QK^T — mfma_f32_32x32x16_bf16 computing mfma(K, Q) so each
-//     lane holds a P column for ONE q row -> softmax is in-register
-//     (16 regs + one __shfl_xor(32) cross-half exchange)
-//   * online softmax (running m, l per q row)
-//   * P -> bf16 via packed cvt + __builtin_amdgcn_permlane32_swap to build
-//     the PV A-fragment without LDS round trips (guide T12)
-//   * K tile LDS-staged with XOR swizzle (guide T2 / Guideline 4), row
-//     stride padded to a multiple of 256 B so the ((row&15)<<4) swizzle is
-//     conflict-free at every head dim
-//   * V tile staged TRANSPOSED in LDS (vt[d][k]) with its own XOR swizzle
-//     so PV B-fragments are contiguous ds_read_b128
+// A workgroup takes 32 query rows of one head per wave and walks K/V in tiles of 64 keys,
+// double-buffered in LDS by direct loads, one barrier a tile. Both products have the query
+// as the accumulator's column, so that a row's maximum, sum and rescaling are per-lane
+// values (flash_tile.h).
 //
-// Varlen (packed THD): per-token doc_start/doc_end arrays (precomputed from
-// cu_seqlens in ops/attention.py) gate the causal mask to the query's own
-// document; KV-tile ranges are clipped per block/wave so cross-document
-// tiles are skipped, giving ONE kernel launch per packed batch.
+// The products of a tile take 1024 cycles of a SIMD's matrix core and its softmax about
+// 900 of the vector unit, so the loop is pipelined over half tiles: while half tile i goes
+// through exp, the matrix core forms the scores of i + 1 and the values of i - 1 (`step`,
+// one basic block). Two waves a SIMD, or two workgroups a CU, fill what one wave leaves.
+// Bound by the dependence of exp on the row maximum and by LDS reads (at 32 rows per wave
+// the four SIMDs ask for 128 B/clk at full rate). 64 rows per wave would halve the LDS
+// reads, but the accumulators leave too few registers: it spilled and ran at 100 TFLOP/s.
+// Measured (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128: 6.52 -> 2.62 ms,
+// 838 TFLOP/s; 2 x 4096: 1030 -> 347 us; 2 x 3072, 16 heads (192, 128): 414 -> 186 us;
+// 4 x 2048, 16/8 heads of 64: 154 -> 67 us.
 //
-// Backward determinism: the dKV kernel's grid is (kv tiles, Hk, B) and each
-// block loops over the GQA query-head group, accumulating dK/dV in registers
-// across the whole q loop — plain stores, no atomicAdd, bitwise
-// run-to-run-identical grads (reference determinism discipline,
-// moe/experts.py:66).
+// Varlen: per-token doc_start gates the causal mask to the query's own document; tiles
+// before a block's first document are skipped.
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 
 #include "common.h"
-#include "flash_attn.h"
+#include "flash_tile.h"
 #include "ops_api.h"
 
 namespace amd_ops {
 
-// ===========================================================================
-// Forward
-// ===========================================================================
+using namespace fa;
+
+struct FwdArgs {
+  const bf16 *q, *k, *v;
+  bf16* out;
+  float* lse;
+  const int* doc_start;
+  const bf16* sink;
+  int B, Sq, Skv, Hq, Hk, q_start;
+  float scale_log2;      // |scale| * log2(e)
+  bool negative;         // scale < 0: q changes sign
+  bool causal;
+};
 
 template <int DQK, int DV, int WAVES, bool VARLEN>
-__global__ __launch_bounds__(WAVES * WAVE_SIZE, 2) void flash_fwd_kernel(
-    const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
-    bf16* __restrict__ out, float* __restrict__ lse, const int* __restrict__ doc_start,
-    const bf16* __restrict__ sink, int B, int Sq, int Skv, int Hq, int Hk, int q_start,
-    float scale, bool causal) {
-  constexpr int KB = pad256(DQK * 2);     // K tile row stride (bytes)
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* k_lds = smem;                               // KVBLK*KB
-  char* v_img = smem + KVBLK * KB;                  // subtiled [DV/16][32][16]
-  float* bcast = reinterpret_cast<float*>(smem + KVBLK * KB + sub_img_bytes<DV>());
-  int* bcast_skip = reinterpret_cast<int*>(bcast + WAVES * 32);
+struct Fwd {
+  static constexpr int BM = WAVES * 32;
+  static constexpr int KT = 64 * row_bytes(DQK), VT = 64 * row_bytes(DV);   // tile bytes
+  static constexpr int SMEM = 2 * KT + 2 * VT;
+  static constexpr int NC = DQK / 16, NT = DV / 32;
 
-  const int tid = threadIdx.x;
-  const int lane = tid & (WAVE_SIZE - 1);
-  const int wid = tid / WAVE_SIZE;
-  const int col = lane & 31;           // q row within wave tile (QK layout)
-  const int half = lane >> 5;
+  char* smem;
+  unsigned kbase, vbase;
+  float c;               // scale * log2(e)
+  bf16x8_t qf[NC];
+  f32x16_t o[NT];
+  float m, l;            // maximum (unscaled) and this half-wave's sum of its row
+  int qpos, qdoc, skv;
+  bool causal;
 
-  const int qblk0 = blockIdx.x * (WAVES * QBLK);
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
-  const int kvh = h / (Hq / Hk);
-
-  const long q_base = (((long)b * Sq) * Hq + h) * DQK;
-  const long k_base = (((long)b * Skv) * Hk + kvh) * DQK;
-  const long v_base = (((long)b * Skv) * Hk + kvh) * DV;
-  const long o_base = (((long)b * Sq) * Hq + h) * DV;
-  const long q_rs = (long)Hq * DQK, k_rs = (long)Hk * DQK;
-  const long v_rs = (long)Hk * DV, o_rs = (long)Hq * DV;
-
-  const int q0 = qblk0 + wid * QBLK;   // this wave's first q row
-
-  // ---- load Q fragments to registers: lane holds Q[q0+col][8*half + j + 16*c]
-  bf16x8_v qfrag[DQK / 16];
+  // scores of the 32 keys `sub` of a K tile
+  __device__ __forceinline__ void scores(f32x16_t& s, unsigned ktile, int sub) {
+    s = zero16();
 #pragma unroll
-  for (int c = 0; c < DQK / 16; ++c) {
-    const bf16* src = q + q_base + (long)(q0 + col) * q_rs + c * 16 + half * 8;
-    qfrag[c] = *reinterpret_cast<const bf16x8_v*>(src);
+    for (int ch = 0; ch < NC; ++ch) s = mma(read_rows<DQK>(smem, ktile, kbase, sub, ch), qf[ch], s);
   }
 
-  // varlen doc bounds: lane's q row is fixed for the whole kernel
-  const int qg_lane = q_start + q0 + col;
-  const int ds_lane = VARLEN ? doc_start[qg_lane] : 0;        // lane's doc start
-  const int ds_wave = VARLEN ? doc_start[q_start + q0] : 0;   // wave min (non-decreasing)
-
-  // ---- accumulators
-  f32x16 o_acc[DV / 32];
+  __device__ __forceinline__ void values(const bf16x8_t (&p)[2], unsigned vtile, int sub) {
 #pragma unroll
-  for (int t = 0; t < DV / 32; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o_acc[t][r] = 0.f;
-  float m_run = -1e30f, l_run = 0.f;
+      for (int ch = 0; ch < 2; ++ch)
+        o[t] = mma(read_cols<DV>(smem, vtile, vbase, sub, ch, t), p[ch], o[t]);
+  }
 
-  const int q_block_max = q_start + qblk0 + WAVES * QBLK - 1;
-  const int n_tiles = causal ? (min(q_block_max, Skv - 1) / KVBLK + 1)
-                             : (Skv + KVBLK - 1) / KVBLK;
-  // block-uniform start tile (varlen: nothing before the block's first doc)
-  const int jt0 = VARLEN ? doc_start[q_start + qblk0] / KVBLK : 0;
-
-  for (int jt = jt0; jt < n_tiles; ++jt) {
-    const int k0 = jt * KVBLK;
-    // ---- stage K tile (swizzled) and V^T tile cooperatively
-    {
-      constexpr int KCH = DQK / 8;     // 16-B chunks per K row
-      for (int idx = tid; idx < KVBLK * KCH; idx += WAVES * WAVE_SIZE) {
-        const int row = idx / KCH, c0 = (idx % KCH) * 8;
-        const int ks = min(k0 + row, Skv - 1);  // overhang rows masked later
-        *reinterpret_cast<bf16x8*>(k_lds + row_lds_off(row, c0 * 2, KB)) =
-            *reinterpret_cast<const bf16x8*>(k + k_base + (long)ks * k_rs + c0);
-      }
-      constexpr int VCH = DV / 8;
-      for (int idx = tid; idx < KVBLK * VCH; idx += WAVES * WAVE_SIZE) {
-        const int row = idx / VCH, c0 = (idx % VCH) * 8;
-        const int ks = min(k0 + row, Skv - 1);
-        // vectorized subtile store (the round-1 path scatter-stored 8
-        // scalars per vector to build a transposed image)
-        *reinterpret_cast<bf16x8*>(v_img + sub_off(row, c0)) =
-            *reinterpret_cast<const bf16x8*>(v + v_base + (long)ks * v_rs + c0);
-      }
-    }
-    __syncthreads();
-
-    const bool tile_live = (!causal || (k0 <= q_start + q0 + QBLK - 1)) &&
-                           (!VARLEN || (k0 + KVBLK > ds_wave));
-    float alpha = 1.f;
-    bf16x8_v pa0, pa1;
-    if (tile_live) {
-      // ---- QK^T swapped: P[k][q] = sum_d K[k][d] * Q[q][d]
-      f32x16 p;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = 0.f;
-#pragma unroll
-      for (int c = 0; c < DQK / 16; ++c) {
-        bf16x8_v ka = *reinterpret_cast<const bf16x8_v*>(
-            k_lds + row_lds_off(col, (c * 16 + half * 8) * 2, KB));
-        p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, qfrag[c], p, 0, 0, 0);
-      }
-
-      // ---- masked online softmax, IN PLACE in the p accumulator
-      const int qg = qg_lane;
-      float tile_max = -1e30f;
+  // Scores `s` of keys k0.. become probabilities `p`; `meanwhile` holds products that do
+  // not depend on them. The maximum is kept while no row grows by more than 2^12 over it:
+  // the f32 sums have room for that, and the pass over the output is skipped.
+  template <bool MASK, typename Meanwhile>
+  __device__ __forceinline__ void softmax(f32x16_t& s, int k0, bf16x8_t (&p)[2], Meanwhile meanwhile) {
+    const int half = (threadIdx.x >> 5) & 1;
+    if constexpr (MASK) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int kg = k0 + (r & 3) + 8 * (r >> 2) + 4 * half;
-        float sv = p[r] * scale;
-        if ((causal && kg > qg) || kg >= Skv || (VARLEN && kg < ds_lane)) sv = -1e30f;
-        p[r] = sv;
-        tile_max = fmaxf(tile_max, sv);
-      }
-      tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
-      // defer-max (guide T13, THR=8): if no row's max grew past m+THR, keep
-      // the old max and skip the O-wide rescale pass — P is then bounded by
-      // e^8 instead of 1, which the f32 accumulator tolerates. Wave-uniform
-      // decision taken BEFORE this tile's P is exponentiated (the textbook-
-      // safe order; guide T13 correctness hazard).
-      const bool need_rescale = !__all(tile_max <= m_run + 8.0f);
-      const float m_new = need_rescale ? fmaxf(m_run, tile_max) : m_run;
-      alpha = need_rescale ? __expf(m_run - m_new) : 1.f;
-      float psum = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float e = __expf(p[r] - m_new);
-        p[r] = e;
-        psum += e;
-      }
-      psum += __shfl_xor(psum, 32);
-      l_run = l_run * alpha + psum;
-      m_run = m_new;
-
-      // ---- P f32 -> bf16 packed pairs, permlane32_swap into A-fragment layout
-      unsigned int pk[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        unsigned lo = __builtin_bit_cast(unsigned short, f2bf(p[2 * i]));
-        unsigned hi = __builtin_bit_cast(unsigned short, f2bf(p[2 * i + 1]));
-        pk[i] = lo | (hi << 16);
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        auto r02 = __builtin_amdgcn_permlane32_swap(pk[4 * i + 0], pk[4 * i + 2], false, false);
-        auto r13 = __builtin_amdgcn_permlane32_swap(pk[4 * i + 1], pk[4 * i + 3], false, false);
-        unsigned frag[4] = {(unsigned)r02[0], (unsigned)r13[0], (unsigned)r02[1], (unsigned)r13[1]};
-        if (i == 0) pa0 = __builtin_bit_cast(bf16x8_v, *reinterpret_cast<ulonglong2*>(frag));
-        else pa1 = __builtin_bit_cast(bf16x8_v, *reinterpret_cast<ulonglong2*>(frag));
-      }
-
-      // ---- broadcast alpha to O layout via LDS (sign bit of slot 0 set
-      // when the whole wave deferred, so the rescale pass can be skipped)
-      if (lane < 32) bcast[wid * 32 + lane] = alpha;
-      if (lane == 0) bcast_skip[wid] = need_rescale ? 1 : 0;
-    }
-    // (waves with dead tiles skip compute but still hit the barriers)
-    __syncthreads();
-
-    if (tile_live) {
-      // ---- rescale O by alpha (skipped on deferred tiles, guide T13)
-      if (bcast_skip[wid]) {
-#pragma unroll
-        for (int t = 0; t < DV / 32; ++t) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int row = (r & 3) + 8 * (r >> 2) + 4 * half;
-            o_acc[t][r] *= bcast[wid * 32 + row];
-          }
-        }
-      }
-      // software-pipelined tr16 PV: tile t+1's four transpose reads are in
-      // flight during tile t's MFMAs; the counted s_waitcnt takes the
-      // fragment registers as "+v" operands so the consuming MFMAs cannot
-      // be scheduled past it. lgkmcnt(4) is conservative-safe: compiler-
-      // issued LDS ops between ours only strengthen the wait.
-      const unsigned v_base_a = lds_addr(v_img);
-      if constexpr (DV > 128) {
-#pragma unroll
-        for (int t = 0; t < DV / 32; ++t) {
-          bf16x8_v vb0 = tr16_frag(v_base_a, t, half, lane);
-          bf16x8_v vb1 = tr16_frag(v_base_a, t, half + 2, lane);
-          o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa0, vb0, o_acc[t], 0, 0, 0);
-          o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa1, vb1, o_acc[t], 0, 0, 0);
-        }
-      } else {
-      unsigned long long f0a, f0b, f1a, f1b, g0a, g0b, g1a, g1b;
-      auto tr_issue = [&](int t, unsigned long long& r0a, unsigned long long& r0b,
-                          unsigned long long& r1a, unsigned long long& r1b) {
-        const unsigned base = v_base_a +
-            (unsigned)((t * 2 + ((lane >> 4) & 1)) * 1152 + (lane & 15) * 8);
-        const unsigned klo = (unsigned)(8 * half) * 32;
-        const unsigned khi = (unsigned)(8 * (half + 2)) * 32;
-        asm volatile("ds_read_b64_tr_b16 %0, %4\n\t"
-                     "ds_read_b64_tr_b16 %1, %4 offset:128\n\t"
-                     "ds_read_b64_tr_b16 %2, %5\n\t"
-                     "ds_read_b64_tr_b16 %3, %5 offset:128"
-                     : "=v"(r0a), "=v"(r0b), "=v"(r1a), "=v"(r1b)
-                     : "v"(base + klo), "v"(base + khi));
-      };
-      tr_issue(0, f0a, f0b, f1a, f1b);
-#pragma unroll
-      for (int t = 0; t < DV / 32; ++t) {
-        unsigned long long& c0a = (t & 1) ? g0a : f0a;
-        unsigned long long& c0b = (t & 1) ? g0b : f0b;
-        unsigned long long& c1a = (t & 1) ? g1a : f1a;
-        unsigned long long& c1b = (t & 1) ? g1b : f1b;
-        if (t + 1 < DV / 32) {
-          tr_issue(t + 1, (t & 1) ? f0a : g0a, (t & 1) ? f0b : g0b,
-                   (t & 1) ? f1a : g1a, (t & 1) ? f1b : g1b);
-          asm volatile("s_waitcnt lgkmcnt(4)"
-                       : "+v"(c0a), "+v"(c0b), "+v"(c1a), "+v"(c1b));
-        } else {
-          asm volatile("s_waitcnt lgkmcnt(0)"
-                       : "+v"(c0a), "+v"(c0b), "+v"(c1a), "+v"(c1b));
-        }
-        ulonglong2 u0{c0a, c0b}, u1{c1a, c1b};
-        bf16x8_v vb0 = __builtin_bit_cast(bf16x8_v, u0);
-        bf16x8_v vb1 = __builtin_bit_cast(bf16x8_v, u1);
-        o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa0, vb0, o_acc[t], 0, 0, 0);
-        o_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa1, vb1, o_acc[t], 0, 0, 0);
-      }
+        const int key = k0 + acc_row(r, half);
+        const bool dead = (causal && key > qpos) || key >= skv || (VARLEN && key < qdoc);
+        s[r] = dead ? -INFINITY : s[r];
       }
     }
-    __syncthreads();
-  }
-
-  // ---- epilogue: normalize by l, write O and LSE. A sink is one more logit in
-  // the denominator, without a key (m_run bounds the scores, so that only a
-  // sink far above all of them can overflow: the output is 0 then, as it is)
-  if (sink) l_run += __expf(bf2f(sink[h]) - m_run);
-  if (lane < 32) bcast[wid * 32 + lane] = (l_run > 0.f) ? 1.f / l_run : 0.f;
-  __syncthreads();
-
-  const int qg = q0 + col;
-  if (lane < 32 && qg < Sq) {
-    lse[((long)b * Hq + h) * Sq + qg] = (l_run > 0.f) ? m_run + __logf(l_run) : -1e30f;
-  }
+    float mx = s[0];
 #pragma unroll
-  for (int t = 0; t < DV / 32; ++t) {
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    mx = max_halves(mx);
+    const bool rescale = __any((mx - m) * c > 12.f);
+    meanwhile();
+    const float mn = rescale ? fmaxf(m, mx) : m;
+    const float alpha = __builtin_amdgcn_exp2f((m - mn) * c);
+    const float mc = mn * c;
+    float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int row = (r & 3) + 8 * (r >> 2) + 4 * half;  // q row in wave tile
-      const int qrow = q0 + row;
-      if (qrow < Sq) {
-        const float inv_l = bcast[wid * 32 + row];
-        out[o_base + (long)qrow * o_rs + t * 32 + col] = f2bf(o_acc[t][r] * inv_l);
+      s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], c, -mc));
+      sum += s[r];
+    }
+    l = l * alpha + sum;
+    m = mn;
+    p[0] = pack8(s, 0);
+    p[1] = pack8(s, 1);
+    if (rescale) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+    }
+  }
+};
+
+// PIPE: as above. Without (head dim 256, whose accumulators leave no room for a second
+// half tile in flight) scores, softmax and values follow one another.
+template <int DQK, int DV, int WAVES, int OCC, bool PIPE, bool VARLEN>
+__global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArgs a) {
+  using F = Fwd<DQK, DV, WAVES, VARLEN>;
+  constexpr int KT = F::KT, VT = F::VT;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  F f;
+  f.smem = smem;
+  f.kbase = rows_base<DQK>();
+  f.vbase = cols_base<DV>();
+  f.c = a.scale_log2;
+  f.skv = a.Skv;
+  f.causal = a.causal;
+
+  const Place at = place_block((a.Sq + F::BM - 1) / F::BM, a.Hq, a.B, a.causal);
+  const int lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = at.head, b = at.batch, kvh = h / (a.Hq / a.Hk);
+  const int qblk = at.tile * F::BM;                   // block's, wave's first query row
+  const int q0 = qblk + wid * 32;
+
+  const unsigned k_rs = (unsigned)a.Hk * DQK * 2, v_rs = (unsigned)a.Hk * DV * 2;
+  const char* kp = reinterpret_cast<const char*>(a.k + ((long)b * a.Skv * a.Hk + kvh) * DQK);
+  const char* vp = reinterpret_cast<const char*>(a.v + ((long)b * a.Skv * a.Hk + kvh) * DV);
+
+  {
+    const int row = min(q0 + col, a.Sq - 1);          // rows beyond Sq are not stored
+    const bf16* src = a.q + (((long)b * a.Sq + row) * a.Hq + h) * DQK + half * 8;
+#pragma unroll
+    for (int ch = 0; ch < F::NC; ++ch) {
+      uint4 w = *reinterpret_cast<const uint4*>(src + ch * 16);
+      if (a.negative) {
+        w.x ^= 0x80008000u; w.y ^= 0x80008000u; w.z ^= 0x80008000u; w.w ^= 0x80008000u;
       }
+      f.qf[ch] = __builtin_bit_cast(bf16x8_t, w);
+    }
+    f.qpos = a.q_start + q0 + col;
+    f.qdoc = VARLEN ? a.doc_start[a.q_start + row] : 0;
+    f.m = -1e30f;
+    f.l = 0.f;
+#pragma unroll
+    for (int t = 0; t < F::NT; ++t) f.o[t] = zero16();
+  }
+
+  // tiles of the block and of the wave (doc_start does not decrease)
+  const int last = a.q_start + min(qblk + F::BM, a.Sq) - 1;
+  const int last_w = a.q_start + min(q0 + 32, a.Sq) - 1;
+  const int all = (a.Skv + 63) / 64;
+  const int t1 = a.causal ? min(last / 64 + 1, all) : all;
+  const int t1w = q0 >= a.Sq ? 0 : a.causal ? min(last_w / 64 + 1, all) : all;
+  int t0 = 0, t0w = 0, doc_w = 0;
+  if (VARLEN) {
+    t0 = __builtin_amdgcn_readfirstlane(a.doc_start[a.q_start + qblk]) / 64;
+    t0w = __builtin_amdgcn_readfirstlane(a.doc_start[a.q_start + min(q0, a.Sq - 1)]) / 64;
+    doc_w = __builtin_amdgcn_readfirstlane(a.doc_start[last_w]);
+  }
+  // first tile with a key that some row of the wave must not see (from the diagonal on)
+  const int t_diag = a.causal ? (a.q_start + q0 + 1) / 64 : all;
+
+  auto load_k = [&](int t) {
+    load_tile<DQK, 64, WAVES>(kp + (long)t * 64 * k_rs, k_rs, a.Skv - t * 64, (t & 1) * KT);
+  };
+  auto load_v = [&](int t) {
+    load_tile<DV, 64, WAVES>(vp + (long)t * 64 * v_rs, v_rs, a.Skv - t * 64, 2 * KT + (t & 1) * VT);
+  };
+  f32x16_t s0, s1;
+  bf16x8_t p0[2], p1[2];
+
+  if (t0 < t1) {
+    load_k(t0);
+    if constexpr (PIPE) {
+      wait_loads();
+      barrier();
+      if (t0 + 1 < t1) load_k(t0 + 1);
+    }
+    load_v(t0);
+  }
+  for (int t = t0; t < t1; ++t) {
+    const bool live = t >= t0w && t < t1w;
+    const unsigned kt = (t & 1) * KT, kn = KT - kt;
+    const unsigned vt = 2 * KT + (t & 1) * VT, vo = 4 * KT + VT - vt;
+    const bool mask = t >= t_diag || t * 64 + 64 > a.Skv || (VARLEN && t * 64 < doc_w);
+    if constexpr (PIPE) {
+      if (live) {
+        auto next = [&] { f.scores(s1, kt, 1); };
+        auto both = [&] { f.scores(s1, kt, 1); f.values(p1, vo, 1); };
+        if (t == t0w) {
+          f.scores(s0, kt, 0);
+          f.template softmax<true>(s0, t * 64, p0, next);
+        } else if (mask) {
+          f.template softmax<true>(s0, t * 64, p0, both);
+        } else {
+          f.template softmax<false>(s0, t * 64, p0, both);
+        }
+      }
+      wait_loads();     // K of t + 1, V of t; the buffers of K of t, V of t - 1 are free
+      barrier();
+      if (t + 1 < t1) load_v(t + 1);
+      if (t + 2 < t1) load_k(t + 2);
+      if (live) {
+        // (the scores of the tile after a wave's last one are formed and not used)
+        auto both = [&] { f.scores(s0, kn, 0); f.values(p0, vt, 0); };
+        if (mask) f.template softmax<true>(s1, t * 64 + 32, p1, both);
+        else f.template softmax<false>(s1, t * 64 + 32, p1, both);
+        if (t == t1w - 1) f.values(p1, vt, 1);
+      }
+    } else {
+      wait_loads();     // K and V of t; the other buffers are free
+      barrier();
+      if (t + 1 < t1) {
+        load_k(t + 1);
+        load_v(t + 1);
+      }
+      if (live) {
+#pragma unroll 1
+        for (int sub = 0; sub < 2; ++sub) {
+          f.scores(s0, kt, sub);
+          __builtin_amdgcn_sched_barrier(0);
+          if (mask) f.template softmax<true>(s0, t * 64 + 32 * sub, p0, [] {});
+          else f.template softmax<false>(s0, t * 64 + 32 * sub, p0, [] {});
+          __builtin_amdgcn_sched_barrier(0);
+          f.values(p0, vt, sub);
+        }
+      }
+    }
+  }
+
+  // ---- normalise, then through LDS (the tiles are done with) to whole-row stores. A
+  // sink is one more logit in the denominator, without a key.
+  constexpr int RB = row_bytes(DV);
+  static_assert(F::SMEM >= F::BM * RB, "output tile fits the K/V buffers");
+  barrier();
+  char* mine = smem + wid * 32 * RB;
+  const float l = sum_halves(f.l), m2 = f.m * f.c;    // maximum in units of log2
+  const float ls = a.sink ? l + __builtin_amdgcn_exp2f(bf2f(a.sink[h]) * LOG2E - m2) : l;
+  const float inv = ls > 0.f ? 1.f / ls : 0.f;
+  if (half == 0 && q0 + col < a.Sq)
+    a.lse[((long)b * a.Hq + h) * a.Sq + q0 + col] = ls > 0.f ? m2 * LN2 + __logf(ls) : -1e30f;
+#pragma unroll
+  for (int t = 0; t < F::NT; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {                     // columns 32 t + 8 g + 4 half + 0..3
+      bf16x4_t w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = (__bf16)(f.o[t][4 * g + j] * inv);
+      *reinterpret_cast<bf16x4_t*>(mine + col * RB + (((t * 4 + g) ^ swz<DV>(col)) << 4) + half * 8) = w;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // a wave reads what it wrote itself
+  constexpr int CH = DV / 8, PER = 64 / CH;           // 16-byte pieces of a row, rows per store
+  bf16* op = a.out + (((long)b * a.Sq + q0) * a.Hq + h) * DV;
+  if (lane < PER * CH) {
+    for (int r = lane / CH; r < 32 && q0 + r < a.Sq; r += PER) {
+      const int ch = lane % CH;
+      *reinterpret_cast<uint4*>(op + (long)r * a.Hq * DV + ch * 8) =
+          *reinterpret_cast<const uint4*>(mine + r * RB + ((ch ^ swz<DV>(r)) << 4));
     }
   }
 }
 
-template <int DQK, int DV, int WAVES, bool VARLEN>
-static void launch_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
-                       at::Tensor& out, at::Tensor& lse, const int* doc_start,
-                       const bf16* sink, int B, int Sq, int Skv, int Hq, int Hk, int q_start,
-                       float scale, bool causal, hipStream_t stream) {
-  const dim3 grid(Sq / (WAVES * QBLK), Hq, B);
-  const size_t smem = KVBLK * pad256(DQK * 2) + sub_img_bytes<DV>() +
-                      WAVES * 33 * sizeof(float);
-  hipLaunchKernelGGL((flash_fwd_kernel<DQK, DV, WAVES, VARLEN>), grid,
-                     dim3(WAVES * WAVE_SIZE), smem, stream,
-                     reinterpret_cast<const bf16*>(q.data_ptr()),
-                     reinterpret_cast<const bf16*>(k.data_ptr()),
-                     reinterpret_cast<const bf16*>(v.data_ptr()),
-                     reinterpret_cast<bf16*>(out.data_ptr()), lse.data_ptr<float>(),
-                     doc_start, sink, B, Sq, Skv, Hq, Hk, q_start, scale, causal);
+template <int DQK, int DV, int WAVES, int OCC, bool PIPE, bool VARLEN>
+static void launch_fwd(const FwdArgs& a, hipStream_t stream) {
+  using F = Fwd<DQK, DV, WAVES, VARLEN>;
+  const long blocks = (long)((a.Sq + F::BM - 1) / F::BM) * a.Hq * a.B;
+  hipLaunchKernelGGL((flash_fwd_kernel<DQK, DV, WAVES, OCC, PIPE, VARLEN>), dim3((unsigned)blocks),
+                     dim3(64 * WAVES), F::SMEM, stream, a);
   HIP_CHECK_KERNEL();
 }
 
@@ -318,43 +295,47 @@ std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
   const int B = q.size(0), Sq = q.size(1), Hq = q.size(2), Dqk = q.size(3);
   const int Skv = k.size(1), Hk = k.size(2), Dv = v.size(3);
   TORCH_CHECK(Hq % Hk == 0, "flash_attn_fwd: Hq must be divisible by Hk");
-  TORCH_CHECK(Sq % (4 * QBLK) == 0, "flash_attn_fwd: Sq must be a multiple of 128");
-  TORCH_CHECK(Skv % KVBLK == 0, "flash_attn_fwd: Skv must be a multiple of 32");
+  TORCH_CHECK(Sq % 128 == 0, "flash_attn_fwd: Sq must be a multiple of 128");
+  TORCH_CHECK(Skv % 32 == 0, "flash_attn_fwd: Skv must be a multiple of 32");
   const bool varlen = doc_start.has_value();
-  const int* ds_ptr = varlen ? doc_start->data_ptr<int>() : nullptr;
   if (varlen) TORCH_CHECK(causal && B == 1, "varlen flash is causal with B==1");
   if (sink)
     TORCH_CHECK(sink->is_cuda() && sink->is_contiguous() && sink->numel() == Hq &&
                     sink->scalar_type() == at::kBFloat16, "flash_attn_fwd: sink [Hq] bf16");
-  const bf16* sk_ptr = sink ? reinterpret_cast<const bf16*>(sink->data_ptr()) : nullptr;
   auto out = at::empty({B, Sq, Hq, Dv}, q.options());
   auto lse = at::empty({B, Hq, Sq}, q.options().dtype(at::kFloat));
   auto stream = c10::hip::getCurrentHIPStream().stream();
+  FwdArgs a;
+  a.q = reinterpret_cast<const bf16*>(q.data_ptr());
+  a.k = reinterpret_cast<const bf16*>(k.data_ptr());
+  a.v = reinterpret_cast<const bf16*>(v.data_ptr());
+  a.out = reinterpret_cast<bf16*>(out.data_ptr());
+  a.lse = lse.data_ptr<float>();
+  a.doc_start = varlen ? doc_start->data_ptr<int>() : nullptr;
+  a.sink = sink ? reinterpret_cast<const bf16*>(sink->data_ptr()) : nullptr;
+  a.B = B; a.Sq = Sq; a.Skv = Skv; a.Hq = Hq; a.Hk = Hk; a.q_start = (int)q_start;
+  // a scale of zero: equal weights, whatever the scores (masked ones stay masked)
+  a.scale_log2 = std::max((float)std::fabs(scale) * LOG2E, 1e-37f);
+  a.negative = scale < 0;
+  a.causal = causal;
 
+  // Waves per workgroup and per SIMD: as many as the registers of the accumulators and
+  // the two K/V tiles in LDS allow. (192, 128) fits one workgroup a CU, so it has 8 waves
+  // (186 us; 240 with 4 waves at one a SIMD); (192, 192) would spill at two a SIMD (457
+  // against 178 us).
   bool done = false;
-#define FA_FWD_CASE(A, C)                                                             \
-  if (!done && Dqk == A && Dv == C) {                                                 \
-    done = true;                                                                      \
-    if (varlen && Sq % (8 * QBLK) == 0) {                                             \
-      launch_fwd<A, C, 8, true>(q, k, v, out, lse, ds_ptr, sk_ptr, B, Sq, Skv, Hq, Hk, \
-                                (int)q_start, (float)scale, causal, stream);          \
-    } else if (varlen) {                                                              \
-      launch_fwd<A, C, 4, true>(q, k, v, out, lse, ds_ptr, sk_ptr, B, Sq, Skv, Hq, Hk, \
-                                (int)q_start, (float)scale, causal, stream);          \
-    } else if (Sq % (8 * QBLK) == 0) {                                                \
-      launch_fwd<A, C, 8, false>(q, k, v, out, lse, nullptr, sk_ptr, B, Sq, Skv, Hq, Hk, \
-                                 (int)q_start, (float)scale, causal, stream);         \
-    } else {                                                                          \
-      launch_fwd<A, C, 4, false>(q, k, v, out, lse, nullptr, sk_ptr, B, Sq, Skv, Hq, Hk, \
-                                 (int)q_start, (float)scale, causal, stream);         \
-    }                                                                                 \
+#define FA_FWD_CASE(A, C, W, OCC, PIPE)                             \
+  if (!done && Dqk == A && Dv == C) {                               \
+    done = true;                                                    \
+    if (varlen) launch_fwd<A, C, W, OCC, PIPE, true>(a, stream);    \
+    else launch_fwd<A, C, W, OCC, PIPE, false>(a, stream);          \
   }
-  FA_FWD_CASE(64, 64)
-  FA_FWD_CASE(96, 96)
-  FA_FWD_CASE(128, 128)
-  FA_FWD_CASE(192, 128)
-  FA_FWD_CASE(192, 192)
-  FA_FWD_CASE(256, 256)
+  FA_FWD_CASE(64, 64, 4, 3, true)
+  FA_FWD_CASE(96, 96, 4, 2, true)
+  FA_FWD_CASE(128, 128, 4, 2, true)
+  FA_FWD_CASE(192, 128, 8, 2, true)
+  FA_FWD_CASE(192, 192, 4, 1, true)
+  FA_FWD_CASE(256, 256, 4, 1, false)
 #undef FA_FWD_CASE
   TORCH_CHECK(done, "flash_attn_fwd: unsupported head dims (Dqk=", Dqk, ", Dv=", Dv,
               "); supported pairs: (64,64),(96,96),(128,128),(192,128),(192,192),(256,256)");

@@ -1,0 +1,60 @@
+"""Flash attention at the edges of its tiles, against plain f32 attention."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")]
+
+
+def _reference(q, k, v, causal, q_start, doc_start, scale):
+    G = q.shape[2] // k.shape[2]
+    q, k, v = (t.float().transpose(1, 2) for t in (q, k, v))
+    k, v = (t.repeat_interleave(G, 1) for t in (k, v))
+    s = (q @ k.transpose(-1, -2).contiguous()) * scale
+    qpos = torch.arange(q_start, q_start + q.shape[2], device="cuda")[:, None]
+    kpos = torch.arange(k.shape[2], device="cuda")[None]
+    keep = (kpos <= qpos) if causal else torch.ones_like(kpos <= qpos)
+    if doc_start is not None:
+        keep = keep & (kpos >= doc_start[qpos])
+    s = s.masked_fill(~keep, -math.inf)
+    return (s.softmax(-1) @ v).transpose(1, 2), s.logsumexp(-1)
+
+
+def _docs(cuts, total):
+    start = torch.empty(total, dtype=torch.int32)
+    end = torch.empty(total, dtype=torch.int32)
+    for a, b in zip([0, *cuts], [*cuts, total]):
+        start[a:b], end[a:b] = a, b
+    return start.cuda(), end.cuda()
+
+
+# probabilities and the output are each rounded to bf16 once (2^-9 of a value at most)
+FWD = 2 * 2.0 ** -9
+
+
+@pytest.mark.parametrize("dims", [(64, 64), (96, 96), (128, 128), (192, 128), (192, 192), (256, 256)])
+@pytest.mark.parametrize("sq,skv,causal,q_start,cuts,scale", [
+    (128, 128, True, 0, None, 1.0),
+    (384, 352, False, 0, None, 1.0),            # last tile half empty, three blocks
+    (256, 640, True, 384, None, 1.0),           # a chunk behind a prefix
+    (640, 640, True, 0, (1, 63, 64, 65, 130, 500), 1.0),
+    (256, 768, True, 256, (100, 300, 301), 1.0),
+    (256, 256, True, 0, None, -1.0),
+    (256, 256, True, 0, None, 0.0),
+])
+def test_forward(dims, sq, skv, causal, q_start, cuts, scale):
+    torch.manual_seed(0)
+    q = torch.randn(1, sq, 4, dims[0], device="cuda").bfloat16() * 2
+    k = torch.randn(1, skv, 2, dims[0], device="cuda").bfloat16()
+    v = torch.randn(1, skv, 2, dims[1], device="cuda").bfloat16()
+    k[:, skv // 3] *= 8                         # scores that stand out: the maximum moves
+    scale *= dims[0] ** -0.5
+    start = None if cuts is None else _docs(cuts, skv)[0]
+    from automodel_amd.ops._backend import hip_ops
+
+    o, lse = hip_ops().flash_attn_fwd(q, k, v, scale, causal, q_start, start)
+    ro, rlse = _reference(q, k, v, causal, q_start, start, scale)
+    assert (o.float() - ro).norm() / ro.norm() < FWD
+    assert (lse - rlse).abs().max() < 1e-5 * max(1.0, float(rlse.abs().max()))
