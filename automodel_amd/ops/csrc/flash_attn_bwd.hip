@@ -1,512 +1,471 @@
-// Flash attention backward (CDNA4, gfx950): deterministic dKV (kv-parallel) and
-// dQ (q-parallel) kernels of the forward in flash_attn.hip, plus the MFMA and
-// transpose-read layout probes.
+// Flash attention backward (CDNA4, gfx950): deterministic dK/dV (kv-parallel) and dQ
+// (q-parallel) kernels of the forward in flash_attn.hip, plus the MFMA and transpose-read
+// layout probes.
+//
+// Both kernels recompute the scores (7 products instead of the 5 of a fused kernel, which
+// would have to add dQ with atomics: gradients here are the same bits in every run).
+//   bwd_stats: -rowsum(dO * O) and the row's log-sum-exp in units of log2
+//   bwd_dkv:   a wave holds 32 K/V rows and their gradients; Q and dO pass by in tiles of
+//              64 rows, for all query heads of the group. S[q][k] and dP[q][k] have the
+//              key as the accumulator's column, so P and dS are operands of
+//              dV^T += dO^T P and dK^T += Q^T dS as they lie (flash_tile.h).
+//   bwd_dq:    a wave holds 32 Q/dO rows; K and V pass by; dQ^T += K^T dS^T.
+// Tiles come by direct LDS loads into three buffers with one barrier a tile. The loop is
+// pipelined over half tiles: while the vector unit turns scores into P and dS, the matrix
+// core forms the scores of the next half tile and adds the products of the previous one
+// (PIPE; three tiles of head dim 192/192 or 256 do not fit LDS: there two buffers, and the
+// phases follow one another).
+// Bound by LDS reads (32 rows per wave: 128 B/clk at full MFMA rate) and the matrix cores.
+// Measured, dK/dV + dQ + stats (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128:
+// 21.25 -> 7.90 ms (4932 + 2811 us); 2 x 4096: 2960 -> 1150 us; 2 x 3072, 16 heads (192, 128):
+// 1725 -> 489 us; 4 x 2048, 16/8 heads of 64: 616 -> 176 us; 2 x 4096, 16/8 heads of 256:
+// 5.99 -> 1.35 ms.
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 
 #include "common.h"
-#include "flash_attn.h"
+#include "flash_tile.h"
 #include "ops_api.h"
 
 namespace amd_ops {
 
-// ===========================================================================
-// Backward: flash-attention-2 style split.
-//   delta kernel: delta[b,h,s] = rowsum(dO * O)
-//   kernel A (kv-parallel, DETERMINISTIC): grid over (kv tiles, Hk, B); each
-//     block loops the GQA query-head group and all q tiles, accumulating
-//     dK/dV in registers; plain bf16 stores (no atomics -> bitwise
-//     reproducible grads).
-//   kernel B (q-parallel): recompute S in [q][k] layout, accumulate dQ.
-// ===========================================================================
+using namespace fa;
 
-__global__ void fa_delta_kernel(const bf16* __restrict__ dout, const bf16* __restrict__ o,
-                                float* __restrict__ delta, int S, int Hq, int DV,
-                                long rows) {
-  // row r = ((b*S + s)*Hq + h); one wave per row
-  const long row = ((long)blockIdx.x * blockDim.x + threadIdx.x) / WAVE_SIZE;
-  if (row >= rows) return;
-  const int lane = threadIdx.x & (WAVE_SIZE - 1);
-  const bf16* dp = dout + row * DV;
-  const bf16* op = o + row * DV;
-  float acc = 0.f;
-  for (int j = lane * 2; j < DV; j += 2 * WAVE_SIZE) {
-    acc += bf2f(dp[j]) * bf2f(op[j]) + bf2f(dp[j + 1]) * bf2f(op[j + 1]);
+// stats[0][b][h][s] = lse * log2(e), stats[1][b][h][s] = -rowsum(dO * O), rows padded to
+// sp = a multiple of 64; padding rows get a log-sum-exp whose probabilities are 0. A block
+// takes 64 rows of one head: 16-byte loads, DV / 8 lanes a row, coalesced stores.
+template <int DV>
+__global__ __launch_bounds__(256) void bwd_stats_kernel(const bf16* __restrict__ dout,
+                                                        const bf16* __restrict__ o,
+                                                        const float* __restrict__ lse,
+                                                        float* __restrict__ stats, int Sq, int sp,
+                                                        int Hq, long plane) {
+  constexpr int LANES = DV <= 64 ? 8 : DV <= 128 ? 16 : 32, ROWS = 256 / LANES;
+  __shared__ float sum[64];
+  const int h = blockIdx.y, b = blockIdx.z, s0 = blockIdx.x * 64;
+  const int l = threadIdx.x % LANES;
+#pragma unroll
+  for (int i = threadIdx.x / LANES; i < 64; i += ROWS) {
+    float acc = 0.f;
+    if (s0 + i < Sq && l < DV / 8) {
+      const long at = (((long)b * Sq + s0 + i) * Hq + h) * DV + l * 8;
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(dout + at);
+      const bf16x8 y = *reinterpret_cast<const bf16x8*>(o + at);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc = fmaf(bf2f(x.v[j]), bf2f(y.v[j]), acc);
+    }
+#pragma unroll
+    for (int off = LANES / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+    if (l == 0) sum[i] = acc;
   }
-  acc = wave_reduce_sum(acc);
-  if (lane == 0) {
-    const long h = row % Hq;
-    const long bs = row / Hq;
-    const long b = bs / S, s = bs % S;
-    delta[(b * Hq + h) * S + s] = acc;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const int s = s0 + threadIdx.x;
+    const long at = ((long)b * Hq + h) * sp + s;
+    stats[at] = s < Sq ? lse[((long)b * Hq + h) * Sq + s] * LOG2E : 1e30f;
+    stats[plane + at] = -sum[threadIdx.x];
   }
 }
 
-template <int DQK, int DV, int WAVES, bool VARLEN>
-__global__ __launch_bounds__(WAVES * WAVE_SIZE, occ_dkv(DQK, DV)) void flash_bwd_dkv_kernel(
-    const bf16* __restrict__ dout, const bf16* __restrict__ q, const bf16* __restrict__ k,
-    const bf16* __restrict__ v, const float* __restrict__ lse, const float* __restrict__ delta,
-    bf16* __restrict__ dk, bf16* __restrict__ dv, const int* __restrict__ doc_end,
-    int B, int Sq, int Skv, int Hq, int Hk, int q_start, float scale, bool causal) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* q_img = smem;                                    // subtiled [DQK/16][32][16]
-  char* do_img = smem + sub_img_bytes<DQK>();            // subtiled [DV/16][32][16]
-  char* tbuf = do_img + sub_img_bytes<DV>();             // WAVES*2048
+struct BwdArgs {
+  const bf16 *dout, *q, *k, *v;
+  const float* stats;              // two planes of B * Hq * sp
+  bf16 *dq, *dk, *dv;
+  const int *doc_start, *doc_end;
+  int B, Sq, Skv, Hq, Hk, q_start, sp;
+  long plane;
+  float scale;
+  bool causal;
+};
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid / 64;
-  const int col = lane & 31;
-  const int half = lane >> 5;
-
-  const int kvb = blockIdx.x * (WAVES * 32);
-  const int kvh = blockIdx.y;
-  const int b = blockIdx.z;
-  const int G = Hq / Hk;               // GQA group size
-  const int kv0 = kvb + wid * 32;      // this wave's kv rows
-
-  const long k_base = (((long)b * Skv) * Hk + kvh) * DQK;
-  const long v_base = (((long)b * Skv) * Hk + kvh) * DV;
-  const long k_rs = (long)Hk * DQK, v_rs = (long)Hk * DV;
-  const long q_rs = (long)Hq * DQK, do_rs = (long)Hq * DV;
-
-  // K/V rows of this wave -> A fragments in registers
-  bf16x8_v kfrag[DQK / 16], vfrag[DV / 16];
+// rows r of a wave's transposed accumulators [D / 32] (column = row of the result), scaled,
+// through LDS to whole-row stores of bf16
+template <int D>
+__device__ __forceinline__ void store_rows(const f32x16_t (&acc)[D / 32], float scale, char* mine,
+                                           bf16* dst, long row_stride, int rows) {
+  constexpr int RB = row_bytes(D), CH = D / 8, PER = 64 / CH;
+  const int lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
 #pragma unroll
-  for (int c = 0; c < DQK / 16; ++c)
-    kfrag[c] = *reinterpret_cast<const bf16x8_v*>(
-        k + k_base + (long)(kv0 + col) * k_rs + c * 16 + half * 8);
+  for (int t = 0; t < D / 32; ++t)
 #pragma unroll
-  for (int c = 0; c < DV / 16; ++c)
-    vfrag[c] = *reinterpret_cast<const bf16x8_v*>(
-        v + v_base + (long)(kv0 + col) * v_rs + c * 16 + half * 8);
+    for (int g = 0; g < 4; ++g) {
+      bf16x4_t w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = (__bf16)(acc[t][4 * g + j] * scale);
+      *reinterpret_cast<bf16x4_t*>(mine + col * RB + (((t * 4 + g) ^ swz<D>(col)) << 4) + half * 8) = w;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // a wave reads what it wrote itself
+  if (lane < PER * CH) {
+    const int ch = lane % CH;
+    for (int r = lane / CH; r < 32 && r < rows; r += PER)
+      *reinterpret_cast<uint4*>(dst + (long)r * row_stride + ch * 8) =
+          *reinterpret_cast<const uint4*>(mine + r * RB + ((ch ^ swz<D>(r)) << 4));
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
 
-  // varlen: per-element doc_end for this wave's 16 kv rows (fixed all kernel)
-  int dend[16];
-  int dend_wave = Sq;                  // max over the wave's rows
+template <int D>
+__device__ __forceinline__ void load_row_frags(bf16x8_t (&f)[D / 16], const bf16* row) {
+  const int half = (threadIdx.x >> 5) & 1;
+#pragma unroll
+  for (int c = 0; c < D / 16; ++c)
+    f[c] = *reinterpret_cast<const bf16x8_t*>(row + c * 16 + half * 8);
+}
+
+// ------------------------------------------------------------------------------- dK, dV
+template <int DQK, int DV, bool PIPE>
+struct Dkv {
+  static constexpr int QT = 64 * row_bytes(DQK), OT = 64 * row_bytes(DV), ST = 1024;
+  static constexpr int BUF = QT + OT + ST, NBUF = PIPE ? 3 : 2, SMEM = NBUF * BUF;
+  char* smem;
+  unsigned qrow, orow, qcol, ocol;
+  float c;
+  bf16x8_t kf[DQK / 16], vf[DV / 16];
+  f32x16_t dk[DQK / 32], dv[DV / 32];
+  int kpos, kend;
+  bool causal;
+
+  // S and dP - delta of the 32 rows `sub` of the tile at byte `buf`
+  __device__ __forceinline__ void scores(f32x16_t& s, f32x16_t& dp, unsigned buf, int sub) {
+    const int half = (threadIdx.x >> 5) & 1;
+    const float* nd = reinterpret_cast<const float*>(smem + buf + QT + OT + 256) + sub * 32 + 4 * half;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 w = *reinterpret_cast<const float4*>(nd + 8 * g);
+      dp[4 * g] = w.x; dp[4 * g + 1] = w.y; dp[4 * g + 2] = w.z; dp[4 * g + 3] = w.w;
+    }
+    s = zero16();
+#pragma unroll
+    for (int ch = 0; ch < DQK / 16; ++ch) s = mma(read_rows<DQK>(smem, buf, qrow, sub, ch), kf[ch], s);
+#pragma unroll
+    for (int ch = 0; ch < DV / 16; ++ch) dp = mma(read_rows<DV>(smem, buf + QT, orow, sub, ch), vf[ch], dp);
+  }
+
+  __device__ __forceinline__ void grads(const bf16x8_t (&p)[2], const bf16x8_t (&ds)[2], unsigned buf,
+                                        int sub) {
+#pragma unroll
+    for (int t = 0; t < DV / 32; ++t)
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch)
+        dv[t] = mma(read_cols<DV>(smem, buf + QT, ocol, sub, ch, t), p[ch], dv[t]);
+#pragma unroll
+    for (int t = 0; t < DQK / 32; ++t)
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch)
+        dk[t] = mma(read_cols<DQK>(smem, buf, qcol, sub, ch, t), ds[ch], dk[t]);
+  }
+
+  // scores of 32 rows at position q0.. become the operands P and dS
+  template <bool MASK, bool VARLEN>
+  __device__ __forceinline__ void probs(f32x16_t& s, f32x16_t& dp, unsigned buf, int sub, int q0,
+                                        bf16x8_t (&p)[2], bf16x8_t (&ds)[2]) {
+    const int half = (threadIdx.x >> 5) & 1;
+    const float* l2 = reinterpret_cast<const float*>(smem + buf + QT + OT) + sub * 32 + 4 * half;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 w = *reinterpret_cast<const float4*>(l2 + 8 * g);
+      const float l[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int r = 4 * g + j, q = q0 + acc_row(r, half);
+        float e = __builtin_amdgcn_exp2f(fmaf(s[r], c, -l[j]));
+        if (MASK && ((causal && kpos > q) || (VARLEN && q >= kend))) e = 0.f;
+        s[r] = e;
+        dp[r] *= e;
+      }
+    }
+    p[0] = pack8(s, 0); p[1] = pack8(s, 1);
+    ds[0] = pack8(dp, 0); ds[1] = pack8(dp, 1);
+  }
+};
+
+template <int DQK, int DV, int WAVES, int OCC, bool PIPE, bool VARLEN>
+__global__ __launch_bounds__(64 * WAVES, OCC) void bwd_dkv_kernel(const BwdArgs a) {
+  using F = Dkv<DQK, DV, PIPE>;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  constexpr int BM = WAVES * 32;
+  F f;
+  f.smem = smem;
+  f.qrow = rows_base<DQK>(); f.orow = rows_base<DV>();
+  f.qcol = cols_base<DQK>(); f.ocol = cols_base<DV>();
+  f.c = a.scale * LOG2E;
+  f.causal = a.causal;
+
+  const Place at = place_block((a.Skv + BM - 1) / BM, a.Hk, a.B, false);
+  const int lane = threadIdx.x & 63, col = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kvh = at.head, b = at.batch, G = a.Hq / a.Hk;
+  const int kvb = at.tile * BM, kv0 = kvb + wid * 32;
+  const int row = min(kv0 + col, a.Skv - 1);            // rows beyond Skv are not stored
+  load_row_frags<DQK>(f.kf, a.k + (((long)b * a.Skv + row) * a.Hk + kvh) * DQK);
+  load_row_frags<DV>(f.vf, a.v + (((long)b * a.Skv + row) * a.Hk + kvh) * DV);
+#pragma unroll
+  for (int t = 0; t < DQK / 32; ++t) f.dk[t] = zero16();
+#pragma unroll
+  for (int t = 0; t < DV / 32; ++t) f.dv[t] = zero16();
+  f.kpos = kv0 + col;
+  f.kend = VARLEN ? a.doc_end[row] : 0;
+
+  // query tiles that see some row of the block, and a wave's first masked positions
+  const int j0 = a.causal && kvb > a.q_start ? (kvb - a.q_start) / 64 : 0;
+  int j1 = (a.Sq + 63) / 64, end_w = 0x7fffffff;
   if (VARLEN) {
+    const int de = __builtin_amdgcn_readfirstlane(a.doc_end[min(kvb + BM, a.Skv) - 1]);
+    j1 = min(j1, (de - a.q_start + 63) / 64);
+    end_w = __builtin_amdgcn_readfirstlane(a.doc_end[min(kv0, a.Skv - 1)]);
+  }
+  const int nt = max(j1 - j0, 0), total = nt * G;
+  const unsigned q_rs = (unsigned)a.Hq * DQK * 2, o_rs = (unsigned)a.Hq * DV * 2;
+
+  auto load = [&](int u, unsigned buf) {
+    const int h = kvh * G + u / nt, q0 = (j0 + u % nt) * 64;
+    load_tile<DQK, 64, WAVES>(a.q + (((long)b * a.Sq + q0) * a.Hq + h) * DQK, q_rs, a.Sq - q0, buf);
+    load_tile<DV, 64, WAVES>(a.dout + (((long)b * a.Sq + q0) * a.Hq + h) * DV, o_rs, a.Sq - q0, buf + F::QT);
+    if (wid == 0) {      // 64 rows of both statistics, 16 bytes a lane (lanes 32.. repeat)
+      const float* src = a.stats + ((long)b * a.Hq + h) * a.sp + q0;
+      const float* mine = src + (lane & 15) * 4 + ((lane >> 4) & 1) * a.plane;
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                   :: "s"(buf + (unsigned)(F::QT + F::OT)), "v"(mine) : "memory");
+    }
+  };
+  auto masked = [&](int u) {
+    const int q0 = a.q_start + (j0 + u % nt) * 64;
+    return (a.causal && q0 < kv0 + 31) || (VARLEN && q0 + 63 >= end_w);
+  };
+  auto pos = [&](int u) { return a.q_start + (j0 + u % nt) * 64; };
+
+  if (total > 0) {
+    f32x16_t s0, d0;
+    bf16x8_t p0[2], e0[2];
+    load(0, 0);
+    if constexpr (PIPE) {
+      f32x16_t s1, d1;
+      bf16x8_t p1[2], e1[2];
+      if (total > 1) load(1, F::BUF);
+      wait_loads();
+      barrier();
+      f.scores(s0, d0, 0, 0);
+      unsigned prev = 0, cur = 0, next = F::BUF, free = 2 * F::BUF;
+      for (int u = 0; u < total; ++u) {
+        const bool mask = masked(u);
+        f.scores(s1, d1, cur, 1);
+        if (u > 0) f.grads(p1, e1, prev, 1);
+        if (mask) f.template probs<true, VARLEN>(s0, d0, cur, 0, pos(u), p0, e0);
+        else f.template probs<false, VARLEN>(s0, d0, cur, 0, pos(u), p0, e0);
+        wait_loads();     // the tile u + 1; the buffer of u - 1 is free
+        barrier();
+        if (u + 2 < total) load(u + 2, free);
+        f.scores(s0, d0, next, 0);    // (after the last tile: not used)
+        f.grads(p0, e0, cur, 0);
+        if (mask) f.template probs<true, VARLEN>(s1, d1, cur, 1, pos(u) + 32, p1, e1);
+        else f.template probs<false, VARLEN>(s1, d1, cur, 1, pos(u) + 32, p1, e1);
+        prev = cur; cur = next; next = free; free = prev;
+      }
+      f.grads(p1, e1, prev, 1);
+    } else {
+      for (int u = 0; u < total; ++u) {
+        const unsigned buf = (u & 1) * F::BUF;
+        const bool mask = masked(u);
+        wait_loads();     // the tile u; the other buffer is free
+        barrier();
+        if (u + 1 < total) load(u + 1, F::BUF - buf);
+#pragma unroll 1
+        for (int sub = 0; sub < 2; ++sub) {
+          f.scores(s0, d0, buf, sub);
+          if (mask) f.template probs<true, VARLEN>(s0, d0, buf, sub, pos(u) + 32 * sub, p0, e0);
+          else f.template probs<false, VARLEN>(s0, d0, buf, sub, pos(u) + 32 * sub, p0, e0);
+          f.grads(p0, e0, buf, sub);
+        }
+      }
+    }
+    barrier();
+  }
+  char* mine = smem + wid * 32 * row_bytes(DQK > DV ? DQK : DV);
+  const long first = ((long)b * a.Skv + kv0) * a.Hk + kvh;
+  store_rows<DQK>(f.dk, a.scale, mine, a.dk + first * DQK, (long)a.Hk * DQK, a.Skv - kv0);
+  store_rows<DV>(f.dv, 1.f, mine, a.dv + first * DV, (long)a.Hk * DV, a.Skv - kv0);
+}
+
+// ----------------------------------------------------------------------------------- dQ
+template <int DQK, int DV, bool PIPE>
+struct Dq {
+  static constexpr int KT = 64 * row_bytes(DQK), VT = 64 * row_bytes(DV);
+  static constexpr int NK = PIPE ? 3 : 2, SMEM = NK * KT + 2 * VT;   // K is read once more, later
+  char* smem;
+  unsigned krow, vrow, kcol;
+  float c, l2, nd;
+  bf16x8_t qf[DQK / 16], of[DV / 16];
+  f32x16_t dq[DQK / 32];
+  int qpos, qdoc, skv;
+  bool causal;
+
+  __device__ __forceinline__ void scores(f32x16_t& s, f32x16_t& dp, unsigned kt, unsigned vt, int sub) {
+    s = zero16();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dp[r] = nd;
+#pragma unroll
+    for (int ch = 0; ch < DQK / 16; ++ch) s = mma(read_rows<DQK>(smem, kt, krow, sub, ch), qf[ch], s);
+#pragma unroll
+    for (int ch = 0; ch < DV / 16; ++ch) dp = mma(read_rows<DV>(smem, vt, vrow, sub, ch), of[ch], dp);
+  }
+  __device__ __forceinline__ void grads(const bf16x8_t (&ds)[2], unsigned kt, int sub) {
+#pragma unroll
+    for (int t = 0; t < DQK / 32; ++t)
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch)
+        dq[t] = mma(read_cols<DQK>(smem, kt, kcol, sub, ch, t), ds[ch], dq[t]);
+  }
+  template <bool MASK, bool VARLEN>
+  __device__ __forceinline__ void probs(f32x16_t& s, f32x16_t& dp, int k0, bf16x8_t (&ds)[2]) {
+    const int half = (threadIdx.x >> 5) & 1;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int kg = kv0 + (r & 3) + 8 * (r >> 2) + 4 * half;
-      dend[r] = doc_end[min(kg, Skv - 1)];
+      const int k = k0 + acc_row(r, half);
+      float e = __builtin_amdgcn_exp2f(fmaf(s[r], c, -l2));
+      if (MASK && ((causal && k > qpos) || k >= skv || (VARLEN && k < qdoc))) e = 0.f;
+      dp[r] *= e;
     }
-    dend_wave = doc_end[min(kv0 + 31, Skv - 1)];
+    ds[0] = pack8(dp, 0); ds[1] = pack8(dp, 1);
   }
+};
 
-  f32x16 dk_acc[DQK / 32], dv_acc[DV / 32];
-#pragma unroll
-  for (int t = 0; t < DQK / 32; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) dk_acc[t][r] = 0.f;
-#pragma unroll
-  for (int t = 0; t < DV / 32; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) dv_acc[t][r] = 0.f;
+template <int DQK, int DV, int WAVES, int OCC, bool PIPE, bool VARLEN>
+__global__ __launch_bounds__(64 * WAVES, OCC) void bwd_dq_kernel(const BwdArgs a) {
+  using F = Dq<DQK, DV, PIPE>;
+  constexpr int KT = F::KT, VT = F::VT, V0 = F::NK * KT;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  constexpr int BM = WAVES * 32;
+  F f;
+  f.smem = smem;
+  f.krow = rows_base<DQK>(); f.vrow = rows_base<DV>(); f.kcol = cols_base<DQK>();
+  f.c = a.scale * LOG2E;
+  f.causal = a.causal;
+  f.skv = a.Skv;
 
-  char* tb = tbuf + wid * 2048;
-  const int jq_start = causal ? (kvb > q_start ? (kvb - q_start) / 32 : 0) : 0;
-  // block-uniform end (varlen: nothing after the block's last doc)
-  int jq_end = Sq / 32;
+  const Place at = place_block((a.Sq + BM - 1) / BM, a.Hq, a.B, a.causal);
+  const int lane = threadIdx.x & 63, col = lane & 31;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = at.head, b = at.batch, kvh = h / (a.Hq / a.Hk);
+  const int qblk = at.tile * BM, q0 = qblk + wid * 32;
+  const int row = min(q0 + col, a.Sq - 1);              // rows beyond Sq are not stored
+  const long qo = ((long)b * a.Sq + row) * a.Hq + h;
+  load_row_frags<DQK>(f.qf, a.q + qo * DQK);
+  load_row_frags<DV>(f.of, a.dout + qo * DV);
+  const float* st = a.stats + ((long)b * a.Hq + h) * a.sp + row;
+  f.l2 = st[0];
+  f.nd = st[a.plane];
+#pragma unroll
+  for (int t = 0; t < DQK / 32; ++t) f.dq[t] = zero16();
+  f.qpos = a.q_start + q0 + col;
+  f.qdoc = VARLEN ? a.doc_start[a.q_start + row] : 0;
+
+  const int last = a.q_start + min(qblk + BM, a.Sq) - 1, all = (a.Skv + 63) / 64;
+  const int t1 = a.causal ? min(last / 64 + 1, all) : all;
+  int t0 = 0, doc_w = 0;
   if (VARLEN) {
-    const int de_blk = doc_end[min(kvb + WAVES * 32 - 1, Skv - 1)];
-    jq_end = min(jq_end, (de_blk - q_start + 31) / 32);
+    t0 = __builtin_amdgcn_readfirstlane(a.doc_start[a.q_start + qblk]) / 64;
+    doc_w = __builtin_amdgcn_readfirstlane(a.doc_start[a.q_start + min(q0 + 32, a.Sq) - 1]);
   }
+  const int t_diag = a.causal ? (a.q_start + q0 + 1) / 64 : all;
+  const unsigned k_rs = (unsigned)a.Hk * DQK * 2, v_rs = (unsigned)a.Hk * DV * 2;
+  const bf16* kp = a.k + ((long)b * a.Skv * a.Hk + kvh) * DQK;
+  const bf16* vp = a.v + ((long)b * a.Skv * a.Hk + kvh) * DV;
+  auto load_k = [&](int t, unsigned to) {
+    load_tile<DQK, 64, WAVES>(kp + (long)t * 64 * a.Hk * DQK, k_rs, a.Skv - t * 64, to);
+  };
+  auto load_v = [&](int t) {
+    load_tile<DV, 64, WAVES>(vp + (long)t * 64 * a.Hk * DV, v_rs, a.Skv - t * 64, V0 + (t & 1) * VT);
+  };
+  auto masked = [&](int t) {
+    return t >= t_diag || t * 64 + 64 > a.Skv || (VARLEN && t * 64 < doc_w);
+  };
 
-  for (int g = 0; g < G; ++g) {
-    const int h = kvh * G + g;
-    const long q_base = (((long)b * Sq) * Hq + h) * DQK;
-    const long do_base = (((long)b * Sq) * Hq + h) * DV;
-    const float* lse_row = lse + ((long)b * Hq + h) * Sq;
-    const float* dlt_row = delta + ((long)b * Hq + h) * Sq;
-
-    for (int jq = jq_start; jq < jq_end; ++jq) {
-      const int q0 = jq * 32;
-      // ---- cooperative stage: ONE subtiled image per tensor (serves both
-      // the row-chunk B-frags and the tr16 transposed B-frags — the round-1
-      // kernel kept a row image AND a scalar-scattered transposed image)
-      {
-        constexpr int QCH = DQK / 8;
-        for (int idx = tid; idx < 32 * QCH; idx += WAVES * 64) {
-          const int rr = idx / QCH, c0 = (idx % QCH) * 8;
-          *reinterpret_cast<bf16x8*>(q_img + sub_off(rr, c0)) =
-              *reinterpret_cast<const bf16x8*>(q + q_base + (long)(q0 + rr) * q_rs + c0);
-        }
-        constexpr int OCH = DV / 8;
-        for (int idx = tid; idx < 32 * OCH; idx += WAVES * 64) {
-          const int rr = idx / OCH, c0 = (idx % OCH) * 8;
-          *reinterpret_cast<bf16x8*>(do_img + sub_off(rr, c0)) =
-              *reinterpret_cast<const bf16x8*>(
-                  dout + do_base + (long)(q0 + rr) * do_rs + c0);
+  if (t0 < t1) {
+    f32x16_t s0, d0;
+    bf16x8_t e0[2];
+    load_k(t0, 0);
+    load_v(t0);
+    if constexpr (PIPE) {
+      f32x16_t s1, d1;
+      bf16x8_t e1[2];
+      wait_loads();
+      barrier();
+      if (t0 + 1 < t1) { load_k(t0 + 1, KT); load_v(t0 + 1); }
+      f.scores(s0, d0, 0, V0 + (t0 & 1) * VT, 0);
+      unsigned prev = 0, cur = 0, next = KT, free = 2 * KT;
+      for (int t = t0; t < t1; ++t) {
+        const bool mask = masked(t);
+        const unsigned vt = V0 + (t & 1) * VT, vn = V0 + ((t + 1) & 1) * VT;
+        f.scores(s1, d1, cur, vt, 1);
+        if (t > t0) f.grads(e1, prev, 1);
+        if (mask) f.template probs<true, VARLEN>(s0, d0, t * 64, e0);
+        else f.template probs<false, VARLEN>(s0, d0, t * 64, e0);
+        wait_loads();     // K and V of t + 1; the buffers of K of t - 1 and V of t are free
+        barrier();
+        if (t + 2 < t1) { load_k(t + 2, free); load_v(t + 2); }
+        f.scores(s0, d0, next, vn, 0);    // (after the last tile: not used)
+        f.grads(e0, cur, 0);
+        if (mask) f.template probs<true, VARLEN>(s1, d1, t * 64 + 32, e1);
+        else f.template probs<false, VARLEN>(s1, d1, t * 64 + 32, e1);
+        prev = cur; cur = next; next = free; free = prev;
+      }
+      f.grads(e1, prev, 1);
+    } else {
+      for (int t = t0; t < t1; ++t) {
+        const bool mask = masked(t);
+        const unsigned kt = ((t - t0) & 1) * KT, vt = V0 + (t & 1) * VT;
+        wait_loads();     // K and V of t; the other buffers are free
+        barrier();
+        if (t + 1 < t1) { load_k(t + 1, KT - kt); load_v(t + 1); }
+#pragma unroll 1
+        for (int sub = 0; sub < 2; ++sub) {
+          f.scores(s0, d0, kt, vt, sub);
+          if (mask) f.template probs<true, VARLEN>(s0, d0, t * 64 + 32 * sub, e0);
+          else f.template probs<false, VARLEN>(s0, d0, t * 64 + 32 * sub, e0);
+          f.grads(e0, kt, sub);
         }
       }
-      __syncthreads();
-
-      const bool live = (!causal || (q_start + q0 + 31 >= kv0)) &&
-                        (!VARLEN || (q_start + q0 < dend_wave));
-      if (live) {
-        const int ql = q0 + col;          // local q row (lse/delta index)
-        const int qg = q_start + ql;      // global position (mask)
-        const float lse_q = lse_row[ql];
-        const float dlt_q = dlt_row[ql];
-
-        // ---- S^T = K Q^T (rows = kv, cols = q)
-        f32x16 st;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) st[r] = 0.f;
-#pragma unroll
-        for (int c = 0; c < DQK / 16; ++c) {
-          bf16x8_v qb = *reinterpret_cast<const bf16x8_v*>(
-              q_img + sub_off(col, c * 16 + half * 8));
-          st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfrag[c], qb, st, 0, 0, 0);
-        }
-        // ---- dP^T = V dO^T
-        f32x16 dpt;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) dpt[r] = 0.f;
-#pragma unroll
-        for (int c = 0; c < DV / 16; ++c) {
-          bf16x8_v db = *reinterpret_cast<const bf16x8_v*>(
-              do_img + sub_off(col, c * 16 + half * 8));
-          dpt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfrag[c], db, dpt, 0, 0, 0);
-        }
-
-        // in place: st becomes P^T, dpt becomes dS^T
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int kg = kv0 + (r & 3) + 8 * (r >> 2) + 4 * half;
-          const bool masked = (causal && kg > qg) || kg >= Skv ||
-                              (VARLEN && qg >= dend[r]);
-          const float pv = masked ? 0.f : __expf(st[r] * scale - lse_q);
-          st[r] = pv;
-          dpt[r] = pv * (dpt[r] - dlt_q) * scale;
-        }
-
-        // ---- transpose P^T -> A-frags via wave-local LDS buffer, accumulate dV
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int krow = (r & 3) + 8 * (r >> 2) + 4 * half;
-          *reinterpret_cast<bf16*>(tb + tb_off(krow, col * 2)) = f2bf(st[r]);
-        }
-        __builtin_amdgcn_wave_barrier();
-        const unsigned do_base_a = lds_addr(do_img);
-        if constexpr (!pipe_ok_dkv(DQK, DV)) {
-#pragma unroll
-          for (int c2 = 0; c2 < 2; ++c2) {
-            bf16x8_v pa = *reinterpret_cast<const bf16x8_v*>(
-                tb + tb_off(col, (c2 * 16 + half * 8) * 2));
-#pragma unroll
-            for (int t = 0; t < DV / 32; ++t) {
-              bf16x8_v dob = tr16_frag(do_base_a, t, c2 * 2 + half, lane);
-              dv_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa, dob, dv_acc[t], 0, 0, 0);
-            }
-          }
-        } else {
-          bf16x8_v paf[2];
-#pragma unroll
-          for (int c2 = 0; c2 < 2; ++c2)
-            paf[c2] = *reinterpret_cast<const bf16x8_v*>(
-                tb + tb_off(col, (c2 * 16 + half * 8) * 2));
-          constexpr int NT = DV / 32;
-          unsigned long long pA, pB, qA, qB;
-          auto addr_f = [&](int i) {
-            const int c2 = i / NT, t = i % NT;
-            return do_base_a + (unsigned)((t * 2 + ((lane >> 4) & 1)) * 1152 +
-                                          (8 * (c2 * 2 + half)) * 32 + (lane & 15) * 8);
-          };
-          tr16_issue2(addr_f(0), pA, pB);
-#pragma unroll
-          for (int i = 0; i < 2 * NT; ++i) {
-            const bool last = (i + 1 == 2 * NT);
-            if (!last) tr16_issue2(addr_f(i + 1), (i & 1) ? pA : qA, (i & 1) ? pB : qB);
-            bf16x8_v dob = tr16_take((i & 1) ? qA : pA, (i & 1) ? qB : pB, !last);
-            dv_acc[i % NT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                paf[i / NT], dob, dv_acc[i % NT], 0, 0, 0);
-          }
-        }
-        // ---- transpose dS^T, accumulate dK
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int krow = (r & 3) + 8 * (r >> 2) + 4 * half;
-          *reinterpret_cast<bf16*>(tb + tb_off(krow, col * 2)) = f2bf(dpt[r]);
-        }
-        __builtin_amdgcn_wave_barrier();
-        const unsigned q_base_a = lds_addr(q_img);
-        if constexpr (!pipe_ok_dkv(DQK, DV)) {
-#pragma unroll
-          for (int c2 = 0; c2 < 2; ++c2) {
-            bf16x8_v da = *reinterpret_cast<const bf16x8_v*>(
-                tb + tb_off(col, (c2 * 16 + half * 8) * 2));
-#pragma unroll
-            for (int t = 0; t < DQK / 32; ++t) {
-              bf16x8_v qb2 = tr16_frag(q_base_a, t, c2 * 2 + half, lane);
-              dk_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(da, qb2, dk_acc[t], 0, 0, 0);
-            }
-          }
-        } else {
-          bf16x8_v daf[2];
-#pragma unroll
-          for (int c2 = 0; c2 < 2; ++c2)
-            daf[c2] = *reinterpret_cast<const bf16x8_v*>(
-                tb + tb_off(col, (c2 * 16 + half * 8) * 2));
-          constexpr int NT = DQK / 32;
-          unsigned long long pA, pB, qA, qB;
-          auto addr_f = [&](int i) {
-            const int c2 = i / NT, t = i % NT;
-            return q_base_a + (unsigned)((t * 2 + ((lane >> 4) & 1)) * 1152 +
-                                         (8 * (c2 * 2 + half)) * 32 + (lane & 15) * 8);
-          };
-          tr16_issue2(addr_f(0), pA, pB);
-#pragma unroll
-          for (int i = 0; i < 2 * NT; ++i) {
-            const bool last = (i + 1 == 2 * NT);
-            if (!last) tr16_issue2(addr_f(i + 1), (i & 1) ? pA : qA, (i & 1) ? pB : qB);
-            bf16x8_v qb2 = tr16_take((i & 1) ? qA : pA, (i & 1) ? qB : pB, !last);
-            dk_acc[i % NT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                daf[i / NT], qb2, dk_acc[i % NT], 0, 0, 0);
-          }
-        }
-      }
-      __syncthreads();
     }
+    barrier();
   }
-
-  // ---- epilogue: plain bf16 stores — each kv row is owned by exactly one
-  // wave of one block (grid is per-Hk), so no cross-block accumulation.
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int krow = (r & 3) + 8 * (r >> 2) + 4 * half;
-    const int kg = kv0 + krow;
-    if (kg < Skv) {
-#pragma unroll
-      for (int t = 0; t < DQK / 32; ++t)
-        dk[k_base + (long)kg * k_rs + t * 32 + col] = f2bf(dk_acc[t][r]);
-#pragma unroll
-      for (int t = 0; t < DV / 32; ++t)
-        dv[v_base + (long)kg * v_rs + t * 32 + col] = f2bf(dv_acc[t][r]);
-    }
-  }
+  store_rows<DQK>(f.dq, a.scale, smem + wid * 32 * row_bytes(DQK),
+                  a.dq + (((long)b * a.Sq + q0) * a.Hq + h) * DQK, (long)a.Hq * DQK, a.Sq - q0);
 }
 
-template <int DQK, int DV, int WAVES, bool VARLEN>
-__global__ __launch_bounds__(WAVES * WAVE_SIZE, occ_dq(DQK, DV)) void flash_bwd_dq_kernel(
-    const bf16* __restrict__ dout, const bf16* __restrict__ q, const bf16* __restrict__ k,
-    const bf16* __restrict__ v, const float* __restrict__ lse, const float* __restrict__ delta,
-    bf16* __restrict__ dq, const int* __restrict__ doc_start, int B, int Sq, int Skv,
-    int Hq, int Hk, int q_start, float scale, bool causal) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* k_img = smem;                                  // subtiled [DQK/16][32][16]
-  char* v_img = smem + sub_img_bytes<DQK>();           // subtiled [DV/16][32][16]
-  char* tbuf = v_img + sub_img_bytes<DV>();            // WAVES*2048
-  float* stats = reinterpret_cast<float*>(tbuf + WAVES * 2048);  // 3*WAVES*32
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid / 64;
-  const int col = lane & 31;
-  const int half = lane >> 5;
-
-  const int qb_blk = blockIdx.x * (WAVES * 32);
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
-  const int kvh = h / (Hq / Hk);
-  const int q0 = qb_blk + wid * 32;
-
-  const long q_base = (((long)b * Sq) * Hq + h) * DQK;
-  const long do_base = (((long)b * Sq) * Hq + h) * DV;
-  const long k_base = (((long)b * Skv) * Hk + kvh) * DQK;
-  const long v_base = (((long)b * Skv) * Hk + kvh) * DV;
-  const long q_rs = (long)Hq * DQK, do_rs = (long)Hq * DV;
-  const long k_rs = (long)Hk * DQK, v_rs = (long)Hk * DV;
-  const float* lse_row = lse + ((long)b * Hq + h) * Sq;
-  const float* dlt_row = delta + ((long)b * Hq + h) * Sq;
-
-  // Q/dO rows of this wave as A-fragments
-  bf16x8_v qfrag[DQK / 16], dofrag[DV / 16];
-#pragma unroll
-  for (int c = 0; c < DQK / 16; ++c)
-    qfrag[c] = *reinterpret_cast<const bf16x8_v*>(
-        q + q_base + (long)(q0 + col) * q_rs + c * 16 + half * 8);
-#pragma unroll
-  for (int c = 0; c < DV / 16; ++c)
-    dofrag[c] = *reinterpret_cast<const bf16x8_v*>(
-        dout + do_base + (long)(q0 + col) * do_rs + c * 16 + half * 8);
-  // lse/delta(/doc_start) for the block's q rows -> LDS
-  if (tid < WAVES * 32) {
-    stats[tid] = lse_row[qb_blk + tid];
-    stats[WAVES * 32 + tid] = dlt_row[qb_blk + tid];
-    if (VARLEN) stats[2 * WAVES * 32 + tid] = (float)doc_start[q_start + qb_blk + tid];
-  }
-
-  f32x16 dq_acc[DQK / 32];
-#pragma unroll
-  for (int t = 0; t < DQK / 32; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) dq_acc[t][r] = 0.f;
-
-  char* tb = tbuf + wid * 2048;
-  const int ds_wave = VARLEN ? doc_start[q_start + q0] : 0;
-  const int block_q_max = q_start + qb_blk + WAVES * 32 - 1;
-  const int n_tiles = causal ? (min(block_q_max, Skv - 1) / 32 + 1) : (Skv + 31) / 32;
-  const int jk0 = VARLEN ? doc_start[q_start + qb_blk] / 32 : 0;
-
-  for (int jk = jk0; jk < n_tiles; ++jk) {
-    const int k0 = jk * 32;
-    // ---- stage K and V as subtiled images (one image serves both the
-    // row-chunk and the tr16 transposed reads)
-    {
-      constexpr int KCH = DQK / 8;
-      for (int idx = tid; idx < 32 * KCH; idx += WAVES * 64) {
-        const int rr = idx / KCH, c0 = (idx % KCH) * 8;
-        const int ks = min(k0 + rr, Skv - 1);  // overhang masked in compute
-        *reinterpret_cast<bf16x8*>(k_img + sub_off(rr, c0)) =
-            *reinterpret_cast<const bf16x8*>(k + k_base + (long)ks * k_rs + c0);
-      }
-      constexpr int VCH = DV / 8;
-      for (int idx = tid; idx < 32 * VCH; idx += WAVES * 64) {
-        const int rr = idx / VCH, c0 = (idx % VCH) * 8;
-        const int ks = min(k0 + rr, Skv - 1);
-        *reinterpret_cast<bf16x8*>(v_img + sub_off(rr, c0)) =
-            *reinterpret_cast<const bf16x8*>(v + v_base + (long)ks * v_rs + c0);
-      }
-    }
-    __syncthreads();
-
-    const bool live = (!causal || (k0 <= q_start + q0 + 31)) &&
-                      (!VARLEN || (k0 + 31 >= ds_wave));
-    if (live) {
-      // ---- S[q][k] = Q K^T : A=Q rows, B from k_rows (contiguous d)
-      f32x16 s;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = 0.f;
-#pragma unroll
-      for (int c = 0; c < DQK / 16; ++c) {
-        bf16x8_v kb = *reinterpret_cast<const bf16x8_v*>(
-            k_img + sub_off(col, c * 16 + half * 8));
-        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qfrag[c], kb, s, 0, 0, 0);
-      }
-      // ---- dP[q][k] = dO V^T
-      f32x16 dp;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) dp[r] = 0.f;
-#pragma unroll
-      for (int c = 0; c < DV / 16; ++c) {
-        bf16x8_v vb = *reinterpret_cast<const bf16x8_v*>(
-            v_img + sub_off(col, c * 16 + half * 8));
-        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dofrag[c], vb, dp, 0, 0, 0);
-      }
-
-      const int kg = k0 + col;   // cols = k here
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qrow = (r & 3) + 8 * (r >> 2) + 4 * half;  // block-local + wid*32
-        const int qg = q_start + q0 + qrow;
-        const bool masked = (causal && kg > qg) || kg >= Skv ||
-                            (VARLEN && kg < (int)stats[2 * WAVES * 32 + wid * 32 + qrow]);
-        const float p = masked ? 0.f : __expf(s[r] * scale - stats[wid * 32 + qrow]);
-        s[r] = p * (dp[r] - stats[WAVES * 32 + wid * 32 + qrow]) * scale;  // dS in place
-      }
-
-      // ---- transpose dS (cols=k -> A-frag rows=q), accumulate dQ
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qrow = (r & 3) + 8 * (r >> 2) + 4 * half;
-        *reinterpret_cast<bf16*>(tb + tb_off(qrow, col * 2)) = f2bf(s[r]);
-      }
-      __builtin_amdgcn_wave_barrier();
-      const unsigned k_base_a = lds_addr(k_img);
-      if constexpr (!pipe_ok_dq(DQK, DV)) {
-#pragma unroll
-        for (int c2 = 0; c2 < 2; ++c2) {
-          bf16x8_v da = *reinterpret_cast<const bf16x8_v*>(
-              tb + tb_off(col, (c2 * 16 + half * 8) * 2));
-#pragma unroll
-          for (int t = 0; t < DQK / 32; ++t) {
-            bf16x8_v ktb = tr16_frag(k_base_a, t, c2 * 2 + half, lane);
-            dq_acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(da, ktb, dq_acc[t], 0, 0, 0);
-          }
-        }
-      } else {
-        bf16x8_v daf[2];
-#pragma unroll
-        for (int c2 = 0; c2 < 2; ++c2)
-          daf[c2] = *reinterpret_cast<const bf16x8_v*>(
-              tb + tb_off(col, (c2 * 16 + half * 8) * 2));
-        constexpr int NT = DQK / 32;
-        unsigned long long pA, pB, qA, qB;
-        auto addr_f = [&](int i) {
-          const int c2 = i / NT, t = i % NT;
-          return k_base_a + (unsigned)((t * 2 + ((lane >> 4) & 1)) * 1152 +
-                                       (8 * (c2 * 2 + half)) * 32 + (lane & 15) * 8);
-        };
-        tr16_issue2(addr_f(0), pA, pB);
-#pragma unroll
-        for (int i = 0; i < 2 * NT; ++i) {
-          const bool last = (i + 1 == 2 * NT);
-          if (!last) tr16_issue2(addr_f(i + 1), (i & 1) ? pA : qA, (i & 1) ? pB : qB);
-          bf16x8_v ktb = tr16_take((i & 1) ? qA : pA, (i & 1) ? qB : pB, !last);
-          dq_acc[i % NT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              daf[i / NT], ktb, dq_acc[i % NT], 0, 0, 0);
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-    __syncthreads();
-  }
-
-  // ---- epilogue: plain bf16 stores (q rows exclusive to this block)
-#pragma unroll
-  for (int t = 0; t < DQK / 32; ++t) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int qrow = q0 + (r & 3) + 8 * (r >> 2) + 4 * half;
-      if (qrow < Sq) {
-        dq[q_base + (long)qrow * q_rs + t * 32 + col] = f2bf(dq_acc[t][r]);
-      }
-    }
-  }
-}
-
-template <int DQK, int DV, int WAVES, bool VARLEN>
-static void launch_dkv(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k,
-                       const at::Tensor& v, const at::Tensor& lse, const at::Tensor& delta,
-                       at::Tensor& dk, at::Tensor& dv, const int* doc_end, int B, int Sq,
-                       int Skv, int Hq, int Hk, int q_start, float scale, bool causal,
-                       hipStream_t stream) {
-  const dim3 grid(Skv / (WAVES * 32), Hk, B);
-  const size_t smem = sub_img_bytes<DQK>() + sub_img_bytes<DV>() + WAVES * 2048;
-  hipLaunchKernelGGL((flash_bwd_dkv_kernel<DQK, DV, WAVES, VARLEN>), grid,
-                     dim3(WAVES * WAVE_SIZE), smem, stream,
-                     reinterpret_cast<const bf16*>(dout.data_ptr()),
-                     reinterpret_cast<const bf16*>(q.data_ptr()),
-                     reinterpret_cast<const bf16*>(k.data_ptr()),
-                     reinterpret_cast<const bf16*>(v.data_ptr()),
-                     lse.data_ptr<float>(), delta.data_ptr<float>(),
-                     reinterpret_cast<bf16*>(dk.data_ptr()),
-                     reinterpret_cast<bf16*>(dv.data_ptr()), doc_end,
-                     B, Sq, Skv, Hq, Hk, q_start, scale, causal);
+template <int DV>
+static void launch_stats(const BwdArgs& a, const bf16* o, const float* lse, float* stats,
+                         hipStream_t stream) {
+  hipLaunchKernelGGL((bwd_stats_kernel<DV>), dim3(a.sp / 64, a.Hq, a.B), dim3(256), 0, stream, a.dout, o,
+                     lse, stats, a.Sq, a.sp, a.Hq, a.plane);
   HIP_CHECK_KERNEL();
 }
 
-template <int DQK, int DV, int WAVES, bool VARLEN>
-static void launch_dq(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k,
-                      const at::Tensor& v, const at::Tensor& lse, const at::Tensor& delta,
-                      at::Tensor& dq, const int* doc_start, int B, int Sq, int Skv, int Hq,
-                      int Hk, int q_start, float scale, bool causal, hipStream_t stream) {
-  const dim3 grid(Sq / (WAVES * 32), Hq, B);
-  const size_t smem = sub_img_bytes<DQK>() + sub_img_bytes<DV>() +
-                      WAVES * 2048 + 3 * WAVES * 32 * sizeof(float);
-  hipLaunchKernelGGL((flash_bwd_dq_kernel<DQK, DV, WAVES, VARLEN>), grid,
-                     dim3(WAVES * WAVE_SIZE), smem, stream,
-                     reinterpret_cast<const bf16*>(dout.data_ptr()),
-                     reinterpret_cast<const bf16*>(q.data_ptr()),
-                     reinterpret_cast<const bf16*>(k.data_ptr()),
-                     reinterpret_cast<const bf16*>(v.data_ptr()),
-                     lse.data_ptr<float>(), delta.data_ptr<float>(),
-                     reinterpret_cast<bf16*>(dq.data_ptr()), doc_start,
-                     B, Sq, Skv, Hq, Hk, q_start, scale, causal);
+template <int DQK, int DV, int WAVES, int OCC, bool PIPE>
+static void launch_dkv(const BwdArgs& a, hipStream_t stream) {
+  const long blocks = (long)((a.Skv + WAVES * 32 - 1) / (WAVES * 32)) * a.Hk * a.B;
+  // (the results leave through the same memory)
+  constexpr int smem = std::max(Dkv<DQK, DV, PIPE>::SMEM, WAVES * 32 * row_bytes(DQK > DV ? DQK : DV));
+  if (a.doc_end)
+    hipLaunchKernelGGL((bwd_dkv_kernel<DQK, DV, WAVES, OCC, PIPE, true>), dim3((unsigned)blocks),
+                       dim3(64 * WAVES), smem, stream, a);
+  else
+    hipLaunchKernelGGL((bwd_dkv_kernel<DQK, DV, WAVES, OCC, PIPE, false>), dim3((unsigned)blocks),
+                       dim3(64 * WAVES), smem, stream, a);
+  HIP_CHECK_KERNEL();
+}
+
+template <int DQK, int DV, int WAVES, int OCC, bool PIPE>
+static void launch_dq(const BwdArgs& a, hipStream_t stream) {
+  const long blocks = (long)((a.Sq + WAVES * 32 - 1) / (WAVES * 32)) * a.Hq * a.B;
+  constexpr int smem = std::max(Dq<DQK, DV, PIPE>::SMEM, WAVES * 32 * row_bytes(DQK));
+  if (a.doc_start)
+    hipLaunchKernelGGL((bwd_dq_kernel<DQK, DV, WAVES, OCC, PIPE, true>), dim3((unsigned)blocks),
+                       dim3(64 * WAVES), smem, stream, a);
+  else
+    hipLaunchKernelGGL((bwd_dq_kernel<DQK, DV, WAVES, OCC, PIPE, false>), dim3((unsigned)blocks),
+                       dim3(64 * WAVES), smem, stream, a);
   HIP_CHECK_KERNEL();
 }
 
@@ -520,62 +479,47 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
               "flash_attn_bwd: Sq%128==0, Skv%128==0 required");
   const bool varlen = doc_start.has_value();
   TORCH_CHECK(varlen == doc_end.has_value(), "doc_start and doc_end go together");
-  const int* ds_ptr = varlen ? doc_start->data_ptr<int>() : nullptr;
-  const int* de_ptr = varlen ? doc_end->data_ptr<int>() : nullptr;
   auto stream = c10::hip::getCurrentHIPStream().stream();
-
-  auto delta = at::empty({B, Hq, Sq}, q.options().dtype(at::kFloat));
-  {
-    const long rows = (long)B * Sq * Hq;
-    const int block = 256;
-    const long grid = (rows * WAVE_SIZE + block - 1) / block;
-    hipLaunchKernelGGL(fa_delta_kernel, dim3((unsigned)grid), dim3(block), 0, stream,
-                       reinterpret_cast<const bf16*>(dout.data_ptr()),
-                       reinterpret_cast<const bf16*>(o.data_ptr()),
-                       delta.data_ptr<float>(), Sq, Hq, Dv, rows);
-    HIP_CHECK_KERNEL();
-  }
-
   auto dq = at::empty_like(q);
   auto dk = at::empty_like(k);
   auto dv = at::empty_like(v);
+  BwdArgs a;
+  a.dout = reinterpret_cast<const bf16*>(dout.data_ptr());
+  a.q = reinterpret_cast<const bf16*>(q.data_ptr());
+  a.k = reinterpret_cast<const bf16*>(k.data_ptr());
+  a.v = reinterpret_cast<const bf16*>(v.data_ptr());
+  a.dq = reinterpret_cast<bf16*>(dq.data_ptr());
+  a.dk = reinterpret_cast<bf16*>(dk.data_ptr());
+  a.dv = reinterpret_cast<bf16*>(dv.data_ptr());
+  a.doc_start = varlen ? doc_start->data_ptr<int>() : nullptr;
+  a.doc_end = varlen ? doc_end->data_ptr<int>() : nullptr;
+  a.B = B; a.Sq = Sq; a.Skv = Skv; a.Hq = Hq; a.Hk = Hk; a.q_start = (int)q_start;
+  a.sp = (Sq + 63) / 64 * 64;
+  a.plane = (long)B * Hq * a.sp;
+  a.scale = (float)scale;
+  a.causal = causal;
+  auto stats = at::empty({2, B, Hq, a.sp}, q.options().dtype(at::kFloat));
+  a.stats = stats.data_ptr<float>();
+  const bf16* op = reinterpret_cast<const bf16*>(o.data_ptr());
 
+  // Waves per SIMD and pipelining by what fits the registers and LDS; dK/dV need one wave a
+  // SIMD from head dim 96 on (at two a SIMD it spills: 1620 against 680 us at 2 x 4096, 32/8
+  // heads of 128). dQ of 128/128 at two waves a SIMD overlaps as well without the third K
+  // buffer (379 against 392 us); (192, 128) would spill there (461 against 203 us).
   bool done = false;
-  // kv-parallel dKV: 8-wave only where two waves/SIMD fit (occ_dkv == 2)
-#define FA_BWD_CASE(A, C)                                                                \
-  if (!done && Dqk == A && Dv == C) {                                                    \
-    done = true;                                                                         \
-    if (varlen) {                                                                        \
-      launch_dkv<A, C, 4, true>(dout, q, k, v, lse, delta, dk, dv, de_ptr, B, Sq, Skv,   \
-                                Hq, Hk, (int)q_start, (float)scale, causal, stream);     \
-      launch_dq<A, C, 4, true>(dout, q, k, v, lse, delta, dq, ds_ptr, B, Sq, Skv, Hq,    \
-                               Hk, (int)q_start, (float)scale, causal, stream);          \
-    } else {                                                                             \
-      if (occ_dkv(A, C) == 2 && Skv % 256 == 0) {                                        \
-        launch_dkv<A, C, (occ_dkv(A, C) == 2 ? 8 : 4), false>(                           \
-            dout, q, k, v, lse, delta, dk, dv, nullptr, B, Sq, Skv, Hq, Hk,              \
-            (int)q_start, (float)scale, causal, stream);                                 \
-      } else {                                                                           \
-        launch_dkv<A, C, 4, false>(dout, q, k, v, lse, delta, dk, dv, nullptr, B, Sq,    \
-                                   Skv, Hq, Hk, (int)q_start, (float)scale, causal,      \
-                                   stream);                                              \
-      }                                                                                  \
-      if (occ_dq(A, C) == 2 && Sq % 256 == 0) {                                          \
-        launch_dq<A, C, (occ_dq(A, C) == 2 ? 8 : 4), false>(                             \
-            dout, q, k, v, lse, delta, dq, nullptr, B, Sq, Skv, Hq, Hk, (int)q_start,    \
-            (float)scale, causal, stream);                                               \
-      } else {                                                                           \
-        launch_dq<A, C, 4, false>(dout, q, k, v, lse, delta, dq, nullptr, B, Sq, Skv,    \
-                                  Hq, Hk, (int)q_start, (float)scale, causal, stream);   \
-      }                                                                                  \
-    }                                                                                    \
+#define FA_BWD_CASE(A, C, KV_OCC, KV_PIPE, Q_OCC, Q_PIPE)                                 \
+  if (!done && Dqk == A && Dv == C) {                                                     \
+    done = true;                                                                          \
+    launch_stats<C>(a, op, lse.data_ptr<float>(), stats.data_ptr<float>(), stream);       \
+    launch_dkv<A, C, 4, KV_OCC, KV_PIPE>(a, stream);                                      \
+    launch_dq<A, C, 4, Q_OCC, Q_PIPE>(a, stream);                                         \
   }
-  FA_BWD_CASE(64, 64)
-  FA_BWD_CASE(96, 96)
-  FA_BWD_CASE(128, 128)
-  FA_BWD_CASE(192, 128)
-  FA_BWD_CASE(192, 192)
-  FA_BWD_CASE(256, 256)
+  FA_BWD_CASE(64, 64, 2, true, 2, true)
+  FA_BWD_CASE(96, 96, 1, true, 2, true)
+  FA_BWD_CASE(128, 128, 1, true, 2, false)
+  FA_BWD_CASE(192, 128, 1, true, 1, true)
+  FA_BWD_CASE(192, 192, 1, false, 1, false)
+  FA_BWD_CASE(256, 256, 1, false, 1, false)
 #undef FA_BWD_CASE
   TORCH_CHECK(done, "flash_attn_bwd: unsupported head dims (Dqk=", Dqk, ", Dv=", Dv, ")");
   return {dq, dk, dv};
@@ -585,13 +529,13 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
 __global__ void mfma_probe_kernel(const bf16* a, const bf16* b, float* d) {
   const int lane = threadIdx.x & 63;
   const int half = lane >> 5;
-  bf16x8_v af, bf_;
+  bf16x8_t af, bf_;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     af[j] = (__bf16)a[(lane & 31) * 16 + half * 8 + j];   // A[i=l&31][k=8*half+j]
     bf_[j] = (__bf16)b[(half * 8 + j) * 32 + (lane & 31)];  // B[k=8*half+j][j=l&31]
   }
-  f32x16 acc;
+  f32x16_t acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bf_, acc, 0, 0, 0);

@@ -30,6 +30,11 @@ def _docs(cuts, total):
     return start.cuda(), end.cuda()
 
 
+def _grads(fn, args, dout):
+    args = [t.detach().clone().requires_grad_() for t in args]
+    return torch.autograd.grad(fn(*args), args, dout)
+
+
 # probabilities and the output are each rounded to bf16 once (2^-9 of a value at most)
 FWD = 2 * 2.0 ** -9
 
@@ -58,3 +63,34 @@ def test_forward(dims, sq, skv, causal, q_start, cuts, scale):
     ro, rlse = _reference(q, k, v, causal, q_start, start, scale)
     assert (o.float() - ro).norm() / ro.norm() < FWD
     assert (lse - rlse).abs().max() < 1e-5 * max(1.0, float(rlse.abs().max()))
+
+
+# dS is rounded to bf16 once and so is each gradient; P and the delta of a bf16 output bring
+# about the same again
+BWD = 4 * 2.0 ** -9
+
+
+@pytest.mark.parametrize("dims", [(64, 64), (96, 96), (128, 128), (192, 128), (192, 192), (256, 256)])
+@pytest.mark.parametrize("sq,skv,causal,q_start,cuts,scale", [
+    (128, 128, True, 0, None, 1.0),
+    (384, 256, False, 0, None, 1.0),
+    (256, 640, True, 384, None, 1.0),
+    (640, 640, True, 0, (1, 63, 64, 65, 130, 500), 1.0),
+    (256, 768, True, 256, (100, 300, 301), 1.0),
+    (256, 256, True, 0, None, -1.0),
+])
+def test_backward(dims, sq, skv, causal, q_start, cuts, scale):
+    torch.manual_seed(0)
+    q = torch.randn(2 if cuts is None else 1, sq, 4, dims[0], device="cuda").bfloat16()
+    k = torch.randn(q.shape[0], skv, 2, dims[0], device="cuda").bfloat16()
+    v = torch.randn(q.shape[0], skv, 2, dims[1], device="cuda").bfloat16()
+    do = torch.randn(q.shape[0], sq, 4, dims[1], device="cuda").bfloat16()
+    scale *= dims[0] ** -0.5
+    start, end = (None, None) if cuts is None else _docs(cuts, skv)
+    from automodel_amd.ops.attention import _FlashAttnHip
+
+    got = _grads(lambda *t: _FlashAttnHip.apply(*t, causal, scale, q_start, start, end), (q, k, v), do)
+    ref = _grads(lambda *t: _reference(*t, causal, q_start, start, scale)[0],
+                 (q.float(), k.float(), v.float()), do.float())
+    for name, g, r in zip(("dq", "dk", "dv"), got, ref):
+        assert (g.float() - r).norm() / r.norm() < BWD, name
