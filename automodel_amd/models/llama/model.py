@@ -225,7 +225,12 @@ class LlamaAttention(nn.Module):
             from automodel_amd.utils.kv_cache import active_kv_cache, maybe_update_kv
 
             cache = active_kv_cache()
-            if cache is not None and getattr(cache, "is_static", False):
+            o = None
+            if cache is not None and self.backend.attn == "hip":
+                o = cache.attend(q, k, v, attn_scale)
+            if o is not None:
+                pass
+            elif cache is not None and getattr(cache, "is_static", False):
                 # static-shape decode (hipGraph capture): full-buffer KV +
                 # additive mask from the device position counter
                 from automodel_amd.ops.attention import sdpa_masked
@@ -233,11 +238,14 @@ class LlamaAttention(nn.Module):
                 k, v, _ = maybe_update_kv(k, v)
                 o = sdpa_masked(q, k, v, cache.attn_mask(), scale=attn_scale)
             else:
+                new_k, new_v = k, v
                 k, v, cache_pos = maybe_update_kv(k, v)
-                # cached decode: q is short (often 1) and prompts are
-                # arbitrary lengths — sdpa is the right tool (GEMV-bound;
-                # the flash kernel's 128-row tiling wants training shapes)
-                attn_backend = "sdpa" if cache is not None else self.backend.attn
+                attn_backend = self.backend.attn
+                if cache is not None and (cache_pos > 0 or q.dtype != torch.bfloat16):
+                    # several tokens behind a prefix: any lengths, few rows
+                    attn_backend = "sdpa"
+                elif cache is not None:
+                    k, v = new_k, new_v       # a whole prompt: the cache holds the same
                 o = flash_attention(q, k, v, causal=True, scale=attn_scale,
                                     backend=attn_backend, q_start=cache_pos)
         return self.o_proj(o.reshape(B, S, -1))
@@ -369,6 +377,7 @@ class LlamaForCausalLM(nn.Module):
                         "HeliumForCausalLM", "SeedOssForCausalLM",
                         "HunYuanDenseV1ForCausalLM", "ApertusForCausalLM")
     config_class = LlamaConfig
+    selects_logit_rows = True       # forward takes ``logit_rows``
 
     @staticmethod
     def config_from_hf(hf_cfg) -> LlamaConfig:
@@ -406,12 +415,15 @@ class LlamaForCausalLM(nn.Module):
         labels: torch.Tensor | None = None,
         position_ids: torch.Tensor | None = None,
         return_hidden: bool = False,
+        logit_rows: torch.Tensor | None = None,
         **_: Any,
     ) -> torch.Tensor:
         """labels given -> token-sum loss; return_hidden -> [B,S,H]; else logits.
 
         ``labels`` must already be shifted (labels[t] is the target of
         position t), matching the reference's dataset convention.
+        ``logit_rows``: indices into the flattened [B*S] tokens whose logits are
+        wanted -> [n, vocab]; the head then runs on those rows only.
         """
         hidden = self.model(input_ids, position_ids)
         if self.config.logits_scaling != 1.0 and not return_hidden:
@@ -422,6 +434,8 @@ class LlamaForCausalLM(nn.Module):
             return self.loss_fn(hidden, self.lm_head.weight, labels)
         if return_hidden:
             return hidden
+        if logit_rows is not None:
+            hidden = hidden.flatten(0, 1)[logit_rows]
         return self.lm_head(hidden)
 
     @torch.no_grad()

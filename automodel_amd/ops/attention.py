@@ -121,31 +121,21 @@ class _FlashAttnHip(torch.autograd.Function):
 
 def _flash_hip(q, k, v, causal, scale, q_start, doc_start=None, doc_end=None):
     """Dispatch to the HIP kernel, zero-padding head dims to a supported
-    kernel pair and (for plain causal) sequence lengths to the kernel's
-    tile granularity — pad/slice sit outside the Function so autograd
-    routes gradients through them."""
+    kernel pair — pad/slice sit outside the Function so autograd routes
+    gradients through them. The kernels take any sequence lengths."""
     dqk, dv = q.shape[-1], v.shape[-1]
     tq, tv = _target_dims(dqk, dv)
     if tq != dqk or tv != dv:
         q, k, v = _pad_head(q, tq), _pad_head(k, tq), _pad_head(v, tv)
-    sq, skv = q.shape[1], k.shape[1]
-    pad_q = (-sq) % 128
-    pad_kv = (-skv) % 128 if doc_start is None else (-skv) % 32
-    if pad_q or pad_kv:
-        # safe only for plain causal from position 0: padded KV rows sit at
-        # positions above every real q row, so the causal mask excludes them
-        assert causal and q_start == 0 and doc_start is None, \
-            "flash: Sq%128/Skv%32 required for q_start/varlen/non-causal calls"
-        F = torch.nn.functional.pad
-        if pad_q:
-            q = F(q, (0, 0, 0, 0, 0, pad_q))
-        if pad_kv:
-            k = F(k, (0, 0, 0, 0, 0, pad_kv))
-            v = F(v, (0, 0, 0, 0, 0, pad_kv))
     o = _FlashAttnHip.apply(q, k, v, causal, scale, q_start, doc_start, doc_end)
-    if pad_q:
-        o = o[:, :sq]
     return o[..., :dv] if tv != dv else o
+
+
+def _check_lengths(q, k, causal, q_start) -> None:
+    """Chunks with an offset and non-causal calls come in whole tiles."""
+    if q.shape[1] % 128 or k.shape[1] % 128:
+        assert causal and q_start == 0, \
+            "flash: Sq%128/Skv%128 required for q_start/non-causal calls"
 
 
 _VARLEN_CU: torch.Tensor | None = None
@@ -163,6 +153,8 @@ def doc_bounds_from_cu(cu_seqlens: torch.Tensor, total: int) -> tuple[torch.Tens
     """Per-token document bounds for the varlen kernels: doc_start[t] /
     doc_end[t] of the packed document containing token t. Tokens in
     [cu[-1], total) (seq-length padding) form their own trailing doc."""
+    if cu_seqlens.is_cuda:
+        return hip_ops().doc_bounds(cu_seqlens.to(torch.int32).contiguous(), total)
     cu = cu_seqlens.to(torch.long)
     lengths = cu[1:] - cu[:-1]
     ds = torch.repeat_interleave(cu[:-1], lengths)
@@ -188,17 +180,8 @@ def flash_attention_varlen(q, k, v, cu_seqlens: torch.Tensor, scale: float | Non
     assert q.shape[0] == 1, "varlen expects a packed THD batch [1, T, H, D]"
     scale = scale if scale is not None else 1.0 / math.sqrt(q.shape[-1])
     if backend == "hip" and q.is_cuda:
-        T = q.shape[1]
-        pad = (-T) % 128
-        Tp = T + pad
-        cu_dev = cu_seqlens.to(q.device)
-        ds, de = doc_bounds_from_cu(cu_dev, Tp)
-        if pad:
-            q = torch.nn.functional.pad(q, (0, 0, 0, 0, 0, pad))
-            k = torch.nn.functional.pad(k, (0, 0, 0, 0, 0, pad))
-            v = torch.nn.functional.pad(v, (0, 0, 0, 0, 0, pad))
-        o = _flash_hip(q, k, v, True, scale, 0, ds, de)
-        return o[:, :T]
+        ds, de = doc_bounds_from_cu(cu_seqlens.to(q.device), q.shape[1])
+        return _flash_hip(q, k, v, True, scale, 0, ds, de)
     from automodel_amd.datasets.llm.packed_sequence import block_causal_mask
 
     mask = block_causal_mask(cu_seqlens.cpu(), q.shape[1]).to(q.device)
@@ -222,6 +205,7 @@ def flash_attention(
         return flash_attention_varlen(q, k, v, _VARLEN_CU, scale, backend)
     scale = scale if scale is not None else 1.0 / math.sqrt(q.shape[-1])
     if backend == "hip" and q.is_cuda:
+        _check_lengths(q, k, causal, q_start)
         return _flash_hip(q, k, v, causal, scale, q_start)
     if backend == "eager":
         return attention_ref(q, k, v, causal, scale, q_start)

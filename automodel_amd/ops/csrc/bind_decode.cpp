@@ -20,6 +20,13 @@ TORCH_LIBRARY_FRAGMENT(amd_ops, m) {
       "gemm_skinny_bf16(Tensor x, Tensor w, bool relu2, bool out_f32, int group_n=0) -> Tensor");
   m.impl("gemm_skinny_bf16", &amd_ops::gemm_skinny_bf16);
 
+  m.def("doc_bounds(Tensor cu, int total) -> (Tensor, Tensor)");
+  m.impl("doc_bounds", &amd_ops::doc_bounds);
+  m.def(
+      "kv_decode_attn(Tensor q, Tensor k_new, Tensor v_new, Tensor(a!) k_cache, "
+      "Tensor(b!) v_cache, int pos, Tensor? pos_dev, float scale) -> Tensor");
+  m.impl("kv_decode_attn", &amd_ops::kv_decode_attn);
+
   m.def("embed_rms_norm(Tensor ids, Tensor table, Tensor w, float eps) -> Tensor");
   m.impl("embed_rms_norm", &amd_ops::embed_rms_norm);
   m.def("residual_rms_norm(Tensor x, Tensor w, float eps) -> Tensor");

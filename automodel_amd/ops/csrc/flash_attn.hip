@@ -277,6 +277,33 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArg
   }
 }
 
+// document [start, end) of every token of a packed row, by bisection of cu; what lies
+// beyond cu's last entry is a document of its own
+__global__ void doc_bounds_kernel(const int* __restrict__ cu, int n, int total, int* __restrict__ start,
+                                  int* __restrict__ end) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= total) return;
+  int lo = 0, hi = n;                   // first entry greater than t
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    if (cu[mid] > t) hi = mid; else lo = mid + 1;
+  }
+  start[t] = lo > 0 ? cu[lo - 1] : 0;
+  end[t] = lo < n ? cu[lo] : total;
+}
+
+std::tuple<at::Tensor, at::Tensor> doc_bounds(const at::Tensor& cu, int64_t total) {
+  TORCH_CHECK(cu.is_cuda() && cu.dim() == 1 && cu.scalar_type() == at::kInt && cu.is_contiguous() &&
+                  cu.numel() >= 1 && total >= 0, "doc_bounds: cu_seqlens int32 [n + 1]");
+  auto start = at::empty({total}, cu.options()), end = at::empty({total}, cu.options());
+  if (total == 0) return {start, end};
+  hipLaunchKernelGGL(doc_bounds_kernel, dim3(ceil_div_i(total, 256)), dim3(256), 0,
+                     c10::hip::getCurrentHIPStream().stream(), cu.data_ptr<int>(), (int)cu.numel(),
+                     (int)total, start.data_ptr<int>(), end.data_ptr<int>());
+  HIP_CHECK_KERNEL();
+  return {start, end};
+}
+
 template <int DQK, int DV, int WAVES, int OCC, bool PIPE, bool VARLEN>
 static void launch_fwd(const FwdArgs& a, hipStream_t stream) {
   using F = Fwd<DQK, DV, WAVES, VARLEN>;
@@ -295,9 +322,13 @@ std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
   const int B = q.size(0), Sq = q.size(1), Hq = q.size(2), Dqk = q.size(3);
   const int Skv = k.size(1), Hk = k.size(2), Dv = v.size(3);
   TORCH_CHECK(Hq % Hk == 0, "flash_attn_fwd: Hq must be divisible by Hk");
-  TORCH_CHECK(Sq % 128 == 0, "flash_attn_fwd: Sq must be a multiple of 128");
-  TORCH_CHECK(Skv % 32 == 0, "flash_attn_fwd: Skv must be a multiple of 32");
+  TORCH_CHECK(k.size(0) == B && v.size(0) == B && k.size(3) == Dqk && v.size(1) == Skv && v.size(2) == Hk &&
+                  q.is_contiguous() && k.is_contiguous() && v.is_contiguous(),
+              "flash_attn_fwd: contiguous k [B,Skv,Hk,Dqk], v [B,Skv,Hk,Dv]");
+  TORCH_CHECK(Sq >= 1 && Skv >= 1, "flash_attn_fwd: empty sequences");
   const bool varlen = doc_start.has_value();
+  if (varlen)
+    TORCH_CHECK(doc_start->numel() >= q_start + Sq, "flash_attn_fwd: doc_start for every query position");
   if (varlen) TORCH_CHECK(causal && B == 1, "varlen flash is causal with B==1");
   if (sink)
     TORCH_CHECK(sink->is_cuda() && sink->is_contiguous() && sink->numel() == Hq &&

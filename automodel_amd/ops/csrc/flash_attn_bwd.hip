@@ -475,10 +475,15 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
     const std::optional<at::Tensor>& doc_start, const std::optional<at::Tensor>& doc_end) {
   const int B = q.size(0), Sq = q.size(1), Hq = q.size(2), Dqk = q.size(3);
   const int Skv = k.size(1), Hk = k.size(2), Dv = v.size(3);
-  TORCH_CHECK(Sq % 128 == 0 && Skv % 128 == 0,
-              "flash_attn_bwd: Sq%128==0, Skv%128==0 required");
+  TORCH_CHECK(q.is_contiguous() && k.is_contiguous() && v.is_contiguous() && o.is_contiguous() &&
+                  dout.is_contiguous() && dout.sizes() == o.sizes() && lse.is_contiguous() &&
+                  lse.numel() == (long)B * Hq * Sq && k.size(3) == Dqk && v.size(1) == Skv && v.size(2) == Hk,
+              "flash_attn_bwd: contiguous tensors of the forward's shapes");
   const bool varlen = doc_start.has_value();
   TORCH_CHECK(varlen == doc_end.has_value(), "doc_start and doc_end go together");
+  if (varlen)
+    TORCH_CHECK(doc_start->numel() >= q_start + Sq && doc_end->numel() >= Skv,
+                "flash_attn_bwd: doc_start and doc_end for every position");
   auto stream = c10::hip::getCurrentHIPStream().stream();
   auto dq = at::empty_like(q);
   auto dk = at::empty_like(k);

@@ -87,10 +87,15 @@ class DecodeSession:
                 if self.live or len(set(lens)) != 1:
                     raise ValueError("a dense K/V cache takes one batch of equal prompts")
                 handles = list(range(len(prompts)))
-                full = self.model(torch.tensor([list(p) for p in prompts], device=self.device))
+                ids = torch.tensor([list(p) for p in prompts], device=self.device)
+                if getattr(self.model, "selects_logit_rows", False):
+                    rows = [i * lens[0] + j % lens[0] for i, w in enumerate(want) for j in w]
+                    logits = self.model(ids, logit_rows=torch.tensor(rows, device=self.device))
+                else:
+                    full = self.model(ids)
+                    logits = torch.cat([full[i, w] for i, w in enumerate(want)])
                 self._check_dense()
                 cache.advance(lens[0])
-                logits = torch.cat([full[i, w] for i, w in enumerate(want)])
         self.live += handles
         return handles, logits
 

@@ -62,6 +62,29 @@ class KVCache:
         self.v[i][:, self.pos : self.pos + S] = v_new
         return (self.k[i][:, : self.pos + S], self.v[i][:, : self.pos + S])
 
+    def attend(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+               scale: float | None) -> torch.Tensor | None:
+        """One new token per sequence, q/k/v [B, 1, heads, D], against all that the
+        layer has of it, which this records as ``update`` does: one pass over the cache
+        (csrc/kv_decode.hip). None where that kernel does not apply, and nothing is done."""
+        kc, D = self.k[self._layer], q.shape[-1]
+        if not (q.is_cuda and q.shape[1] == 1 and not torch.is_grad_enabled()
+                and q.dtype == kc.dtype == torch.bfloat16
+                and D % 8 == 0 and D <= 256 and q.shape[0] == kc.shape[0]):
+            return None
+        from automodel_amd.ops._backend import hip_ops
+
+        pos_dev = self._device_position()
+        assert pos_dev is not None or self.pos < self.max_len, "KV cache overflow"
+        o = hip_ops().kv_decode_attn(
+            q.contiguous(), k.contiguous(), v.contiguous(), kc, self.v[self._layer],
+            self.pos, pos_dev, D ** -0.5 if scale is None else scale)
+        self._layer += 1
+        return o
+
+    def _device_position(self) -> torch.Tensor | None:
+        return None
+
     def advance(self, n: int) -> None:
         self.pos += n
 
@@ -112,6 +135,9 @@ class StaticKVCache(KVCache):
             self.k[i].index_copy_(1, idx, k_new)
             self.v[i].index_copy_(1, idx, v_new)
         return self.k[i], self.v[i]          # full static buffers
+
+    def _device_position(self) -> torch.Tensor | None:
+        return self.pos_dev
 
     def position_ids(self) -> torch.Tensor:
         """[1, 1] device position for rope indexing inside the graph."""

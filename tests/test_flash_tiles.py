@@ -48,6 +48,9 @@ FWD = 2 * 2.0 ** -9
     (256, 768, True, 256, (100, 300, 301), 1.0),
     (256, 256, True, 0, None, -1.0),
     (256, 256, True, 0, None, 0.0),
+    (1, 1, True, 0, None, 1.0),
+    (129, 129, True, 0, None, 1.0),
+    (333, 333, True, 0, (5, 200, 201), 1.0),
 ])
 def test_forward(dims, sq, skv, causal, q_start, cuts, scale):
     torch.manual_seed(0)
@@ -78,6 +81,9 @@ BWD = 4 * 2.0 ** -9
     (640, 640, True, 0, (1, 63, 64, 65, 130, 500), 1.0),
     (256, 768, True, 256, (100, 300, 301), 1.0),
     (256, 256, True, 0, None, -1.0),
+    (17, 17, True, 0, None, 1.0),
+    (129, 129, True, 0, None, 1.0),
+    (333, 333, True, 0, (5, 200, 201), 1.0),
 ])
 def test_backward(dims, sq, skv, causal, q_start, cuts, scale):
     torch.manual_seed(0)
@@ -94,3 +100,12 @@ def test_backward(dims, sq, skv, causal, q_start, cuts, scale):
                  (q.float(), k.float(), v.float()), do.float())
     for name, g, r in zip(("dq", "dk", "dv"), got, ref):
         assert (g.float() - r).norm() / r.norm() < BWD, name
+
+
+def test_document_bounds():
+    from automodel_amd.ops.attention import doc_bounds_from_cu
+
+    for cu, total in ([0, 3, 3, 7, 300], 300), ([0, 5, 260], 301), ([0, 1], 1):
+        cu = torch.tensor(cu, dtype=torch.int32)
+        for got, want in zip(doc_bounds_from_cu(cu.cuda(), total), doc_bounds_from_cu(cu, total)):
+            assert got.dtype == want.dtype and torch.equal(got.cpu(), want)
