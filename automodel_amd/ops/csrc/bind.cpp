@@ -63,6 +63,8 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("fp8_cast", &amd_ops::fp8_cast);
   m.def("fp8_transpose(Tensor x8) -> Tensor");
   m.impl("fp8_transpose", &amd_ops::fp8_transpose);
+  m.def("lora_apply(Tensor? y, Tensor x, Tensor A, Tensor B, float scale) -> (Tensor, Tensor)");
+  m.impl("lora_apply", &amd_ops::lora_apply);
   m.def("lora_fused_fwd(Tensor x, Tensor A, Tensor B, float scale) -> Tensor");
   m.impl("lora_fused_fwd", &amd_ops::lora_fused_fwd);
   m.def("sgmv_fused_fwd(Tensor x, Tensor A, Tensor B, Tensor scales, Tensor offs, Tensor tile_map, Tensor? n_tiles=None) -> Tensor");

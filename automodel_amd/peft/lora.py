@@ -39,30 +39,28 @@ class PeftConfig:
 
 
 class _FusedLoRAFn(torch.autograd.Function):
-    """Fused delta = (x @ A^T) @ B^T * scale (csrc/lora.hip — one kernel,
-    the [M, r] intermediate never hits HBM; reference _peft/lora_kernel.py
-    lora_forward_kernel). Backward recomputes t with two skinny GEMMs."""
+    """y + (x @ A^T) @ B^T * scale (csrc/lora.hip; reference _peft/lora_kernel.py
+    lora_forward_kernel): one pass over y, the sum rounded once."""
 
     @staticmethod
-    def forward(ctx, x2, wa, wb, scale):
+    def forward(ctx, y, x2, wa, wb, scale):
         from automodel_amd.ops._backend import hip_ops
 
-        delta = hip_ops().lora_fused_fwd(x2, wa, wb, scale)
-        ctx.save_for_backward(x2, wa, wb)
+        out, t = hip_ops().lora_apply(y, x2, wa.contiguous(), wb.contiguous(), scale)
+        ctx.save_for_backward(x2, wa, wb, t)
         ctx.scale = scale
-        return delta
+        return out
 
     @staticmethod
     def backward(ctx, g):
-        x2, wa, wb = ctx.saved_tensors
+        x2, wa, wb, t = ctx.saved_tensors
         s = ctx.scale
         g = g.contiguous()
-        t = x2 @ wa.t()                  # [M, r] recompute
         dt = (g @ wb) * s
         dx = dt.to(x2.dtype) @ wa
         da = dt.t().to(x2.dtype) @ x2
-        db = (g.t() @ t.to(g.dtype)) * s
-        return dx, da.to(wa.dtype), db.to(wb.dtype), None
+        db = (g.t() @ t) * s
+        return g, dx, da.to(wa.dtype), db.to(wb.dtype), None
 
 
 class LinearLoRA(nn.Module):
@@ -118,14 +116,15 @@ class LinearLoRA(nn.Module):
             y = torch.nn.functional.linear(x, w, self.base.bias)
             return y
         wa, wb = self.lora_A.weight, self.lora_B.weight
+        y = self.base(x)
         if (x.is_cuda and x.dtype == torch.bfloat16 and not self.training_dropout()
                 and wa.shape[0] in (32, 64) and wa.shape[1] % 64 == 0
-                and wb.shape[0] % 64 == 0
+                and wb.shape[0] % 64 == 0 and wa.dtype == y.dtype == torch.bfloat16
                 and (x.numel() // x.shape[-1]) % 8 == 0):
             x2 = x.reshape(-1, x.shape[-1]).contiguous()
-            delta = _FusedLoRAFn.apply(x2, wa, wb, self.scale)
-            return self.base(x) + delta.view(*x.shape[:-1], wb.shape[0])
-        return self.base(x) + self.lora_B(self.lora_A(self.dropout(x))) * self.scale
+            y2 = y.reshape(-1, wb.shape[0]).contiguous()
+            return _FusedLoRAFn.apply(y2, x2, wa, wb, self.scale).view(y.shape)
+        return y + self.lora_B(self.lora_A(self.dropout(x))) * self.scale
 
     def training_dropout(self) -> bool:
         return self.training and not isinstance(self.dropout, nn.Identity)
