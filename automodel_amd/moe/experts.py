@@ -173,14 +173,17 @@ class GroupedExperts(nn.Module):
             and x_perm.numel() > 0
         )
         if use_grouped:
-            from automodel_amd.ops.grouped_gemm import grouped_linear, make_group_plan
+            from automodel_amd.ops.grouped_gemm import grouped_linear, make_group_plan, tile_rows
 
             if torch.is_tensor(counts) and counts.is_cuda:
                 # device-side plan shared by all three projections — the
-                # routing counts never touch the host;
+                # routing counts never touch the host; the fp8 kernels have
                 # 256-row tiles when every projection width allows
-                bm = 256 if (self.intermediate_size % 256 == 0
-                             and self.hidden_size % 256 == 0) else 128
+                if self.fp8:
+                    bm = 256 if (self.intermediate_size % 256 == 0
+                                 and self.hidden_size % 256 == 0) else 128
+                else:
+                    bm = tile_rows(x_perm.shape[0], self.n_experts)
                 plan = (*make_group_plan(counts, x_perm.shape[0], bm), bm)
                 cl = counts
             else:

@@ -74,14 +74,12 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("build_group_plan", &amd_ops::build_group_plan);
   m.def("grouped_gemm_nt(Tensor x, Tensor w, Tensor offs, Tensor tile_map, Tensor? n_tiles=None, int bm=128) -> Tensor");
   m.impl("grouped_gemm_nt", &amd_ops::grouped_gemm_nt);
-  m.def("grouped_gemm_nn(Tensor g, Tensor w, Tensor offs, Tensor tile_map, Tensor? n_tiles=None) -> Tensor");
+  m.def("grouped_gemm_nn(Tensor g, Tensor w, Tensor offs, Tensor tile_map, Tensor? n_tiles=None, int bm=128) -> Tensor");
   m.impl("grouped_gemm_nn", &amd_ops::grouped_gemm_nn);
   m.def("grouped_gemm_tn(Tensor g, Tensor x, Tensor offs, int E) -> Tensor");
   m.impl("grouped_gemm_tn", &amd_ops::grouped_gemm_tn);
   m.def("grouped_gemm_nt_fp8(Tensor x8, Tensor w8, Tensor offs, Tensor tile_map, Tensor scale, Tensor? n_tiles=None, int bm=128) -> Tensor");
   m.impl("grouped_gemm_nt_fp8", &amd_ops::grouped_gemm_nt_fp8);
-  m.def("transpose_bf16(Tensor x) -> Tensor");
-  m.impl("transpose_bf16", &amd_ops::transpose_bf16);
   m.def("permute_gather(Tensor x, Tensor src) -> Tensor");
   m.impl("permute_gather", &amd_ops::permute_gather);
   m.def("unpermute_combine(Tensor yp, Tensor pos, Tensor probs) -> Tensor");

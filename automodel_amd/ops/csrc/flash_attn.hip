@@ -133,7 +133,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArg
   f.causal = a.causal;
 
   const Place at = place_block((a.Sq + F::BM - 1) / F::BM, a.Hq, a.B, a.causal);
-  const int lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
+  const int half = (threadIdx.x >> 5) & 1, col = threadIdx.x & 31;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = at.head, b = at.batch, kvh = h / (a.Hq / a.Hk);
   const int qblk = at.tile * F::BM;                   // block's, wave's first query row
@@ -256,25 +256,8 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArg
   const float inv = ls > 0.f ? 1.f / ls : 0.f;
   if (half == 0 && q0 + col < a.Sq)
     a.lse[((long)b * a.Hq + h) * a.Sq + q0 + col] = ls > 0.f ? m2 * LN2 + __logf(ls) : -1e30f;
-#pragma unroll
-  for (int t = 0; t < F::NT; ++t)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {                     // columns 32 t + 8 g + 4 half + 0..3
-      bf16x4_t w;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = (__bf16)(f.o[t][4 * g + j] * inv);
-      *reinterpret_cast<bf16x4_t*>(mine + col * RB + (((t * 4 + g) ^ swz<DV>(col)) << 4) + half * 8) = w;
-    }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // a wave reads what it wrote itself
-  constexpr int CH = DV / 8, PER = 64 / CH;           // 16-byte pieces of a row, rows per store
-  bf16* op = a.out + (((long)b * a.Sq + q0) * a.Hq + h) * DV;
-  if (lane < PER * CH) {
-    for (int r = lane / CH; r < 32 && q0 + r < a.Sq; r += PER) {
-      const int ch = lane % CH;
-      *reinterpret_cast<uint4*>(op + (long)r * a.Hq * DV + ch * 8) =
-          *reinterpret_cast<const uint4*>(mine + r * RB + ((ch ^ swz<DV>(r)) << 4));
-    }
-  }
+  store_rows<DV>(f.o, inv, mine, a.out + (((long)b * a.Sq + q0) * a.Hq + h) * DV, (long)a.Hq * DV,
+                 a.Sq - q0);
 }
 
 // document [start, end) of every token of a packed row, by bisection of cu; what lies

@@ -80,32 +80,6 @@ struct BwdArgs {
   bool causal;
 };
 
-// rows r of a wave's transposed accumulators [D / 32] (column = row of the result), scaled,
-// through LDS to whole-row stores of bf16
-template <int D>
-__device__ __forceinline__ void store_rows(const f32x16_t (&acc)[D / 32], float scale, char* mine,
-                                           bf16* dst, long row_stride, int rows) {
-  constexpr int RB = row_bytes(D), CH = D / 8, PER = 64 / CH;
-  const int lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
-#pragma unroll
-  for (int t = 0; t < D / 32; ++t)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      bf16x4_t w;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = (__bf16)(acc[t][4 * g + j] * scale);
-      *reinterpret_cast<bf16x4_t*>(mine + col * RB + (((t * 4 + g) ^ swz<D>(col)) << 4) + half * 8) = w;
-    }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // a wave reads what it wrote itself
-  if (lane < PER * CH) {
-    const int ch = lane % CH;
-    for (int r = lane / CH; r < 32 && r < rows; r += PER)
-      *reinterpret_cast<uint4*>(dst + (long)r * row_stride + ch * 8) =
-          *reinterpret_cast<const uint4*>(mine + r * RB + ((ch ^ swz<D>(r)) << 4));
-  }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-}
-
 template <int D>
 __device__ __forceinline__ void load_row_frags(bf16x8_t (&f)[D / 16], const bf16* row) {
   const int half = (threadIdx.x >> 5) & 1;

@@ -57,11 +57,16 @@ __device__ __forceinline__ int acc_row(int r, int half) { return (r & 3) + 8 * (
 
 // 16-byte direct loads of ROWS x D into the tile at LDS byte offset `lds`: rows
 // row0.. of a tensor whose rows are `stride` bytes apart, clamped to the last of `left`
-// remaining rows (callers mask what lies beyond). The loads are asm because the
-// compiler would wait for every load in flight before any LDS read; they write no
-// register. `wait_loads` and a barrier come before the tile is read.
+// remaining rows and to the first `chunks` 16-byte pieces of a row (callers mask what lies
+// beyond). The loads are asm because the compiler would wait for every load in flight
+// before any LDS read; they write no register. `wait_loads` and a barrier come before the
+// tile is read.
 template <int D, int ROWS, int WAVES>
-__device__ __forceinline__ void load_tile(const void* base, unsigned stride, int left, unsigned lds) {
+constexpr int tile_loads() { return ROWS * row_bytes(D) / 1024 / WAVES; }   // per wave
+
+template <int D, int ROWS, int WAVES>
+__device__ __forceinline__ void load_tile(const void* base, unsigned stride, int left, unsigned lds,
+                                          int chunks = D / 8) {
   constexpr int RB = row_bytes(D), PER = 1024 / RB;     // rows of one wave's load
   constexpr int N = ROWS * RB / 1024;
   static_assert(N % WAVES == 0, "every wave issues the same number of loads");
@@ -73,7 +78,7 @@ __device__ __forceinline__ void load_tile(const void* base, unsigned stride, int
     const int j = i * WAVES + wid;
     const int row = j * PER + lane / (RB / 16);
     int chunk = slot ^ swz<D>(row);
-    if (D * 2 < RB && chunk >= D / 8) chunk = 0;        // padding columns: any valid address
+    if (chunk >= chunks) chunk = 0;                     // any valid address
     const unsigned off = (unsigned)min(row, left - 1) * stride + chunk * 16;
     const unsigned to = lds + j * 1024;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -81,7 +86,11 @@ __device__ __forceinline__ void load_tile(const void* base, unsigned stride, int
   }
 }
 
-__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// waits until at most LATER of the wave's loads, the last ones issued, are in flight
+template <int LATER = 0>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(LATER) : "memory");
+}
 
 // barrier behind which every wave's LDS reads so far are complete
 __device__ __forceinline__ void barrier() {
@@ -121,6 +130,25 @@ __device__ __forceinline__ bf16x8_t read_cols(const char* smem, unsigned tile, u
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
+// the same with rows 16 c + 8 half + 0..7, the order of read_rows' columns, for products of
+// a row-read with a column-read tile
+template <int D>
+__device__ __forceinline__ unsigned cols_base_natural() {
+  const int lane = threadIdx.x & 63, i = lane & 15, half = lane >> 5;
+  const int row = 8 * half + (i >> 2), slot = ((lane >> 4) & 1) * 2 + ((i & 3) >> 1);
+  return row * row_bytes(D) + ((slot ^ swz<D>(row)) << 4) + (i & 1) * 8;
+}
+template <int D>
+__device__ __forceinline__ bf16x8_t read_cols_natural(const char* smem, unsigned tile, unsigned base,
+                                                      int c, int t) {
+  typedef __attribute__((address_space(3))) bf16x4_t* lds_ptr;
+  const char* p = smem + tile + (base ^ (t << 6)) + c * 16 * row_bytes(D);
+  const char* p4 = smem + tile + (base ^ (t << 6) ^ 16) + (c * 16 + 4) * row_bytes(D);
+  const bf16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_ptr)p);
+  const bf16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_ptr)p4);
+  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
 // registers 8 c .. 8 c + 7 of an accumulator as the operand of the next product
 __device__ __forceinline__ bf16x8_t pack8(const f32x16_t& p, int c) {
   bf16x8_t out;
@@ -141,6 +169,33 @@ __device__ __forceinline__ float max_halves(float x) {
 __device__ __forceinline__ float sum_halves(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// a wave's transposed accumulators [D / 32] (column = row of the result), scaled, through
+// 32 rows of LDS of its own to whole-row stores of bf16: the first `rows` rows and `chunks`
+// 16-byte pieces of a row
+template <int D>
+__device__ __forceinline__ void store_rows(const f32x16_t (&acc)[D / 32], float scale, char* mine,
+                                           bf16* dst, long row_stride, int rows, int chunks = D / 8) {
+  constexpr int RB = row_bytes(D), CH = D / 8, PER = 64 / CH;
+  const int lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
+#pragma unroll
+  for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      bf16x4_t w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = (__bf16)(acc[t][4 * g + j] * scale);
+      *reinterpret_cast<bf16x4_t*>(mine + col * RB + (((t * 4 + g) ^ swz<D>(col)) << 4) + half * 8) = w;
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // a wave reads what it wrote itself
+  if (lane < PER * CH) {
+    const int ch = lane % CH;
+    for (int r = lane / CH; r < 32 && r < rows && ch < chunks; r += PER)
+      *reinterpret_cast<uint4*>(dst + (long)r * row_stride + ch * 8) =
+          *reinterpret_cast<const uint4*>(mine + r * RB + ((ch ^ swz<D>(r)) << 4));
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
 // Block -> (tile, head, batch). Consecutive blocks go to the 8 XCDs in turn; the

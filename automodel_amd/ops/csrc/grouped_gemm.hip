@@ -1,0 +1,315 @@
+// Grouped GEMM for stacked expert weights (CDNA4, bf16, f32 accumulation): rows of x are
+// sorted by expert, expert e owns rows offs[e] .. offs[e+1].
+//
+//   nt (forward)  y[m, n]  = sum_k x[m, k] w[e(m), n, k]
+//   nn (dx)      dx[m, k]  = sum_n g[m, n] w[e(m), n, k]
+//   tn (dw)   dw[e, n, k]  = sum_{m of e} g[m, n] x[m, k]
+//
+// One kernel for the three: 8 waves compute BM x 256 of the output, 64 x 64 or 64 x 128
+// each, over steps of 64 of the summed index. What differs is which index of an
+// operand is contiguous: tiles whose rows are output rows or columns are read by rows,
+// tiles whose rows are the summed index by columns, with the transposing LDS reads
+// (flash_tile.h). So dw takes g and x as they are, and dx takes w as it is.
+//
+// Direct loads fill three LDS buffers two steps ahead (256 x 256: two, one ahead, which is
+// what fits), one barrier a step. Blocks are dealt to the 8 XCDs in contiguous stretches of
+// the tile list, column tiles of one row tile next to each other: an expert's weights and a
+// row tile stay in one L2.
+//
+// Bound by LDS (at full MFMA rate 64 x 128 wave tiles read and load 128 B/clk, 64 x 64 ones
+// more: 256 x 256 is the faster tile) against padding of the groups' last row tiles: nt and
+// nn take 256 rows from 512 rows per expert on (the caller's plan: 128 experts x 512 rows: 328 against
+// 334 us; 64 x 281: 192 against 179), tn, whose tiles have no padding, always. 4 waves of
+// 64 x 128, one a SIMD, wait for LDS more than they save (128 x 256: 374 against 345 us).
+// Measured, nt / nn / tn, before (tn with its transposes) -> now: 65536 rows, 128 experts,
+// 768 x 2048: 515 / 607 / 742 -> 328 / 331 / 311 us; 2048 x 768: 502 / 691 / 757 -> 300 / 287 /
+// 287 us; 18018 rows, 64 experts, 1408 x 2048: 284 / 369 / 403 -> 179 / 168 / 197 us; 16384 rows,
+// 8 experts, 4096 x 2048: 495 / 779 / 639 -> 296 / 329 / 269 us (929 / 834 / 1022 TFLOP/s).
+
+#include <torch/library.h>
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+
+#include "common.h"
+#include "flash_tile.h"
+#include "ops_api.h"
+
+namespace amd_ops {
+
+using namespace fa;
+
+namespace {
+
+enum Mode { NT, NN, TN };
+constexpr int STEP = 64;               // of the summed index
+
+struct GroupedArgs {
+  const bf16 *r, *c;                   // operands of the output's rows and columns
+  bf16* out;
+  const int *tile_map, *offs, *n_tiles;
+  int n_mtiles, N, K, E;               // tile_map's capacity; w is [E, N, K]
+};
+
+}  // namespace
+
+template <Mode MODE, int BM, int BN, int WAVES, int BUFS>
+__global__ __launch_bounds__(64 * WAVES, 1) void grouped_gemm_kernel(const GroupedArgs a) {
+  constexpr int WR = BM / 64, WC = WAVES / WR, WN = BN / WC;    // waves down, across; columns of one
+  constexpr bool RC = MODE == TN, CC = MODE != NT;              // operand read by columns
+  // tiles: [BM][STEP] or, read by columns, [STEP][BM]
+  constexpr int RT = RC ? STEP * row_bytes(BM) : BM * row_bytes(STEP);
+  constexpr int CT = CC ? STEP * row_bytes(BN) : BN * row_bytes(STEP);
+  constexpr int BUF = RT + CT, LOADS = BUF / 1024 / WAVES;
+  static_assert(BM % 64 == 0 && WAVES % WR == 0 && (WN == 64 || WN == 128), "wave tiles");
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+
+  // ---- tile of the block
+  const int rows_out = MODE == TN ? a.N : 0, cols_out = MODE == NT ? a.N : a.K;
+  const int nr = (rows_out + BM - 1) / BM, nc = (cols_out + BN - 1) / BN;
+  const int total = MODE == TN ? a.E * nr * nc : (a.n_tiles ? a.n_tiles[0] : a.n_mtiles) * nc;
+  const int per = (total + 7) / 8, slot = blockIdx.x >> 3, id = (blockIdx.x & 7) * per + slot;
+  if (slot >= per || id >= total) return;
+  int e, r0, c0, sum, r_left;          // expert; first row, column; length of the sum; rows left
+  const bf16 *rp, *cp;                 // first element of either operand
+  if constexpr (MODE == TN) {
+    e = id / (nr * nc);
+    r0 = id / nc % nr * BM;
+    c0 = id % nc * BN;
+    const int m0 = a.offs[e];
+    sum = a.offs[e + 1] - m0;
+    r_left = a.N - r0;
+    rp = a.r + (long)m0 * a.N + r0;
+    cp = a.c + (long)m0 * a.K + c0;
+  } else {
+    const int t = id / nc;
+    e = a.tile_map[2 * t];
+    r0 = a.tile_map[2 * t + 1];
+    c0 = id % nc * BN;
+    sum = MODE == NT ? a.K : a.N;
+    r_left = a.offs[e + 1] - r0;
+    rp = a.r + (long)r0 * sum;
+    cp = a.c + (long)e * a.N * a.K + (MODE == NT ? (long)c0 * a.K : c0);
+  }
+  const int c_left = cols_out - c0;
+  const unsigned r_rs = (MODE == TN ? a.N : sum) * 2, c_rs = a.K * 2;
+
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wid / WC, wc = wid % WC;
+
+  auto load = [&](int s, unsigned buf) {
+    const int left = sum - s * STEP;   // of the summed index (a multiple of STEP but for tn)
+    if constexpr (RC) load_tile<BM, STEP, WAVES>(rp + (long)s * STEP * a.N, r_rs, left, buf, r_left / 8);
+    else load_tile<STEP, BM, WAVES>(rp + s * STEP, r_rs, r_left, buf);
+    if constexpr (CC) load_tile<BN, STEP, WAVES>(cp + (long)s * STEP * a.K, c_rs, left, buf + RT, c_left / 8);
+    else load_tile<STEP, BN, WAVES>(cp + s * STEP, c_rs, c_left, buf + RT);
+  };
+  const unsigned rrow = rows_base<STEP>(), crow = rows_base<STEP>();
+  const unsigned rcol = cols_base_natural<BM>(), ccol = cols_base_natural<BN>();
+
+  f32x16_t acc[2][WN / 32];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < WN / 32; ++j) acc[i][j] = zero16();
+
+  const int steps = (sum + STEP - 1) / STEP;
+  unsigned cur = 0, next = BUF, after = 2 * BUF;
+  if (steps > 0) load(0, cur);
+  if (BUFS == 3 && steps > 1) load(1, next);
+  for (int s = 0; s < steps; ++s) {
+    if (BUFS == 3 && s + 1 < steps) wait_loads<LOADS>();
+    else wait_loads();
+    barrier();                         // the step's tiles are there; those of s - 1 are done with
+    if (s + BUFS - 1 < steps) load(s + BUFS - 1, BUFS == 3 ? after : next);
+    if constexpr (MODE == TN) {
+      // rows of the next expert, or beyond the end: clamped by the load, zeroed here
+      const int left = sum - s * STEP;
+      if (left < STEP) {
+        for (int i = threadIdx.x; i < (STEP - left) * (row_bytes(BM) / 16); i += 64 * WAVES)
+          *reinterpret_cast<uint4*>(smem + cur + left * row_bytes(BM) + i * 16) = uint4{0, 0, 0, 0};
+        barrier();
+      }
+    }
+#pragma unroll
+    for (int ch = 0; ch < STEP / 16; ++ch) {
+      bf16x8_t rf[2], cf[WN / 32];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        rf[i] = RC ? read_cols_natural<BM>(smem, cur, rcol, ch, wr * 2 + i)
+                   : read_rows<STEP>(smem, cur + wr * 64 * row_bytes(STEP), rrow, i, ch);
+#pragma unroll
+      for (int j = 0; j < WN / 32; ++j)
+        cf[j] = CC ? read_cols_natural<BN>(smem, cur + RT, ccol, ch, wc * (WN / 32) + j)
+                   : read_rows<STEP>(smem, cur + RT + wc * WN * row_bytes(STEP), crow, j, ch);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < WN / 32; ++j) acc[i][j] = mma(cf[j], rf[i], acc[i][j]);
+    }
+    const unsigned t = cur;
+    cur = next;
+    next = BUFS == 3 ? after : t;
+    after = t;
+  }
+  barrier();                           // the buffers are the waves' output tiles now
+
+  char* mine = smem + wid * 32 * row_bytes(WN);
+  const int cw = c0 + wc * WN, cols = min(cols_out - cw, WN);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int rw = wr * 64 + i * 32;   // row of the block's tile
+    const long row = MODE == TN ? (long)e * a.N + r0 + rw : r0 + rw;
+    if (cols > 0)
+      store_rows<WN>(acc[i], 1.f, mine, a.out + row * cols_out + cw, cols_out, r_left - rw, cols / 8);
+  }
+}
+
+// Offsets and (expert, first row) tiles of the groups, from counts on the device, so that
+// routing never waits for the host. One workgroup: thread t sums a stretch of experts, a
+// scan over the threads gives every stretch its first row and tile. (A single thread took
+// 26 us for 128 experts, now 11 with the launch.)
+__global__ __launch_bounds__(256) void build_group_plan_kernel(const int* __restrict__ counts, int E,
+                                                               int* __restrict__ offs,
+                                                               int* __restrict__ tile_map,
+                                                               int* __restrict__ n_tiles, int bm,
+                                                               int capacity) {
+  __shared__ int rows[256], tiles[256];
+  const int t = threadIdx.x, per = (E + 255) / 256, e0 = min(t * per, E), e1 = min(e0 + per, E);
+  int r = 0, n = 0;
+  for (int e = e0; e < e1; ++e) {
+    r += counts[e];
+    n += (counts[e] + bm - 1) / bm;
+  }
+  rows[t] = r;
+  tiles[t] = n;
+  __syncthreads();
+  for (int off = 1; off < 256; off <<= 1) {
+    const int rr = t >= off ? rows[t - off] : 0, nn = t >= off ? tiles[t - off] : 0;
+    __syncthreads();
+    rows[t] += rr;
+    tiles[t] += nn;
+    __syncthreads();
+  }
+  if (t == 255) n_tiles[0] = min(tiles[255], capacity);
+  if (t == 0) offs[0] = 0;
+  r = rows[t] - r;
+  n = tiles[t] - n;
+  for (int e = e0; e < e1; ++e) {
+    for (int m = 0; m < counts[e]; m += bm, ++n)
+      if (n < capacity) {
+        tile_map[2 * n] = e;
+        tile_map[2 * n + 1] = r + m;
+      }
+    r += counts[e];
+    offs[e + 1] = r;
+  }
+}
+
+std::tuple<at::Tensor, at::Tensor, at::Tensor> build_group_plan(
+    const at::Tensor& counts, int64_t M, int64_t bm) {
+  TORCH_CHECK(counts.is_cuda() && counts.scalar_type() == at::kInt,
+              "build_group_plan: counts int32 on GPU");
+  const int E = counts.size(0);
+  const long max_tiles = M / bm + E + 1;
+  auto opts = counts.options();
+  auto offs = at::empty({E + 1}, opts);
+  auto tile_map = at::empty({max_tiles, 2}, opts);
+  auto n_tiles = at::empty({1}, opts);
+  auto stream = c10::hip::getCurrentHIPStream();
+  hipLaunchKernelGGL(build_group_plan_kernel, dim3(1), dim3(256), 0, stream.stream(),
+                     counts.data_ptr<int>(), E, offs.data_ptr<int>(),
+                     tile_map.data_ptr<int>(), n_tiles.data_ptr<int>(), (int)bm, (int)max_tiles);
+  HIP_CHECK_KERNEL();
+  return {offs, tile_map, n_tiles};
+}
+
+namespace {
+
+template <Mode MODE, int BM, int BN, int WAVES, int BUFS>
+void launch(const GroupedArgs& a) {
+  constexpr int rt = MODE == TN ? STEP * row_bytes(BM) : BM * row_bytes(STEP);
+  constexpr int ct = MODE != NT ? STEP * row_bytes(BN) : BN * row_bytes(STEP);
+  constexpr int wn = BN * BM / 64 / WAVES;
+  constexpr int smem = std::max(BUFS * (rt + ct), WAVES * 32 * row_bytes(wn));
+  const int nc = ((MODE == NT ? a.N : a.K) + BN - 1) / BN;
+  const long tiles = MODE == TN ? (long)a.E * ((a.N + BM - 1) / BM) * nc : (long)a.n_mtiles * nc;
+  TORCH_CHECK(tiles < (1l << 31) - 8, "grouped_gemm: too many tiles");
+  // the stretches of the 8 XCDs are rounded up: up to 7 workgroups beyond the tiles
+  hipLaunchKernelGGL((grouped_gemm_kernel<MODE, BM, BN, WAVES, BUFS>), dim3((unsigned)((tiles + 7) / 8 * 8)),
+                     dim3(64 * WAVES), smem, c10::hip::getCurrentHIPStream().stream(), a);
+  HIP_CHECK_KERNEL();
+}
+
+GroupedArgs grouped_args(const at::Tensor& r, const at::Tensor& c, at::Tensor& out,
+                         const at::Tensor& offs) {
+  TORCH_CHECK(r.is_cuda() && r.is_contiguous() && c.is_contiguous() && r.scalar_type() == at::kBFloat16 &&
+                  c.scalar_type() == at::kBFloat16, "grouped_gemm: contiguous bf16 operands");
+  TORCH_CHECK(offs.scalar_type() == at::kInt && offs.is_contiguous(), "grouped_gemm: offs int32");
+  GroupedArgs a{};
+  a.r = reinterpret_cast<const bf16*>(r.data_ptr());
+  a.c = reinterpret_cast<const bf16*>(c.data_ptr());
+  a.out = reinterpret_cast<bf16*>(out.data_ptr());
+  a.offs = offs.data_ptr<int>();
+  return a;
+}
+
+void set_tiles(GroupedArgs& a, const at::Tensor& w, const at::Tensor& offs, const at::Tensor& tile_map,
+               const std::optional<at::Tensor>& n_tiles) {
+  TORCH_CHECK(tile_map.scalar_type() == at::kInt && tile_map.is_contiguous(), "tile_map int32 [n, 2]");
+  TORCH_CHECK(offs.numel() == w.size(0) + 1, "offs [E + 1]");
+  a.tile_map = tile_map.data_ptr<int>();
+  a.n_tiles = n_tiles.has_value() ? n_tiles->data_ptr<int>() : nullptr;
+  a.n_mtiles = tile_map.size(0);
+  a.E = w.size(0);
+  a.N = w.size(1);
+  a.K = w.size(2);
+}
+
+}  // namespace
+
+at::Tensor grouped_gemm_nt(const at::Tensor& x, const at::Tensor& w,
+                           const at::Tensor& offs, const at::Tensor& tile_map,
+                           const std::optional<at::Tensor>& n_tiles, int64_t bm) {
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 3 && x.size(1) == w.size(2), "grouped_gemm_nt: x [M,K], w [E,N,K]");
+  TORCH_CHECK(w.size(2) % STEP == 0 && w.size(1) % 128 == 0, "need K%64==0, N%128==0");
+  TORCH_CHECK(bm == 128 || bm == 256, "grouped_gemm_nt: tiles of 128 or 256 rows");
+  auto y = at::empty({x.size(0), w.size(1)}, x.options());
+  if (tile_map.size(0) == 0 || x.size(0) == 0) return y;
+  auto a = grouped_args(x, w, y, offs);
+  set_tiles(a, w, offs, tile_map, n_tiles);
+  if (bm == 256) launch<NT, 256, 256, 8, 2>(a);
+  else launch<NT, 128, 256, 8, 3>(a);
+  return y;
+}
+
+at::Tensor grouped_gemm_nn(const at::Tensor& g, const at::Tensor& w,
+                           const at::Tensor& offs, const at::Tensor& tile_map,
+                           const std::optional<at::Tensor>& n_tiles, int64_t bm) {
+  TORCH_CHECK(g.dim() == 2 && w.dim() == 3 && g.size(1) == w.size(1), "grouped_gemm_nn: g [M,N], w [E,N,K]");
+  TORCH_CHECK(bm == 128 || bm == 256, "grouped_gemm_nn: tiles of 128 or 256 rows");
+  TORCH_CHECK(w.size(1) % STEP == 0 && w.size(2) % 128 == 0, "need N%64==0, K%128==0");
+  auto dx = at::empty({g.size(0), w.size(2)}, g.options());
+  if (tile_map.size(0) == 0 || g.size(0) == 0) return dx;
+  auto a = grouped_args(g, w, dx, offs);
+  set_tiles(a, w, offs, tile_map, n_tiles);
+  if (bm == 256) launch<NN, 256, 256, 8, 2>(a);
+  else launch<NN, 128, 256, 8, 3>(a);
+  return dx;
+}
+
+at::Tensor grouped_gemm_tn(const at::Tensor& g, const at::Tensor& x, const at::Tensor& offs, int64_t E) {
+  TORCH_CHECK(g.dim() == 2 && x.dim() == 2 && g.size(0) == x.size(0) && offs.numel() == E + 1,
+              "grouped_gemm_tn: g [M,N], x [M,K], offs [E+1]");
+  TORCH_CHECK(g.size(1) % 128 == 0 && x.size(1) % 128 == 0, "need N%128==0, K%128==0");
+  auto dw = at::empty({E, g.size(1), x.size(1)}, g.options());
+  if (dw.numel() == 0) return dw;
+  auto a = grouped_args(g, x, dw, offs);
+  a.E = E;
+  a.N = g.size(1);
+  a.K = x.size(1);
+  launch<TN, 256, 256, 8, 2>(a);
+  return dw;
+}
+
+}  // namespace amd_ops

@@ -2,7 +2,7 @@
 
 ``grouped_linear(x_perm, w, counts)`` computes y[rows of group e] =
 x[rows] @ w[e].T with autograd. Forward runs the in-tree CDNA4 kernel
-(csrc/moe_kernels.hip grouped_gemm_nt); backward runs the single-kernel
+(csrc/grouped_gemm.hip grouped_gemm_nt); backward runs the single-kernel
 grouped dx (NN) and dw (TN) kernels — no per-expert loop, no atomics.
 
 With ``counts`` as a DEVICE int tensor the (offs, tile_map, n_tiles) plan is
@@ -41,6 +41,13 @@ def make_group_plan(counts: torch.Tensor, M: int, bm: int = 128):
     return hip_ops().build_group_plan(counts.to(torch.int32), M, bm)
 
 
+def tile_rows(rows: int, experts: int) -> int:
+    """Row tile of the bf16 kernels: 256 is the faster tile, but the last one of
+    every group is padding for half of it on average (measured in
+    csrc/grouped_gemm.hip)."""
+    return 256 if rows >= 512 * experts else 128
+
+
 def _loop_gemm_nt(x, w, counts):
     outs, start = [], 0
     for e, n in enumerate(counts):
@@ -76,20 +83,8 @@ class _GroupedLinear(torch.autograd.Function):
         # kernel needs N%128 and K%128
         if ctx.use_hip and w.shape[1] % 128 == 0 and w.shape[2] % 128 == 0:
             ops = hip_ops()
-            if ctx.bm != 128:
-                # nn rides 128-row tiles; rebuild its plan on device (cheap)
-                if torch.is_tensor(ctx.counts) and ctx.counts.is_cuda:
-                    offs, tile_map, n_tiles = make_group_plan(ctx.counts, g.shape[0], 128)
-                else:
-                    cl = list(ctx.counts)
-                    tile_map, offs = _build_tile_map([int(c) for c in cl])
-                    tile_map, offs, n_tiles = tile_map.to(g.device), offs.to(g.device), None
-            dx = ops.grouped_gemm_nn(g, w.contiguous(), offs, tile_map, n_tiles)
-            # TN operands pre-transposed (m contiguous) by the tiled HIP
-            # transpose — torch's strided transpose measured 6x off roofline
-            dw = ops.grouped_gemm_tn(ops.transpose_bf16(g),
-                                     ops.transpose_bf16(x.contiguous()),
-                                     offs, w.shape[0])
+            dx = ops.grouped_gemm_nn(g, w.contiguous(), offs, tile_map, n_tiles, ctx.bm)
+            dw = ops.grouped_gemm_tn(g, x.contiguous(), offs, w.shape[0])
             return dx, dw, None, None, None, None, None
         cl = ctx.counts.tolist() if torch.is_tensor(ctx.counts) else list(ctx.counts)
         dx = torch.empty_like(x)
@@ -118,21 +113,17 @@ def grouped_linear(x_perm: torch.Tensor, w: torch.Tensor, counts,
         # caller-provided plan carries its tile height: (offs, tm, nt, bm)
         offs, tile_map, n_tiles, bm = plan
         return _GroupedLinear.apply(x_perm, w, counts, offs, tile_map, n_tiles, bm)
-    # 256x256 big-tile forward when the output width allows (+27% measured,
-    # benchmarks/gg_micro.py)
-    bm = 256 if (hip_eligible and w.shape[1] % 256 == 0
-                 and torch.is_tensor(counts) and counts.is_cuda) else 128
+    bm = 128
     if hip_eligible:
         if torch.is_tensor(counts) and counts.is_cuda:
+            bm = tile_rows(x_perm.shape[0], w.shape[0])
             offs, tile_map, n_tiles = make_group_plan(counts, x_perm.shape[0], bm)
         else:
             cl = counts.tolist() if torch.is_tensor(counts) else list(counts)
             tile_map, offs = _build_tile_map([int(c) for c in cl])
             tile_map, offs, n_tiles = tile_map.to(x_perm.device), offs.to(x_perm.device), None
-            bm = 128
     else:
         offs = tile_map = n_tiles = None
-        bm = 128
     return _GroupedLinear.apply(x_perm, w, counts, offs, tile_map, n_tiles, bm)
 
 

@@ -14,7 +14,6 @@ x = torch.randn(M, H, device="cuda", dtype=torch.bfloat16)
 g = torch.randn(M, I, device="cuda", dtype=torch.bfloat16)
 w = torch.randn(E, I, H, device="cuda", dtype=torch.bfloat16) * 0.02
 offs, tm, ntl = make_group_plan(counts, M)
-gt, xt = g.t().contiguous(), x.t().contiguous()
 
 def timeit(name, fn, flops, iters=10):
     for _ in range(3): fn()
@@ -34,11 +33,7 @@ y_big = ops.grouped_gemm_nt(x, w3, offs_b, tm_b, ntl_b, 256)
 y_ref = ops.grouped_gemm_nt(x, w3, offs, tm, ntl)
 print("big-vs-128 maxdiff:", float((y_big.float()-y_ref.float()).abs().max()))
 timeit("nn  (dx=g@w)", lambda: ops.grouped_gemm_nn(g, w, offs, tm, ntl), fl)
-timeit("tn  (dw=gTx)", lambda: ops.grouped_gemm_tn(gt, xt, offs, E), fl)
-timeit("tn+torch-transpose", lambda: ops.grouped_gemm_tn(g.t().contiguous(), x.t().contiguous(), offs, E), fl)
-timeit("tn+hip-transpose", lambda: ops.grouped_gemm_tn(ops.transpose_bf16(g), ops.transpose_bf16(x), offs, E), fl)
-xtr = ops.transpose_bf16(x)
-assert torch.equal(xtr, x.t().contiguous()), "transpose mismatch"
+timeit("tn  (dw=gTx)", lambda: ops.grouped_gemm_tn(g, x, offs, E), fl)
 # hipBLASLt ceiling: one dense GEMM of the same FLOPs
 xb = torch.randn(M, H, device="cuda", dtype=torch.bfloat16)
 wb = torch.randn(I, H, device="cuda", dtype=torch.bfloat16)
