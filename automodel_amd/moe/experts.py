@@ -51,49 +51,53 @@ class _FusedPermuteGather(torch.autograd.Function):
         return dx, None, None, None
 
 
+_ROUTE_MAX_EXPERTS = 4096       # csrc/moe_kernels.hip
+
+
 def fused_dispatch_combine(x, probs, indices, n_experts, expert_fn):
-    """GPU MoE glue: argsort routing, HIP gather, expert_fn over permuted
+    """GPU MoE glue: device-side routing plan, HIP gather, expert_fn over permuted
     rows, HIP combine — one gather + one combine instead of
     repeat_interleave + fancy-index + scatter (reference fused permute/
-    unpermute, moe_utils.py:31/115)."""
+    unpermute, moe_utils.py:31/115). Nothing waits for the host."""
+    from automodel_amd.ops._backend import hip_ops
+
     T, K = indices.shape
-    flat = indices.reshape(-1)
-    sort_idx = flat.argsort(stable=True)
-    counts = torch.bincount(flat, minlength=n_experts).to(torch.int32)
-    src = (sort_idx // K).to(torch.int32)
-    inv = torch.empty_like(sort_idx)
-    inv[sort_idx] = torch.arange(T * K, device=x.device)
-    pos = inv.to(torch.int32).view(T, K)
-    perm_probs = probs.reshape(-1).float()[sort_idx]     # prob per perm slot
+    with torch.no_grad():
+        probs32 = probs.detach().float().contiguous()
+        if n_experts <= _ROUTE_MAX_EXPERTS:
+            counts, order, src, pos, perm_probs = hip_ops().route_plan(
+                indices.long().contiguous(), probs32, n_experts)
+        else:
+            order = indices.reshape(-1).argsort(stable=True)
+            counts = torch.bincount(indices.reshape(-1), minlength=n_experts).to(torch.int32)
+            src = (order // K).to(torch.int32)
+            pos = torch.empty_like(order)
+            pos[order] = torch.arange(T * K, device=x.device)
+            pos, order = pos.to(torch.int32).view(T, K), order.to(torch.int32)
+            perm_probs = probs32.reshape(-1)[order]
     x_perm = _FusedPermuteGather.apply(x, src, pos, K)
     y_perm = expert_fn(x_perm, counts)
-    # combine with prob routing; dprobs via scatter of per-slot dots
-    return _CombineWithProbs.apply(y_perm, pos, probs, src, perm_probs, sort_idx)
+    return _CombineWithProbs.apply(y_perm, pos, probs, src, perm_probs, order)
 
 
 class _CombineWithProbs(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, y_perm, pos, probs, src, perm_probs, sort_idx):
+    def forward(ctx, y_perm, pos, probs, src, perm_probs, order):
         from automodel_amd.ops._backend import hip_ops
 
-        out = hip_ops().unpermute_combine(y_perm.contiguous(), pos,
-                                          probs.float().contiguous())
-        ctx.save_for_backward(y_perm, src, perm_probs, sort_idx)
-        ctx.shape_tk = probs.shape
+        y_perm = y_perm.contiguous()
+        out = hip_ops().unpermute_combine(y_perm, pos, probs.float().contiguous())
+        ctx.save_for_backward(y_perm, src, perm_probs, order)
+        ctx.probs_shape, ctx.probs_dtype = probs.shape, probs.dtype
         return out
 
     @staticmethod
     def backward(ctx, g):
         from automodel_amd.ops._backend import hip_ops
 
-        y_perm, src, perm_probs, sort_idx = ctx.saved_tensors
-        g = g.contiguous()
-        g_gath = hip_ops().permute_gather(g, src)       # [T*K, H] perm order
-        dy = (g_gath.float() * perm_probs.unsqueeze(1)).to(y_perm.dtype)
-        s = (g_gath.float() * y_perm.float()).sum(-1)   # [T*K] perm order
-        dprobs = torch.empty_like(s)
-        dprobs.scatter_(0, sort_idx, s)
-        return dy, None, dprobs.view(ctx.shape_tk).to(torch.float32), None, None, None
+        y_perm, src, perm_probs, order = ctx.saved_tensors
+        dy, dprobs = hip_ops().combine_bwd(g.contiguous(), y_perm, src, order, perm_probs)
+        return dy, None, dprobs.view(ctx.probs_shape).to(ctx.probs_dtype), None, None, None
 
 
 def unpermute_tokens(y_perm: torch.Tensor, sort_idx: torch.Tensor,
@@ -173,7 +177,12 @@ class GroupedExperts(nn.Module):
             and x_perm.numel() > 0
         )
         if use_grouped:
-            from automodel_amd.ops.grouped_gemm import grouped_linear, make_group_plan, tile_rows
+            from automodel_amd.ops.grouped_gemm import (
+                grouped_linear,
+                grouped_linear_pair,
+                make_group_plan,
+                tile_rows,
+            )
 
             if torch.is_tensor(counts) and counts.is_cuda:
                 # device-side plan shared by all three projections — the
@@ -216,8 +225,11 @@ class GroupedExperts(nn.Module):
                                        st["up"], x8, sx)
                 h = swiglu(g, u)
                 return grouped_linear_fp8(h, self.down_proj, cl, plan, st["down"])
-            g = grouped_linear(x_perm, self.gate_proj, cl, plan=plan)
-            u = grouped_linear(x_perm, self.up_proj, cl, plan=plan)
+            if plan is not None:
+                g, u = grouped_linear_pair(x_perm, self.gate_proj, self.up_proj, cl, plan)
+            else:
+                g = grouped_linear(x_perm, self.gate_proj, cl)
+                u = grouped_linear(x_perm, self.up_proj, cl)
             h = swiglu(g, u)
             return grouped_linear(h, self.down_proj, cl, plan=plan)
         return self._expert_mlp_loop(x_perm, counts)

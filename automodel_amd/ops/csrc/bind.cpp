@@ -80,6 +80,14 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("grouped_gemm_tn", &amd_ops::grouped_gemm_tn);
   m.def("grouped_gemm_nt_fp8(Tensor x8, Tensor w8, Tensor offs, Tensor tile_map, Tensor scale, Tensor? n_tiles=None, int bm=128) -> Tensor");
   m.impl("grouped_gemm_nt_fp8", &amd_ops::grouped_gemm_nt_fp8);
+  m.def("route_plan(Tensor indices, Tensor probs, int E) -> (Tensor, Tensor, Tensor, Tensor, Tensor)");
+  m.impl("route_plan", &amd_ops::route_plan);
+  m.def("combine_bwd(Tensor g, Tensor y, Tensor src, Tensor order, Tensor probs) -> (Tensor, Tensor)");
+  m.impl("combine_bwd", &amd_ops::combine_bwd);
+  m.def(
+      "grouped_gemm_nn2(Tensor g1, Tensor w1, Tensor g2, Tensor w2, Tensor offs, Tensor tile_map, "
+      "Tensor? n_tiles=None, int bm=128) -> Tensor");
+  m.impl("grouped_gemm_nn2", &amd_ops::grouped_gemm_nn2);
   m.def("permute_gather(Tensor x, Tensor src) -> Tensor");
   m.impl("permute_gather", &amd_ops::permute_gather);
   m.def("unpermute_combine(Tensor yp, Tensor pos, Tensor probs) -> Tensor");

@@ -2,7 +2,8 @@
 // sorted by expert, expert e owns rows offs[e] .. offs[e+1].
 //
 //   nt (forward)  y[m, n]  = sum_k x[m, k] w[e(m), n, k]
-//   nn (dx)      dx[m, k]  = sum_n g[m, n] w[e(m), n, k]
+//   nn (dx)      dx[m, k]  = sum_n g[m, n] w[e(m), n, k], optionally over two pairs of g and
+//                w (gate and up): one sum in the accumulators instead of an addition after
 //   tn (dw)   dw[e, n, k]  = sum_{m of e} g[m, n] x[m, k]
 //
 // One kernel for the three: 8 waves compute BM x 256 of the output, 64 x 64 or 64 x 128
@@ -45,6 +46,7 @@ constexpr int STEP = 64;               // of the summed index
 
 struct GroupedArgs {
   const bf16 *r, *c;                   // operands of the output's rows and columns
+  const bf16 *r2, *c2;                 // nn: a second pair, added to the sum
   bf16* out;
   const int *tile_map, *offs, *n_tiles;
   int n_mtiles, N, K, E;               // tile_map's capacity; w is [E, N, K]
@@ -70,7 +72,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void grouped_gemm_kernel(const Group
   const int per = (total + 7) / 8, slot = blockIdx.x >> 3, id = (blockIdx.x & 7) * per + slot;
   if (slot >= per || id >= total) return;
   int e, r0, c0, sum, r_left;          // expert; first row, column; length of the sum; rows left
-  const bf16 *rp, *cp;                 // first element of either operand
+  const bf16 *rp, *cp, *rp2 = nullptr, *cp2 = nullptr;          // first element of either operand
   if constexpr (MODE == TN) {
     e = id / (nr * nc);
     r0 = id / nc % nr * BM;
@@ -89,6 +91,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void grouped_gemm_kernel(const Group
     r_left = a.offs[e + 1] - r0;
     rp = a.r + (long)r0 * sum;
     cp = a.c + (long)e * a.N * a.K + (MODE == NT ? (long)c0 * a.K : c0);
+    if (MODE == NN && a.r2) {
+      rp2 = a.r2 + (long)r0 * sum;
+      cp2 = a.c2 + (long)e * a.N * a.K + c0;
+    }
   }
   const int c_left = cols_out - c0;
   const unsigned r_rs = (MODE == TN ? a.N : sum) * 2, c_rs = a.K * 2;
@@ -97,12 +103,19 @@ __global__ __launch_bounds__(64 * WAVES, 1) void grouped_gemm_kernel(const Group
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wid / WC, wc = wid % WC;
 
+  const int once = (sum + STEP - 1) / STEP, steps = MODE == NN && rp2 ? 2 * once : once;
   auto load = [&](int s, unsigned buf) {
+    const bf16 *r = rp, *c = cp;
+    if (MODE == NN && s >= once) {
+      r = rp2;
+      c = cp2;
+      s -= once;
+    }
     const int left = sum - s * STEP;   // of the summed index (a multiple of STEP but for tn)
-    if constexpr (RC) load_tile<BM, STEP, WAVES>(rp + (long)s * STEP * a.N, r_rs, left, buf, r_left / 8);
-    else load_tile<STEP, BM, WAVES>(rp + s * STEP, r_rs, r_left, buf);
-    if constexpr (CC) load_tile<BN, STEP, WAVES>(cp + (long)s * STEP * a.K, c_rs, left, buf + RT, c_left / 8);
-    else load_tile<STEP, BN, WAVES>(cp + s * STEP, c_rs, c_left, buf + RT);
+    if constexpr (RC) load_tile<BM, STEP, WAVES>(r + (long)s * STEP * a.N, r_rs, left, buf, r_left / 8);
+    else load_tile<STEP, BM, WAVES>(r + s * STEP, r_rs, r_left, buf);
+    if constexpr (CC) load_tile<BN, STEP, WAVES>(c + (long)s * STEP * a.K, c_rs, left, buf + RT, c_left / 8);
+    else load_tile<STEP, BN, WAVES>(c + s * STEP, c_rs, c_left, buf + RT);
   };
   const unsigned rrow = rows_base<STEP>(), crow = rows_base<STEP>();
   const unsigned rcol = cols_base_natural<BM>(), ccol = cols_base_natural<BN>();
@@ -113,7 +126,6 @@ __global__ __launch_bounds__(64 * WAVES, 1) void grouped_gemm_kernel(const Group
 #pragma unroll
     for (int j = 0; j < WN / 32; ++j) acc[i][j] = zero16();
 
-  const int steps = (sum + STEP - 1) / STEP;
   unsigned cur = 0, next = BUF, after = 2 * BUF;
   if (steps > 0) load(0, cur);
   if (BUFS == 3 && steps > 1) load(1, next);
@@ -283,19 +295,37 @@ at::Tensor grouped_gemm_nt(const at::Tensor& x, const at::Tensor& w,
   return y;
 }
 
-at::Tensor grouped_gemm_nn(const at::Tensor& g, const at::Tensor& w,
-                           const at::Tensor& offs, const at::Tensor& tile_map,
-                           const std::optional<at::Tensor>& n_tiles, int64_t bm) {
+static at::Tensor nn(const at::Tensor& g, const at::Tensor& w, const at::Tensor* g2, const at::Tensor* w2,
+                     const at::Tensor& offs, const at::Tensor& tile_map,
+                     const std::optional<at::Tensor>& n_tiles, int64_t bm) {
   TORCH_CHECK(g.dim() == 2 && w.dim() == 3 && g.size(1) == w.size(1), "grouped_gemm_nn: g [M,N], w [E,N,K]");
   TORCH_CHECK(bm == 128 || bm == 256, "grouped_gemm_nn: tiles of 128 or 256 rows");
   TORCH_CHECK(w.size(1) % STEP == 0 && w.size(2) % 128 == 0, "need N%64==0, K%128==0");
   auto dx = at::empty({g.size(0), w.size(2)}, g.options());
   if (tile_map.size(0) == 0 || g.size(0) == 0) return dx;
   auto a = grouped_args(g, w, dx, offs);
+  if (g2) {
+    TORCH_CHECK(g2->sizes() == g.sizes() && w2->sizes() == w.sizes(), "grouped_gemm_nn2: two equal pairs");
+    auto b = grouped_args(*g2, *w2, dx, offs);
+    a.r2 = b.r;
+    a.c2 = b.c;
+  }
   set_tiles(a, w, offs, tile_map, n_tiles);
   if (bm == 256) launch<NN, 256, 256, 8, 2>(a);
   else launch<NN, 128, 256, 8, 3>(a);
   return dx;
+}
+
+at::Tensor grouped_gemm_nn(const at::Tensor& g, const at::Tensor& w,
+                           const at::Tensor& offs, const at::Tensor& tile_map,
+                           const std::optional<at::Tensor>& n_tiles, int64_t bm) {
+  return nn(g, w, nullptr, nullptr, offs, tile_map, n_tiles, bm);
+}
+
+at::Tensor grouped_gemm_nn2(const at::Tensor& g1, const at::Tensor& w1, const at::Tensor& g2,
+                            const at::Tensor& w2, const at::Tensor& offs, const at::Tensor& tile_map,
+                            const std::optional<at::Tensor>& n_tiles, int64_t bm) {
+  return nn(g1, w1, &g2, &w2, offs, tile_map, n_tiles, bm);
 }
 
 at::Tensor grouped_gemm_tn(const at::Tensor& g, const at::Tensor& x, const at::Tensor& offs, int64_t E) {

@@ -97,6 +97,14 @@ at::Tensor grouped_gemm_nt_fp8(const at::Tensor& x8, const at::Tensor& w8,
                                const at::Tensor& scale,
                                const std::optional<at::Tensor>& n_tiles = std::nullopt,
                                int64_t bm = 128);
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor> route_plan(
+    const at::Tensor& indices, const at::Tensor& probs, int64_t E);
+std::tuple<at::Tensor, at::Tensor> combine_bwd(const at::Tensor& g, const at::Tensor& y,
+                                               const at::Tensor& src, const at::Tensor& order,
+                                               const at::Tensor& probs);
+at::Tensor grouped_gemm_nn2(const at::Tensor& g1, const at::Tensor& w1, const at::Tensor& g2,
+                            const at::Tensor& w2, const at::Tensor& offs, const at::Tensor& tile_map,
+                            const std::optional<at::Tensor>& n_tiles, int64_t bm);
 at::Tensor permute_gather(const at::Tensor& x, const at::Tensor& src);
 at::Tensor unpermute_combine(const at::Tensor& yp, const at::Tensor& pos,
                              const at::Tensor& probs);

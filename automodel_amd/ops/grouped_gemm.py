@@ -127,6 +127,39 @@ def grouped_linear(x_perm: torch.Tensor, w: torch.Tensor, counts,
     return _GroupedLinear.apply(x_perm, w, counts, offs, tile_map, n_tiles, bm)
 
 
+class _GroupedPair(torch.autograd.Function):
+    """(x @ w1[e].T, x @ w2[e].T): two projections of one input, whose gradient is
+    one product over both (bf16 kernels only)."""
+
+    @staticmethod
+    def forward(ctx, x, w1, w2, offs, tile_map, n_tiles, bm):
+        x, w1, w2 = x.contiguous(), w1.contiguous(), w2.contiguous()
+        ctx.save_for_backward(x, w1, w2, offs, tile_map, n_tiles)
+        ctx.bm = bm
+        ops = hip_ops()
+        return (ops.grouped_gemm_nt(x, w1, offs, tile_map, n_tiles, bm),
+                ops.grouped_gemm_nt(x, w2, offs, tile_map, n_tiles, bm))
+
+    @staticmethod
+    def backward(ctx, g1, g2):
+        x, w1, w2, offs, tile_map, n_tiles = ctx.saved_tensors
+        ops, need = hip_ops(), ctx.needs_input_grad
+        g1, g2 = g1.contiguous(), g2.contiguous()
+        dx = ops.grouped_gemm_nn2(g1, w1, g2, w2, offs, tile_map, n_tiles, ctx.bm) if need[0] else None
+        d1 = ops.grouped_gemm_tn(g1, x, offs, w1.shape[0]) if need[1] else None
+        d2 = ops.grouped_gemm_tn(g2, x, offs, w2.shape[0]) if need[2] else None
+        return dx, d1, d2, None, None, None, None
+
+
+def grouped_linear_pair(x_perm, w1, w2, counts, plan):
+    """``grouped_linear`` of two equal stacks with a device plan."""
+    if (x_perm.is_cuda and x_perm.dtype == w1.dtype == w2.dtype == torch.bfloat16
+            and w1.shape == w2.shape and w1.shape[1] % 128 == 0 and w1.shape[2] % 128 == 0):
+        return _GroupedPair.apply(x_perm, w1, w2, *plan)
+    return (grouped_linear(x_perm, w1, counts, plan=plan),
+            grouped_linear(x_perm, w2, counts, plan=plan))
+
+
 # ===========================================================================
 # fp8 grouped forward (SURVEY §2.5 MXFP8-grouped equivalent): tensorwise
 # delayed scaling exactly like quantization/fp8.py Float8Linear — the step's
