@@ -130,6 +130,19 @@ class LlamaConfig:
         )
 
 
+def _project(backend: BackendConfig, lins: list[nn.Module], x: torch.Tensor) -> list[torch.Tensor]:
+    """``[lin(x) for lin in lins]``; the few rows of a decode step in one launch."""
+    from automodel_amd.utils.kv_cache import active_kv_cache
+
+    if active_kv_cache() is not None and backend.attn == "hip":
+        from automodel_amd.serving.decode_linear import decode_rows
+
+        ys = decode_rows(lins, x)
+        if ys is not None:
+            return ys
+    return [lin(x) for lin in lins]
+
+
 class LlamaAttention(nn.Module):
     def __init__(self, cfg: LlamaConfig, backend: BackendConfig,
                  use_rope: bool = True):
@@ -160,7 +173,7 @@ class LlamaAttention(nn.Module):
 
         B, S, _ = x.shape
         if self.cfg.fused_qkv:
-            qkv = self.qkv_proj(x)
+            (qkv,) = _project(self.backend, [self.qkv_proj], x)
             q, k, v = qkv.split([self.num_heads * self.head_dim,
                                  self.num_kv_heads * self.head_dim,
                                  self.num_kv_heads * self.head_dim], dim=-1)
@@ -168,14 +181,13 @@ class LlamaAttention(nn.Module):
             k = k.contiguous().view(B, S, -1, self.head_dim)
             v = v.contiguous().view(B, S, -1, self.head_dim)
         else:
-            q = self.q_proj(x)
-            k = self.k_proj(x)
+            q, k, v = _project(self.backend, [self.q_proj, self.k_proj, self.v_proj], x)
             if self.cfg.qk_norm_full:   # OLMoE: norm over the flat projection
                 q = self.q_norm(q)
                 k = self.k_norm(k)
             q = q.view(B, S, -1, self.head_dim)
             k = k.view(B, S, -1, self.head_dim)
-            v = self.v_proj(x).view(B, S, -1, self.head_dim)
+            v = v.view(B, S, -1, self.head_dim)
         if self.cfg.qk_norm and not self.cfg.qk_norm_after_rope:
             q = self.q_norm(q)
             k = self.k_norm(k)
@@ -248,7 +260,7 @@ class LlamaAttention(nn.Module):
                     k, v = new_k, new_v       # a whole prompt: the cache holds the same
                 o = flash_attention(q, k, v, causal=True, scale=attn_scale,
                                     backend=attn_backend, q_start=cache_pos)
-        return self.o_proj(o.reshape(B, S, -1))
+        return _project(self.backend, [self.o_proj], o.reshape(B, S, -1))[0]
 
 
 class LlamaMLP(nn.Module):
@@ -266,6 +278,15 @@ class LlamaMLP(nn.Module):
         self.down_proj = nn.Linear(cfg.intermediate_size, cfg.hidden_size, bias=bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        from automodel_amd.utils.kv_cache import active_kv_cache
+
+        if active_kv_cache() is not None and self.backend.attn == "hip":
+            from automodel_amd.serving.decode_linear import decode_rows
+
+            lins = [self.gate_up_proj] if self.fused else [self.gate_proj, self.up_proj]
+            act = decode_rows(lins, x, glu=True)
+            if act is not None:
+                return _project(self.backend, [self.down_proj], act[0])[0]
         if self.fused:
             return self.down_proj(swiglu_cat(self.gate_up_proj(x)))
         return self.down_proj(swiglu(self.gate_proj(x), self.up_proj(x)))
@@ -436,7 +457,7 @@ class LlamaForCausalLM(nn.Module):
             return hidden
         if logit_rows is not None:
             hidden = hidden.flatten(0, 1)[logit_rows]
-        return self.lm_head(hidden)
+        return _project(self.backend, [self.lm_head], hidden)[0]
 
     @torch.no_grad()
     def forward_with_aux(

@@ -19,6 +19,8 @@ TORCH_LIBRARY_FRAGMENT(amd_ops, m) {
   m.def(
       "gemm_skinny_bf16(Tensor x, Tensor w, bool relu2, bool out_f32, int group_n=0) -> Tensor");
   m.impl("gemm_skinny_bf16", &amd_ops::gemm_skinny_bf16);
+  m.def("decode_rows(Tensor x, Tensor[] ws, bool glu=False) -> Tensor[]");
+  m.impl("decode_rows", &amd_ops::decode_rows);
 
   m.def("doc_bounds(Tensor cu, int total) -> (Tensor, Tensor)");
   m.impl("doc_bounds", &amd_ops::doc_bounds);

@@ -1,22 +1,24 @@
-// Skinny-batch bf16 GEMV for KV-cached decode: y[B,N] = x[B,K] @ W[N,K]^T.
+// Linear layers of decode steps: y[B, N] = x[B, K] W[N, K]^T for few rows x.
 //
-// Decode-step linears are m<=16 GEMMs — pure weight-streaming. hipBLASLt's
-// GEMV path measures ~23% of HBM bandwidth on these shapes (profiled in
-// profiles/decode_*.json); this kernel streams each W row once with b128
-// loads (guide Guideline 13) and broadcasts the tiny x through L2:
-//   * one wave per output row, lanes cover K in 16-byte chunks
-//     (lane l reads W[row, l*8 + i*512 .. +8) — 1 KB/instruction/wave,
-//     fully coalesced);
-//   * batch columns (B) accumulate in registers in the same pass, so W
-//     traffic is independent of B;
-//   * fp32 dot accumulation + wave reduce, lane 0 stores;
-//   * the epilogue can apply max(y, 0)^2 and can store f32 (residual inputs,
-//     logits) instead of bf16.
-// Grid = N/4 workgroups of 4 waves: N=4096 -> 1024 blocks >> 256 CUs.
+// The weights are read once and are all the traffic there is; both kernels are
+// bound by how many of their loads are in flight. Up to 2 rows (4 with a bias) a
+// wave takes a row of W and its lanes run along K; above that the matrix cores
+// take 16 rows of W against 16 rows of x per instruction, since a dot product
+// per row of x would cost more than the load (4 rows, 14336 x 4096: 27 us against
+// 21 us). Weight loads leave no trace in the caches (nontemporal).
+//
+// One launch can take several weights of the same input (q, k and v; gate and
+// up), each with an output of its own, and can return silu(gate) * up instead of
+// gate and up; one weight can also be split into groups of rows that take
+// different inputs. A launch of a small weight alone does not reach the memory's
+// rate: 1024 x 4096 takes 5 us, 1.7 us of them for its bytes.
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+
+#include <climits>
+#include <type_traits>
 
 #include "common.h"
 #include "ops_api.h"
@@ -27,244 +29,387 @@ typedef __bf16 gemv_bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 gemv_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float gemv_f32x4 __attribute__((ext_vector_type(4)));
 
+constexpr int MAX_SEGMENTS = 3;
+
+// What a launch computes: weights [n[s], K] whose blocks begin at first[s]. With a
+// gated product, w[0] and w[1] are gate and up and there is one output.
+struct Rows {
+  const bf16* x;
+  const bf16* w[MAX_SEGMENTS];
+  bf16* y[MAX_SEGMENTS];
+  int n[MAX_SEGMENTS];
+  int first[MAX_SEGMENTS];   // INT_MAX: no such segment
+  const bf16* bias;          // of a single weight
+  float* yf;                 // of a single weight: float32 output instead of y[0]
+  bool relu2;                // max(y, 0)^2
+  int K;
+  int group_n;               // > 0: every group_n rows of w take the next B rows of x
+};
+
 __device__ __forceinline__ float dot2(const bf16x8& a, const bf16x8& b, int j, float c) {
   const gemv_bf16x8 av = __builtin_bit_cast(gemv_bf16x8, a), bv = __builtin_bit_cast(gemv_bf16x8, b);
   return __builtin_amdgcn_fdot2_f32_bf16(gemv_bf16x2{av[2 * j], av[2 * j + 1]},
                                          gemv_bf16x2{bv[2 * j], bv[2 * j + 1]}, c, false);
 }
 
-// Two rows per wave: doubles outstanding b128 loads per wave (latency
-// hiding for the short 8-iteration K sweep at K=4096).
-template <int B>
-__global__ __launch_bounds__(256, 4) void gemv_bf16_kernel(
-    const bf16* __restrict__ W, const bf16* __restrict__ x,
-    const bf16* __restrict__ bias, bf16* __restrict__ y, float* __restrict__ yf, bool relu2,
-    int N, int K, int group_n) {
+__device__ __forceinline__ bf16x8 load_stream(const bf16* p) {
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)));
+}
+
+__device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.f + __expf(-g)) * u; }
+
+__device__ __forceinline__ int segment_of(const Rows& p, int block) {
+  return (block >= p.first[1]) + (block >= p.first[2]);
+}
+
+// A wave takes R rows of W, or with GLU one row of gate and the same of up, and
+// has 512 U columns of each in flight. One row and U = 8 reach the highest rate
+// for one row of x: 14336 x 4096 in 18.6 us (6.3 TB/s) against 23.1 with two rows
+// and U = 2, and 24.2 with two rows and U = 1.
+template <int B, int R, int U, bool GLU>
+__global__ __launch_bounds__(256) void gemv_bf16_kernel(const Rows p) {
+  static_assert(!GLU || R == 2);
+  constexpr int STEP = GLU ? 1 : R;               // rows of output per wave
+  const int seg = segment_of(p, blockIdx.x), K = p.K, N = p.n[seg];
   const int lane = threadIdx.x & (WAVE_SIZE - 1);
-  const int wid = blockIdx.x * (blockDim.x / WAVE_SIZE) + (threadIdx.x / WAVE_SIZE);
-  const int row0 = 2 * wid;
+  const int row0 = ((blockIdx.x - p.first[seg]) * 4 + threadIdx.x / WAVE_SIZE) * STEP;
   if (row0 >= N) return;
-  const bool two = row0 + 1 < N;
-  float acc0[B], acc1[B];
+  float acc[R][B];
+  const bf16* w[R];
 #pragma unroll
-  for (int b = 0; b < B; ++b) acc0[b] = acc1[b] = 0.f;
-  const bf16* wrow0 = W + (long)row0 * K;
-  const bf16* wrow1 = wrow0 + (two ? K : 0);
-  if (group_n) x += (long)(row0 / group_n) * B * K;   // group_n is even
-  for (int k = lane * 8; k < K; k += WAVE_SIZE * 8) {
-    const bf16x8 w0 = *reinterpret_cast<const bf16x8*>(wrow0 + k);
-    const bf16x8 w1 = *reinterpret_cast<const bf16x8*>(wrow1 + k);
+  for (int r = 0; r < R; ++r) {
+    w[r] = GLU ? p.w[r] + (long)row0 * K : p.w[seg] + (long)min(row0 + r, N - 1) * K;
 #pragma unroll
-    for (int b = 0; b < B; ++b) {
-      const bf16x8 xv = *reinterpret_cast<const bf16x8*>(x + (long)b * K + k);
-      float d0 = 0.f, d1 = 0.f;
+    for (int b = 0; b < B; ++b) acc[r][b] = 0.f;
+  }
+  const bf16* x = p.x;
+  if (p.group_n) x += (long)(row0 / p.group_n) * B * K;   // group_n is a multiple of R
+  auto part = [&](int k, auto depth) {
+    constexpr int D = decltype(depth)::value;
+    bf16x8 wv[D][R];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {               // v_dot2_f32_bf16: f32 accumulation
-        d0 = dot2(w0, xv, j, d0);
-        d1 = dot2(w1, xv, j, d1);
+    for (int u = 0; u < D; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r) wv[u][r] = load_stream(w[r] + k + u * 512);
+#pragma unroll
+    for (int u = 0; u < D; ++u)
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const bf16x8 xv = *reinterpret_cast<const bf16x8*>(x + (long)b * K + k + u * 512);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          float d = 0.f;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) d = dot2(wv[u][r], xv, j, d);   // f32 accumulation
+          acc[r][b] += d;
+        }
       }
-      acc0[b] += d0;
-      acc1[b] += d1;
+  };
+  int k = lane * 8;                               // K % 8 == 0: all 8 columns or none
+  for (; k + 512 * (U - 1) < K; k += 512 * U) part(k, std::integral_constant<int, U>{});
+  if constexpr (U > 4) {
+    if (k + 512 * 3 < K) {
+      part(k, std::integral_constant<int, 4>{});
+      k += 512 * 4;
     }
   }
+  for (; k < K; k += 512) part(k, std::integral_constant<int, 1>{});
 #pragma unroll
   for (int b = 0; b < B; ++b) {
-    const float t0 = wave_reduce_sum(acc0[b]);
-    const float t1 = wave_reduce_sum(acc1[b]);
-    if (lane == 0) {
+    float t[R];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        if (i && !two) break;
-        float t = (i ? t1 : t0) + (bias ? bf2f(bias[row0 + i]) : 0.f);
-        if (relu2) {
-          t = fmaxf(t, 0.f);
-          t *= t;
+    for (int r = 0; r < R; ++r) t[r] = wave_reduce_sum(acc[r][b]);
+    if (lane != 0) continue;
+    if constexpr (GLU) {
+      p.y[0][(long)b * N + row0] = f2bf(silu_mul(t[0], t[1]));
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if (row0 + r >= N) break;
+        if (p.bias) t[r] += bf2f(p.bias[row0 + r]);
+        if (p.relu2) {
+          t[r] = fmaxf(t[r], 0.f);
+          t[r] *= t[r];
         }
-        if (yf) yf[(long)b * N + row0 + i] = t;
-        else y[(long)b * N + row0 + i] = f2bf(t);
+        if (p.yf) p.yf[(long)b * N + row0 + r] = t[r];
+        else p.y[seg][(long)b * N + row0 + r] = f2bf(t[r]);
       }
     }
   }
 }
+
+// A workgroup takes 16 RT rows of W (GLU: 16 of gate and the same 16 of up) and
+// 16 NB rows of x; its waves take every WAVES-th tile of K and add up through LDS
+// at the end, so that N = 1024 fills the chip too. Matrix fragments want one row
+// per lane, memory wants consecutive lanes on consecutive bytes: each wave moves
+// its tiles of W and x with coalesced loads into LDS of its own, with the next
+// DEPTH tiles' loads in flight. No workgroup barrier in the loop.
+constexpr int SK_KC = 128;                        // K per tile
+constexpr int SK_STRIDE = SK_KC * 2 + 16;         // LDS bytes per row
+
+template <int NB, int WAVES, int RT, int DEPTH, bool GLU>
+__global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(const Rows p, int B) {
+  static_assert(!GLU || RT == 2);
+  constexpr int OUT = GLU ? 16 : 16 * RT;         // rows of output per workgroup
+  constexpr int RS = 16 * NB + 1;
+  constexpr int RED = WAVES * 16 * RT * RS * 4;
+  constexpr int TILE = 16 * (RT + NB) * SK_STRIDE;
+  __shared__ __attribute__((aligned(16))) char lds[WAVES * TILE > RED ? WAVES * TILE : RED];
+  const int lane = threadIdx.x & (WAVE_SIZE - 1), wid = threadIdx.x / WAVE_SIZE;
+  const int lo16 = lane & 15, hi4 = lane >> 4;
+  const int seg = segment_of(p, blockIdx.x), K = p.K, N = p.n[seg];
+  const int n0 = (blockIdx.x - p.first[seg]) * OUT;
+  const bf16* x = p.x;
+  if (p.group_n) x += (long)(n0 / p.group_n) * B * K;   // group_n % OUT == 0
+  char* wl = lds + wid * TILE;                    // [16 RT][SK_STRIDE]
+  char* xl = wl + 16 * RT * SK_STRIDE;            // [16 NB][SK_STRIDE]
+
+  gemv_f32x4 acc[RT][NB];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[r][b] = gemv_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int tiles = (K + SK_KC - 1) / SK_KC;
+
+  // load j covers rows 4j + hi4, 16 bytes per lane at column 8 lo16
+  bf16x8 wr[DEPTH][4 * RT], xr[DEPTH][4 * NB];
+  auto fetch = [&](int t, int d) {
+    const int k = t * SK_KC + lo16 * 8;
+    const bool in = k < K;                        // K % 8 == 0: all 8 or none
+#pragma unroll
+    for (int j = 0; j < 4 * RT; ++j) {
+      wr[d][j] = bf16x8{};
+      const bf16* w = GLU ? p.w[j / 4] : p.w[seg];
+      const int row = n0 + 4 * (GLU ? j % 4 : j) + hi4;
+      if (in) wr[d][j] = load_stream(w + (long)min(row, N - 1) * K + k);
+    }
+#pragma unroll
+    for (int j = 0; j < 4 * NB; ++j) {
+      xr[d][j] = bf16x8{};
+      if (in)
+        xr[d][j] = *reinterpret_cast<const bf16x8*>(x + (long)min(4 * j + hi4, B - 1) * K + k);
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) fetch(wid + d * WAVES, d);
+  for (int t0 = wid; t0 < tiles; t0 += WAVES * DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      const int t = t0 + d * WAVES;
+      if (t >= tiles) break;
+#pragma unroll
+      for (int j = 0; j < 4 * RT; ++j)
+        *reinterpret_cast<bf16x8*>(wl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = wr[d][j];
+#pragma unroll
+      for (int j = 0; j < 4 * NB; ++j)
+        *reinterpret_cast<bf16x8*>(xl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = xr[d][j];
+      __builtin_amdgcn_wave_barrier();
+      fetch(t + WAVES * DEPTH, d);
+#pragma unroll
+      for (int kk = 0; kk < SK_KC / 32; ++kk) {
+        const int off = lo16 * SK_STRIDE + kk * 64 + hi4 * 16;
+        gemv_bf16x8 xv[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          xv[b] = *reinterpret_cast<const gemv_bf16x8*>(xl + b * 16 * SK_STRIDE + off);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          const gemv_bf16x8 wv = *reinterpret_cast<const gemv_bf16x8*>(wl + r * 16 * SK_STRIDE + off);
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+            acc[r][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, xv[b], acc[r][b], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();            // the tile is overwritten next
+    }
+  }
+  __syncthreads();                                // tiles become the reduction buffer
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        red[((wid * RT + r) * 16 + hi4 * 4 + i) * RS + b * 16 + lo16] = acc[r][b][i];
+  __syncthreads();
+  auto total = [&](int row, int col) {
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) t += red[(w * 16 * RT + row) * RS + col];
+    return t;
+  };
+  for (int i = threadIdx.x; i < OUT * 16 * NB; i += WAVES * WAVE_SIZE) {
+    const int row = i % OUT, col = i / OUT;
+    if (n0 + row >= N || col >= B) continue;
+    const long o = (long)col * N + n0 + row;
+    float t = total(row, col);
+    if constexpr (GLU) t = silu_mul(t, total(16 + row, col));
+    if (p.relu2) {
+      t = fmaxf(t, 0.f);
+      t *= t;
+    }
+    if (p.yf) p.yf[o] = t;
+    else p.y[seg][o] = f2bf(t);
+  }
+}
+
+namespace {
+
+const bf16* data(const at::Tensor& t) { return reinterpret_cast<const bf16*>(t.data_ptr()); }
+
+// Gives each segment its blocks of ``per`` rows of output; -> blocks in all.
+int place(Rows& p, int segments, int per) {
+  int blocks = 0;
+  for (int s = 0; s < MAX_SEGMENTS; ++s) {
+    p.first[s] = s < segments ? blocks : INT_MAX;
+    if (s < segments) blocks += (p.n[s] + per - 1) / per;
+  }
+  return blocks;
+}
+
+template <int B, int R, int U, bool GLU = false>
+void launch_gemv(Rows p, int segments) {
+  const int blocks = place(p, segments, 4 * (GLU ? 1 : R));
+  gemv_bf16_kernel<B, R, U, GLU>
+      <<<dim3(blocks), dim3(256), 0, c10::hip::getCurrentHIPStream()>>>(p);
+}
+
+template <int NB, int WAVES, int RT, int DEPTH, bool GLU = false>
+void launch_skinny(Rows p, int segments, int B) {
+  const int blocks = place(p, segments, GLU ? 16 : 16 * RT);
+  gemm_skinny_kernel<NB, WAVES, RT, DEPTH, GLU>
+      <<<dim3(blocks), dim3(WAVES * WAVE_SIZE), 0, c10::hip::getCurrentHIPStream()>>>(p, B);
+}
+
+// Up to 16 rows the loads in flight decide: 8 waves, and 2 tiles ahead, for a K
+// that has that many (8 rows, 14336 x 4096: 21.4 us, 23.0 with 1 tile ahead and W
+// through the caches; K < 2048 keeps 4 waves). Above that the x rows of each
+// workgroup weigh as much as its rows of W: 64 rows of W per workgroup once that
+// still leaves 128 workgroups (32 rows, 14336 x 4096: 28.1 us, 16 rows each 34.9;
+// at 4096 x 4096 22.2 against 11.4). A gated pair has 32 rows of W anyway.
+void skinny(const Rows& p, int segments, int B, bool glu) {
+  int rows = 0;
+  for (int s = 0; s < segments; ++s) rows += p.n[s];
+  const bool wide = rows >= 8192 && p.group_n % 64 == 0;
+  if (B <= 16) {
+    if (glu) launch_skinny<1, 4, 2, 1, true>(p, segments, B);
+    else if (p.K >= 2048) launch_skinny<1, 8, 1, 2>(p, segments, B);
+    else launch_skinny<1, 4, 1, 1>(p, segments, B);
+  } else if (B <= 32) {
+    if (glu) launch_skinny<2, 4, 2, 1, true>(p, segments, B);
+    else if (wide) launch_skinny<2, 4, 4, 1>(p, segments, B);
+    else launch_skinny<2, 8, 1, 1>(p, segments, B);
+  } else {
+    if (glu) launch_skinny<4, 2, 2, 1, true>(p, segments, B);
+    else if (wide) launch_skinny<4, 4, 4, 1>(p, segments, B);
+    else launch_skinny<4, 4, 1, 1>(p, segments, B);
+  }
+}
+
+// One weight, [B, K] per group of its rows -> (its part of a launch, output).
+std::pair<Rows, at::Tensor> single(const char* name, const at::Tensor& x, const at::Tensor& w,
+                                   bool relu2, bool out_f32, int64_t group_n, int unit,
+                                   int& B) {
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.dtype() == at::kBFloat16 &&
+                  w.dtype() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2,
+              name, ": x [B,K], w [N,K] bf16 on the GPU");
+  const int K = (int)x.size(1), N = (int)w.size(0);
+  const int groups = group_n > 0 ? (int)((N + group_n - 1) / group_n) : 1;
+  TORCH_CHECK(group_n >= 0 && group_n % unit == 0 && x.size(0) % groups == 0, name,
+              ": group_n in multiples of ", unit, ", and one [B,K] input per group");
+  TORCH_CHECK(w.size(1) == K && K % 8 == 0 && K >= 8 && N >= 1, name, ": K % 8 == 0");
+  B = (int)x.size(0) / groups;
+  auto y = at::empty({B, N}, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
+  Rows p{};
+  p.x = data(x);
+  p.w[0] = data(w);
+  p.n[0] = N;
+  if (out_f32) p.yf = y.data_ptr<float>();
+  else p.y[0] = reinterpret_cast<bf16*>(y.data_ptr());
+  p.relu2 = relu2;
+  p.K = K;
+  p.group_n = (int)group_n;
+  return {p, y};
+}
+
+}  // namespace
 
 // group_n > 0: x holds several [B, K] inputs one after another, and every
 // group_n rows of w take the next one.
 at::Tensor gemv_bf16(const at::Tensor& x, const at::Tensor& w,
                      const c10::optional<at::Tensor>& bias, bool relu2, bool out_f32,
                      int64_t group_n) {
-  TORCH_CHECK(x.is_cuda() && w.is_cuda(), "gemv_bf16: GPU tensors required");
-  TORCH_CHECK(x.dtype() == at::kBFloat16 && w.dtype() == at::kBFloat16,
-              "gemv_bf16: bf16 only");
-  TORCH_CHECK(x.dim() == 2 && w.dim() == 2, "gemv_bf16: x [B,K], w [N,K]");
-  const int K = (int)x.size(1), N = (int)w.size(0);
-  const int groups = group_n > 0 ? (int)((N + group_n - 1) / group_n) : 1;
-  TORCH_CHECK(group_n >= 0 && group_n % 2 == 0 && x.size(0) % groups == 0,
-              "gemv_bf16: an even group_n, and one [B,K] input per group");
-  const int B = (int)x.size(0) / groups;
-  TORCH_CHECK(w.size(1) == K, "K mismatch");
+  const auto xc = x.contiguous(), wc = w.contiguous();
+  at::Tensor bc;
+  int B = 0;
+  auto [p, y] = single("gemv_bf16", xc, wc, relu2, out_f32, group_n, 2, B);
   TORCH_CHECK(B >= 1 && B <= 16, "gemv_bf16: B in [1,16], got ", B,
               " (larger batches belong on hipBLASLt)");
-  TORCH_CHECK(K % 8 == 0, "gemv_bf16: K % 8 == 0, got ", K);
-  auto xc = x.contiguous(), wc = w.contiguous();
-  auto y = at::empty({B, N}, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
-  const bf16* bptr = nullptr;
   if (bias.has_value()) {
-    TORCH_CHECK(bias->numel() == N && bias->dtype() == at::kBFloat16, "bias [N] bf16");
-    bptr = reinterpret_cast<const bf16*>(bias->contiguous().data_ptr());
+    TORCH_CHECK(bias->numel() == p.n[0] && bias->dtype() == at::kBFloat16, "bias [N] bf16");
+    bc = bias->contiguous();
+    p.bias = data(bc);
   }
-  const int waves_per_block = 4;
-  const int rows_per_block = 2 * waves_per_block;
-  const dim3 grid((N + rows_per_block - 1) / rows_per_block);
-  auto stream = c10::hip::getCurrentHIPStream();
-#define LAUNCH(BB)                                                             \
-  gemv_bf16_kernel<BB><<<grid, dim3(waves_per_block * WAVE_SIZE), 0, stream>>>( \
-      reinterpret_cast<const bf16*>(wc.data_ptr()),                            \
-      reinterpret_cast<const bf16*>(xc.data_ptr()), bptr,                      \
-      out_f32 ? nullptr : reinterpret_cast<bf16*>(y.data_ptr()),               \
-      out_f32 ? y.data_ptr<float>() : nullptr, relu2, N, K, (int)group_n)
   switch (B) {
-    case 1: LAUNCH(1); break;
-    case 2: LAUNCH(2); break;
-    case 3: LAUNCH(3); break;
-    case 4: LAUNCH(4); break;
-    case 8: LAUNCH(8); break;
-    case 16: LAUNCH(16); break;
+    case 1: launch_gemv<1, 1, 8>(p, 1); break;
+    case 2: launch_gemv<2, 1, 4>(p, 1); break;
+    case 3: launch_gemv<3, 2, 1>(p, 1); break;
+    case 4: launch_gemv<4, 2, 1>(p, 1); break;
+    case 8: launch_gemv<8, 2, 1>(p, 1); break;
+    case 16: launch_gemv<16, 2, 1>(p, 1); break;
     default: TORCH_CHECK(false, "gemv_bf16: pad B to one of 1,2,3,4,8,16 (python wrapper does)");
   }
-#undef LAUNCH
   HIP_CHECK_KERNEL();
   return y;
-}
-
-// ---------------------------------------------------------------------------
-// Skinny GEMM for decode batches of 5..64 rows: the same weight stream, with
-// the products on the matrix cores. A workgroup owns 16 rows of W; its waves
-// split K and reduce through LDS at the end, so that even N = 4096 fills the
-// chip. Matrix fragments want one row per lane, memory wants consecutive lanes
-// on consecutive bytes: each wave moves its 16 x 128 tile of W (and the x rows
-// of the same K range) with coalesced loads into LDS of its own, the next
-// tile's loads in flight meanwhile. No workgroup barrier in the loop.
-// ---------------------------------------------------------------------------
-constexpr int SK_KC = 128;                        // K per tile
-constexpr int SK_STRIDE = SK_KC * 2 + 16;         // LDS bytes per row
-
-template <int NB, int WAVES>
-__global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(
-    const bf16* __restrict__ W, const bf16* __restrict__ x, bf16* __restrict__ y,
-    float* __restrict__ yf, bool relu2, int B, int N, int K, int group_n) {
-  constexpr int RED = WAVES * 16 * (16 * NB + 1) * 4;
-  constexpr int TILE = 16 * (1 + NB) * SK_STRIDE;
-  __shared__ __attribute__((aligned(16))) char lds[WAVES * TILE > RED ? WAVES * TILE : RED];
-  const int lane = threadIdx.x & (WAVE_SIZE - 1), wid = threadIdx.x / WAVE_SIZE;
-  const int lo16 = lane & 15, hi4 = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-  if (group_n) x += (long)(n0 / group_n) * B * K;       // group_n % 16 == 0
-  char* wl = lds + wid * TILE;                    // [16][SK_STRIDE]
-  char* xl = wl + 16 * SK_STRIDE;                 // [16 NB][SK_STRIDE]
-
-  gemv_f32x4 acc[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) acc[b] = gemv_f32x4{0.f, 0.f, 0.f, 0.f};
-  const int tiles = (K + SK_KC - 1) / SK_KC;
-  const int per = (tiles + WAVES - 1) / WAVES;
-  const int t_lo = wid * per, t_hi = min(t_lo + per, tiles);
-
-  // load j covers rows 4j + hi4, 16 bytes per lane at column 8 lo16
-  gemv_bf16x8 wr[4], xr[4 * NB];
-  auto fetch = [&](int t) {
-    const int k = t * SK_KC + lo16 * 8;
-    const bool in = k < K;                        // K % 8 == 0: all 8 or none
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      wr[j] = gemv_bf16x8{};
-      if (in)
-        wr[j] = *reinterpret_cast<const gemv_bf16x8*>(
-            W + (long)min(n0 + 4 * j + hi4, N - 1) * K + k);
-    }
-#pragma unroll
-    for (int j = 0; j < 4 * NB; ++j) {
-      xr[j] = gemv_bf16x8{};
-      if (in)
-        xr[j] = *reinterpret_cast<const gemv_bf16x8*>(x + (long)min(4 * j + hi4, B - 1) * K + k);
-    }
-  };
-  if (t_lo < t_hi) fetch(t_lo);
-  for (int t = t_lo; t < t_hi; ++t) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<gemv_bf16x8*>(wl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = wr[j];
-#pragma unroll
-    for (int j = 0; j < 4 * NB; ++j)
-      *reinterpret_cast<gemv_bf16x8*>(xl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = xr[j];
-    __builtin_amdgcn_wave_barrier();
-    if (t + 1 < t_hi) fetch(t + 1);
-#pragma unroll
-    for (int kk = 0; kk < SK_KC / 32; ++kk) {
-      const int off = lo16 * SK_STRIDE + kk * 64 + hi4 * 16;
-      const gemv_bf16x8 w = *reinterpret_cast<const gemv_bf16x8*>(wl + off);
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const gemv_bf16x8 v = *reinterpret_cast<const gemv_bf16x8*>(xl + b * 16 * SK_STRIDE + off);
-        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, v, acc[b], 0, 0, 0);
-      }
-    }
-    __builtin_amdgcn_wave_barrier();              // the tile is overwritten next
-  }
-  __syncthreads();                                // tiles become the reduction buffer
-  float* red = reinterpret_cast<float*>(lds);
-  constexpr int RS = 16 * NB + 1;
-#pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) red[(wid * 16 + hi4 * 4 + i) * RS + b * 16 + lo16] = acc[b][i];
-  __syncthreads();
-  for (int i = threadIdx.x; i < 256 * NB; i += WAVES * WAVE_SIZE) {
-    const int row = i & 15, col = i >> 4;
-    if (n0 + row >= N || col >= B) continue;
-    float t = 0.f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) t += red[(w * 16 + row) * RS + col];
-    if (relu2) {
-      t = fmaxf(t, 0.f);
-      t *= t;
-    }
-    const long o = (long)col * N + n0 + row;
-    if (yf) yf[o] = t;
-    else y[o] = f2bf(t);
-  }
 }
 
 at::Tensor gemm_skinny_bf16(const at::Tensor& x, const at::Tensor& w, bool relu2, bool out_f32,
                             int64_t group_n) {
-  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.dtype() == at::kBFloat16 &&
-                  w.dtype() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2,
-              "gemm_skinny_bf16: x [B,K], w [N,K] bf16 on the GPU");
-  const int K = (int)x.size(1), N = (int)w.size(0);
-  const int groups = group_n > 0 ? (int)((N + group_n - 1) / group_n) : 1;
-  TORCH_CHECK(group_n >= 0 && group_n % 16 == 0 && x.size(0) % groups == 0,
-              "gemm_skinny_bf16: group_n in whole tiles of 16, one [B,K] input per group");
-  const int B = (int)x.size(0) / groups;
-  TORCH_CHECK(w.size(1) == K && K % 8 == 0 && K >= 8 && N >= 1, "gemm_skinny_bf16: K % 8 == 0");
+  const auto xc = x.contiguous(), wc = w.contiguous();
+  int B = 0;
+  auto [p, y] = single("gemm_skinny_bf16", xc, wc, relu2, out_f32, group_n, 16, B);
   TORCH_CHECK(B >= 1 && B <= 64, "gemm_skinny_bf16: 1..64 rows, got ", B);
-  auto xc = x.contiguous(), wc = w.contiguous();
-  auto y = at::empty({B, N}, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
-  auto stream = c10::hip::getCurrentHIPStream();
-#define LAUNCH(NB, WAVES)                                                                    \
-  gemm_skinny_kernel<NB, WAVES>                                                              \
-      <<<dim3((N + 15) / 16), dim3(WAVES * WAVE_SIZE), 0, stream>>>(                         \
-          reinterpret_cast<const bf16*>(wc.data_ptr()),                                      \
-          reinterpret_cast<const bf16*>(xc.data_ptr()),                                      \
-          out_f32 ? nullptr : reinterpret_cast<bf16*>(y.data_ptr()),                         \
-          out_f32 ? y.data_ptr<float>() : nullptr, relu2, B, N, K, (int)group_n)
-  // waves per workgroup: enough of them across the chip, each with K left to
-  // stream; LDS grows with the x rows
-  const bool deep = K >= 2048;
-  if (B <= 16) { if (deep) LAUNCH(1, 8); else LAUNCH(1, 4); }
-  else if (B <= 32) { LAUNCH(2, 4); }
-  else { LAUNCH(4, 2); }
-#undef LAUNCH
+  skinny(p, 1, B, false);
   HIP_CHECK_KERNEL();
   return y;
+}
+
+// x [B, K] against up to three weights [n, K] in one launch -> [B, n] each; glu:
+// against gate and up -> silu(x gate^T) * (x up^T) alone.
+std::vector<at::Tensor> decode_rows(const at::Tensor& x, at::TensorList ws, bool glu) {
+  const int64_t B = x.size(0), K = x.size(-1);
+  TORCH_CHECK(x.is_cuda() && x.dtype() == at::kBFloat16 && x.dim() == 2 && x.is_contiguous() &&
+                  B >= 1 && B <= 64 && K >= 8 && K % 8 == 0,
+              "decode_rows: x [1..64, K] bf16, K % 8 == 0");
+  TORCH_CHECK(ws.size() >= 1 && ws.size() <= MAX_SEGMENTS, "decode_rows: 1 to 3 weights");
+  TORCH_CHECK(!glu || (ws.size() == 2 && ws[0].sizes() == ws[1].sizes()),
+              "decode_rows: gate and up of one shape");
+  Rows p{};
+  p.x = data(x);
+  p.K = (int)K;
+  std::vector<at::Tensor> out;
+  for (size_t s = 0; s < ws.size(); ++s) {
+    const auto& w = ws[s];
+    TORCH_CHECK(w.device() == x.device() && w.dtype() == at::kBFloat16 && w.dim() == 2 &&
+                    w.is_contiguous() && w.size(1) == K && w.size(0) >= 1 &&
+                    w.size(0) < INT_MAX / 2,
+                "decode_rows: weights [n, K] bf16, rows one after another");
+    p.w[s] = data(w);
+    p.n[s] = (int)w.size(0);
+    if (glu && s == 1) break;
+    out.push_back(at::empty({B, w.size(0)}, x.options()));
+    p.y[s] = reinterpret_cast<bf16*>(out.back().data_ptr());
+  }
+  const int segments = (int)out.size();
+  if (B > 2) skinny(p, segments, (int)B, glu);
+  else if (B == 1 && glu) launch_gemv<1, 2, 4, true>(p, 1);
+  else if (B == 1) launch_gemv<1, 1, 8>(p, segments);
+  else if (glu) launch_gemv<2, 2, 4, true>(p, 1);
+  else launch_gemv<2, 1, 4>(p, segments);
+  HIP_CHECK_KERNEL();
+  return out;
 }
 
 }  // namespace amd_ops

@@ -80,6 +80,7 @@ at::Tensor kv_decode_attn(const at::Tensor& q, const at::Tensor& k_new, const at
                           const std::optional<at::Tensor>& pos_dev, double scale);
 at::Tensor gemm_skinny_bf16(const at::Tensor& x, const at::Tensor& w, bool relu2, bool out_f32,
                             int64_t group_n = 0);
+std::vector<at::Tensor> decode_rows(const at::Tensor& x, at::TensorList ws, bool glu);
 
 std::tuple<at::Tensor, at::Tensor, at::Tensor> build_group_plan(
     const at::Tensor& counts, int64_t M, int64_t bm = 128);
