@@ -21,7 +21,7 @@ import torch.nn as nn
 
 from automodel_amd.models.common.backend import BackendConfig
 from automodel_amd.ops.attention import flash_attention
-from automodel_amd.ops.rms_norm import RMSNorm
+from automodel_amd.ops.rms_norm import RMSNorm, add_norm
 from automodel_amd.ops.rope import apply_rope, build_rope_cache
 from automodel_amd.ops.swiglu import swiglu, swiglu_cat
 
@@ -351,9 +351,11 @@ class LlamaDecoderLayer(nn.Module):
             x = x + self.post_attention_layernorm(self.self_attn(x, cos, sin))
             return x + self.post_feedforward_layernorm(self.mlp(x))
         r = self.residual_multiplier
-        x = x + self.self_attn(self.input_layernorm(x), cos, sin) * r
-        x = x + self.mlp(self.post_attention_layernorm(x)) * r
-        return x
+        x, h = add_norm(self.input_layernorm, x)
+        h = self.self_attn(h, cos, sin)
+        x, h = add_norm(self.post_attention_layernorm, x, h if r == 1.0 else h * r)
+        h = self.mlp(h)
+        return x + (h if r == 1.0 else h * r)
 
 
 class LlamaModel(nn.Module):

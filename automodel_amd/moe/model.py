@@ -18,7 +18,7 @@ from automodel_amd.models.llama.model import LlamaAttention, LlamaConfig
 from automodel_amd.moe.config import MoEConfig
 from automodel_amd.moe.layers import MoE, Gate, SharedExpert
 from automodel_amd.moe.state_dict_adapter import MoEStateDictAdapter
-from automodel_amd.ops.rms_norm import RMSNorm
+from automodel_amd.ops.rms_norm import RMSNorm, add_norm
 from automodel_amd.ops.rope import build_rope_cache
 
 
@@ -183,9 +183,11 @@ class MoEDecoderLayer(nn.Module):
         if self.cfg.olmo2_layout:
             x = x + self.post_attention_layernorm(self.self_attn(x, cos, sin)) * r
             return x + self.post_feedforward_layernorm(self.mlp(x)) * r
-        x = x + self.self_attn(self.input_layernorm(x), cos, sin) * r
-        x = x + self.mlp(self.post_attention_layernorm(x)) * r
-        return x
+        x, h = add_norm(self.input_layernorm, x)
+        h = self.self_attn(h, cos, sin)
+        x, h = add_norm(self.post_attention_layernorm, x, h if r == 1.0 else h * r)
+        h = self.mlp(h)
+        return x + (h if r == 1.0 else h * r)
 
 
 class MoEForCausalLM(nn.Module):

@@ -10,7 +10,11 @@
 TORCH_LIBRARY(amd_ops, m) {
   m.def("rms_norm_fwd(Tensor x, Tensor w, float eps) -> (Tensor, Tensor)");
   m.impl("rms_norm_fwd", &amd_ops::rms_norm_fwd);
-  m.def("rms_norm_bwd(Tensor dy, Tensor x, Tensor w, Tensor invrms) -> (Tensor, Tensor)");
+  m.def("add_rms_norm_fwd(Tensor x, Tensor delta, Tensor w, float eps) -> (Tensor, Tensor, Tensor)");
+  m.impl("add_rms_norm_fwd", &amd_ops::add_rms_norm_fwd);
+  m.def(
+      "rms_norm_bwd(Tensor dy, Tensor x, Tensor w, Tensor invrms, Tensor? dres=None, "
+      "bool want_dw=True) -> (Tensor, Tensor)");
   m.impl("rms_norm_bwd", &amd_ops::rms_norm_bwd);
 
   m.def("rope_fwd(Tensor q, Tensor k, Tensor cos, Tensor sin, bool backward) -> (Tensor, Tensor)");

@@ -8,8 +8,13 @@ namespace amd_ops {
 
 std::tuple<at::Tensor, at::Tensor> rms_norm_fwd(const at::Tensor& x, const at::Tensor& w,
                                                 double eps);
+std::tuple<at::Tensor, at::Tensor, at::Tensor> add_rms_norm_fwd(const at::Tensor& x,
+                                                                const at::Tensor& delta,
+                                                                const at::Tensor& w, double eps);
 std::tuple<at::Tensor, at::Tensor> rms_norm_bwd(const at::Tensor& dy, const at::Tensor& x,
-                                                const at::Tensor& w, const at::Tensor& invrms);
+                                                const at::Tensor& w, const at::Tensor& invrms,
+                                                const std::optional<at::Tensor>& dres = std::nullopt,
+                                                bool want_dw = true);
 
 std::tuple<at::Tensor, at::Tensor> rope_fwd(const at::Tensor& q, const at::Tensor& k,
                                             const at::Tensor& cosb, const at::Tensor& sinb,

@@ -8,6 +8,10 @@
 // buffer and a second kernel adds them up in a fixed order. Atomic adds into one row of H
 // sums, 1024 deep on each, were the bound before: 263 us for 8192 x 4096, 219 us for
 // 6001 x 2048 and 54 us for 256 x 256; now 44, 24 and 12 us with the sum.
+//
+// Around a norm stands a residual stream: the sum that is normed, and in the backward the
+// gradient that reaches the stream by its other way. Both take that operand here, so that
+// the sum and the gradients' sum are no passes of their own.
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -32,9 +36,12 @@ __device__ __forceinline__ float row_sum(float x, float* red) {
   }
 }
 
-// x: [T, H], w: [H] -> y: [T, H], invrms: [T] f32
-template <int LPR, int ITERS>
+// x: [T, H], w: [H] -> y: [T, H], invrms: [T] f32; with ADD of sum = x + delta, which is
+// rounded to bf16 and stored first
+template <int LPR, int ITERS, bool ADD>
 __global__ __launch_bounds__(256) void rms_norm_fwd_kernel(const bf16* __restrict__ x,
+                                                           const bf16* __restrict__ delta,
+                                                           bf16* __restrict__ sum,
                                                            const bf16* __restrict__ w,
                                                            bf16* __restrict__ y,
                                                            float* __restrict__ invrms, long T, int H,
@@ -51,6 +58,23 @@ __global__ __launch_bounds__(256) void rms_norm_fwd_kernel(const bf16* __restric
   for (int it = 0; it < ITERS; ++it) {
     const int i = (l + it * LPR) * 8;
     if (i < H) xv[it] = *reinterpret_cast<const bf16x8*>(xr + i);
+  }
+  if constexpr (ADD) {
+    bf16x8 dv[ITERS];
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+      const int i = (l + it * LPR) * 8;
+      if (i < H) dv[it] = *reinterpret_cast<const bf16x8*>(delta + row * H + i);
+    }
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+      const int i = (l + it * LPR) * 8;
+      if (i < H) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) xv[it].v[j] = f2bf(bf2f(xv[it].v[j]) + bf2f(dv[it].v[j]));
+        *reinterpret_cast<bf16x8*>(sum + row * H + i) = xv[it];
+      }
+    }
   }
 #pragma unroll
   for (int it = 0; it < ITERS; ++it)
@@ -107,13 +131,15 @@ __global__ __launch_bounds__(256) void rms_norm_fwd_long_kernel(const bf16* __re
   }
 }
 
-// dx_i = inv * dy_i*w_i - x_i * inv^3 / H * sum_j(dy_j*w_j*x_j)
+// dx_i = inv * dy_i*w_i - x_i * inv^3 / H * sum_j(dy_j*w_j*x_j) + dres_i
 // part[block][i] = sum over the block's rows of dy_i * x_i * inv
+// dres (the other gradient of x) and part (wanted weight gradient) may be null
 template <int LPR, int ITERS>
 __global__ __launch_bounds__(256) void rms_norm_bwd_kernel(const bf16* __restrict__ dy,
                                                            const bf16* __restrict__ x,
                                                            const bf16* __restrict__ w,
                                                            const float* __restrict__ invrms,
+                                                           const bf16* __restrict__ dres,
                                                            bf16* __restrict__ dx,
                                                            float* __restrict__ part, long T, int H) {
   constexpr int ROWS = 256 / LPR;      // rows at a time
@@ -128,11 +154,13 @@ __global__ __launch_bounds__(256) void rms_norm_bwd_kernel(const bf16* __restric
 
   for (long row = (long)blockIdx.x * ROWS + threadIdx.x / LPR; row < T; row += (long)gridDim.x * ROWS) {
     const float inv = invrms[row];
-    bf16x8 xv[ITERS], dv[ITERS];
+    bf16x8 xv[ITERS], dv[ITERS], rv[ITERS];
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
       const int i = (l + it * LPR) * 8;
+      rv[it] = bf16x8{};
       if (i < H) {
+        if (dres) rv[it] = *reinterpret_cast<const bf16x8*>(dres + row * H + i);
         xv[it] = *reinterpret_cast<const bf16x8*>(x + row * H + i);
         dv[it] = *reinterpret_cast<const bf16x8*>(dy + row * H + i);
       }
@@ -161,12 +189,14 @@ __global__ __launch_bounds__(256) void rms_norm_bwd_kernel(const bf16* __restric
         bf16x8 out;
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          out.v[j] = f2bf(inv * bf2f(dv[it].v[j]) * bf2f(wv.v[j]) - bf2f(xv[it].v[j]) * c);
+          out.v[j] = f2bf(inv * bf2f(dv[it].v[j]) * bf2f(wv.v[j]) - bf2f(xv[it].v[j]) * c +
+                          bf2f(rv[it].v[j]));
         *reinterpret_cast<bf16x8*>(dx + row * H + i) = out;
       }
     }
   }
 
+  if (!part) return;
   // the block's sums: over the wave's parts by shuffles, over the waves in LDS
   float* to = part + (long)blockIdx.x * H;
 #pragma unroll
@@ -241,6 +271,27 @@ constexpr int MAX_IN_REGISTERS = 16384;
 
 }  // namespace
 
+namespace {
+
+const bf16* data(const at::Tensor& t) { return reinterpret_cast<const bf16*>(t.data_ptr()); }
+bf16* out(const at::Tensor& t) { return reinterpret_cast<bf16*>(t.data_ptr()); }
+
+template <bool ADD>
+void launch_fwd(const at::Tensor& x, const bf16* delta, bf16* sum, const at::Tensor& w,
+                const at::Tensor& y, const at::Tensor& invrms, double eps) {
+  const long T = x.size(0);
+  const int H = x.size(1);
+  by_row_size(H, [&](auto lpr, auto iters) {
+    constexpr int LPR = lpr.value, ITERS = iters.value;
+    hipLaunchKernelGGL((rms_norm_fwd_kernel<LPR, ITERS, ADD>), dim3(ceil_div_i(T, 256 / LPR)),
+                       dim3(256), 0, c10::hip::getCurrentHIPStream().stream(), data(x), delta, sum,
+                       data(w), out(y), invrms.data_ptr<float>(), T, H, (float)eps);
+  });
+  HIP_CHECK_KERNEL();
+}
+
+}  // namespace
+
 std::tuple<at::Tensor, at::Tensor> rms_norm_fwd(const at::Tensor& x,
                                                 const at::Tensor& w,
                                                 double eps) {
@@ -251,35 +302,51 @@ std::tuple<at::Tensor, at::Tensor> rms_norm_fwd(const at::Tensor& x,
   TORCH_CHECK(H % 8 == 0, "rms_norm_fwd: H must be a multiple of 8, got ", H);
   auto y = at::empty_like(x);
   auto invrms = at::empty({T}, x.options().dtype(at::kFloat));
-  auto stream = c10::hip::getCurrentHIPStream().stream();
   if (H > MAX_IN_REGISTERS) {
-    hipLaunchKernelGGL(rms_norm_fwd_long_kernel, dim3(T), dim3(256), 0, stream,
-                       reinterpret_cast<const bf16*>(x.data_ptr()),
-                       reinterpret_cast<const bf16*>(w.data_ptr()),
-                       reinterpret_cast<bf16*>(y.data_ptr()), invrms.data_ptr<float>(), H, (float)eps);
+    hipLaunchKernelGGL(rms_norm_fwd_long_kernel, dim3(T), dim3(256), 0,
+                       c10::hip::getCurrentHIPStream().stream(), data(x), data(w), out(y),
+                       invrms.data_ptr<float>(), H, (float)eps);
     HIP_CHECK_KERNEL();
     return {y, invrms};
   }
-  by_row_size(H, [&](auto lpr, auto iters) {
-    constexpr int LPR = lpr.value, ITERS = iters.value;
-    hipLaunchKernelGGL((rms_norm_fwd_kernel<LPR, ITERS>), dim3(ceil_div_i(T, 256 / LPR)), dim3(256), 0,
-                       stream, reinterpret_cast<const bf16*>(x.data_ptr()),
-                       reinterpret_cast<const bf16*>(w.data_ptr()),
-                       reinterpret_cast<bf16*>(y.data_ptr()), invrms.data_ptr<float>(), T, H,
-                       (float)eps);
-  });
-  HIP_CHECK_KERNEL();
+  launch_fwd<false>(x, nullptr, nullptr, w, y, invrms, eps);
   return {y, invrms};
 }
 
+// -> x + delta, its norm, invrms
+std::tuple<at::Tensor, at::Tensor, at::Tensor> add_rms_norm_fwd(const at::Tensor& x,
+                                                                const at::Tensor& delta,
+                                                                const at::Tensor& w, double eps) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.scalar_type() == at::kBFloat16 &&
+                  x.is_contiguous() && x.size(0) >= 1,
+              "add_rms_norm_fwd: x [T, H] bf16");
+  TORCH_CHECK(delta.device() == x.device() && delta.sizes() == x.sizes() &&
+                  delta.scalar_type() == at::kBFloat16 && delta.is_contiguous(),
+              "add_rms_norm_fwd: delta as x");
+  TORCH_CHECK(w.device() == x.device() && w.scalar_type() == at::kBFloat16 && w.dim() == 1 &&
+                  w.size(0) == x.size(1) && w.is_contiguous() && x.size(1) % 8 == 0 &&
+                  x.size(1) <= MAX_IN_REGISTERS,
+              "add_rms_norm_fwd: w [H] bf16, H a multiple of 8 and at most ", MAX_IN_REGISTERS);
+  auto sum = at::empty_like(x), y = at::empty_like(x);
+  auto invrms = at::empty({x.size(0)}, x.options().dtype(at::kFloat));
+  launch_fwd<true>(x, data(delta), out(sum), w, y, invrms, eps);
+  return {sum, y, invrms};
+}
+
+// -> dx (+ dres), dw (undefined if it is not wanted)
 std::tuple<at::Tensor, at::Tensor> rms_norm_bwd(const at::Tensor& dy,
                                                 const at::Tensor& x,
                                                 const at::Tensor& w,
-                                                const at::Tensor& invrms) {
+                                                const at::Tensor& invrms,
+                                                const std::optional<at::Tensor>& dres,
+                                                bool want_dw) {
   const long T = x.size(0);
   const int H = x.size(1);
+  TORCH_CHECK(!dres || (dres->device() == x.device() && dres->sizes() == x.sizes() &&
+                        dres->scalar_type() == at::kBFloat16 && dres->is_contiguous()),
+              "rms_norm_bwd: dres as x");
   auto dx = at::empty_like(x);
-  auto dw = at::empty({H}, x.options());
+  at::Tensor dw, part;
   auto stream = c10::hip::getCurrentHIPStream().stream();
   by_row_size(H, [&](auto lpr, auto iters) {
     constexpr int LPR = lpr.value, ITERS = iters.value;
@@ -287,14 +354,17 @@ std::tuple<at::Tensor, at::Tensor> rms_norm_bwd(const at::Tensor& dy,
     // read again (8192 x 4096: 52 us with 512, 44 with 1024, 53 with 2048; 6001 x 2048,
     // where a wave has a row of its own: 28 with 256, 24 with 512, 29 with 1024)
     const int blocks = (int)std::min<long>((T + 256 / LPR - 1) / (256 / LPR), LPR > 64 ? 1024 : 512);
-    auto part = at::empty({blocks, H}, x.options().dtype(at::kFloat));
+    if (want_dw) {
+      dw = at::empty({H}, x.options());
+      part = at::empty({blocks, H}, x.options().dtype(at::kFloat));
+    }
     hipLaunchKernelGGL((rms_norm_bwd_kernel<LPR, ITERS>), dim3(blocks), dim3(256), 0, stream,
-                       reinterpret_cast<const bf16*>(dy.data_ptr()),
-                       reinterpret_cast<const bf16*>(x.data_ptr()),
-                       reinterpret_cast<const bf16*>(w.data_ptr()), invrms.data_ptr<float>(),
-                       reinterpret_cast<bf16*>(dx.data_ptr()), part.data_ptr<float>(), T, H);
-    hipLaunchKernelGGL(rms_norm_dw_kernel, dim3(ceil_div_i(H, 64)), dim3(256), 0, stream,
-                       part.data_ptr<float>(), reinterpret_cast<bf16*>(dw.data_ptr()), blocks, H);
+                       data(dy), data(x), data(w), invrms.data_ptr<float>(),
+                       dres ? data(*dres) : nullptr, out(dx),
+                       want_dw ? part.data_ptr<float>() : nullptr, T, H);
+    if (want_dw)
+      hipLaunchKernelGGL(rms_norm_dw_kernel, dim3(ceil_div_i(H, 64)), dim3(256), 0, stream,
+                         part.data_ptr<float>(), out(dw), blocks, H);
   });
   HIP_CHECK_KERNEL();
   return {dx, dw};
