@@ -2,14 +2,15 @@
 
 MI355X-native equivalent of the reference's cut-cross-entropy path
 (nemo_automodel/components/loss/linear_ce.py:130-265): the [T, V] logits tensor
-(V≈128k for Llama-3 → 2 GB per microbatch at T=8k, bf16) is never stored.
+(V≈128k for Llama-3 → 2 GB per microbatch at T=8k, bf16) is not stored, apart from
+what the backward's memory has room for anyway (see ``_kept_chunks``).
 
 Three implementations behind one autograd Function interface:
   * "hip_fused": csrc/fused_ce.hip — single-pass vocab-tiled MFMA stats GEMM
     forward (no logits tensor at any point); backward recomputes chunked
     through hipBLASLt + in-place HIP CE epilogue, reusing the forward's lse.
   * "hybrid": chunked hipBLASLt GEMM + HIP CE-epilogue kernels fwd AND bwd
-    (one [chunk, V] bf16 buffer alive at a time).
+    (one [chunk, V] bf16 buffer alive at a time beside the kept chunks).
   * "chunked": token-chunked torch path (CPU tests + fallback).
 
 Both return the SUM of per-token losses over labels != ignore_index.
@@ -67,48 +68,79 @@ class _ChunkedLinearCE(torch.autograd.Function):
         return dh, dw.to(weight.dtype), None, None
 
 
-class _HybridLinearCE(torch.autograd.Function):
-    """hipBLASLt GEMMs + HIP CE-epilogue kernels (csrc/ce_logits.hip).
+def _kept_chunks(T: int, H: int, V: int, chunk_size: int) -> int:
+    """How many leading chunks' logits stay until the backward, instead of their GEMM
+    being run again.
 
-    The [T, V] logits tensor never exists — only one [chunk, V] bf16 buffer.
-    Backward recomputes the chunk logits (GEMM), turns them into d(logits)
-    in place (one bf16 pass), then dH / dW are plain bf16 GEMMs.
-    """
+    Kept logits add to the backward's peak, so they get what it no longer takes: it used
+    to hold the weight's gradient in float32, a bf16 part of it and that part in float32,
+    10 V H bytes in all, now 6 V H. 8192 rows x 4096, V = 32768: 1.6 ms less GEMM of a
+    step with 8 of them."""
+    return min(4 * V * H // (2 * chunk_size * V), -(-T // chunk_size))
+
+
+def _chunk_grads(ctx, dloss: torch.Tensor):
+    """d(hidden), d(weight) of the summed loss, chunk by chunk: logits (kept, or a GEMM
+    again), d(logits) over them in one bf16 pass, then two plain bf16 GEMMs."""
+    ops = hip_ops()
+    hidden, weight, labels, lse_all, *kept = ctx.saved_tensors
+    need_h, need_w = ctx.needs_input_grad[:2]
+    T, chunk_size = hidden.shape[0], ctx.chunk_size
+    dh = torch.empty_like(hidden) if need_h else None
+    dw = None
+    d = dloss.reshape(1).float().contiguous()
+    chunks = range(0, T, chunk_size)
+    for i, s in enumerate(chunks):
+        rows = slice(s, s + chunk_size)
+        h, y, lse = hidden[rows], labels[rows], lse_all[rows]
+        if i < len(kept):                      # stays as it is: the graph may be run again
+            g = ops.ce_grad_logits(kept[i], y, lse, d, 0)
+        else:
+            g = h @ weight.t()
+            ops.ce_bwd_logits(g, y, lse, d, 0)
+        if need_h:
+            dh[rows] = g @ weight
+        if need_w:
+            part = g.t() @ h
+            # sums of three and more parts in float32; of two, rounding their float32 sum
+            # once is what a bf16 addition does
+            if dw is None:
+                dw = part.float() if len(chunks) > 2 else part
+            else:
+                dw += part
+        del g
+    if need_w:
+        dw = torch.zeros_like(weight) if dw is None else dw.to(weight.dtype)
+    return dh, dw
+
+
+class _HybridLinearCE(torch.autograd.Function):
+    """hipBLASLt GEMMs + HIP CE-epilogue kernels (csrc/ce_logits.hip)."""
 
     @staticmethod
     def forward(ctx, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor,
-                chunk_size: int):
+                chunk_size: int, keep: bool):
         ops = hip_ops()
-        T = hidden.shape[0]
+        T, H = hidden.shape
         loss_sum = torch.zeros(1, dtype=torch.float32, device=hidden.device)
         lse_all = torch.empty(T, dtype=torch.float32, device=hidden.device)
         wt = weight.t()
-        for s in range(0, T, chunk_size):
+        n_kept = _kept_chunks(T, H, weight.shape[0], chunk_size) if keep else 0
+        kept = []
+        for i, s in enumerate(range(0, T, chunk_size)):
             logits = hidden[s : s + chunk_size] @ wt
             lse, _ = ops.ce_fwd_logits(logits, labels[s : s + chunk_size], loss_sum)
             lse_all[s : s + chunk_size] = lse
-        ctx.save_for_backward(hidden, weight, labels, lse_all)
+            if i < n_kept:
+                kept.append(logits)
+            del logits
+        ctx.save_for_backward(hidden, weight, labels, lse_all, *kept)
         ctx.chunk_size = chunk_size
         return loss_sum.squeeze(0)
 
     @staticmethod
     def backward(ctx, dloss: torch.Tensor):
-        ops = hip_ops()
-        hidden, weight, labels, lse_all = ctx.saved_tensors
-        chunk_size = ctx.chunk_size
-        T = hidden.shape[0]
-        dh = torch.empty_like(hidden)
-        dw = torch.zeros_like(weight, dtype=torch.float32)
-        d = dloss.reshape(1).float().contiguous()
-        wt = weight.t()
-        for s in range(0, T, chunk_size):
-            h = hidden[s : s + chunk_size]
-            y = labels[s : s + chunk_size]
-            logits = h @ wt                       # recompute (bf16 GEMM)
-            ops.ce_bwd_logits(logits, y, lse_all[s : s + chunk_size], d, 0)
-            dh[s : s + chunk_size] = logits @ weight
-            dw += (logits.t() @ h).float()
-        return dh, dw.to(weight.dtype), None, None
+        return *_chunk_grads(ctx, dloss), None, None, None
 
 
 class _FusedLinearCEHip(torch.autograd.Function):
@@ -129,22 +161,7 @@ class _FusedLinearCEHip(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dloss):
-        ops = hip_ops()
-        hidden, weight, labels, lse_all = ctx.saved_tensors
-        chunk_size = ctx.chunk_size
-        T = hidden.shape[0]
-        dh = torch.empty_like(hidden)
-        dw = torch.zeros_like(weight, dtype=torch.float32)
-        d = dloss.reshape(1).float().contiguous()
-        wt = weight.t()
-        for s in range(0, T, chunk_size):
-            h = hidden[s : s + chunk_size]
-            y = labels[s : s + chunk_size]
-            logits = h @ wt                       # recompute (bf16 GEMM)
-            ops.ce_bwd_logits(logits, y, lse_all[s : s + chunk_size], d, 0)
-            dh[s : s + chunk_size] = logits @ weight
-            dw += (logits.t() @ h).float()
-        return dh, dw.to(weight.dtype), None, None
+        return *_chunk_grads(ctx, dloss), None, None
 
 
 def fused_linear_cross_entropy(
@@ -153,27 +170,35 @@ def fused_linear_cross_entropy(
     labels: torch.Tensor,
     backend: str = "hybrid",
     chunk_size: int = 4096,
+    keep_logits: bool = True,
 ) -> torch.Tensor:
-    """hidden [*, H] -> flattened [T, H]; labels [*] -> [T]. Returns loss SUM."""
+    """hidden [*, H] -> flattened [T, H]; labels [*] -> [T]. Returns loss SUM.
+
+    ``keep_logits=False``: none stay from the forward for the backward ("hybrid"), for
+    callers that run many forwards before their backwards."""
     hidden = hidden.reshape(-1, hidden.shape[-1])
     labels = labels.reshape(-1)
     if hidden.is_cuda and backend == "hip_fused":
         return _FusedLinearCEHip.apply(hidden, weight, labels.to(torch.long), chunk_size)
     if hidden.is_cuda and backend == "hybrid":
-        return _HybridLinearCE.apply(hidden, weight, labels, chunk_size)
+        keep = keep_logits and torch.is_grad_enabled()
+        return _HybridLinearCE.apply(hidden, weight, labels, chunk_size, keep)
     return _ChunkedLinearCE.apply(hidden, weight, labels, chunk_size)
 
 
 class FusedLinearCrossEntropy(torch.nn.Module):
     """Loss module the recipe calls with (hidden_states, lm_head_weight, labels)."""
 
-    def __init__(self, backend: str = "hybrid", chunk_size: int = 4096):
+    def __init__(self, backend: str = "hybrid", chunk_size: int = 4096,
+                 keep_logits: bool = True):
         super().__init__()
         self.backend = backend
         self.chunk_size = chunk_size
+        self.keep_logits = keep_logits
 
     def forward(self, hidden, weight, labels):
         backend = self.backend if hidden.is_cuda else "chunked"
         return fused_linear_cross_entropy(
-            hidden, weight, labels, backend=backend, chunk_size=self.chunk_size
+            hidden, weight, labels, backend=backend, chunk_size=self.chunk_size,
+            keep_logits=self.keep_logits
         )

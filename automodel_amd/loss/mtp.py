@@ -52,7 +52,7 @@ def calculate_mtp_loss(
     mtp_hidden = mtp_head(h, nxt)
     mtp_labels = labels[:, 1:].contiguous()
     return fused_linear_cross_entropy(
-        mtp_hidden, lm_head_weight, mtp_labels, backend=loss_backend)
+        mtp_hidden, lm_head_weight, mtp_labels, backend=loss_backend, keep_logits=False)
 
 
 def _roll_mask(t: torch.Tensor, k: int, fill) -> torch.Tensor:
@@ -115,7 +115,7 @@ def calculate_mtp_loss_multi(
         cur = mtp_heads.heads[k - 1](cur, embed_tokens(ids_k))
         lk = fused_linear_cross_entropy(cur, lm_head_weight,
                                         labels_k.contiguous(),
-                                        backend=loss_backend)
+                                        backend=loss_backend, keep_logits=False)
         per_depth.append(lk)
         total = lk if total is None else total + lk
     total = total * scaling_factor

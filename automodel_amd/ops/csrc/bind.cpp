@@ -50,6 +50,8 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("ce_fwd_logits", &amd_ops::ce_fwd_logits);
   m.def("ce_bwd_logits(Tensor(a!) logits, Tensor labels, Tensor lse, Tensor dloss, int vocab_offset=0) -> ()");
   m.impl("ce_bwd_logits", &amd_ops::ce_bwd_logits);
+  m.def("ce_grad_logits(Tensor logits, Tensor labels, Tensor lse, Tensor dloss, int vocab_offset=0) -> Tensor");
+  m.impl("ce_grad_logits", &amd_ops::ce_grad_logits);
   m.def("ce_stats_logits(Tensor logits) -> (Tensor, Tensor)");
   m.impl("ce_stats_logits", &amd_ops::ce_stats_logits);
 

@@ -8,10 +8,11 @@
 //     torch ops measured in profiles/bench8b round-1).
 //   ce_bwd_logits: overwrites logits IN PLACE with d(logits) =
 //     (softmax - onehot(label)) * dloss — single bf16 read+write pass.
+//     ce_grad_logits: the same into a new buffer.
 //
 // Together with the GEMMs this is the MI355X equivalent of cut-cross-entropy
-// (reference loss/linear_ce.py:253): the full [T, V] logits tensor never
-// exists, only one [chunk, V] bf16 buffer.
+// (reference loss/linear_ce.py:253): one [chunk, V] bf16 buffer at a time, and
+// the chunks that the caller chooses to keep for the backward.
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -107,8 +108,8 @@ __global__ void ce_stats_logits_kernel(const bf16* __restrict__ logits,
   }
 }
 
-// grad in place: g = (exp(x - lse) - onehot) * dloss ; ignored rows -> 0.
-__global__ void ce_bwd_logits_kernel(bf16* __restrict__ logits,
+// g = (exp(x - lse) - onehot) * dloss ; ignored rows -> 0. grad may be logits.
+__global__ void ce_bwd_logits_kernel(const bf16* logits, bf16* grad,
                                      const long* __restrict__ labels,
                                      const float* __restrict__ lse,
                                      const float* __restrict__ dloss,
@@ -118,11 +119,11 @@ __global__ void ce_bwd_logits_kernel(bf16* __restrict__ logits,
   const long y = (y_raw == ignore_index) ? ignore_index : y_raw - vocab_offset;
   const float d = dloss[0];
   const float l = lse[row];
-  bf16* x = logits + row * (long)V;
+  const bf16* x = logits + row * (long)V;
   const bool ignored = (y_raw == ignore_index);
   for (int i = (blockIdx.x * blockDim.x + threadIdx.x) * 8; i < V;
        i += gridDim.x * blockDim.x * 8) {
-    bf16x8 xv = *reinterpret_cast<bf16x8*>(x + i);
+    bf16x8 xv = *reinterpret_cast<const bf16x8*>(x + i);
     bf16x8 out;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -131,7 +132,7 @@ __global__ void ce_bwd_logits_kernel(bf16* __restrict__ logits,
       if ((long)(i + j) == y) p -= 1.f;
       out.v[j] = f2bf(p * d);
     }
-    *reinterpret_cast<bf16x8*>(x + i) = out;
+    *reinterpret_cast<bf16x8*>(grad + row * (long)V + i) = out;
   }
 }
 
@@ -156,8 +157,8 @@ std::tuple<at::Tensor, at::Tensor> ce_fwd_logits(const at::Tensor& logits,
   return {lse, loss_sum};
 }
 
-void ce_bwd_logits(at::Tensor logits, const at::Tensor& labels, const at::Tensor& lse,
-                   const at::Tensor& dloss, int64_t vocab_offset) {
+static void ce_grad(const at::Tensor& logits, const at::Tensor& grad, const at::Tensor& labels,
+                    const at::Tensor& lse, const at::Tensor& dloss, int64_t vocab_offset) {
   const long T = logits.size(0);
   const int V = logits.size(1);
   TORCH_CHECK(V % 8 == 0, "ce_bwd_logits: V must be a multiple of 8");
@@ -165,10 +166,26 @@ void ce_bwd_logits(at::Tensor logits, const at::Tensor& labels, const at::Tensor
   const int gx = std::min(64, (V / 8 + block - 1) / block);
   auto stream = c10::hip::getCurrentHIPStream();
   hipLaunchKernelGGL(ce_bwd_logits_kernel, dim3(gx, T), dim3(block), 0, stream.stream(),
-                     reinterpret_cast<bf16*>(logits.data_ptr()),
-                     labels.data_ptr<long>(), lse.data_ptr<float>(),
-                     dloss.data_ptr<float>(), V, -100, vocab_offset);
+                     reinterpret_cast<const bf16*>(logits.data_ptr()),
+                     reinterpret_cast<bf16*>(grad.data_ptr()), labels.data_ptr<long>(),
+                     lse.data_ptr<float>(), dloss.data_ptr<float>(), V, -100, vocab_offset);
   HIP_CHECK_KERNEL();
+}
+
+void ce_bwd_logits(at::Tensor logits, const at::Tensor& labels, const at::Tensor& lse,
+                   const at::Tensor& dloss, int64_t vocab_offset) {
+  ce_grad(logits, logits, labels, lse, dloss, vocab_offset);
+}
+
+at::Tensor ce_grad_logits(const at::Tensor& logits, const at::Tensor& labels,
+                          const at::Tensor& lse, const at::Tensor& dloss, int64_t vocab_offset) {
+  TORCH_CHECK(logits.is_cuda() && logits.dim() == 2 && logits.is_contiguous() &&
+                  logits.scalar_type() == at::kBFloat16 && labels.numel() == logits.size(0) &&
+                  lse.numel() == logits.size(0),
+              "ce_grad_logits: logits [T,V] bf16, labels and lse [T]");
+  auto grad = at::empty_like(logits);
+  ce_grad(logits, grad, labels, lse, dloss, vocab_offset);
+  return grad;
 }
 
 std::tuple<at::Tensor, at::Tensor> ce_stats_logits(const at::Tensor& logits) {

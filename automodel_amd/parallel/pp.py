@@ -28,6 +28,8 @@ from torch.distributed.device_mesh import DeviceMesh
 from torch.distributed.pipelining import PipelineStage, Schedule1F1B, ScheduleGPipe
 from torch.distributed.pipelining.schedules import ScheduleInterleaved1F1B
 
+from automodel_amd.loss.linear_ce import FusedLinearCrossEntropy
+
 
 @dataclass
 class PipelineConfig:
@@ -145,7 +147,11 @@ class AutoPipeline:
 
         def schedule_loss(output, target):
             # last-stage hidden -> fused linear CE against lm_head weight
-            return last_mod.loss_fn(output, last_mod.lm_head.weight, target)
+            loss = last_mod.loss_fn
+            if config.schedule == "gpipe" and isinstance(loss, FusedLinearCrossEntropy):
+                # every forward comes before the first backward: keep no logits meanwhile
+                loss = FusedLinearCrossEntropy(loss.backend, loss.chunk_size, keep_logits=False)
+            return loss(output, last_mod.lm_head.weight, target)
 
         sched_cls = {
             "1f1b": Schedule1F1B,
