@@ -25,109 +25,10 @@ namespace amd_ops {
 void latent_check_rope(const at::Tensor& cos, const at::Tensor& sin, int64_t rot);
 void latent_check_cache(const at::Tensor& cache, at::ScalarType dt, int64_t rank, int64_t rot);
 
-// ---------------------------------------------------------------------------
-// prep: blockIdx.x < H * NC absorbs 16*V latent columns of one head for RT
-// rows (16 column groups x 16 slices of the head dim, then a reduction);
-// the last blockIdx.x writes the rows' latents into the cache.
-// ---------------------------------------------------------------------------
-template <typename T, int V, int RT>
-__global__ __launch_bounds__(256) void latent_decode_prep_kernel(
-    const T* __restrict__ qkv, const T* __restrict__ w_uk, const T* __restrict__ w_norm, float eps,
-    const float* __restrict__ cosb, const float* __restrict__ sinb, int n_pos, int cs_stride,
-    const int* __restrict__ pos, const int* __restrict__ slot, T* __restrict__ cache, int n_slots,
-    int max_len, T* __restrict__ q_out, int R, int H, int dn, int dr, int rank, int NC) {
-  extern __shared__ float sm[];
-  const int tid = threadIdx.x;
-  const int r0 = blockIdx.y * RT;
-  const int hd = dn + dr, RP = pad32(rank), C = RP + pad32(dr);
-  const long N = (long)H * hd + rank + dr;
-  if ((int)blockIdx.x == H * NC) {
-    for (int r = r0; r < min(r0 + RT, R); ++r) {
-      const int p = min(max(pos[r], 0), n_pos - 1);
-      const long cr = cache_row(slot[r], pos[r], n_slots, max_len);
-      latent_token<T>(qkv + r * N + (long)H * hd, w_norm, eps, cosb + (long)p * cs_stride,
-                      sinb + (long)p * cs_stride, rank, dr, cr >= 0 ? cache + cr * C : nullptr,
-                      (T*)nullptr, (T*)nullptr, sm);
-    }
-    return;
-  }
-  const int h = blockIdx.x / NC, nc = blockIdx.x % NC;
-  float* qs = sm;                                 // [RT][dn]
-  float* part = sm + RT * dn;                     // [4 waves][RT][16*V]
-  for (int i = tid; i < RT * dn; i += 256) {
-    const int r = r0 + i / dn;
-    qs[i] = r < R ? lat_f(qkv[r * N + h * hd + i % dn]) : 0.f;
-  }
-  if (nc == 0) {                                  // rotated part and zero padding
-    const int half = dr / 2;
-    for (int rr = 0; rr < RT; ++rr) {
-      const int r = r0 + rr;
-      if (r >= R) break;
-      T* o = q_out + ((long)r * H + h) * C;
-      const T* src = qkv + r * N + h * hd + dn;
-      const int p = min(max(pos[r], 0), n_pos - 1);
-      for (int i = tid; i < half; i += 256) {
-        const float c = cosb[(long)p * cs_stride + i], s = sinb[(long)p * cs_stride + i];
-        const float u = lat_f(src[i]), v = lat_f(src[half + i]);
-        o[RP + i] = lat_t<T>(u * c - v * s);
-        o[RP + half + i] = lat_t<T>(v * c + u * s);
-      }
-      for (int i = rank + tid; i < RP; i += 256) o[i] = lat_t<T>(0.f);
-      for (int i = RP + dr + tid; i < C; i += 256) o[i] = lat_t<T>(0.f);
-    }
-  }
-  __syncthreads();
-  const int vec = tid & 15, slice = tid >> 4;     // 16 columns groups x 16 slices
-  const int col = (nc * 16 + vec) * V;
-  float acc[RT][V];
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int j = 0; j < V; ++j) acc[r][j] = 0.f;
-  if (col < rank) {                               // V divides rank
-    const T* wp = w_uk + (long)h * dn * rank + col;
-#pragma unroll 4
-    for (int d = slice; d < dn; d += 16) {
-      const LatPack<T, V> w = *reinterpret_cast<const LatPack<T, V>*>(wp + (long)d * rank);
-#pragma unroll
-      for (int r = 0; r < RT; ++r) {
-        const float qv = qs[r * dn + d];
-#pragma unroll
-        for (int j = 0; j < V; ++j) acc[r][j] = fmaf(qv, lat_f(w.v[j]), acc[r][j]);
-      }
-    }
-  }
-  const int lane = tid & 63, wid = tid >> 6;
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int j = 0; j < V; ++j) {
-      float a = acc[r][j];
-      a += __shfl_xor(a, 16);
-      a += __shfl_xor(a, 32);
-      if (lane < 16) part[(wid * RT + r) * 16 * V + vec * V + j] = a;
-    }
-  __syncthreads();
-  for (int i = tid; i < RT * 16 * V; i += 256) {
-    const int r = r0 + i / (16 * V), c = nc * 16 * V + i % (16 * V);
-    if (r >= R || c >= rank) continue;
-    float a = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) a += part[w * RT * 16 * V + i];
-    q_out[((long)r * H + h) * C + c] = lat_t<T>(a);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// attention over the cache. grid (splits, head groups of 16*HT, rows)
-// ---------------------------------------------------------------------------
 typedef __bf16 lat_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 lat_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float lat_f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned lat_u32x4 __attribute__((ext_vector_type(4)));    // 16 bytes in flight
-
-constexpr int LD_KEYS = 64;           // keys per tile: 4 waves x 16
-constexpr int LD_PSTRIDE = LD_KEYS * 2 + 16;
 
 // hardware-transposed read: 16 lanes fetch a [4 keys][16 columns] block, lane g
 // receives column g (each lane supplies the address of its own 8 bytes)
@@ -137,28 +38,224 @@ __device__ __forceinline__ lat_bf16x4 lds_tr16(const char* p) {
       (lds_ptr)(__attribute__((address_space(3))) char*)const_cast<char*>(p));
 }
 
-// HT: head tiles (of 16 heads) per workgroup, four waves each; they share the
-// staged keys. NCT: 16-column value tiles per wave (4 waves cover RP <= 64 *
-// NCT). NPM: bound on the 16-byte pieces of a key tile per thread. The next
-// tile travels through registers while the current one is used.
-template <int HT, int NCT, int NPM>
-__global__ __launch_bounds__(256 * HT) void latent_decode_attn_kernel(
+// ---------------------------------------------------------------------------
+// prep: blockIdx.x < H * NC absorbs 8*V latent columns of one head for RT rows
+// (8 column groups x 32 slices of the head dim, then a reduction); RT more
+// workgroups each write a row's latent into the cache. All of it is latency:
+// 64 columns per workgroup, so that 32 heads give one to each CU, and no loop
+// over rows where a row ends in a barrier (8 rows, 32 heads, rank 512: 13.5 us
+// with one workgroup for all rows' latents, 11.3 now).
+// ---------------------------------------------------------------------------
+constexpr int LP_VECS = 8;
+template <typename T, int V, int RT>
+__global__ __launch_bounds__(256) void latent_decode_prep_kernel(
+    const T* __restrict__ qkv, const T* __restrict__ w_uk, const T* __restrict__ w_norm, float eps,
+    const float* __restrict__ cosb, const float* __restrict__ sinb, int n_pos, int cs_stride,
+    const int* __restrict__ pos, const int* __restrict__ slot, T* __restrict__ cache, int n_slots,
+    int max_len, T* __restrict__ q_out, int R, int H, int dn, int dr, int rank, int NC) {
+  extern __shared__ float sm[];
+  constexpr int COLS = LP_VECS * V, SLICES = 256 / LP_VECS;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int r0 = blockIdx.y * RT;
+  const int hd = dn + dr, RP = pad32(rank), C = RP + pad32(dr);
+  const long N = (long)H * hd + rank + dr;
+  if ((int)blockIdx.x >= H * NC) {
+    const int r = r0 + blockIdx.x - H * NC;
+    if (r >= R) return;
+    const int p = min(max(pos[r], 0), n_pos - 1);
+    const long cr = cache_row(slot[r], pos[r], n_slots, max_len);
+    latent_token<T>(qkv + r * N + (long)H * hd, w_norm, eps, cosb + (long)p * cs_stride,
+                    sinb + (long)p * cs_stride, rank, dr, cr >= 0 ? cache + cr * C : nullptr,
+                    (T*)nullptr, (T*)nullptr, sm);
+    return;
+  }
+  const int h = blockIdx.x / NC, nc = blockIdx.x % NC;
+  float* qs = sm;                                 // [RT][dn]
+  float* part = sm + RT * dn;                     // [4 waves][RT][COLS]
+#pragma unroll
+  for (int rr = wid; rr < RT; rr += 4)
+    for (int i = lane; i < dn; i += 64)
+      qs[rr * dn + i] = r0 + rr < R ? lat_f(qkv[(r0 + rr) * N + h * hd + i]) : 0.f;
+  if (nc == 0) {                                  // rotated part and zero padding
+    const int half = dr / 2;
+#pragma unroll
+    for (int rr = wid; rr < RT; rr += 4) {
+      const int r = r0 + rr;
+      if (r >= R) break;
+      T* o = q_out + ((long)r * H + h) * C;
+      const T* src = qkv + r * N + h * hd + dn;
+      const int p = min(max(pos[r], 0), n_pos - 1);
+      for (int i = lane; i < half; i += 64) {
+        const float c = cosb[(long)p * cs_stride + i], s = sinb[(long)p * cs_stride + i];
+        const float u = lat_f(src[i]), v = lat_f(src[half + i]);
+        o[RP + i] = lat_t<T>(u * c - v * s);
+        o[RP + half + i] = lat_t<T>(v * c + u * s);
+      }
+      for (int i = rank + lane; i < RP; i += 64) o[i] = lat_t<T>(0.f);
+      for (int i = RP + dr + lane; i < C; i += 64) o[i] = lat_t<T>(0.f);
+    }
+  }
+  __syncthreads();
+  const int vec = tid % LP_VECS, slice = tid / LP_VECS;
+  const int col = nc * COLS + vec * V;
+  float acc[RT][V];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc[r][j] = 0.f;
+  if (col < rank) {                               // V divides rank
+    const T* wp = w_uk + (long)h * dn * rank + col;
+#pragma unroll 4
+    for (int d = slice; d < dn; d += SLICES) {
+      const LatPack<T, V> w = *reinterpret_cast<const LatPack<T, V>*>(wp + (long)d * rank);
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        const float qv = qs[r * dn + d];
+#pragma unroll
+        for (int j = 0; j < V; ++j) acc[r][j] = fmaf(qv, lat_f(w.v[j]), acc[r][j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      float a = acc[r][j];
+#pragma unroll
+      for (int d = LP_VECS; d < 64; d *= 2) a += __shfl_xor(a, d);
+      if (lane < LP_VECS) part[(wid * RT + r) * COLS + vec * V + j] = a;
+    }
+  __syncthreads();
+  for (int i = tid; i < RT * COLS; i += 256) {
+    const int r = r0 + i / COLS, c = nc * COLS + i % COLS;
+    if (r >= R || c >= rank) continue;
+    float a = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) a += part[w * RT * COLS + i];
+    q_out[((long)r * H + h) * C + c] = lat_t<T>(a);
+  }
+}
+
+// The same on the matrix cores, for bf16, a head dim in steps of 32 and rows in
+// whole 16-byte pieces: 16 rows at once, 64 columns of one head per workgroup, 16
+// per wave; W_uk goes through LDS to be read transposed. With rows in registers the
+// instructions themselves, each run once, took most of the time: 11.3 us for 8 rows,
+// 32 heads, 4.7 here; 1 row, 16 heads 3.6 and 3.4.
+constexpr int LPM_STRIDE = 64 * 2 + 16;           // LDS bytes per row of W_uk
+__global__ __launch_bounds__(256) void latent_decode_prep_mfma_kernel(
+    const bf16* __restrict__ qkv, const bf16* __restrict__ w_uk, const bf16* __restrict__ w_norm,
+    float eps, const float* __restrict__ cosb, const float* __restrict__ sinb, int n_pos,
+    int cs_stride, const int* __restrict__ pos, const int* __restrict__ slot,
+    bf16* __restrict__ cache, int n_slots, int max_len, bf16* __restrict__ q_out, int R, int H,
+    int dn, int dr, int rank, int NC) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];    // [dn][LPM_STRIDE]
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int lo16 = lane & 15, hi4 = lane >> 4;
+  const int r0 = blockIdx.y * 16;
+  const int hd = dn + dr, RP = pad32(rank), C = RP + pad32(dr);
+  const long N = (long)H * hd + rank + dr;
+  if ((int)blockIdx.x >= H * NC) {                // a row's latent
+    const int r = r0 + blockIdx.x - H * NC;
+    if (r >= R) return;
+    const int p = min(max(pos[r], 0), n_pos - 1);
+    const long cr = cache_row(slot[r], pos[r], n_slots, max_len);
+    latent_token<bf16>(qkv + r * N + (long)H * hd, w_norm, eps, cosb + (long)p * cs_stride,
+                       sinb + (long)p * cs_stride, rank, dr, cr >= 0 ? cache + cr * C : nullptr,
+                       (bf16*)nullptr, (bf16*)nullptr, reinterpret_cast<float*>(lds));
+    return;
+  }
+  const int h = blockIdx.x / NC, nc = blockIdx.x % NC;
+  const bf16* wp = w_uk + (long)h * dn * rank;
+#pragma unroll 4
+  for (int i = tid; i < dn * 8; i += 256) {
+    const int d = i >> 3, col = nc * 64 + (i & 7) * 8;
+    lat_u32x4 x = {0u, 0u, 0u, 0u};
+    if (col < rank) x = *reinterpret_cast<const lat_u32x4*>(wp + (long)d * rank + col);
+    *reinterpret_cast<lat_u32x4*>(lds + d * LPM_STRIDE + (i & 7) * 16) = x;
+  }
+  // the head's NC workgroups share the rows' rotated part and zero padding
+  for (int rr = nc * 4 + wid; rr < 16 && r0 + rr < R; rr += 4 * NC) {
+    const int r = r0 + rr, half = dr / 2;
+    bf16* o = q_out + ((long)r * H + h) * C;
+    const bf16* src = qkv + r * N + h * hd + dn;
+    const int p = min(max(pos[r], 0), n_pos - 1);
+    for (int i = lane; i < half; i += 64) {
+      const float c = cosb[(long)p * cs_stride + i], s = sinb[(long)p * cs_stride + i];
+      const float u = bf2f(src[i]), v = bf2f(src[half + i]);
+      o[RP + i] = f2bf(u * c - v * s);
+      o[RP + half + i] = f2bf(v * c + u * s);
+    }
+    for (int i = rank + lane; i < RP; i += 64) o[i] = f2bf(0.f);
+    for (int i = RP + dr + lane; i < C; i += 64) o[i] = f2bf(0.f);
+  }
+  __syncthreads();
+  const int r = r0 + lo16;
+  const bf16* qp = qkv + min(r, R - 1) * N + h * hd + hi4 * 8;
+  const char* wl = lds + (hi4 * 8 + (lo16 >> 2)) * LPM_STRIDE + wid * 32 + (lo16 & 3) * 8;
+  lat_f32x4 acc = {0.f, 0.f, 0.f, 0.f};           // D[column = 4 hi4 + i][row = lo16]
+#pragma unroll 4
+  for (int d = 0; d < dn; d += 32) {
+    const lat_bf16x8 qv = __builtin_bit_cast(lat_bf16x8, *reinterpret_cast<const lat_u32x4*>(qp + d));
+    const lat_bf16x4 w0 = lds_tr16(wl + d * LPM_STRIDE), w1 = lds_tr16(wl + (d + 4) * LPM_STRIDE);
+    const lat_bf16x8 wv = __builtin_shufflevector(w0, w1, 0, 1, 2, 3, 4, 5, 6, 7);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, qv, acc, 0, 0, 0);
+  }
+  const int col = nc * 64 + wid * 16 + hi4 * 4;
+  if (r < R && col < rank) {                      // rank % 8 == 0: all 4 columns or none
+    bf16x4 y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y.v[i] = f2bf(acc[i]);
+    *reinterpret_cast<bf16x4*>(q_out + ((long)r * H + h) * C + col) = y;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// attention over the cache. grid (splits, head groups of 16, rows)
+// ---------------------------------------------------------------------------
+constexpr int LD_KEYS = 64;           // keys per tile: 4 waves x 16
+constexpr int LD_PSTRIDE = LD_KEYS * 2 + 16;
+
+// 16 heads per workgroup (32, on the same staged keys, were no faster at 128 heads
+// and slower at 32). NCT: 16-column value tiles per wave (4 waves cover RP <= 64 *
+// NCT). NPM: bound on the 32-column steps of a row. One tile in LDS: a second
+// buffer for the next one was no faster, also at 8 tiles per split, and takes the
+// room of a second workgroup.
+//
+// A split is a tile or two, so this is a chain of latencies, and of instructions
+// that run once: both products put the head in the lane (columns of the
+// accumulator), so that the running maximum and scale are one value a lane, P goes
+// to LDS in one piece and the partial results leave in 16-byte stores; keys go to
+// LDS without registers in between; the queries sit in registers, which leaves LDS
+// for two workgroups per CU. With heads in the accumulator's rows, keys through
+// registers and queries in LDS: 9.7 us for 1 row, 16 heads, 200 keys and 20.9 for 8
+// rows, 32 heads, 1500 keys; now 7.0 and 12.4 (and 46 -> 49 for 8 rows of 16000).
+template <int NCT, int NPM>
+__global__ __launch_bounds__(256) void latent_decode_attn_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ cache, const int* __restrict__ slot,
     const int* __restrict__ pos, float* __restrict__ part_o, float* __restrict__ part_ml,
     int n_slots, int max_len, int H, int RP, int C, float scale) {
-  constexpr int NT = 256 * HT;
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  const int KS = C * 2 + 16;                      // LDS row stride: conflict-free b128 reads
+  const int KS = C * 2;
   char* kt = lds;                                 // [64][KS]
-  char* qt = kt + LD_KEYS * KS;                   // [16 HT][KS]
-  char* pt = qt + 16 * HT * KS;                   // [16 HT][LD_PSTRIDE]
-  float* red = reinterpret_cast<float*>(pt + 16 * HT * LD_PSTRIDE);   // [HT][4][16]
+  const unsigned kt_at = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  char* pt = kt + LD_KEYS * KS;                   // [16][LD_PSTRIDE]
+  float* red = reinterpret_cast<float*>(pt + 16 * LD_PSTRIDE);   // [4][16]
 
-  const int tid = threadIdx.x, lane = tid & 63, wid = (tid >> 6) & 3, ht = tid >> 8;
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lo16 = lane & 15, hi4 = lane >> 4;
   const int split = blockIdx.x, n_split = gridDim.x;
-  const int h0 = blockIdx.y * 16 * HT;
+  const int h = blockIdx.y * 16 + lo16;           // this lane's head
   const int r = blockIdx.z;
+
+  const int steps = C / 32;
+  lat_bf16x8 qf[NPM];                             // step j: columns 32j + 8 hi4 of head h
+  {
+    const bf16* qp = q + ((long)r * H + min(h, H - 1)) * C + hi4 * 8;
+#pragma unroll
+    for (int j = 0; j < NPM; ++j)
+      if (j < steps)                              // uniform
+        qf[j] = __builtin_bit_cast(lat_bf16x8, *reinterpret_cast<const lat_u32x4*>(qp + j * 32));
+  }
 
   const int sl = slot[r];
   const int n = (sl < 0 || sl >= n_slots) ? 0 : min(max(pos[r] + 1, 0), max_len);
@@ -167,109 +264,96 @@ __global__ __launch_bounds__(256 * HT) void latent_decode_attn_kernel(
   const int t_lo = split * per, t_hi = min(t_lo + per, tiles);
   const bf16* base = cache + (long)(n > 0 ? sl : 0) * max_len * C;
 
-  const int vecs = C / 8;                         // 16-byte pieces per row
-  const int pieces = LD_KEYS * vecs, np = (pieces + NT - 1) / NT;
+  // A tile lies in LDS without padding, row after row; piece c of row r sits at
+  // c ^ swz(r), which spreads the 16 rows of a read over the banks: the rows'
+  // starts repeat every 16 / g rows, g pieces apart (g: the largest power of two in
+  // a row's pieces, 16 at most)
+  const int vecs = C / 8;                         // 16-byte pieces per row, a multiple of 4
+  const int lg = min(__builtin_ctz(vecs), 4), sh = 4 - lg, gm = (1 << lg) - 1;
   const unsigned magic = ((1u << 20) + vecs - 1) / vecs;    // i / vecs, exact for i < 128 vecs
-  lat_u32x4 pre[NPM];
-  auto fetch = [&](int t) {
-#pragma unroll
-    for (int j = 0; j < NPM; ++j) {
-      if (j < np) {                               // uniform
-        const unsigned i = tid + j * NT, row = (i * magic) >> 20, c = i - row * vecs;
-        const int key = min(t * LD_KEYS + (int)row, n - 1);   // rows past the end: masked below
-        pre[j] = *reinterpret_cast<const lat_u32x4*>(base + (long)key * C + c * 8);
-      }
+  auto stage = [&](int t) {
+    const bf16* tile = base + (long)t * LD_KEYS * C;
+    const int left = n - t * LD_KEYS;             // rows past the end: masked below
+#pragma unroll 2
+    for (int j = wid; j < vecs; j += 4) {         // a kilobyte each
+      const unsigned i = j * 64 + lane, row = (i * magic) >> 20, c = i - row * vecs;
+      const unsigned off = (unsigned)min((int)row, left - 1) * C * 2 + ((c ^ ((row >> sh) & gm)) << 4);
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                   :: "s"(kt_at + j * 1024), "v"(off), "s"(tile) : "memory");
     }
   };
-  if (t_lo < t_hi) fetch(t_lo);
-  for (int i0 = tid; i0 < 16 * HT * vecs; i0 += 4 * NT) {      // this workgroup's queries
-    lat_u32x4 x[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const unsigned i = i0 + j * NT, row = (i * magic) >> 20, c = i - row * vecs;
-      x[j] = lat_u32x4{0u, 0u, 0u, 0u};
-      if (i < 16u * HT * vecs && h0 + (int)row < H)
-        x[j] = *reinterpret_cast<const lat_u32x4*>(q + ((long)r * H + h0 + row) * C + c * 8);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const unsigned i = i0 + j * NT, row = (i * magic) >> 20, c = i - row * vecs;
-      if (i < 16u * HT * vecs) *reinterpret_cast<lat_u32x4*>(qt + row * KS + c * 16) = x[j];
-    }
-  }
+  // pieces of this lane's reads: row lo16 of a wave's keys; rows hi4 * 8 + lo16 / 4 and 4 on
+  const int ks_swz = (lo16 >> sh) & gm;
+  const int v_row = (hi4 & 1) * 8 + (lo16 >> 2), v_swz0 = (v_row >> sh) & gm,
+            v_swz1 = ((v_row + 4) >> sh) & gm;
 
   lat_f32x4 acc[NCT];
-  float m_run[4], l_run[4];
+  float m_run = -1e30f, l_run = 0.f;
 #pragma unroll
   for (int c = 0; c < NCT; ++c) acc[c] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) m_run[i] = -1e30f, l_run[i] = 0.f;
-  float* my_red = red + ht * 64;
-  char* my_pt = pt + ht * 16 * LD_PSTRIDE;
 
   for (int t = t_lo; t < t_hi; ++t) {
     const int k0 = t * LD_KEYS;
-#pragma unroll
-    for (int j = 0; j < NPM; ++j) {
-      if (j < np) {
-        const unsigned i = tid + j * NT, row = (i * magic) >> 20, c = i - row * vecs;
-        if ((int)i < pieces) *reinterpret_cast<lat_u32x4*>(kt + row * KS + c * 16) = pre[j];
-      }
-    }
+    stage(t);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (t + 1 < t_hi) fetch(t + 1);
 
-    // scores: D[head = 4*hi4 + i][key = lo16] of this wave's 16 keys
+    // scores: D[key = 4 hi4 + i][head = lo16] of this wave's 16 keys
     lat_f32x4 s = {0.f, 0.f, 0.f, 0.f};
-    const char* kp = kt + (wid * 16 + lo16) * KS + hi4 * 16;
-    const char* qp = qt + (ht * 16 + lo16) * KS + hi4 * 16;
-#pragma unroll 6
-    for (int c = 0; c < C * 2; c += 64) {
-      const lat_bf16x8 b = *reinterpret_cast<const lat_bf16x8*>(kp + c);
-      const lat_bf16x8 x = *reinterpret_cast<const lat_bf16x8*>(qp + c);
-      s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, b, s, 0, 0, 0);
-    }
-    const bool live = k0 + wid * 16 + lo16 < n;
-    float mx[4];
+    const char* kp = kt + (wid * 16 + lo16) * KS;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s[i] = mx[i] = live ? s[i] * scale : -1e30f;
-#pragma unroll
-    for (int d = 1; d < 16; d *= 2)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], d));
-    if (lo16 == 0)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) my_red[wid * 16 + hi4 * 4 + i] = mx[i];
-    __syncthreads();
+    for (int j = 0; j < NPM; ++j)
+      if (j < steps) {
+        const lat_bf16x8 k =
+            *reinterpret_cast<const lat_bf16x8*>(kp + (((j * 4 + hi4) ^ ks_swz) << 4));
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[j], s, 0, 0, 0);
+      }
+    float mx = -1e30f;
+    bool live[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int row = hi4 * 4 + i;
-      float mn = m_run[i];
-#pragma unroll
-      for (int w = 0; w < 4; ++w) mn = fmaxf(mn, my_red[w * 16 + row]);
-      const float alpha = __expf(m_run[i] - mn);
-      const float p = live ? __expf(s[i] - mn) : 0.f;
-      l_run[i] = l_run[i] * alpha + p;
-      m_run[i] = mn;
-      *reinterpret_cast<bf16*>(my_pt + row * LD_PSTRIDE + (wid * 16 + lo16) * 2) = f2bf(p);
-#pragma unroll
-      for (int c = 0; c < NCT; ++c) acc[c][i] *= alpha;
+      live[i] = k0 + wid * 16 + hi4 * 4 + i < n;
+      s[i] = live[i] ? s[i] * scale : -1e30f;
+      mx = fmaxf(mx, s[i]);
     }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    if (hi4 == 0) red[wid * 16 + lo16] = mx;
+    __syncthreads();
+    float mn = m_run;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) mn = fmaxf(mn, red[w * 16 + lo16]);
+    const float alpha = __expf(m_run - mn);
+    m_run = mn;
+    bf16x4 p;
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float e = live[i] ? __expf(s[i] - mn) : 0.f;
+      sum += e;
+      p.v[i] = f2bf(e);
+    }
+    l_run = l_run * alpha + sum;
+    *reinterpret_cast<bf16x4*>(pt + lo16 * LD_PSTRIDE + (wid * 16 + hi4 * 4) * 2) = p;
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) acc[c] *= alpha;
     __syncthreads();
 
-    // O[head][column] += P[head][key] V[key][column], V = the tile's latents
-#pragma unroll
+    // O[column][head] += V[key][column] P[head][key], V = the tile's latents
+#pragma unroll 1
     for (int ks = 0; ks < LD_KEYS / 32; ++ks) {
-      const lat_bf16x8 p = *reinterpret_cast<const lat_bf16x8*>(my_pt + lo16 * LD_PSTRIDE +
-                                                                (ks * 32 + hi4 * 8) * 2);
+      const lat_bf16x8 p8 = *reinterpret_cast<const lat_bf16x8*>(pt + lo16 * LD_PSTRIDE +
+                                                                 (ks * 32 + hi4 * 8) * 2);
 #pragma unroll
       for (int c = 0; c < NCT; ++c) {
         const int n0 = (wid * NCT + c) * 16;
         if (n0 < RP) {                            // wave-uniform
-          const char* vp = kt + (ks * 32 + hi4 * 8 + (lo16 >> 2)) * KS + (n0 + (lo16 & 3) * 4) * 2;
-          const lat_bf16x4 v0 = lds_tr16(vp), v1 = lds_tr16(vp + 4 * KS);
+          const char* vp = kt + (ks * 32 + hi4 * 8 + (lo16 >> 2)) * KS + (lo16 & 1) * 8;
+          const int piece = n0 / 8 + ((lo16 & 3) >> 1);
+          const lat_bf16x4 v0 = lds_tr16(vp + ((piece ^ v_swz0) << 4));
+          const lat_bf16x4 v1 = lds_tr16(vp + 4 * KS + ((piece ^ v_swz1) << 4));
           const lat_bf16x8 v = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-          acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p, v, acc[c], 0, 0, 0);
+          acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, p8, acc[c], 0, 0, 0);
         }
       }
     }
@@ -277,31 +361,23 @@ __global__ __launch_bounds__(256 * HT) void latent_decode_attn_kernel(
   }
 
   // partial results of this split; an empty split stores zeros
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float l = l_run[i];
-#pragma unroll
-    for (int d = 1; d < 16; d *= 2) l += __shfl_xor(l, d);
-    if (lo16 == 0) my_red[wid * 16 + hi4 * 4 + i] = l;
-  }
+  l_run += __shfl_xor(l_run, 16);
+  l_run += __shfl_xor(l_run, 32);
+  if (hi4 == 0) red[wid * 16 + lo16] = l_run;
   __syncthreads();
+  if (h >= H) return;
+  const long o = ((long)r * H + h) * n_split + split;
+  if (wid == 0 && hi4 == 0) {
+    float l = 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = hi4 * 4 + i, h = h0 + ht * 16 + row;
-    if (h >= H) continue;
-    const long o = ((long)r * H + h) * n_split + split;
-    if (wid == 0 && lo16 == 0) {
-      float l = 0.f;
+    for (int w = 0; w < 4; ++w) l += red[w * 16 + lo16];
+    part_ml[o * 2] = m_run;
+    part_ml[o * 2 + 1] = l;
+  }
 #pragma unroll
-      for (int w = 0; w < 4; ++w) l += my_red[w * 16 + row];
-      part_ml[o * 2] = m_run[i];
-      part_ml[o * 2 + 1] = l;
-    }
-#pragma unroll
-    for (int c = 0; c < NCT; ++c) {
-      const int n0 = (wid * NCT + c) * 16;
-      if (n0 < RP) part_o[o * RP + n0 + lo16] = acc[c][i];
-    }
+  for (int c = 0; c < NCT; ++c) {
+    const int n0 = (wid * NCT + c) * 16;
+    if (n0 < RP) *reinterpret_cast<lat_f32x4*>(part_o + o * RP + n0 + hi4 * 4) = acc[c];
   }
 }
 
@@ -405,6 +481,98 @@ __global__ __launch_bounds__(256) void latent_decode_value_kernel(
     out[((long)(r0 + rr) * H + h) * dv + v0 + v] = lat_t<T>(acc[0]);
 }
 
+// The same on the matrix cores, for bf16 weights and a rank in whole 16-byte
+// pieces: grid (value chunks of 16, H, row groups of 16), the four waves share
+// the rank. The outputs stay float32: as the sum of three bf16 parts, 24 bits,
+// they enter the products exactly. 8 rows, 32 heads, 24 splits: 18.9 us with the
+// merge above by the kernel above, 8.3 now.
+__global__ __launch_bounds__(256) void latent_decode_value_mfma_kernel(
+    const float* __restrict__ o_lat, const bf16* __restrict__ w_uv, bf16* __restrict__ out, int R,
+    int H, int dv, int rank, int stride) {
+  __shared__ float red[4][16][17];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int lo16 = lane & 15, hi4 = lane >> 4;
+  const int h = blockIdx.y, v0 = blockIdx.x * 16, r0 = blockIdx.z * 16;
+  const float* o = o_lat + ((long)min(r0 + lo16, R - 1) * H + h) * stride;
+  const bf16* w = w_uv + ((long)h * dv + min(v0 + lo16, dv - 1)) * rank;
+  lat_f32x4 acc = {0.f, 0.f, 0.f, 0.f};           // D[value = 4 hi4 + i][row = lo16]
+#pragma unroll 2
+  for (int k0 = wid * 32; k0 < rank; k0 += 128) {
+    const int k = k0 + hi4 * 8;
+    lat_bf16x8 wv = {}, part[3] = {};
+    if (k < rank) {                               // all 8 columns or none
+      wv = __builtin_bit_cast(lat_bf16x8, *reinterpret_cast<const lat_u32x4*>(w + k));
+      const lat_f32x4 x[2] = {*reinterpret_cast<const lat_f32x4*>(o + k),
+                              *reinterpret_cast<const lat_f32x4*>(o + k + 4)};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float f = x[j / 4][j % 4];
+        part[0][j] = (__bf16)f;
+        // nothing is left of an infinity
+        const float mid = __builtin_isfinite(f) ? f - (float)part[0][j] : 0.f;
+        part[1][j] = (__bf16)mid;
+        part[2][j] = (__bf16)(mid - (float)part[1][j]);
+      }
+    }
+#pragma unroll
+    for (int i = 2; i >= 0; --i)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, part[i], acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[wid][lo16][hi4 * 4 + i] = acc[i];
+  __syncthreads();
+  const int r = tid >> 4, v = tid & 15;
+  if (r0 + r < R && v0 + v < dv)
+    out[((long)(r0 + r) * H + h) * dv + v0 + v] =
+        f2bf(red[0][r][v] + red[1][r][v] + red[2][r][v] + red[3][r][v]);
+}
+
+// Few rows and splits: merge and up-projection in one launch, grid (value chunks of
+// 16, H, R). A lane adds up the splits of its own columns, which no other lane of
+// the wave needs, and every workgroup does so again. 1 row, 16 heads, 4 splits: 7.6 us
+// in two launches, 4.1 now; 24 splits, 32 heads 8.2, and 7.4 by the kernels above.
+__global__ __launch_bounds__(256) void latent_decode_value_fold_kernel(
+    const float* __restrict__ part_o, const float* __restrict__ part_ml,
+    const bf16* __restrict__ w_uv, bf16* __restrict__ out, int H, int dv, int rank, int stride,
+    int S) {
+  constexpr int V = 8, NV = 4;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int h = blockIdx.y, v0 = blockIdx.x * 16 + wid * NV;
+  const long rh = (long)blockIdx.z * H + h;
+  const float* ml = part_ml + rh * S * 2;
+  const bf16* w[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) w[v] = w_uv + ((long)h * dv + min(v0 + v, dv - 1)) * rank;
+  float acc[NV] = {};
+  float m = -1e30f, l = 0.f;
+  for (int s = 0; s < S; ++s) m = fmaxf(m, ml[2 * s]);
+  for (int s = 0; s < S; ++s) l = fmaf(__expf(ml[2 * s] - m), ml[2 * s + 1], l);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  for (int c = lane * V; c < rank; c += 64 * V) {           // V divides rank
+    LatPack<bf16, V> x[NV];
+    LatPack<float, V> o = {};
+#pragma unroll
+    for (int v = 0; v < NV; ++v) x[v] = *reinterpret_cast<const LatPack<bf16, V>*>(w[v] + c);
+#pragma unroll 4
+    for (int s = 0; s < S; ++s) {
+      const float e = __expf(ml[2 * s] - m) * inv;
+      const LatPack<float, V> po =
+          *reinterpret_cast<const LatPack<float, V>*>(part_o + (rh * S + s) * stride + c);
+#pragma unroll
+      for (int j = 0; j < V; ++j) o.v[j] = fmaf(e, po.v[j], o.v[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) acc[v] = fmaf(bf2f(x[v].v[j]), o.v[j], acc[v]);
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const float t = wave_reduce_sum(acc[v]);
+    if (lane == 0 && v0 + v < dv) out[rh * dv + v0 + v] = f2bf(t);
+  }
+}
+
 // ---------------------------------------------------------------------------
 namespace {
 bool dec_t(const at::Tensor& x) {
@@ -415,6 +583,7 @@ bool dec_i32(const at::Tensor& x, int64_t n) {
   return x.is_cuda() && x.is_contiguous() && x.scalar_type() == at::kInt && x.numel() == n;
 }
 constexpr size_t LDS_MAX = 160 * 1024;
+bool aligned(const at::Tensor& x) { return reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0; }
 }  // namespace
 
 #define ROW_TILE(R, ...)                                   \
@@ -444,11 +613,25 @@ at::Tensor latent_decode_prep(const at::Tensor& qkv, const at::Tensor& w_uk,
   if (R == 0) return q;
   auto stream = c10::hip::getCurrentHIPStream();
   const bool vec = rank % 8 == 0;
-  const int cols = vec ? 128 : 16;
+  if (dt == at::kBFloat16 && vec && dn % 32 == 0 && dn <= 256 && (dn + dr) % 8 == 0 &&
+      qkv.size(1) % 8 == 0 && aligned(qkv) && aligned(w_uk)) {
+    const int NC = (int)((rank + 63) / 64);
+    latent_decode_prep_mfma_kernel<<<dim3(heads * NC + std::min<int64_t>(R, 16), (R + 15) / 16),
+                                     dim3(256), dn * LPM_STRIDE, stream>>>(
+        reinterpret_cast<const bf16*>(qkv.data_ptr()), reinterpret_cast<const bf16*>(w_uk.data_ptr()),
+        reinterpret_cast<const bf16*>(w_norm.data_ptr()), (float)eps, cos.data_ptr<float>(),
+        sin.data_ptr<float>(), (int)cos.size(0), (int)cos.size(1), pos.data_ptr<int>(),
+        slot.data_ptr<int>(), reinterpret_cast<bf16*>(cache.data_ptr()), (int)cache.size(0),
+        (int)cache.size(1), reinterpret_cast<bf16*>(q.data_ptr()), (int)R, (int)heads, (int)dn,
+        (int)dr, (int)rank, NC);
+    HIP_CHECK_KERNEL();
+    return q;
+  }
+  const int cols = LP_VECS * (vec ? 8 : 1);
   const int NC = (int)((rank + cols - 1) / cols);
 #define LAUNCH(TT, VV)                                                                           \
   latent_decode_prep_kernel<TT, VV, RT>                                                          \
-      <<<dim3(heads * NC + 1, (R + RT - 1) / RT), dim3(256), smem, stream>>>(                    \
+      <<<dim3(heads * NC + RT, (R + RT - 1) / RT), dim3(256), smem, stream>>>(                   \
           reinterpret_cast<const TT*>(qkv.data_ptr()),                                           \
           reinterpret_cast<const TT*>(w_uk.data_ptr()),                                          \
           reinterpret_cast<const TT*>(w_norm.data_ptr()), (float)eps, cos.data_ptr<float>(),     \
@@ -486,34 +669,26 @@ std::tuple<at::Tensor, at::Tensor> latent_decode_attn(const at::Tensor& q, const
   auto part_ml = at::empty({R, H, splits, 2}, part_o.options());
   if (R == 0) return {part_o, part_ml};
   auto stream = c10::hip::getCurrentHIPStream();
-  // head tiles per workgroup: both share the staged keys, but two workgroups
-  // are better where the splits alone leave CUs idle
-  const bool two = H > 16 && R * splits * ((H + 31) / 32) >= 256;
-#define LAUNCH1(HT, NCT, NPM)                                                                    \
+  const size_t smem = LD_KEYS * C * 2 + 16 * (LD_PSTRIDE + 16);
+  TORCH_CHECK(smem <= LDS_MAX, "latent_decode_attn: tile exceeds LDS");
+#define LAUNCH(NCT, NPM)                                                                         \
   do {                                                                                           \
-    const size_t smem = (LD_KEYS + 16 * HT) * (C * 2 + 16) + 16 * HT * (LD_PSTRIDE + 16);        \
-    TORCH_CHECK(smem <= LDS_MAX, "latent_decode_attn: tile exceeds LDS");                        \
     static const hipError_t attr_ = hipFuncSetAttribute(                                         \
-        reinterpret_cast<const void*>(&latent_decode_attn_kernel<HT, NCT, NPM>),                 \
+        reinterpret_cast<const void*>(&latent_decode_attn_kernel<NCT, NPM>),                     \
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_MAX);                               \
     TORCH_CHECK(attr_ == hipSuccess, "latent_decode_attn: LDS attribute");                       \
-    latent_decode_attn_kernel<HT, NCT, NPM>                                                      \
-        <<<dim3(splits, (H + 16 * HT - 1) / (16 * HT), R), dim3(256 * HT), smem, stream>>>(      \
+    latent_decode_attn_kernel<NCT, NPM>                                                          \
+        <<<dim3(splits, (H + 15) / 16, R), dim3(256), smem, stream>>>(                           \
             reinterpret_cast<const bf16*>(q.data_ptr()),                                         \
             reinterpret_cast<const bf16*>(cache.data_ptr()), slot.data_ptr<int>(),               \
             pos.data_ptr<int>(), part_o.data_ptr<float>(), part_ml.data_ptr<float>(),            \
             (int)cache.size(0), (int)cache.size(1), (int)H, (int)RP, (int)C, (float)scale);      \
-  } while (0)
-#define LAUNCH(NCT, NPM)                                                                         \
-  do {                                                                                           \
-    if (two) LAUNCH1(2, NCT, (NPM + 1) / 2); else LAUNCH1(1, NCT, NPM);                          \
   } while (0)
   TORCH_CHECK(C / 32 <= 26, "latent_decode_attn: latent and rotated key too wide");
   if (RP <= 128 && C <= 256) LAUNCH(2, 8);
   else if (RP <= 256 && C <= 384) LAUNCH(4, 12);
   else if (C <= 640) LAUNCH(8, 20);
   else LAUNCH(8, 26);
-#undef LAUNCH1
 #undef LAUNCH
   HIP_CHECK_KERNEL();
   return {part_o, part_ml};
@@ -541,15 +716,34 @@ at::Tensor latent_decode_combine(const at::Tensor& part_o,
   if (R == 0) return out;
   auto stream = c10::hip::getCurrentHIPStream();
   const bool vec = rank % 8 == 0;
+  const bool wide = vec && w_uv.scalar_type() == at::kBFloat16 && n % 4 == 0 && aligned(part_o) &&
+                    aligned(w_uv);
+  TORCH_CHECK(!part_ml || (n % 32 == 0 && S <= 1024),
+              "latent_decode_combine: padded rank, splits <= 1024");
+  if (wide && part_ml && R * S <= 20) {
+    latent_decode_value_fold_kernel<<<dim3((dv + 15) / 16, H, R), dim3(256), 0, stream>>>(
+        part_o.data_ptr<float>(), part_ml->data_ptr<float>(),
+        reinterpret_cast<const bf16*>(w_uv.data_ptr()), reinterpret_cast<bf16*>(out.data_ptr()),
+        (int)H, (int)dv, (int)rank, (int)n, (int)S);
+    HIP_CHECK_KERNEL();
+    return out;
+  }
   at::Tensor o_lat = part_o;
   if (part_ml) {
-    TORCH_CHECK(n % 32 == 0 && S <= 1024, "latent_decode_combine: padded rank, splits <= 1024");
     o_lat = at::empty({R, H, n}, part_o.options());
     latent_decode_merge_kernel<<<dim3((n + LM_COLS - 1) / LM_COLS, H, R), dim3(256),
                                  ((S + 3) / 4 * 4 + 1024) * sizeof(float), stream>>>(
         part_o.data_ptr<float>(), part_ml->data_ptr<float>(), o_lat.data_ptr<float>(), (int)H,
         (int)n, (int)S);
     HIP_CHECK_KERNEL();
+  }
+  if (wide) {
+    latent_decode_value_mfma_kernel<<<dim3((dv + 15) / 16, H, (R + 15) / 16), dim3(256), 0,
+                                      stream>>>(
+        o_lat.data_ptr<float>(), reinterpret_cast<const bf16*>(w_uv.data_ptr()),
+        reinterpret_cast<bf16*>(out.data_ptr()), (int)R, (int)H, (int)dv, (int)rank, (int)n);
+    HIP_CHECK_KERNEL();
+    return out;
   }
 #define LAUNCH(TT, VV)                                                                          \
   latent_decode_value_kernel<TT, VV, RT>                                                        \
