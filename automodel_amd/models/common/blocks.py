@@ -90,6 +90,10 @@ class SandwichLayer(nn.Module):
 
     def forward(self, x: torch.Tensor, h: torch.Tensor, next_norm: torch.Tensor | None,
                 *mixer_args) -> tuple[torch.Tensor, torch.Tensor | None]:
+        decode = getattr(self.self_attn, "decode_layer", None)
+        done = decode(self, x, h, next_norm, *mixer_args) if decode is not None else None
+        if done is not None:
+            return done
         y = self.self_attn(h, *mixer_args)
         if self.mlp is None:
             return residual_add_norm(x, y, self.post_attention_layernorm.weight, self.mult,

@@ -346,7 +346,51 @@ class LlamaDecoderLayer(nn.Module):
             self.input_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps, backend.rms_norm)
             self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps, backend.rms_norm)
 
+    def _decode_step(self, x: torch.Tensor, cos: torch.Tensor,
+                     sin: torch.Tensor) -> torch.Tensor | None:
+        """One token per sequence behind a K/V cache, all of the layer's kernels issued by
+        one native call (csrc/llama_layer.cpp). None for layers and inputs that it does not
+        take, and nothing is done."""
+        from automodel_amd.parallel.cp import active_cp
+        from automodel_amd.serving.decode_linear import plain_linears, unobserved
+        from automodel_amd.utils.kv_cache import KVCache, StaticKVCache, active_kv_cache
+
+        cache, attn, mlp = active_kv_cache(), self.self_attn, self.mlp
+        if not (type(cache) in (KVCache, StaticKVCache) and not self.olmo2 and type(x) is torch.Tensor
+                and x.is_cuda and x.shape[1] == 1 and x.dtype == torch.bfloat16
+                and not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
+                and type(attn) is LlamaAttention and type(mlp) is LlamaMLP):
+            return None
+        cfg, norms = attn.cfg, (self.input_layernorm, self.post_attention_layernorm)
+        if (self.residual_multiplier != 1.0 or cfg.qk_norm or cfg.qk_norm_full
+                or cfg.rope_interleaved or cfg.sliding_window is not None or cfg.bidirectional
+                or not attn.use_rope or attn.backend.attn != "hip" or attn.backend.rope != "hip"
+                or active_cp() is not None
+                or any(type(n) is not RMSNorm or n.backend != "hip" for n in norms)):
+            return None
+        qkv = [attn.qkv_proj] if cfg.fused_qkv else [attn.q_proj, attn.k_proj, attn.v_proj]
+        glu = [mlp.gate_up_proj] if mlp.fused else [mlp.gate_proj, mlp.up_proj]
+        lins = [attn.o_proj, mlp.down_proj, *qkv, *glu]
+        if not (plain_linears(*lins) and unobserved(attn, mlp, *norms)
+                and all(type(n.weight) in (nn.Parameter, torch.Tensor) for n in norms)):
+            return None
+        from automodel_amd.ops._backend import hip_ops
+
+        keys, values, pos, pos_dev = cache.next_entry()
+        scale = attn.head_dim ** -0.5 if cfg.attention_multiplier is None else cfg.attention_multiplier
+        y = hip_ops().llama_decode_layer(
+            x, [m.weight for m in (*norms, *lins)], cos, sin, keys, values, pos, pos_dev, scale,
+            norms[0].variance_epsilon, norms[1].variance_epsilon, attn.num_heads,
+            attn.num_kv_heads, cfg.fused_qkv, mlp.fused)
+        if not y:
+            return None
+        cache.entry_used()
+        return y[0]
+
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
+        y = self._decode_step(x, cos, sin)
+        if y is not None:
+            return y
         if self.olmo2:
             x = x + self.post_attention_layernorm(self.self_attn(x, cos, sin))
             return x + self.post_feedforward_layernorm(self.mlp(x))

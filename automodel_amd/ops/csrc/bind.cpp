@@ -10,6 +10,11 @@
 TORCH_LIBRARY(amd_ops, m) {
   m.def("rms_norm_fwd(Tensor x, Tensor w, float eps) -> (Tensor, Tensor)");
   m.impl("rms_norm_fwd", &amd_ops::rms_norm_fwd);
+  m.def(
+      "llama_decode_layer(Tensor x, Tensor[] ws, Tensor cos, Tensor sin, Tensor(a!) k_cache, "
+      "Tensor(b!) v_cache, int pos, Tensor? pos_dev, float scale, float eps_in, float eps_mid, "
+      "int heads, int kv_heads, bool fused_qkv, bool fused_gate_up) -> Tensor[]");
+  m.impl("llama_decode_layer", &amd_ops::llama_decode_layer);
   m.def("add_rms_norm_fwd(Tensor x, Tensor delta, Tensor w, float eps) -> (Tensor, Tensor, Tensor)");
   m.impl("add_rms_norm_fwd", &amd_ops::add_rms_norm_fwd);
   m.def(

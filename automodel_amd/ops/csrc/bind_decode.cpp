@@ -19,7 +19,9 @@ TORCH_LIBRARY_FRAGMENT(amd_ops, m) {
   m.def(
       "gemm_skinny_bf16(Tensor x, Tensor w, bool relu2, bool out_f32, int group_n=0) -> Tensor");
   m.impl("gemm_skinny_bf16", &amd_ops::gemm_skinny_bf16);
-  m.def("decode_rows(Tensor x, Tensor[] ws, bool glu=False) -> Tensor[]");
+  m.def(
+      "decode_rows(Tensor x, Tensor[] ws, bool glu=False, bool relu2=False, "
+      "Tensor? residual=None) -> Tensor[]");
   m.impl("decode_rows", &amd_ops::decode_rows);
 
   m.def("doc_bounds(Tensor cu, int total) -> (Tensor, Tensor)");
@@ -28,6 +30,12 @@ TORCH_LIBRARY_FRAGMENT(amd_ops, m) {
       "kv_decode_attn(Tensor q, Tensor k_new, Tensor v_new, Tensor(a!) k_cache, "
       "Tensor(b!) v_cache, int pos, Tensor? pos_dev, float scale) -> Tensor");
   m.impl("kv_decode_attn", &amd_ops::kv_decode_attn);
+
+  m.def(
+      "latent_decode_layer(Tensor(a!) x, Tensor h, Tensor[] ws, Tensor? w_next, Tensor cos, "
+      "Tensor sin, Tensor pos, Tensor slot, Tensor(b!) cache, float eps, float latent_eps, "
+      "float mult, float scale, int heads, int dn, int dr, int splits) -> Tensor[]");
+  m.impl("latent_decode_layer", &amd_ops::latent_decode_layer);
 
   m.def("embed_rms_norm(Tensor ids, Tensor table, Tensor w, float eps) -> Tensor");
   m.impl("embed_rms_norm", &amd_ops::embed_rms_norm);

@@ -41,6 +41,7 @@ struct Rows {
   int first[MAX_SEGMENTS];   // INT_MAX: no such segment
   const bf16* bias;          // of a single weight
   float* yf;                 // of a single weight: float32 output instead of y[0]
+  const bf16* res;           // of a single weight: added to y
   bool relu2;                // max(y, 0)^2
   int K;
   int group_n;               // > 0: every group_n rows of w take the next B rows of x
@@ -132,6 +133,7 @@ __global__ __launch_bounds__(256) void gemv_bf16_kernel(const Rows p) {
           t[r] = fmaxf(t[r], 0.f);
           t[r] *= t[r];
         }
+        if (p.res) t[r] += bf2f(p.res[(long)b * N + row0 + r]);
         if (p.yf) p.yf[(long)b * N + row0 + r] = t[r];
         else p.y[seg][(long)b * N + row0 + r] = f2bf(t[r]);
       }
@@ -250,6 +252,7 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(const Ro
       t = fmaxf(t, 0.f);
       t *= t;
     }
+    if (p.res) t += bf2f(p.res[o]);
     if (p.yf) p.yf[o] = t;
     else p.y[seg][o] = f2bf(t);
   }
@@ -377,15 +380,17 @@ at::Tensor gemm_skinny_bf16(const at::Tensor& x, const at::Tensor& w, bool relu2
 }
 
 // x [B, K] against up to three weights [n, K] in one launch -> [B, n] each; glu:
-// against gate and up -> silu(x gate^T) * (x up^T) alone.
-std::vector<at::Tensor> decode_rows(const at::Tensor& x, at::TensorList ws, bool glu) {
+// against gate and up -> silu(x gate^T) * (x up^T) alone. relu2: max(y, 0)^2;
+// residual [B, n] of a single weight: added.
+std::vector<at::Tensor> decode_rows(const at::Tensor& x, at::TensorList ws, bool glu, bool relu2,
+                                    const std::optional<at::Tensor>& residual) {
   const int64_t B = x.size(0), K = x.size(-1);
   TORCH_CHECK(x.is_cuda() && x.dtype() == at::kBFloat16 && x.dim() == 2 && x.is_contiguous() &&
                   B >= 1 && B <= 64 && K >= 8 && K % 8 == 0,
               "decode_rows: x [1..64, K] bf16, K % 8 == 0");
   TORCH_CHECK(ws.size() >= 1 && ws.size() <= MAX_SEGMENTS, "decode_rows: 1 to 3 weights");
-  TORCH_CHECK(!glu || (ws.size() == 2 && ws[0].sizes() == ws[1].sizes()),
-              "decode_rows: gate and up of one shape");
+  TORCH_CHECK(!glu || (ws.size() == 2 && ws[0].sizes() == ws[1].sizes() && !relu2 && !residual),
+              "decode_rows: gate and up of one shape, and nothing after their product");
   Rows p{};
   p.x = data(x);
   p.K = (int)K;
@@ -403,6 +408,14 @@ std::vector<at::Tensor> decode_rows(const at::Tensor& x, at::TensorList ws, bool
     p.y[s] = reinterpret_cast<bf16*>(out.back().data_ptr());
   }
   const int segments = (int)out.size();
+  p.relu2 = relu2;
+  if (residual) {
+    TORCH_CHECK(segments == 1 && residual->device() == x.device() &&
+                    residual->dtype() == at::kBFloat16 && residual->is_contiguous() &&
+                    residual->sizes() == out[0].sizes(),
+                "decode_rows: residual as the one output");
+    p.res = data(*residual);
+  }
   if (B > 2) skinny(p, segments, (int)B, glu);
   else if (B == 1 && glu) launch_gemv<1, 2, 4, true>(p, 1);
   else if (B == 1) launch_gemv<1, 1, 8>(p, segments);

@@ -87,7 +87,19 @@ at::Tensor kv_decode_attn(const at::Tensor& q, const at::Tensor& k_new, const at
                           const std::optional<at::Tensor>& pos_dev, double scale);
 at::Tensor gemm_skinny_bf16(const at::Tensor& x, const at::Tensor& w, bool relu2, bool out_f32,
                             int64_t group_n = 0);
-std::vector<at::Tensor> decode_rows(const at::Tensor& x, at::TensorList ws, bool glu);
+std::vector<at::Tensor> decode_rows(const at::Tensor& x, at::TensorList ws, bool glu = false,
+                                    bool relu2 = false,
+                                    const std::optional<at::Tensor>& residual = std::nullopt);
+std::vector<at::Tensor> llama_decode_layer(
+    const at::Tensor& x, at::TensorList ws, const at::Tensor& cos, const at::Tensor& sin,
+    at::Tensor k_cache, at::Tensor v_cache, int64_t pos, const std::optional<at::Tensor>& pos_dev,
+    double scale, double eps_in, double eps_mid, int64_t heads, int64_t kv_heads, bool fused_qkv,
+    bool fused_gate_up);
+std::vector<at::Tensor> latent_decode_layer(
+    at::Tensor x, const at::Tensor& h, at::TensorList ws, const std::optional<at::Tensor>& w_next,
+    const at::Tensor& cos, const at::Tensor& sin, const at::Tensor& pos, const at::Tensor& slot,
+    at::Tensor cache, double eps, double latent_eps, double mult, double scale, int64_t heads,
+    int64_t dn, int64_t dr, int64_t splits);
 
 std::tuple<at::Tensor, at::Tensor, at::Tensor> build_group_plan(
     const at::Tensor& counts, int64_t M, int64_t bm = 128);

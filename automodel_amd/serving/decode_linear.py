@@ -109,14 +109,20 @@ def grouped_rows(lin: nn.Module, xs: torch.Tensor, sizes: list[int]) -> torch.Te
     return hip_ops().gemm_skinny_bf16(x, w, False, False, group)
 
 
-def _plain(lin: nn.Module) -> bool:
-    """A layer whose call is x W^T and nothing else: no adapter, no bias, no hook of a
-    wrapper or an observer, no sharded weight."""
-    hooks = nn.modules.module
-    return (type(lin) in (nn.Linear, DecodeLinear) and lin.bias is None
-            and type(lin.weight) in (nn.Parameter, torch.Tensor)
-            and not (lin._forward_hooks or lin._forward_pre_hooks
-                     or hooks._global_forward_hooks or hooks._global_forward_pre_hooks))
+def unobserved(*modules: nn.Module) -> bool:
+    """No hook would see these modules' calls, so that kernels may take their place."""
+    every = nn.modules.module
+    if every._global_forward_hooks or every._global_forward_pre_hooks:
+        return False
+    return not any(m._forward_hooks or m._forward_pre_hooks for m in modules)
+
+
+def plain_linears(*lins: nn.Module) -> bool:
+    """Each call is x W^T and nothing else: no adapter, no bias, no hook of a wrapper or an
+    observer, no sharded weight."""
+    return unobserved(*lins) and all(
+        type(lin) in (nn.Linear, DecodeLinear) and lin.bias is None
+        and type(lin.weight) in (nn.Parameter, torch.Tensor) for lin in lins)
 
 
 def decode_rows(lins: list[nn.Module], x: torch.Tensor,
@@ -132,13 +138,15 @@ def decode_rows(lins: list[nn.Module], x: torch.Tensor,
     if not (x.is_cuda and x.dtype == torch.bfloat16 and 1 <= rows <= 32 and K % 8 == 0
             and not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda")
             and type(x) is torch.Tensor and x.is_contiguous() and x.data_ptr() % 16 == 0
-            and all(map(_plain, lins))):
+            and plain_linears(*lins)):
         return None
     ws = [lin.weight for lin in lins]
     if glu and len(ws) == 1:
         ws = list(ws[0].chunk(2))
     if not all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.device == x.device
                and w.data_ptr() % 16 == 0 for w in ws):
+        return None
+    if glu and rows * ws[0].shape[0] % 8:         # the activation kernel refuses these
         return None
     from automodel_amd.ops._backend import hip_ops
 

@@ -74,13 +74,22 @@ class KVCache:
             return None
         from automodel_amd.ops._backend import hip_ops
 
+        keys, values, pos, pos_dev = self.next_entry()
+        o = hip_ops().kv_decode_attn(
+            q.contiguous(), k.contiguous(), v.contiguous(), keys, values, pos, pos_dev,
+            D ** -0.5 if scale is None else scale)
+        self.entry_used()
+        return o
+
+    def next_entry(self) -> tuple[torch.Tensor, torch.Tensor, int, torch.Tensor | None]:
+        """(keys, values, position, its tensor if it lives on the device) of the layer that
+        comes next, for a kernel that records one token there itself; ``entry_used`` after."""
         pos_dev = self._device_position()
         assert pos_dev is not None or self.pos < self.max_len, "KV cache overflow"
-        o = hip_ops().kv_decode_attn(
-            q.contiguous(), k.contiguous(), v.contiguous(), kc, self.v[self._layer],
-            self.pos, pos_dev, D ** -0.5 if scale is None else scale)
+        return self.k[self._layer], self.v[self._layer], self.pos, pos_dev
+
+    def entry_used(self) -> None:
         self._layer += 1
-        return o
 
     def _device_position(self) -> torch.Tensor | None:
         return None
