@@ -13,9 +13,9 @@
 // Bound by the dependence of exp on the row maximum and by LDS reads (at 32 rows per wave
 // the four SIMDs ask for 128 B/clk at full rate). 64 rows per wave would halve the LDS
 // reads, but the accumulators leave too few registers: it spilled and ran at 100 TFLOP/s.
-// Measured (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128: 6.52 -> 2.62 ms,
-// 838 TFLOP/s; 2 x 4096: 1030 -> 347 us; 2 x 3072, 16 heads (192, 128): 414 -> 186 us;
-// 4 x 2048, 16/8 heads of 64: 154 -> 67 us.
+// Measured (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128: 6.52 -> 2.19 ms,
+// 1006 TFLOP/s; 2 x 4096: 1030 -> 289 us; 2 x 3072, 16 heads (192, 128): 414 -> 120 us;
+// 4 x 2048, 16/8 heads of 64: 154 -> 55 us.
 //
 // Varlen: per-token doc_start gates the causal mask to the query's own document; tiles
 // before a block's first document are skipped.
@@ -195,36 +195,64 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArg
     }
     load_v(t0);
   }
-  for (int t = t0; t < t1; ++t) {
-    const bool live = t >= t0w && t < t1w;
-    const unsigned kt = (t & 1) * KT, kn = KT - kt;
-    const unsigned vt = 2 * KT + (t & 1) * VT, vo = 4 * KT + VT - vt;
-    const bool mask = t >= t_diag || t * 64 + 64 > a.Skv || (VARLEN && t * 64 < doc_w);
-    if constexpr (PIPE) {
+  if constexpr (PIPE) {
+    // A tile that every row of the wave sees whole, with neighbours on both sides: the hot
+    // loop, without a branch but the rescaling. At two waves a SIMD instructions are issued
+    // nearly all the time, so that each one less counts: one loop with all of a tile's cases
+    // kept the output in two sets of registers and moved it between them, and buffers
+    // known when this is compiled are offsets in the reads (29 us of the next figure). 16384, 32/8
+    // heads of 128: 2499 -> 2187 us; 2 x 3072, 16 heads of (192, 128): 168 -> 120.
+    auto steady = [&](int t, auto parity) {
+      constexpr int PARITY = decltype(parity)::value;      // of t; -1: any
+      const unsigned odd = PARITY < 0 ? t % 2 : PARITY, kt = odd * KT, kn = KT - kt;
+      const unsigned vt = 2 * KT + odd * VT, vo = 4 * KT + VT - vt;
+      f.template softmax<false>(s0, t * 64, p0, [&] { f.scores(s1, kt, 1); f.values(p1, vo, 1); });
+      wait_loads();       // K of t + 1, V of t; the buffers of K of t, V of t - 1 are free
+      barrier();
+      load_v(t + 1);
+      load_k(min(t + 2, t1 - 1));
+      f.template softmax<false>(s1, t * 64 + 32, p1, [&] { f.scores(s0, kn, 0); f.values(p0, vt, 0); });
+    };
+    auto general = [&](int t) {
+      const bool live = t >= t0w && t < t1w;
+      const unsigned kt = (t & 1) * KT, kn = KT - kt;
+      const unsigned vt = 2 * KT + (t & 1) * VT, vo = 4 * KT + VT - vt;
       if (live) {
-        auto next = [&] { f.scores(s1, kt, 1); };
-        auto both = [&] { f.scores(s1, kt, 1); f.values(p1, vo, 1); };
-        if (t == t0w) {
-          f.scores(s0, kt, 0);
-          f.template softmax<true>(s0, t * 64, p0, next);
-        } else if (mask) {
-          f.template softmax<true>(s0, t * 64, p0, both);
-        } else {
-          f.template softmax<false>(s0, t * 64, p0, both);
-        }
+        if (t == t0w) f.scores(s0, kt, 0);
+        f.template softmax<true>(s0, t * 64, p0, [&] {
+          f.scores(s1, kt, 1);
+          if (t != t0w) f.values(p1, vo, 1);
+        });
       }
-      wait_loads();     // K of t + 1, V of t; the buffers of K of t, V of t - 1 are free
+      wait_loads();
       barrier();
       if (t + 1 < t1) load_v(t + 1);
       if (t + 2 < t1) load_k(t + 2);
       if (live) {
         // (the scores of the tile after a wave's last one are formed and not used)
-        auto both = [&] { f.scores(s0, kn, 0); f.values(p0, vt, 0); };
-        if (mask) f.template softmax<true>(s1, t * 64 + 32, p1, both);
-        else f.template softmax<false>(s1, t * 64 + 32, p1, both);
+        f.template softmax<true>(s1, t * 64 + 32, p1, [&] { f.scores(s0, kn, 0); f.values(p0, vt, 0); });
         if (t == t1w - 1) f.values(p1, vt, 1);
       }
-    } else {
+    };
+    // tiles of the steady kind: [first, end)
+    const int first = max(t0w + 1, VARLEN ? (doc_w + 63) / 64 : 0);
+    const int end = min(min(t_diag, a.Skv / 64), min(t1w, t1) - 1);
+    int t = t0;
+    for (; t < min(first, t1) || (!VARLEN && t < end && t % 2); ++t) general(t);
+    // (pairs leave a tile over at either end; the runs of short documents are too short)
+    if constexpr (VARLEN)
+      for (; t < end; ++t) steady(t, std::integral_constant<int, -1>{});
+    else
+      for (; t + 1 < end; t += 2) {
+        steady(t, std::integral_constant<int, 0>{});
+        steady(t + 1, std::integral_constant<int, 1>{});
+      }
+    for (; t < t1; ++t) general(t);
+  } else {
+    for (int t = t0; t < t1; ++t) {
+      const bool live = t >= t0w && t < t1w;
+      const unsigned kt = (t & 1) * KT, vt = 2 * KT + (t & 1) * VT;
+      const bool mask = t >= t_diag || t * 64 + 64 > a.Skv || (VARLEN && t * 64 < doc_w);
       wait_loads();     // K and V of t; the other buffers are free
       barrier();
       if (t + 1 < t1) {
@@ -335,7 +363,7 @@ std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
 
   // Waves per workgroup and per SIMD: as many as the registers of the accumulators and
   // the two K/V tiles in LDS allow. (192, 128) fits one workgroup a CU, so it has 8 waves
-  // (186 us; 240 with 4 waves at one a SIMD); (192, 192) would spill at two a SIMD (457
+  // (120 us; 4 waves at one a SIMD were 1.3 times slower); (192, 192) would spill at two a SIMD (457
   // against 178 us).
   bool done = false;
 #define FA_FWD_CASE(A, C, W, OCC, PIPE)                             \
