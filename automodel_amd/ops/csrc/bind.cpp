@@ -39,6 +39,11 @@ TORCH_LIBRARY(amd_ops, m) {
       "Tensor(d!) v, int step, float lr, float beta1, float beta2, float eps, "
       "float weight_decay) -> ()");
   m.impl("adamw_step", &amd_ops::adamw_step);
+  m.def(
+      "adamw_steps(Tensor(a!)[] params, Tensor[] grads, Tensor(b!)[] masters, Tensor(c!)[] ms, "
+      "Tensor(d!)[] vs, int[] steps, float lr, float beta1, float beta2, float eps, "
+      "float weight_decay) -> ()");
+  m.impl("adamw_steps", &amd_ops::adamw_steps);
 
   m.def(
       "flash_attn_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, "

@@ -8,11 +8,11 @@
 //
 // The products of a tile take 1024 cycles of a SIMD's matrix core and its softmax about
 // 900 of the vector unit, so the loop is pipelined over half tiles: while half tile i goes
-// through exp, the matrix core forms the scores of i + 1 and the values of i - 1 (`step`,
-// one basic block). Two waves a SIMD, or two workgroups a CU, fill what one wave leaves.
-// Bound by the dependence of exp on the row maximum and by LDS reads (at 32 rows per wave
-// the four SIMDs ask for 128 B/clk at full rate). 64 rows per wave would halve the LDS
-// reads, but the accumulators leave too few registers: it spilled and ran at 100 TFLOP/s.
+// through exp, the matrix core forms the scores of i + 1 and the values of i - 1. Two waves
+// a SIMD, or two workgroups a CU, fill what one wave leaves. Bound by instruction issue (at
+// (128, 128) 96% of the cycles, the matrix core busy 45% and LDS 23% of them, before whole
+// tiles had a loop of their own). 64 rows per wave would halve the LDS reads, but the
+// accumulators leave too few registers: it spilled and ran at 100 TFLOP/s.
 // Measured (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128: 6.52 -> 2.19 ms,
 // 1006 TFLOP/s; 2 x 4096: 1030 -> 289 us; 2 x 3072, 16 heads (192, 128): 414 -> 120 us;
 // 4 x 2048, 16/8 heads of 64: 154 -> 55 us.

@@ -26,6 +26,9 @@ at::Tensor swiglu_cat_bwd(const at::Tensor& dy, const at::Tensor& gu);
 std::tuple<at::Tensor, at::Tensor> swiglu_bwd(const at::Tensor& dy, const at::Tensor& g,
                                               const at::Tensor& u);
 
+void adamw_steps(at::TensorList params, at::TensorList grads, at::TensorList masters,
+                 at::TensorList ms, at::TensorList vs, at::IntArrayRef steps, double lr,
+                 double beta1, double beta2, double eps, double weight_decay);
 void adamw_step(at::Tensor param, at::Tensor grad, at::Tensor master, at::Tensor m,
                 at::Tensor v, int64_t step, double lr, double beta1, double beta2,
                 double eps, double weight_decay);

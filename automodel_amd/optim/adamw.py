@@ -50,6 +50,7 @@ class FusedAdamW(torch.optim.Optimizer):
             lr = group["lr"]
             beta1, beta2 = group["betas"]
             eps, wd = group["eps"], group["weight_decay"]
+            batch = ([], [], [], [], [], [])      # for one launch: p, grad, master, m, v, t
             for p_ in group["params"]:
                 if p_.grad is None:
                     continue
@@ -67,10 +68,12 @@ class FusedAdamW(torch.optim.Optimizer):
                 state["step"] += 1
                 t = state["step"]
                 m, v = state["exp_avg"], state["exp_avg_sq"]
-                if use_hip:
-                    # fp32 states ride the master-weight kernel; bf16 states
-                    # ride the master-free kernel (m passed as placeholder
-                    # for the unused master arg)
+                if use_hip and m.dtype == torch.float32 and "master" in state:
+                    for to, x in zip(batch, (p, grad.to(torch.bfloat16), state["master"], m, v, t)):
+                        to.append(x)
+                elif use_hip:
+                    # bf16 states ride the master-free kernel (m passed as
+                    # placeholder for the unused master arg)
                     hip_ops().adamw_step(
                         p, grad.to(torch.bfloat16), state.get("master", m), m, v,
                         t, lr, beta1, beta2, eps, wd,
@@ -87,6 +90,8 @@ class FusedAdamW(torch.optim.Optimizer):
                     denom = (v.sqrt() / math.sqrt(bc2)).add_(eps)
                     pf.addcdiv_(m, denom, value=-lr / bc1)
                     p.copy_(pf.to(p.dtype))
+            if batch[0]:
+                hip_ops().adamw_steps(*batch, lr, beta1, beta2, eps, wd)
         return loss
 
     def state_dict(self):
