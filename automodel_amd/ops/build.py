@@ -25,7 +25,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 BUILD_DIR = os.path.join(PKG_DIR, "_build")
 SO_PATH = os.path.join(PKG_DIR, "libamd_ops.so")
 DECODE_SO_PATH = os.path.join(PKG_DIR, "libamd_ops_decode.so")
-DECODE_SOURCES = ("bind_decode.cpp", "flash_attn.hip", "gemv.hip", "gqa_attn.hip",
+DECODE_SOURCES = ("bind_decode.cpp", "device_ints.hip", "flash_attn.hip", "gemv.hip", "gqa_attn.hip",
                   "hyper.hip", "kv_decode.hip", "latent_attn.hip", "latent_decode.hip",
                   "latent_layer.cpp", "linear_scan.hip", "residual_norm.hip")
 ARCH = os.environ.get("PYTORCH_ROCM_ARCH", "gfx950")

@@ -24,6 +24,7 @@ TORCH_LIBRARY_FRAGMENT(amd_ops, m) {
       "Tensor? residual=None) -> Tensor[]");
   m.impl("decode_rows", &amd_ops::decode_rows);
 
+  m.def("device_ints(int[] values, Device device) -> Tensor", &amd_ops::device_ints);
   m.def("doc_bounds(Tensor cu, int total) -> (Tensor, Tensor)");
   m.impl("doc_bounds", &amd_ops::doc_bounds);
   m.def(

@@ -84,6 +84,7 @@ at::Tensor sgmv_fused_fwd(const at::Tensor& x, const at::Tensor& A,
 at::Tensor gemv_bf16(const at::Tensor& x, const at::Tensor& w,
                      const c10::optional<at::Tensor>& bias, bool relu2 = false,
                      bool out_f32 = false, int64_t group_n = 0);
+at::Tensor device_ints(at::IntArrayRef values, at::Device device);
 std::tuple<at::Tensor, at::Tensor> doc_bounds(const at::Tensor& cu, int64_t total);
 at::Tensor kv_decode_attn(const at::Tensor& q, const at::Tensor& k_new, const at::Tensor& v_new,
                           at::Tensor k_cache, at::Tensor v_cache, int64_t pos,

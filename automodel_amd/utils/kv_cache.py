@@ -217,7 +217,12 @@ class SlotCache:
         pos = [self.lens[s] for s in slots]
         if not pos or max(pos) >= self.max_len:
             raise RuntimeError("KV cache overflow")
-        both = torch.tensor([pos, slots], dtype=torch.int32).to(self.device)
+        if self.device.type == "cuda":
+            from automodel_amd.ops._backend import hip_ops
+
+            both = hip_ops().device_ints(pos + list(slots), self.device).view(2, len(pos))
+        else:
+            both = torch.tensor([pos, slots], dtype=torch.int32)
         self.step = PackedStep(positions=both[0], slots=both[1], prompt=False)
         self._pending = [(s, 1) for s in slots]
         return self.step
