@@ -98,6 +98,10 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("grouped_gemm_nt_fp8", &amd_ops::grouped_gemm_nt_fp8);
   m.def("route_plan(Tensor indices, Tensor probs, int E) -> (Tensor, Tensor, Tensor, Tensor, Tensor)");
   m.impl("route_plan", &amd_ops::route_plan);
+  m.def("route_topk(Tensor scores, int K) -> Tensor");
+  m.impl("route_topk", &amd_ops::route_topk);
+  m.def("expert_load(Tensor indices, int E) -> Tensor");
+  m.impl("expert_load", &amd_ops::expert_load);
   m.def("combine_bwd(Tensor g, Tensor y, Tensor src, Tensor order, Tensor probs) -> (Tensor, Tensor)");
   m.impl("combine_bwd", &amd_ops::combine_bwd);
   m.def(

@@ -123,6 +123,8 @@ at::Tensor grouped_gemm_nt_fp8(const at::Tensor& x8, const at::Tensor& w8,
                                int64_t bm = 128);
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor> route_plan(
     const at::Tensor& indices, const at::Tensor& probs, int64_t E);
+at::Tensor route_topk(const at::Tensor& scores, int64_t K);
+at::Tensor expert_load(const at::Tensor& indices, int64_t E);
 std::tuple<at::Tensor, at::Tensor> combine_bwd(const at::Tensor& g, const at::Tensor& y,
                                                const at::Tensor& src, const at::Tensor& order,
                                                const at::Tensor& probs);

@@ -58,3 +58,28 @@ def test_two_pairs(counts, N, K, bm):
     want = torch.cat([g1[s].double() @ w1[e].double() + g2[s].double() @ w2[e].double()
                       for e, s in enumerate(slice(a, b) for a, b in zip(at, at[1:]))])
     assert (dx.double() - want).norm() <= 2.0 ** -9 * 1.02 * want.norm()
+
+
+@pytest.mark.parametrize("T,E,K", [(1, 1, 1), (3, 63, 2), (5, 64, 32), (130, 65, 6), (4, 128, 8), (7, 129, 5),
+                                   (2, 257, 8), (6, 512, 32), (33, 512, 1), (9, 8, 8), (0, 16, 2),
+                                   (5, 40, 33), (5, 513, 4)])       # the last two: torch's own
+def test_route_choice(T, E, K):
+    from automodel_amd.moe.layers import _expert_load, _largest
+
+    g = torch.Generator().manual_seed(E)
+    s = torch.rand(T, 2 * E, generator=g).cuda()[:, ::2] - 0.5      # no two equal, not contiguous
+    idx = _largest(s, K)
+    assert torch.equal(idx, s.topk(K, dim=-1)[1])
+    assert torch.equal(_expert_load(idx, E), torch.bincount(idx.reshape(-1), minlength=E).float())
+
+
+def test_route_choice_of_special_values():
+    from automodel_amd.moe.layers import _expert_load, _largest
+
+    inf, nan = float("inf"), float("nan")
+    s = torch.tensor([[-inf, 1.0, -inf, inf, -0.5], [0.0, nan, 2.0, -inf, inf], [3.0, 3.0, 3.0, 4.0, 3.0],
+                      [-inf] * 5, [torch.finfo(torch.float32).min, -inf, 1e-45, 0.0, -1e-45]]).cuda()
+    want = [[3, 1, 4, 0], [1, 4, 2, 0], [3, 0, 1, 2], [0, 1, 2, 3], [2, 3, 4, 0]]    # equal: the lowest first
+    assert _largest(s, 4).tolist() == want
+    many = torch.randint(0, 4096, (4097, 3), device="cuda")
+    assert torch.equal(_expert_load(many.T, 4096), torch.bincount(many.reshape(-1), minlength=4096).float())
