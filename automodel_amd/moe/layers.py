@@ -19,9 +19,46 @@ from automodel_amd.ops.swiglu import swiglu
 def _device_tensor(t: torch.Tensor) -> bool:
     """An ordinary GPU tensor in an eager call: traced, transformed and mode-wrapped calls
     stay with torch's own operations, which those can see into."""
-    return (t.is_cuda and type(t) is torch.Tensor and not torch.compiler.is_compiling()
-            and not torch.jit.is_tracing() and not torch._C._are_functorch_transforms_active()
+    return (t.is_cuda and type(t) in (torch.Tensor, nn.Parameter)
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch._C._are_functorch_transforms_active()
+            and torch.autograd.forward_ad._current_level < 0
             and not torch._C._len_torch_dispatch_stack())
+
+
+class _RouterLinear(torch.autograd.Function):
+    """float32 scores of bf16 tokens and weights, without float32 copies of either."""
+
+    @staticmethod
+    def forward(ctx, x, w):
+        from automodel_amd.ops._backend import hip_ops
+
+        ctx.save_for_backward(x, w)
+        return hip_ops().router_linear(x, w)
+
+    @staticmethod
+    def backward(ctx, g):
+        x, w = ctx.saved_tensors
+        want_dx, want_dw = ctx.needs_input_grad
+        if torch.is_grad_enabled() or not _device_tensor(g):    # a graph of the backward is wanted
+            return ((g @ w.float()).to(x.dtype) if want_dx else None,
+                    (g.t() @ x.float()).to(w.dtype) if want_dw else None)
+        from automodel_amd.ops._backend import hip_ops
+
+        dx, dw = hip_ops().router_linear_bwd(g, x, w, want_dx, want_dw)
+        return dx if want_dx else None, dw if want_dw else None
+
+
+def _router_scores(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x [T, H] times w [E, H] transposed, in float32. The kernel (csrc/router_linear.hip) keeps
+    at most 128 experts' weights in a wave's registers and moves 128 columns at a time."""
+    E, H = w.shape
+    if (x.dtype == w.dtype == torch.bfloat16 and _device_tensor(x) and _device_tensor(w)
+            and x.dim() == 2 and x.device == w.device and x.shape[1] == H and x.shape[0] > 0
+            and E % 8 == 0 and 8 <= E <= 128 and H % 128 == 0 and 128 <= H <= 1 << 20
+            and not torch.is_autocast_enabled("cuda")):
+        return _RouterLinear.apply(x, w)
+    return torch.nn.functional.linear(x.float(), w.float())
 
 
 def _largest(scores: torch.Tensor, k: int) -> torch.Tensor:
@@ -60,7 +97,7 @@ class Gate(nn.Module):
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """x [T, H] -> (probs [T, K], indices [T, K])."""
         cfg = self.cfg
-        logits = torch.nn.functional.linear(x.float(), self.weight.float())
+        logits = _router_scores(x, self.weight)
         if cfg.score_func == "sigmoid":
             scores = logits.sigmoid()
         else:

@@ -98,6 +98,10 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("grouped_gemm_nt_fp8", &amd_ops::grouped_gemm_nt_fp8);
   m.def("route_plan(Tensor indices, Tensor probs, int E) -> (Tensor, Tensor, Tensor, Tensor, Tensor)");
   m.impl("route_plan", &amd_ops::route_plan);
+  m.def("router_linear(Tensor x, Tensor w) -> Tensor");
+  m.impl("router_linear", &amd_ops::router_linear);
+  m.def("router_linear_bwd(Tensor d, Tensor x, Tensor w, bool want_dx, bool want_dw) -> (Tensor, Tensor)");
+  m.impl("router_linear_bwd", &amd_ops::router_linear_bwd);
   m.def("route_topk(Tensor scores, int K) -> Tensor");
   m.impl("route_topk", &amd_ops::route_topk);
   m.def("expert_load(Tensor indices, int E) -> Tensor");

@@ -123,6 +123,9 @@ at::Tensor grouped_gemm_nt_fp8(const at::Tensor& x8, const at::Tensor& w8,
                                int64_t bm = 128);
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor> route_plan(
     const at::Tensor& indices, const at::Tensor& probs, int64_t E);
+at::Tensor router_linear(const at::Tensor& x, const at::Tensor& w);
+std::tuple<at::Tensor, at::Tensor> router_linear_bwd(const at::Tensor& d, const at::Tensor& x,
+                                                     const at::Tensor& w, bool want_dx, bool want_dw);
 at::Tensor route_topk(const at::Tensor& scores, int64_t K);
 at::Tensor expert_load(const at::Tensor& indices, int64_t E);
 std::tuple<at::Tensor, at::Tensor> combine_bwd(const at::Tensor& g, const at::Tensor& y,
