@@ -13,17 +13,21 @@ import torch.nn as nn
 
 from automodel_amd.moe.config import MoEConfig
 from automodel_amd.moe.experts import GroupedExperts
+from automodel_amd.ops._backend import ops_available
 from automodel_amd.ops.swiglu import swiglu
 
 
-def _device_tensor(t: torch.Tensor) -> bool:
-    """An ordinary GPU tensor in an eager call: traced, transformed and mode-wrapped calls
-    stay with torch's own operations, which those can see into."""
-    return (t.is_cuda and type(t) in (torch.Tensor, nn.Parameter)
+def _device_op(name: str, t: torch.Tensor):
+    """The kernel of that name for an ordinary GPU tensor in an eager call, else None: traced,
+    transformed and mode-wrapped calls stay with torch's own operations, which those can see
+    into, and so does a build of the inference kernels alone."""
+    if not (t.is_cuda and type(t) in (torch.Tensor, nn.Parameter)
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and not torch._C._are_functorch_transforms_active()
             and torch.autograd.forward_ad._current_level < 0
-            and not torch._C._len_torch_dispatch_stack())
+            and not torch._C._len_torch_dispatch_stack() and ops_available()):
+        return None
+    return getattr(torch.ops.amd_ops, name, None)
 
 
 class _RouterLinear(torch.autograd.Function):
@@ -31,21 +35,18 @@ class _RouterLinear(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w):
-        from automodel_amd.ops._backend import hip_ops
-
         ctx.save_for_backward(x, w)
-        return hip_ops().router_linear(x, w)
+        return torch.ops.amd_ops.router_linear(x, w)
 
     @staticmethod
     def backward(ctx, g):
         x, w = ctx.saved_tensors
         want_dx, want_dw = ctx.needs_input_grad
-        if torch.is_grad_enabled() or not _device_tensor(g):    # a graph of the backward is wanted
+        op = _device_op("router_linear_bwd", g)
+        if op is None or torch.is_grad_enabled():      # the latter: a graph of the backward is wanted
             return ((g @ w.float()).to(x.dtype) if want_dx else None,
                     (g.t() @ x.float()).to(w.dtype) if want_dw else None)
-        from automodel_amd.ops._backend import hip_ops
-
-        dx, dw = hip_ops().router_linear_bwd(g, x, w, want_dx, want_dw)
+        dx, dw = op(g, x, w, want_dx, want_dw)
         return dx if want_dx else None, dw if want_dw else None
 
 
@@ -53,10 +54,11 @@ def _router_scores(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [T, H] times w [E, H] transposed, in float32. The kernel (csrc/router_linear.hip) keeps
     at most 128 experts' weights in a wave's registers and moves 128 columns at a time."""
     E, H = w.shape
-    if (x.dtype == w.dtype == torch.bfloat16 and _device_tensor(x) and _device_tensor(w)
-            and x.dim() == 2 and x.device == w.device and x.shape[1] == H and x.shape[0] > 0
+    if (x.dtype == w.dtype == torch.bfloat16 and x.dim() == 2 and x.device == w.device
+            and x.shape[1] == H and x.shape[0] > 0
             and E % 8 == 0 and 8 <= E <= 128 and H % 128 == 0 and 128 <= H <= 1 << 20
-            and not torch.is_autocast_enabled("cuda")):
+            and not torch.is_autocast_enabled("cuda")
+            and _device_op("router_linear", x) and _device_op("router_linear", w)):
         return _RouterLinear.apply(x, w)
     return torch.nn.functional.linear(x.float(), w.float())
 
@@ -65,20 +67,18 @@ def _largest(scores: torch.Tensor, k: int) -> torch.Tensor:
     """The indices of each row's k largest scores, the largest first. The kernel holds a row
     in one wave and takes the scores out one by one; its limits are the range over which it
     was measured to be 4 to 9 times faster (csrc/moe_kernels.hip)."""
-    if (_device_tensor(scores) and scores.dtype == torch.float32 and scores.dim() == 2
+    op = _device_op("route_topk", scores)
+    if (op and scores.dtype == torch.float32 and scores.dim() == 2
             and 1 <= k <= min(scores.shape[1], 32) and scores.shape[1] <= 512):
-        from automodel_amd.ops._backend import hip_ops
-
-        return hip_ops().route_topk(scores.detach().contiguous(), k)
+        return op(scores.detach().contiguous(), k)
     return scores.topk(k, dim=-1)[1]
 
 
 def _expert_load(indices: torch.Tensor, n_experts: int) -> torch.Tensor:
     """How often each expert was chosen, float32 [n_experts]."""
-    if _device_tensor(indices) and indices.dtype == torch.long and n_experts <= 4096:
-        from automodel_amd.ops._backend import hip_ops
-
-        return hip_ops().expert_load(indices.contiguous(), n_experts)
+    op = _device_op("expert_load", indices)
+    if op and indices.dtype == torch.long and n_experts <= 4096:
+        return op(indices.contiguous(), n_experts)
     load = torch.zeros(n_experts, device=indices.device)
     return load.scatter_add_(0, indices.reshape(-1),
                              torch.ones(indices.numel(), device=indices.device))

@@ -9,6 +9,7 @@
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
 #include "common.h"
@@ -213,6 +214,7 @@ at::Tensor route_topk(const at::Tensor& scores, int64_t K) {
   TORCH_CHECK(E <= CHOICE_MAX_E && K >= 1 && K <= std::min<long>(E, CHOICE_MAX_K), "route_topk: 1 to ",
               CHOICE_MAX_K, " of at most ", CHOICE_MAX_E, " experts");
   TORCH_CHECK(T < (1l << 31) - 4, "route_topk: too many tokens");
+  const c10::DeviceGuard guard(scores.device());
   auto out = at::empty({T, K}, scores.options().dtype(at::kLong));
   if (!T) return out;
   auto stream = c10::hip::getCurrentHIPStream().stream();
@@ -253,6 +255,7 @@ at::Tensor expert_load(const at::Tensor& indices, int64_t E) {
   TORCH_CHECK(E >= 1 && E <= ROUTE_MAX_E, "expert_load: 1 to ", ROUTE_MAX_E, " experts");
   const long n = indices.numel();
   TORCH_CHECK(n < (1l << 31), "expert_load: too many choices");
+  const c10::DeviceGuard guard(indices.device());
   auto load = at::zeros({E}, indices.options().dtype(at::kFloat));
   if (n)
     hipLaunchKernelGGL(expert_load_kernel, dim3((unsigned)((n + LOAD_CHUNK - 1) / LOAD_CHUNK)), dim3(256),

@@ -15,6 +15,7 @@
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
 #include "common.h"
@@ -263,6 +264,7 @@ void rl_check(const at::Tensor& x, const at::Tensor& w) {
 
 at::Tensor router_linear(const at::Tensor& x_, const at::Tensor& w_) {
   rl_check(x_, w_);
+  const c10::DeviceGuard guard(x_.device());
   auto x = rl_plain(x_), w = rl_plain(w_);
   const int T = (int)x.size(0), H = (int)x.size(1), E = (int)w.size(0);
   auto out = at::empty({T, E}, x.options().dtype(at::kFloat));
@@ -291,6 +293,7 @@ std::tuple<at::Tensor, at::Tensor> router_linear_bwd(const at::Tensor& d_, const
   rl_check(x_, w_);
   TORCH_CHECK(d_.device() == x_.device() && d_.dim() == 2 && d_.scalar_type() == at::kFloat &&
                   d_.size(0) == x_.size(0) && d_.size(1) == w_.size(0), "router_linear_bwd: d [T,E] float32");
+  const c10::DeviceGuard guard(x_.device());
   auto d = rl_plain(d_);
   const int T = (int)x_.size(0), H = (int)x_.size(1), E = (int)w_.size(0);
   auto stream = c10::hip::getCurrentHIPStream().stream();
