@@ -90,7 +90,8 @@ class DecodeSession:
                 ids = torch.tensor([list(p) for p in prompts], device=self.device)
                 if getattr(self.model, "selects_logit_rows", False):
                     rows = [i * lens[0] + j % lens[0] for i, w in enumerate(want) for j in w]
-                    logits = self.model(ids, logit_rows=torch.tensor(rows, device=self.device))
+                    rows = torch.tensor(rows, dtype=torch.long, device=self.device)
+                    logits = self.model(ids, logit_rows=rows)
                 else:
                     full = self.model(ids)
                     logits = torch.cat([full[i, w] for i, w in enumerate(want)])
