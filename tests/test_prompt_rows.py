@@ -24,4 +24,6 @@ def test_wanted_rows(model, want):
     _, logits = DecodeSession(model, 2, 8).prefill(PROMPTS, want)
     with torch.no_grad():
         full = model(torch.tensor(PROMPTS))
-    assert torch.equal(logits, torch.cat([full[i, w] for i, w in enumerate(want)]))
+    # a product of fewer rows may sum in another order: 32 terms of size below 1, in float32
+    torch.testing.assert_close(logits, torch.cat([full[i, w] for i, w in enumerate(want)]),
+                               rtol=0, atol=32 * 2.0 ** -23)
