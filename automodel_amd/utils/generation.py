@@ -89,7 +89,7 @@ class DecodeSession:
                 handles = list(range(len(prompts)))
                 ids = torch.tensor([list(p) for p in prompts], device=self.device)
                 if getattr(self.model, "selects_logit_rows", False):
-                    rows = [i * lens[0] + j % lens[0] for i, w in enumerate(want) for j in w]
+                    rows = [i * lens[0] + range(lens[i])[j] for i, w in enumerate(want) for j in w]
                     rows = torch.tensor(rows, dtype=torch.long, device=self.device)
                     logits = self.model(ids, logit_rows=rows)
                 else:

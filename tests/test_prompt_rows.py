@@ -27,3 +27,11 @@ def test_wanted_rows(model, want):
     # a product of fewer rows may sum in another order: 32 terms of size below 1, in float32
     torch.testing.assert_close(logits, torch.cat([full[i, w] for i, w in enumerate(want)]),
                                rtol=0, atol=32 * 2.0 ** -23)
+
+
+@pytest.mark.parametrize("want", [[[3], [0]], [[5], [1]], [[0], [1, -4]], [[0], [1], [2]]])
+def test_rows_beyond_the_prompt_are_refused(model, want):
+    session = DecodeSession(model, 2, 8)
+    with pytest.raises(IndexError):
+        session.prefill(PROMPTS, want)
+    assert session.live == [] and session.cache.pos == 0
