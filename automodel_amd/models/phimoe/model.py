@@ -164,7 +164,7 @@ class PhimoeSparseMoeBlock(nn.Module):
         xf = x.reshape(-1, H)
         logits = self.router(xf)
         probs, indices = sparsemixer(logits, self.jitter_eps, self.training)
-        return self.experts(xf, probs.to(x.dtype), indices).view(B, S, H)
+        return self.experts(xf, probs.to(x.dtype), indices, checked=True).view(B, S, H)
 
 
 class PhimoeDecoderLayer(nn.Module):

@@ -54,13 +54,24 @@ class _FusedPermuteGather(torch.autograd.Function):
 _ROUTE_MAX_EXPERTS = 4096       # csrc/moe_kernels.hip
 
 
-def fused_dispatch_combine(x, probs, indices, n_experts, expert_fn):
+def check_experts(indices: torch.Tensor, n_experts: int) -> None:
+    """Refuses experts that do not exist; waits for the device that ``indices`` is on."""
+    if indices.numel():
+        low, high = torch.stack(indices.aminmax()).tolist()
+        if low < 0 or high >= n_experts:
+            raise RuntimeError(f"experts {low} to {high} chosen of {n_experts}")
+
+
+def fused_dispatch_combine(x, probs, indices, n_experts, expert_fn, checked=False):
     """GPU MoE glue: device-side routing plan, HIP gather, expert_fn over permuted
     rows, HIP combine — one gather + one combine instead of
     repeat_interleave + fancy-index + scatter (reference fused permute/
-    unpermute, moe_utils.py:31/115). Nothing waits for the host."""
+    unpermute, moe_utils.py:31/115). Nothing waits for the host where ``checked`` says that
+    every index is one of an expert; without it the indices are looked at first."""
     from automodel_amd.ops._backend import hip_ops
 
+    if not checked:
+        check_experts(indices, n_experts)
     T, K = indices.shape
     with torch.no_grad():
         probs32 = probs.detach().float().contiguous()
@@ -234,11 +245,13 @@ class GroupedExperts(nn.Module):
             return grouped_linear(h, self.down_proj, cl, plan=plan)
         return self._expert_mlp_loop(x_perm, counts)
 
-    def forward(self, x: torch.Tensor, probs: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, probs: torch.Tensor, indices: torch.Tensor,
+                checked: bool = False) -> torch.Tensor:
+        """``checked``: the caller knows that every index is one of an expert."""
         if (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[-1] % 8 == 0
                 and self.backend in ("auto", "hip_grouped")):
             return fused_dispatch_combine(x, probs, indices, self.n_experts,
-                                          self.forward_permuted)
+                                          self.forward_permuted, checked)
         x_perm, sort_idx, counts = permute_tokens(x, indices, self.n_experts)
         y_perm = self.forward_permuted(x_perm, counts)
         return unpermute_tokens(y_perm, sort_idx, probs)

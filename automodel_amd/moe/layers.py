@@ -12,7 +12,7 @@ import torch
 import torch.nn as nn
 
 from automodel_amd.moe.config import MoEConfig
-from automodel_amd.moe.experts import GroupedExperts
+from automodel_amd.moe.experts import GroupedExperts, check_experts
 from automodel_amd.ops._backend import ops_available
 from automodel_amd.ops.swiglu import swiglu
 
@@ -122,7 +122,9 @@ class Gate(nn.Module):
 
         rr = active_router_replay()
         if rr is not None and rr.mode == "replay":
-            indices = rr.next_replay().to(x.device)   # R3: replayed routing
+            indices = rr.next_replay()                # R3: replayed routing
+            check_experts(indices, scores.shape[1])   # (a file's or another model's)
+            indices = indices.to(x.device)
         else:
             base = logits if cfg.topk_then_softmax else select_scores
             indices = _largest(base, cfg.n_activated_experts)
@@ -228,6 +230,11 @@ class MoE(nn.Module):
         probs, indices = self.gate(xf)
         with torch.no_grad():
             self.last_expert_load = _expert_load(indices, self.cfg.n_routed_experts)
+        # a router of this file chooses among its experts: they need not be looked at again
+        known = {}
+        if (type(self.experts).forward is GroupedExperts.forward
+                and type(self.gate).forward in (Gate.forward, FakeBalancedGate.forward)):
+            known["checked"] = True
         if self.dispatcher is not None:
             y = self.dispatcher(xf, probs, indices, self.experts)
         elif self.shared_experts is not None and xf.is_cuda:
@@ -241,12 +248,12 @@ class MoE(nn.Module):
                 shared = self.shared_experts(xf)
                 if getattr(self, "shared_expert_gate", None) is not None:
                     shared = torch.sigmoid(self.shared_expert_gate(xf)) * shared
-            y = self.experts(xf, probs, indices)
+            y = self.experts(xf, probs, indices, **known)
             torch.cuda.current_stream().wait_stream(ss)
             shared.record_stream(torch.cuda.current_stream())
             return (y + shared).view(B, S, H)
         else:
-            y = self.experts(xf, probs, indices)
+            y = self.experts(xf, probs, indices, **known)
         if self.shared_experts is not None:
             shared = self.shared_experts(xf)
             if getattr(self, "shared_expert_gate", None) is not None:
