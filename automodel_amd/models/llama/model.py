@@ -20,10 +20,14 @@ import torch
 import torch.nn as nn
 
 from automodel_amd.models.common.backend import BackendConfig
-from automodel_amd.ops.attention import flash_attention
+from automodel_amd.ops import attention as attn_mod
+from automodel_amd.ops.attention import _sdpa, flash_attention, sdpa_masked
 from automodel_amd.ops.rms_norm import RMSNorm, add_norm
 from automodel_amd.ops.rope import apply_rope, build_rope_cache
 from automodel_amd.ops.swiglu import swiglu, swiglu_cat
+from automodel_amd.parallel.cp import active_cp, cp_blockdiag_attention, cp_flash_attention
+from automodel_amd.serving.decode_linear import decode_rows, plain_linears, unobserved
+from automodel_amd.utils.kv_cache import KVCache, StaticKVCache, active_kv_cache, maybe_update_kv
 
 
 @dataclass
@@ -132,11 +136,7 @@ class LlamaConfig:
 
 def _project(backend: BackendConfig, lins: list[nn.Module], x: torch.Tensor) -> list[torch.Tensor]:
     """``[lin(x) for lin in lins]``; the few rows of a decode step in one launch."""
-    from automodel_amd.utils.kv_cache import active_kv_cache
-
     if active_kv_cache() is not None and backend.attn == "hip":
-        from automodel_amd.serving.decode_linear import decode_rows
-
         ys = decode_rows(lins, x)
         if ys is not None:
             return ys
@@ -169,8 +169,6 @@ class LlamaAttention(nn.Module):
             self.k_norm = RMSNorm(Hk * D, cfg.rms_norm_eps, backend.rms_norm)
 
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
-        from automodel_amd.parallel.cp import active_cp, cp_flash_attention
-
         B, S, _ = x.shape
         if self.cfg.fused_qkv:
             (qkv,) = _project(self.backend, [self.qkv_proj], x)
@@ -209,8 +207,6 @@ class LlamaAttention(nn.Module):
         if self.cfg.sliding_window is not None:
             # windowed causal (mistral): explicit mask via sdpa — the flash
             # kernel's full-causal tiling doesn't window (round-2 kernel)
-            from automodel_amd.ops.attention import sdpa_masked
-
             i = torch.arange(S, device=x.device)
             keep = (i[None, :] <= i[:, None]) \
                 & (i[None, :] > i[:, None] - self.cfg.sliding_window)
@@ -218,24 +214,16 @@ class LlamaAttention(nn.Module):
                 .to(q.dtype).reshape(1, 1, S, S)
             o = sdpa_masked(q, k, v, mask, scale=attn_scale)
         elif self.cfg.bidirectional:
-            from automodel_amd.ops.attention import _sdpa
-
             o = _sdpa(q, k, v, causal=False, scale=attn_scale)
         elif active_cp() is not None:
-            from automodel_amd.ops import attention as attn_mod
-
             if attn_mod._VARLEN_CU is not None:
                 # packed documents under CP: block-diagonal-correct path
-                from automodel_amd.parallel.cp import cp_blockdiag_attention
-
                 o = cp_blockdiag_attention(q, k, v, attn_mod._VARLEN_CU,
                                            scale=attn_scale)
             else:
                 o = cp_flash_attention(q, k, v, causal=True, scale=attn_scale,
                                        backend=self.backend.attn)
         else:
-            from automodel_amd.utils.kv_cache import active_kv_cache, maybe_update_kv
-
             cache = active_kv_cache()
             o = None
             if cache is not None and self.backend.attn == "hip":
@@ -245,8 +233,6 @@ class LlamaAttention(nn.Module):
             elif cache is not None and getattr(cache, "is_static", False):
                 # static-shape decode (hipGraph capture): full-buffer KV +
                 # additive mask from the device position counter
-                from automodel_amd.ops.attention import sdpa_masked
-
                 k, v, _ = maybe_update_kv(k, v)
                 o = sdpa_masked(q, k, v, cache.attn_mask(), scale=attn_scale)
             else:
@@ -278,11 +264,7 @@ class LlamaMLP(nn.Module):
         self.down_proj = nn.Linear(cfg.intermediate_size, cfg.hidden_size, bias=bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        from automodel_amd.utils.kv_cache import active_kv_cache
-
         if active_kv_cache() is not None and self.backend.attn == "hip":
-            from automodel_amd.serving.decode_linear import decode_rows
-
             lins = [self.gate_up_proj] if self.fused else [self.gate_proj, self.up_proj]
             act = decode_rows(lins, x, glu=True)
             if act is not None:
@@ -351,10 +333,6 @@ class LlamaDecoderLayer(nn.Module):
         """One token per sequence behind a K/V cache, all of the layer's kernels issued by
         one native call (csrc/llama_layer.cpp). None for layers and inputs that it does not
         take, and nothing is done."""
-        from automodel_amd.parallel.cp import active_cp
-        from automodel_amd.serving.decode_linear import plain_linears, unobserved
-        from automodel_amd.utils.kv_cache import KVCache, StaticKVCache, active_kv_cache
-
         cache, attn, mlp = active_kv_cache(), self.self_attn, self.mlp
         if not (type(cache) in (KVCache, StaticKVCache) and not self.olmo2 and type(x) is torch.Tensor
                 and x.is_cuda and x.shape[1] == 1 and x.dtype == torch.bfloat16
@@ -388,9 +366,10 @@ class LlamaDecoderLayer(nn.Module):
         return y[0]
 
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
-        y = self._decode_step(x, cos, sin)
-        if y is not None:
-            return y
+        if active_kv_cache() is not None:
+            y = self._decode_step(x, cos, sin)
+            if y is not None:
+                return y
         if self.olmo2:
             x = x + self.post_attention_layernorm(self.self_attn(x, cos, sin))
             return x + self.post_feedforward_layernorm(self.mlp(x))
