@@ -262,10 +262,12 @@ at::Tensor kv_decode_attn(const at::Tensor& q, const at::Tensor& k_new, const at
                   v_new.scalar_type() == at::kBFloat16, "kv_decode_attn: new k, v [B,1,Hk,D] bf16");
   TORCH_CHECK(Hq % Hk == 0 && D % 8 == 0 && D >= 8 && D <= 256 && B >= 1 && B <= 65535,
               "kv_decode_attn: whole groups, head dim a multiple of 8 up to 256");
-  TORCH_CHECK(pos_dev ? pos_dev->is_cuda() && pos_dev->scalar_type() == at::kLong && pos_dev->numel() == 1
+  TORCH_CHECK(pos_dev ? pos_dev->device() == q.device() && pos_dev->scalar_type() == at::kLong && pos_dev->numel() == 1
                       : pos >= 0 && pos < max_len, "kv_decode_attn: position outside the cache");
-  for (const at::Tensor* t : {&q, &k_new, &v_new, (const at::Tensor*)&k_cache, (const at::Tensor*)&v_cache})
+  for (const at::Tensor* t : {&q, &k_new, &v_new, (const at::Tensor*)&k_cache, (const at::Tensor*)&v_cache}) {
+    TORCH_CHECK(t->device() == q.device(), "kv_decode_attn: one device");
     TORCH_CHECK((uintptr_t)t->data_ptr() % 16 == 0, "kv_decode_attn: 16-byte alignment");
+  }
 
   const int group = Hq / Hk;
   const int gq = group >= 5 ? 8 : group >= 3 ? 4 : group;

@@ -64,3 +64,15 @@ def test_decode_matches_whole_forward(heads, kv, dim):
     for _ in range(2):
         assert torch.equal(generate_graphed(model, prompt, 12), eager)
     assert torch.equal(generate_cached(model, prompt, 2), eager[:, :22])
+
+
+@pytest.mark.parametrize("elsewhere", [1, 2, 3, 4, 5])
+def test_tensors_elsewhere_are_refused(elsewhere):
+    from automodel_amd.ops._backend import hip_ops
+
+    args = [torch.zeros(1, 1, 2, 64, dtype=torch.bfloat16), torch.zeros(1, 1, 1, 64, dtype=torch.bfloat16),
+            torch.zeros(1, 1, 1, 64, dtype=torch.bfloat16), torch.zeros(1, 9, 1, 64, dtype=torch.bfloat16),
+            torch.zeros(1, 9, 1, 64, dtype=torch.bfloat16), torch.tensor(0)]
+    args = [t if i == elsewhere else t.cuda() for i, t in enumerate(args)]
+    with pytest.raises(RuntimeError):
+        hip_ops().kv_decode_attn(*args[:5], -1, args[5], 0.125)
