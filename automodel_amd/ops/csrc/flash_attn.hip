@@ -177,11 +177,12 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArg
   // first tile with a key that some row of the wave must not see (from the diagonal on)
   const int t_diag = a.causal ? (a.q_start + q0 + 1) / 64 : all;
 
+  const unsigned lds = lds_address(smem);
   auto load_k = [&](int t) {
-    load_tile<DQK, 64, WAVES>(kp + (long)t * 64 * k_rs, k_rs, a.Skv - t * 64, (t & 1) * KT);
+    load_tile<DQK, 64, WAVES>(kp + (long)t * 64 * k_rs, k_rs, a.Skv - t * 64, lds + (t & 1) * KT);
   };
   auto load_v = [&](int t) {
-    load_tile<DV, 64, WAVES>(vp + (long)t * 64 * v_rs, v_rs, a.Skv - t * 64, 2 * KT + (t & 1) * VT);
+    load_tile<DV, 64, WAVES>(vp + (long)t * 64 * v_rs, v_rs, a.Skv - t * 64, lds + 2 * KT + (t & 1) * VT);
   };
   f32x16_t s0, s1;
   bf16x8_t p0[2], p1[2];

@@ -193,15 +193,17 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void bwd_dkv_kernel(const BwdArgs 
   const int nt = max(j1 - j0, 0), total = nt * G;
   const unsigned q_rs = (unsigned)a.Hq * DQK * 2, o_rs = (unsigned)a.Hq * DV * 2;
 
+  const unsigned lds = lds_address(smem);
   auto load = [&](int u, unsigned buf) {
     const int h = kvh * G + u / nt, q0 = (j0 + u % nt) * 64;
-    load_tile<DQK, 64, WAVES>(a.q + (((long)b * a.Sq + q0) * a.Hq + h) * DQK, q_rs, a.Sq - q0, buf);
-    load_tile<DV, 64, WAVES>(a.dout + (((long)b * a.Sq + q0) * a.Hq + h) * DV, o_rs, a.Sq - q0, buf + F::QT);
+    load_tile<DQK, 64, WAVES>(a.q + (((long)b * a.Sq + q0) * a.Hq + h) * DQK, q_rs, a.Sq - q0,
+                              lds + buf);
+    load_tile<DV, 64, WAVES>(a.dout + (((long)b * a.Sq + q0) * a.Hq + h) * DV, o_rs, a.Sq - q0,
+                             lds + buf + F::QT);
     if (wid == 0) {      // 64 rows of both statistics, 16 bytes a lane (lanes 32.. repeat)
       const float* src = a.stats + ((long)b * a.Hq + h) * a.sp + q0;
       const float* mine = src + (lane & 15) * 4 + ((lane >> 4) & 1) * a.plane;
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                   :: "s"(buf + (unsigned)(F::QT + F::OT)), "v"(mine) : "memory");
+      load_lds16(lds + buf + F::QT + F::OT, mine);
     }
   };
   auto masked = [&](int u) {
@@ -346,11 +348,13 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void bwd_dq_kernel(const BwdArgs a
   const unsigned k_rs = (unsigned)a.Hk * DQK * 2, v_rs = (unsigned)a.Hk * DV * 2;
   const bf16* kp = a.k + ((long)b * a.Skv * a.Hk + kvh) * DQK;
   const bf16* vp = a.v + ((long)b * a.Skv * a.Hk + kvh) * DV;
+  const unsigned lds = lds_address(smem);
   auto load_k = [&](int t, unsigned to) {
-    load_tile<DQK, 64, WAVES>(kp + (long)t * 64 * a.Hk * DQK, k_rs, a.Skv - t * 64, to);
+    load_tile<DQK, 64, WAVES>(kp + (long)t * 64 * a.Hk * DQK, k_rs, a.Skv - t * 64, lds + to);
   };
   auto load_v = [&](int t) {
-    load_tile<DV, 64, WAVES>(vp + (long)t * 64 * a.Hk * DV, v_rs, a.Skv - t * 64, V0 + (t & 1) * VT);
+    load_tile<DV, 64, WAVES>(vp + (long)t * 64 * a.Hk * DV, v_rs, a.Skv - t * 64,
+                             lds + V0 + (t & 1) * VT);
   };
   auto masked = [&](int t) {
     return t >= t_diag || t * 64 + 64 > a.Skv || (VARLEN && t * 64 < doc_w);

@@ -18,6 +18,7 @@
 #pragma once
 
 #include "common.h"
+#include "lds_load.h"
 
 namespace amd_ops {
 namespace fa {
@@ -37,10 +38,6 @@ __device__ __forceinline__ int swz(int row) {
   else return ((row & 3) << 2) | ((row >> 2) & 3);
 }
 
-__device__ __forceinline__ unsigned lds_offset(const void* p) {
-  return (unsigned)(unsigned long long)(uintptr_t)p;
-}
-
 __device__ __forceinline__ f32x16_t mma(bf16x8_t a, bf16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
@@ -55,12 +52,10 @@ __device__ __forceinline__ f32x16_t zero16() {
 // row of register r of a 32x32 accumulator
 __device__ __forceinline__ int acc_row(int r, int half) { return (r & 3) + 8 * (r >> 2) + 4 * half; }
 
-// 16-byte direct loads of ROWS x D into the tile at LDS byte offset `lds`: rows
+// 16-byte direct loads of ROWS x D into the tile at LDS address `lds`: rows
 // row0.. of a tensor whose rows are `stride` bytes apart, clamped to the last of `left`
 // remaining rows and to the first `chunks` 16-byte pieces of a row (callers mask what lies
-// beyond). The loads are asm because the compiler would wait for every load in flight
-// before any LDS read; they write no register. `wait_loads` and a barrier come before the
-// tile is read.
+// beyond).
 template <int D, int ROWS, int WAVES>
 constexpr int tile_loads() { return ROWS * row_bytes(D) / 1024 / WAVES; }   // per wave
 
@@ -80,21 +75,8 @@ __device__ __forceinline__ void load_tile(const void* base, unsigned stride, int
     int chunk = slot ^ swz<D>(row);
     if (chunk >= chunks) chunk = 0;                     // any valid address
     const unsigned off = (unsigned)min(row, left - 1) * stride + chunk * 16;
-    const unsigned to = lds + j * 1024;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :: "s"(to), "v"(off), "s"(base) : "memory");
+    load_lds16(lds + j * 1024, base, off);
   }
-}
-
-// waits until at most LATER of the wave's loads, the last ones issued, are in flight
-template <int LATER = 0>
-__device__ __forceinline__ void wait_loads() {
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(LATER) : "memory");
-}
-
-// barrier behind which every wave's LDS reads so far are complete
-__device__ __forceinline__ void barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 // per-lane offsets of the reads; `tile32` and `chunk` are compile-time
@@ -157,11 +139,6 @@ __device__ __forceinline__ bf16x8_t pack8(const f32x16_t& p, int c) {
   return out;
 }
 
-// the other half-wave's value of the same column
-__device__ __forceinline__ float other_half(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
-}
 __device__ __forceinline__ float max_halves(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));

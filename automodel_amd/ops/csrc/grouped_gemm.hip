@@ -110,7 +110,9 @@ __global__ __launch_bounds__(64 * WAVES, 1) void grouped_gemm_kernel(const Group
   const bool live = wr * 64 < r_left && wc * WN < c_left;
 
   const int once = (sum + STEP - 1) / STEP, steps = MODE == NN && rp2 ? 2 * once : once;
+  const unsigned lds = lds_address(smem);
   auto load = [&](int s, unsigned buf) {
+    buf += lds;
     const bf16 *r = rp, *c = cp;
     if (MODE == NN && s >= once) {
       r = rp2;

@@ -18,6 +18,7 @@
 
 #include "common.h"
 #include "latent_attn.h"
+#include "lds_load.h"
 #include "ops_api.h"
 
 namespace amd_ops {
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(256) void latent_decode_attn_kernel(
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int KS = C * 2;
   char* kt = lds;                                 // [64][KS]
-  const unsigned kt_at = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const unsigned kt_at = fa::lds_address(lds);
   char* pt = kt + LD_KEYS * KS;                   // [16][LD_PSTRIDE]
   float* red = reinterpret_cast<float*>(pt + 16 * LD_PSTRIDE);   // [4][16]
 
@@ -278,8 +279,7 @@ __global__ __launch_bounds__(256) void latent_decode_attn_kernel(
     for (int j = wid; j < vecs; j += 4) {         // a kilobyte each
       const unsigned i = j * 64 + lane, row = (i * magic) >> 20, c = i - row * vecs;
       const unsigned off = (unsigned)min((int)row, left - 1) * C * 2 + ((c ^ ((row >> sh) & gm)) << 4);
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                   :: "s"(kt_at + j * 1024), "v"(off), "s"(tile) : "memory");
+      fa::load_lds16(kt_at + j * 1024, tile, off);
     }
   };
   // pieces of this lane's reads: row lo16 of a wave's keys; rows hi4 * 8 + lo16 / 4 and 4 on
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void latent_decode_attn_kernel(
   for (int t = t_lo; t < t_hi; ++t) {
     const int k0 = t * LD_KEYS;
     stage(t);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    fa::wait_loads();
     __syncthreads();
 
     // scores: D[key = 4 hi4 + i][head = lo16] of this wave's 16 keys
