@@ -17,12 +17,12 @@ __device__ __forceinline__ unsigned lds_address(const void* p) {
 // 16 bytes a lane, 1024 consecutive ones of LDS a wave: from `base` + the lane's `off`
 __device__ __forceinline__ void load_lds16(unsigned lds, const void* base, unsigned off) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds), "v"(off), "s"(base) : "memory");
+               :: "s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
 // the same from an address of the lane's own
 __device__ __forceinline__ void load_lds16(unsigned lds, const void* mine) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :: "s"(lds), "v"(mine) : "memory");
+               :: "s"(lds), "v"(mine) : "memory", "m0");
 }
 
 // waits until at most LATER of the wave's loads, the last ones issued, are in flight
