@@ -211,7 +211,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArg
       wait_loads();       // K of t + 1, V of t; the buffers of K of t, V of t - 1 are free
       barrier();
       load_v(t + 1);
-      load_k(min(t + 2, t1 - 1));
+      load_k(t + 2);
       f.template softmax<false>(s1, t * 64 + 32, p1, [&] { f.scores(s0, kn, 0); f.values(p0, vt, 0); });
     };
     auto general = [&](int t) {
@@ -235,9 +235,10 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArg
         if (t == t1w - 1) f.values(p1, vt, 1);
       }
     };
-    // tiles of the steady kind: [first, end)
+    // Tiles of the steady kind: [first, end). There is a tile t + 2 for each of them to load:
+    // the buffer of t + 1, which a step reads, has no load in flight.
     const int first = max(t0w + 1, VARLEN ? (doc_w + 63) / 64 : 0);
-    const int end = min(min(t_diag, a.Skv / 64), min(t1w, t1) - 1);
+    const int end = min(min(t_diag, a.Skv / 64), min(t1w - 1, t1 - 2));
     int t = t0;
     for (; t < min(first, t1) || (!VARLEN && t < end && t % 2); ++t) general(t);
     // (pairs leave a tile over at either end; the runs of short documents are too short)

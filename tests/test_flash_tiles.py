@@ -68,6 +68,23 @@ def test_forward(dims, sq, skv, causal, q_start, cuts, scale):
     assert (lse - rlse).abs().max() < 1e-5 * max(1.0, float(rlse.abs().max()))
 
 
+@pytest.mark.parametrize("dims", [(64, 64), (128, 128), (192, 128)])
+@pytest.mark.parametrize("s,causal,cuts", [(160, True, None), (544, True, None), (701, False, None),
+                                           (832, False, None), (448, True, ()), (1344, True, (40, 1000))])
+def test_last_tiles_without_a_successor(dims, s, causal, cuts):
+    """Waves whose whole tiles reach up to the last one but one."""
+    torch.manual_seed(0)
+    q = torch.randn(1, s, 4, dims[0], device="cuda").bfloat16()
+    k = torch.randn(1, s, 2, dims[0], device="cuda").bfloat16()
+    v = torch.randn(1, s, 2, dims[1], device="cuda").bfloat16()
+    start = None if cuts is None else _docs(cuts, s)[0]
+    from automodel_amd.ops._backend import hip_ops
+
+    o, _ = hip_ops().flash_attn_fwd(q, k, v, dims[0] ** -0.5, causal, 0, start)
+    ro, _ = _reference(q, k, v, causal, 0, start, dims[0] ** -0.5)
+    assert (o.float() - ro).norm() / ro.norm() < FWD
+
+
 # dS is rounded to bf16 once and so is each gradient; P and the delta of a bf16 output bring
 # about the same again
 BWD = 4 * 2.0 ** -9
