@@ -216,36 +216,39 @@ __global__ __launch_bounds__(256) void latent_decode_prep_mfma_kernel(
 constexpr int LD_KEYS = 64;           // keys per tile: 4 waves x 16
 constexpr int LD_PSTRIDE = LD_KEYS * 2 + 16;
 
-// 16 heads per workgroup (32, on the same staged keys, were no faster at 128 heads
-// and slower at 32). NCT: 16-column value tiles per wave (4 waves cover RP <= 64 *
-// NCT). NPM: bound on the 32-column steps of a row. One tile in LDS: a second
-// buffer for the next one was no faster, also at 8 tiles per split, and takes the
-// room of a second workgroup.
+// HT: head tiles of 16 per workgroup, four waves each; they share the staged keys.
+// NCT: 16-column value tiles per wave (4 waves cover RP <= 64 * NCT). NPM: bound on
+// the 32-column steps of a row. One head tile has one tile of keys in LDS, which
+// leaves room for a second workgroup; two have a second buffer, whose loads are in
+// flight while the first one is used.
 //
-// A split is a tile or two, so this is a chain of latencies, and of instructions
-// that run once: both products put the head in the lane (columns of the
+// With few rows a split is a tile or two, so this is a chain of latencies, and of
+// instructions that run once: both products put the head in the lane (columns of the
 // accumulator), so that the running maximum and scale are one value a lane, P goes
 // to LDS in one piece and the partial results leave in 16-byte stores; keys go to
 // LDS without registers in between; the queries sit in registers, which leaves LDS
 // for two workgroups per CU. With heads in the accumulator's rows, keys through
-// registers and queries in LDS: 9.7 us for 1 row, 16 heads, 200 keys and 20.9 for 8
-// rows, 32 heads, 1500 keys; now 7.0 and 12.4 (and 46 -> 49 for 8 rows of 16000).
-template <int NCT, int NPM>
-__global__ __launch_bounds__(256) void latent_decode_attn_kernel(
+// registers and queries in LDS: 9.5 us for 1 row, 16 heads, 200 keys and 21.0 for 8
+// rows, 32 heads, 1500 keys; now 7.2 and 12.3. (Rows of 576 columns, 512 of them
+// latents. 32 rows of 32000 keys, 32 heads, read at the memory's rate: 300 with the
+// launches around it, now 307.)
+template <int NCT, int NPM, int HT>
+__global__ __launch_bounds__(256 * HT) void latent_decode_attn_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ cache, const int* __restrict__ slot,
     const int* __restrict__ pos, float* __restrict__ part_o, float* __restrict__ part_ml,
     int n_slots, int max_len, int H, int RP, int C, float scale) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int KS = C * 2;
-  char* kt = lds;                                 // [64][KS]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wid = wave & 3, ht = wave >> 2;       // part of the keys and columns; head tile
+  const int tile_bytes = LD_KEYS * KS;
+  char* kt = lds;                                 // [64][KS], HT times
   const unsigned kt_at = fa::lds_address(lds);
-  char* pt = kt + LD_KEYS * KS;                   // [16][LD_PSTRIDE]
-  float* red = reinterpret_cast<float*>(pt + 16 * LD_PSTRIDE);   // [4][16]
-
-  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  char* pt = lds + HT * tile_bytes + ht * 16 * (LD_PSTRIDE + 16);   // [16][LD_PSTRIDE]
+  float* red = reinterpret_cast<float*>(pt + 16 * LD_PSTRIDE);      // [4][16]
   const int lo16 = lane & 15, hi4 = lane >> 4;
   const int split = blockIdx.x, n_split = gridDim.x;
-  const int h = blockIdx.y * 16 + lo16;           // this lane's head
+  const int h = (blockIdx.y * HT + ht) * 16 + lo16;   // this lane's head
   const int r = blockIdx.z;
 
   const int steps = C / 32;
@@ -272,14 +275,14 @@ __global__ __launch_bounds__(256) void latent_decode_attn_kernel(
   const int vecs = C / 8;                         // 16-byte pieces per row, a multiple of 4
   const int lg = min(__builtin_ctz(vecs), 4), sh = 4 - lg, gm = (1 << lg) - 1;
   const unsigned magic = ((1u << 20) + vecs - 1) / vecs;    // i / vecs, exact for i < 128 vecs
-  auto stage = [&](int t) {
+  auto stage = [&](int t, int buf) {
     const bf16* tile = base + (long)t * LD_KEYS * C;
     const int left = n - t * LD_KEYS;             // rows past the end: masked below
 #pragma unroll 2
-    for (int j = wid; j < vecs; j += 4) {         // a kilobyte each
+    for (int j = wave; j < vecs; j += 4 * HT) {   // a kilobyte each
       const unsigned i = j * 64 + lane, row = (i * magic) >> 20, c = i - row * vecs;
       const unsigned off = (unsigned)min((int)row, left - 1) * C * 2 + ((c ^ ((row >> sh) & gm)) << 4);
-      fa::load_lds16(kt_at + j * 1024, tile, off);
+      fa::load_lds16(kt_at + buf * tile_bytes + j * 1024, tile, off);
     }
   };
   // pieces of this lane's reads: row lo16 of a wave's keys; rows hi4 * 8 + lo16 / 4 and 4 on
@@ -292,11 +295,15 @@ __global__ __launch_bounds__(256) void latent_decode_attn_kernel(
 #pragma unroll
   for (int c = 0; c < NCT; ++c) acc[c] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
 
+  if (HT == 2 && t_lo < t_hi) stage(t_lo, 0);
   for (int t = t_lo; t < t_hi; ++t) {
     const int k0 = t * LD_KEYS;
-    stage(t);
+    if (HT == 2) kt = lds + ((t - t_lo) & 1) * tile_bytes;
+    else stage(t, 0);
+
     fa::wait_loads();
-    __syncthreads();
+    fa::barrier();
+    if (HT == 2 && t + 1 < t_hi) stage(t + 1, (t + 1 - t_lo) & 1);
 
     // scores: D[key = 4 hi4 + i][head = lo16] of this wave's 16 keys
     lat_f32x4 s = {0.f, 0.f, 0.f, 0.f};
@@ -319,7 +326,7 @@ __global__ __launch_bounds__(256) void latent_decode_attn_kernel(
     mx = fmaxf(mx, __shfl_xor(mx, 16));
     mx = fmaxf(mx, __shfl_xor(mx, 32));
     if (hi4 == 0) red[wid * 16 + lo16] = mx;
-    __syncthreads();
+    fa::barrier();
     float mn = m_run;
 #pragma unroll
     for (int w = 0; w < 4; ++w) mn = fmaxf(mn, red[w * 16 + lo16]);
@@ -337,7 +344,7 @@ __global__ __launch_bounds__(256) void latent_decode_attn_kernel(
     *reinterpret_cast<bf16x4*>(pt + lo16 * LD_PSTRIDE + (wid * 16 + hi4 * 4) * 2) = p;
 #pragma unroll
     for (int c = 0; c < NCT; ++c) acc[c] *= alpha;
-    __syncthreads();
+    fa::barrier();
 
     // O[column][head] += V[key][column] P[head][key], V = the tile's latents
 #pragma unroll 1
@@ -357,14 +364,14 @@ __global__ __launch_bounds__(256) void latent_decode_attn_kernel(
         }
       }
     }
-    __syncthreads();                              // before the tile is overwritten
+    if (HT == 1) fa::barrier();                   // before the tile is overwritten
   }
 
   // partial results of this split; an empty split stores zeros
   l_run += __shfl_xor(l_run, 16);
   l_run += __shfl_xor(l_run, 32);
   if (hi4 == 0) red[wid * 16 + lo16] = l_run;
-  __syncthreads();
+  fa::barrier();
   if (h >= H) return;
   const long o = ((long)r * H + h) * n_split + split;
   if (wid == 0 && hi4 == 0) {
@@ -669,26 +676,39 @@ std::tuple<at::Tensor, at::Tensor> latent_decode_attn(const at::Tensor& q, const
   auto part_ml = at::empty({R, H, splits, 2}, part_o.options());
   if (R == 0) return {part_o, part_ml};
   auto stream = c10::hip::getCurrentHIPStream();
-  const size_t smem = LD_KEYS * C * 2 + 16 * (LD_PSTRIDE + 16);
-  TORCH_CHECK(smem <= LDS_MAX, "latent_decode_attn: tile exceeds LDS");
-#define LAUNCH(NCT, NPM)                                                                         \
+  auto smem_of = [&](int ht) { return (size_t)ht * (LD_KEYS * C * 2 + 16 * (LD_PSTRIDE + 16)); };
+  TORCH_CHECK(smem_of(1) <= LDS_MAX, "latent_decode_attn: tile exceeds LDS");
+  // Pairs of head tiles read every key once for 32 heads and load while they work, but take a
+  // whole CU. They win from 64 rows on, where splits are long (one head tile and pairs, prep
+  // and combine included: 64 rows of 16000 keys, 32 heads 350 and 313 us, 128 heads 1312 and
+  // 1076; of 500 keys 45 and 44, 132 and 125), and lose below (32 rows of 2000 keys, 64 heads
+  // 66.8 and 70.3; 1 of 200, 32 heads 15.6 and 18.6), or where their last round leaves more of the
+  // chip idle (96 rows of 8000, 128 heads, 256 latents: 620 and 712; 128 rows: 918 and 741).
+  auto fill = [&](int ht) {
+    const int64_t round = 256 * (LDS_MAX / smem_of(ht));
+    const int64_t n = R * ((H + 16 * ht - 1) / (16 * ht)) * splits;
+    return (double)n / ((n + round - 1) / round * round);
+  };
+  const bool pairs = H > 16 && R >= 64 && smem_of(2) <= LDS_MAX && fill(2) >= fill(1);
+  const size_t smem = smem_of(pairs ? 2 : 1);
+#define LAUNCH(NCT, NPM, HT)                                                                     \
   do {                                                                                           \
     static const hipError_t attr_ = hipFuncSetAttribute(                                         \
-        reinterpret_cast<const void*>(&latent_decode_attn_kernel<NCT, NPM>),                     \
+        reinterpret_cast<const void*>(&latent_decode_attn_kernel<NCT, NPM, HT>),                 \
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_MAX);                               \
     TORCH_CHECK(attr_ == hipSuccess, "latent_decode_attn: LDS attribute");                       \
-    latent_decode_attn_kernel<NCT, NPM>                                                          \
-        <<<dim3(splits, (H + 15) / 16, R), dim3(256), smem, stream>>>(                           \
+    latent_decode_attn_kernel<NCT, NPM, HT>                                                      \
+        <<<dim3(splits, (H + 16 * HT - 1) / (16 * HT), R), dim3(256 * HT), smem, stream>>>(      \
             reinterpret_cast<const bf16*>(q.data_ptr()),                                         \
             reinterpret_cast<const bf16*>(cache.data_ptr()), slot.data_ptr<int>(),               \
             pos.data_ptr<int>(), part_o.data_ptr<float>(), part_ml.data_ptr<float>(),            \
             (int)cache.size(0), (int)cache.size(1), (int)H, (int)RP, (int)C, (float)scale);      \
   } while (0)
   TORCH_CHECK(C / 32 <= 26, "latent_decode_attn: latent and rotated key too wide");
-  if (RP <= 128 && C <= 256) LAUNCH(2, 8);
-  else if (RP <= 256 && C <= 384) LAUNCH(4, 12);
-  else if (C <= 640) LAUNCH(8, 20);
-  else LAUNCH(8, 26);
+  if (RP <= 128 && C <= 256) { if (pairs) LAUNCH(2, 8, 2); else LAUNCH(2, 8, 1); }
+  else if (RP <= 256 && C <= 384) { if (pairs) LAUNCH(4, 12, 2); else LAUNCH(4, 12, 1); }
+  else if (C <= 640) { if (pairs) LAUNCH(8, 20, 2); else LAUNCH(8, 20, 1); }
+  else LAUNCH(8, 26, 1);
 #undef LAUNCH
   HIP_CHECK_KERNEL();
   return {part_o, part_ml};

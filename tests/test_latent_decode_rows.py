@@ -84,3 +84,32 @@ def test_combine(R, S, H, dv, rank):
         bf16_close(hip_ops().latent_decode_combine(part, None, w, dv),
                    torch.stack([part[:, h, 0, :rank].double() @ wd[h].t().contiguous()
                                 for h in range(H)], 1).reshape(R, -1))
+
+
+@pytest.mark.parametrize("R,H", [(63, 17), (64, 16), (64, 17), (65, 40), (64, 32)])
+@pytest.mark.parametrize("rank,rot,splits", [(512, 64, 1), (512, 64, 3), (256, 32, 1), (128, 16, 2), (512, 128, 2)])
+def test_attention_of_many_rows(R, H, rank, rot, splits):
+    """Heads in pairs of tiles, two buffers of keys: from 64 rows and 17 heads on."""
+    from automodel_amd.ops._backend import hip_ops
+
+    torch.manual_seed(0)
+    RP, C, max_len = pad32(rank), pad32(rank) + pad32(rot), 330
+    q = torch.randn(R, H, C, device="cuda").bfloat16()
+    cache = torch.randn(R, max_len, C, device="cuda").bfloat16()
+    pos = torch.randint(0, max_len, (R,), device="cuda", dtype=torch.int32)
+    pos[:5] = torch.tensor([0, 63, 64, 127, max_len - 1])
+    slot = torch.randperm(R, device="cuda").int()
+    slot[7] = -1                                        # no sequence: zeros
+    scale = C ** -0.5
+    part, ml = hip_ops().latent_decode_attn(q, cache, slot, pos, rank, rot, scale, splits)
+    assert (part[7] == 0).all() and (ml[7, ..., 1] == 0).all()
+    m, l = ml.double().unbind(-1)
+    e = (m - m.amax(-1, keepdim=True)).exp()
+    got = (part.double() * e[..., None]).sum(2) / (e * l).sum(-1)[..., None]
+    for r in range(R):
+        if r != 7:
+            keys = cache[slot[r], :pos[r] + 1].double()
+            p = (q[r].double() @ keys.t().contiguous() * scale).softmax(-1)
+            want = p @ keys[:, :RP]
+            # probabilities are rounded to bf16 once
+            assert (got[r] - want).norm() <= 2.0 ** -9 * 1.05 * (p @ keys[:, :RP].abs()).norm()
