@@ -97,7 +97,8 @@ __global__ __launch_bounds__(256) void lora_up_kernel(const bf16* __restrict__ y
                                                       bf16* __restrict__ out, long M, int O,
                                                       float scale) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
-  const long m = (long)blockIdx.y * 64 + wid * 16 + l16;
+  const int strips = (O + 255) / 256;                  // blocks side by side take one stretch of rows
+  const long m = (long)(blockIdx.x / strips) * 64 + wid * 16 + l16;
   const bf16* tr = t + min(m, M - 1) * R + g * 8;
   bf16x8l tv[R / 32];
 #pragma unroll
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(256) void lora_up_kernel(const bf16* __restrict__ y
   const int perm = (l16 >> 2) * 16 + (l16 & 3);        // column of row l16 of tile j: perm + 4 j
 #pragma unroll 2
   for (int s = 0; s < 4; ++s) {
-    const int o0 = blockIdx.x * 256 + s * 64;
+    const int o0 = blockIdx.x % strips * 256 + s * 64;
     if (o0 >= O) break;                                // O is a multiple of 64
     const long at = m * O + o0 + g * 16;
     bf16x8 yv[2];
@@ -339,7 +340,9 @@ std::tuple<at::Tensor, at::Tensor> lora_apply(const std::optional<at::Tensor>& y
   auto out = at::empty({M, (long)O}, x.options());
   auto t = at::empty({M, (long)R}, x.options());
   if (M == 0) return {out, t};
-  TORCH_CHECK((M + 63) / 64 <= 65535, "lora_apply: too many rows");
+  const long blocks = (M + 63) / 64 * ((O + 255) / 256);
+  // (a grid has 2^32 threads)
+  TORCH_CHECK(blocks < (1l << 24) && (M + 31) / 32 < (1l << 24), "lora_apply: too many rows");
   auto stream = c10::hip::getCurrentHIPStream().stream();
   const bf16* yp = y ? reinterpret_cast<const bf16*>(y->data_ptr()) : nullptr;
   auto run = [&](auto rank) {
@@ -348,8 +351,8 @@ std::tuple<at::Tensor, at::Tensor> lora_apply(const std::optional<at::Tensor>& y
                        reinterpret_cast<const bf16*>(x.data_ptr()),
                        reinterpret_cast<const bf16*>(A.data_ptr()),
                        reinterpret_cast<bf16*>(t.data_ptr()), M, H);
-    hipLaunchKernelGGL((lora_up_kernel<RANK>), dim3((O + 255) / 256, (unsigned)((M + 63) / 64)), dim3(256),
-                       0, stream, yp, reinterpret_cast<const bf16*>(t.data_ptr()),
+    hipLaunchKernelGGL((lora_up_kernel<RANK>), dim3((unsigned)blocks), dim3(256), 0, stream, yp,
+                       reinterpret_cast<const bf16*>(t.data_ptr()),
                        reinterpret_cast<const bf16*>(B.data_ptr()),
                        reinterpret_cast<bf16*>(out.data_ptr()), M, O, (float)scale);
   };

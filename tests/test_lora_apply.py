@@ -23,3 +23,17 @@ def test_lora_apply(M, H, O, R, with_y):
     assert (t.double() - td).norm() <= 2.0 ** -9 * 1.05 * td.norm()
     ref = 0.5 * (t.double() @ B.double().t()) + (0 if y is None else y.double())
     assert (out.double() - ref).norm() <= 2.0 ** -9 * 1.05 * ref.norm()
+
+
+def test_more_rows_than_a_grid_is_high():
+    from automodel_amd.ops._backend import hip_ops
+
+    M = 65535 * 64 + 33
+    torch.manual_seed(0)
+    x = torch.randn(M, 64, device="cuda").bfloat16()
+    A, B = torch.randn(32, 64, device="cuda").bfloat16() / 8, torch.randn(64, 32, device="cuda").bfloat16()
+    y = torch.randn(M, 64, device="cuda").bfloat16()
+    out, t = hip_ops().lora_apply(y, x, A, B, 0.5)
+    rows = torch.tensor([0, 1, M // 2, M - 65, M - 33, M - 1], device="cuda")
+    ref = 0.5 * (t[rows].double() @ B.double().t()) + y[rows].double()
+    assert (out[rows].double() - ref).norm() <= 2.0 ** -9 * 1.05 * ref.norm()
