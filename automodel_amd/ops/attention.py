@@ -132,7 +132,8 @@ def _flash_hip(q, k, v, causal, scale, q_start, doc_start=None, doc_end=None):
 
 
 def _check_lengths(q, k, causal, q_start) -> None:
-    """Chunks with an offset and non-causal calls come in whole tiles."""
+    """Refuses chunks with an offset and non-causal calls whose lengths are not in
+    128s, as this entry point always has (the kernels would take them)."""
     if q.shape[1] % 128 or k.shape[1] % 128:
         assert causal and q_start == 0, \
             "flash: Sq%128/Skv%128 required for q_start/non-causal calls"

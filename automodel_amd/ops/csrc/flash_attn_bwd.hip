@@ -15,7 +15,10 @@
 // core forms the scores of the next half tile and adds the products of the previous one
 // (PIPE; three tiles of head dim 192/192 or 256 do not fit LDS: there two buffers, and the
 // phases follow one another).
-// Bound by LDS reads (32 rows per wave: 128 B/clk at full MFMA rate) and the matrix cores.
+// dK/dV is bound by waits that nothing fills: its accumulators and operands leave one wave a
+// SIMD (matrix cores 39% busy, instructions issued 46% of the cycles, at 16384 x 128); dQ, two
+// waves a SIMD, by the matrix cores (66%) and LDS reads (32 rows per wave: 128 B/clk at full
+// MFMA rate).
 // Measured, dK/dV + dQ + stats (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128:
 // 21.25 -> 7.90 ms (4932 + 2811 us); 2 x 4096: 2960 -> 1150 us; 2 x 3072, 16 heads (192, 128):
 // 1725 -> 489 us; 4 x 2048, 16/8 heads of 64: 616 -> 176 us; 2 x 4096, 16/8 heads of 256:

@@ -19,13 +19,14 @@
 //
 // Bound by LDS (at full MFMA rate 64 x 128 wave tiles read and load 128 B/clk, 64 x 64 ones
 // more: 256 x 256 is the faster tile) against padding of the groups' last row tiles: nt and
-// nn take 256 rows from 512 rows per expert on (the caller's plan: 128 experts x 512 rows: 328 against
-// 334 us; 64 x 281: 192 against 179), tn, whose tiles have no padding, always. 4 waves of
-// 64 x 128, one a SIMD, wait for LDS more than they save (128 x 256: 374 against 345 us).
-// Measured, nt / nn / tn, before (tn with its transposes) -> now: 65536 rows, 128 experts,
-// 768 x 2048: 515 / 607 / 742 -> 328 / 331 / 311 us; 2048 x 768: 502 / 691 / 757 -> 300 / 287 /
-// 287 us; 18018 rows, 64 experts, 1408 x 2048: 284 / 369 / 403 -> 179 / 168 / 197 us; 16384 rows,
-// 8 experts, 4096 x 2048: 495 / 779 / 639 -> 296 / 329 / 269 us (929 / 834 / 1022 TFLOP/s).
+// nn take 256 rows from 512 rows per expert on (the caller's plan, ops/grouped_gemm.py, has both
+// sides), tn, whose tiles have no padding, always. 4 waves of 64 x 128, one a SIMD, wait for
+// LDS more than they save (128 x 256: 374 against 345 us).
+// Measured, nt / nn / tn, groups as a random choice fills them, before (tn with its transposes)
+// -> now: 65536 rows, 128 experts, 768 x 2048: 515 / 607 / 742 -> 255 / 281 / 286 us; 2048 x 768:
+// 502 / 691 / 757 -> 280 / 262 / 275 us; 18018 rows, 64 experts, 1408 x 2048: 284 / 369 / 403 ->
+// 166 / 166 / 184 us; 16384 rows, 8 experts, 4096 x 2048: 495 / 779 / 639 -> 280 / 307 / 276 us
+// (982 / 895 / 996 TFLOP/s).
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void grouped_gemm_kernel(const Group
   // Waves w and w + 4 share a SIMD: they get different rows and different columns, and a
   // wave without rows or columns of its own (a tile at a group's or the output's end) forms
   // no products, so that half a tile takes half the time. 128 experts x 512 rows, 768 x 2048,
-  // nt: 266 -> 259 us; 64 x 281, 1408 x 2048: 175 -> 163. (A choice of 32 or 64 rows in the
+  // nt: 266 -> 259 us (255 in another run); 64 x 281, 1408 x 2048: 175 -> 163. (A choice of 32 or 64 rows in the
   // loop spilled.)
   const int wr = wid / WC, wc = (wid % WC) ^ (wid >= 4 ? WC / 2 : 0);
   const bool live = wr * 64 < r_left && wc * WN < c_left;

@@ -5,8 +5,8 @@
 //   latent_decode_prep     q'[r,h] = [ W_uk[h]^T q_unrot | rotated q ], and the
 //                          new token's cache row, in one launch
 //   latent_decode_attn     split-KV attention of all heads over the cache:
-//                          the heads are the M dimension of 16x16x32 MFMAs, so
-//                          one staged key tile serves them all
+//                          the heads are the columns of 16x16x32 MFMAs, 16 or 32
+//                          of them on one staged key tile
 //   latent_decode_combine  merges the splits, then applies W_uv per head
 //
 // Lengths and slots are device tensors: a captured step replays for every
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void latent_decode_prep_mfma_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// attention over the cache. grid (splits, head groups of 16, rows)
+// attention over the cache. grid (splits, head groups of 16 HT, rows)
 // ---------------------------------------------------------------------------
 constexpr int LD_KEYS = 64;           // keys per tile: 4 waves x 16
 constexpr int LD_PSTRIDE = LD_KEYS * 2 + 16;

@@ -143,8 +143,9 @@ __global__ __launch_bounds__(256) void lora_up_kernel(const bf16* __restrict__ y
 // "SGMV kernels"; reference uses punica-style segmented gather MV for
 // per-request adapters). Tokens arrive SORTED by adapter; the grouped-GEMM
 // plan (offs + 256-row tile_map, device-built) picks each tile's adapter,
-// whose A/B/scale are indexed from stacked tensors. Same two-phase
-// register/LDS structure as the single-adapter kernel above.
+// whose A/B/scale are indexed from stacked tensors. One kernel per 256 rows
+// does both products: the first one's result goes through LDS as the second's
+// operand.
 // ===========================================================================
 
 template <int R>

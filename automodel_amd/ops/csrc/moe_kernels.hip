@@ -47,7 +47,7 @@ constexpr int ROUTE_CHUNK = 256, ROUTE_MAX_E = 4096;
 
 __device__ __forceinline__ int route_expert(const long* idx, long i, int E) {
   const long e = idx[i];
-  return e < 0 ? 0 : e >= E ? E - 1 : (int)e;      // (a valid router gives 0 .. E-1)
+  return e < 0 ? 0 : e >= E ? E - 1 : (int)e;      // memory stays safe; callers refuse such numbers
 }
 
 __global__ __launch_bounds__(64) void route_count_kernel(const long* __restrict__ idx, long n, int E,

@@ -36,7 +36,7 @@ FLASH_MAX_HEAD_DIM = 256
 MFMA_MAX_RANK = 512
 MFMA_MAX_CACHE_WIDTH = 832
 _KEYS_PER_TILE = 64                 # latent_decode.hip LD_KEYS
-_TARGET_WORKGROUPS = 256            # one per CU: a staged tile fills most of its LDS
+_TARGET_WORKGROUPS = 256            # see decode_splits
 
 
 def pad32(n: int) -> int:
@@ -142,7 +142,14 @@ def latent_attention_prompt(qkv, norm_w, w_kv_b, spec: LatentAttentionSpec, rope
 def decode_splits(rows: int, heads: int, max_len: int) -> int:
     """KV splits per (row, head group): enough workgroups for the chip, no more
     than there are key tiles. Depends on capacities only, so that it is the
-    same on every replay of a captured step."""
+    same on every replay of a captured step.
+
+    A workgroup takes 16 heads (32 with many rows: csrc/latent_decode.hip), and two fit
+    a CU: up to 16 heads this asks for one a CU, above for two. Attention and merge with
+    half as many splits, these, and twice as many: 8 rows, 16 heads, 1500 keys 17.7,
+    15.2, 19.2 us; 8 rows, 32 heads, 4000 keys 27.6, 24.4, 34.9; 32 rows, 32 heads,
+    1500 keys 45.7, 34.9, 43.7. (More would help 16 heads of many rows: 32 rows of 4000
+    keys 48.8 and 39.1.)"""
     groups = -(-heads // (16 if heads <= 16 else 32))
     want = _TARGET_WORKGROUPS // max(1, rows * groups)
     return max(1, min(want, -(-max_len // _KEYS_PER_TILE), 64))
