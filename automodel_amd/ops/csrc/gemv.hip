@@ -5,7 +5,9 @@
 // wave takes a row of W and its lanes run along K; above that the matrix cores
 // take 16 rows of W against 16 rows of x per instruction, since a dot product
 // per row of x would cost more than the load (4 rows, 14336 x 4096: 27 us against
-// 21 us). Weight loads leave no trace in the caches (nontemporal).
+// 21 us). Weight loads leave no trace in the caches (nontemporal): a model's weights are gone
+// from them before its next step (5 rows, 2048 x 2048: 4.7 us, 5.0 through the caches). Weights of
+// a model that the last-level cache could hold pay for it (16 rows, 1024 x 4096: 7.7 and 6.2).
 //
 // One launch can take several weights of the same input (q, k and v; gate and
 // up), each with an output of its own, and can return silu(gate) * up instead of
@@ -60,27 +62,40 @@ __device__ __forceinline__ bf16x8 load_stream(const bf16* p) {
 
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.f + __expf(-g)) * u; }
 
-__device__ __forceinline__ int segment_of(const Rows& p, int block) {
-  return (block >= p.first[1]) + (block >= p.first[2]);
+// The segment of a block, by selection: an index into the arguments would be one more load
+// in the chain that every launch begins with.
+struct Segment {
+  const bf16* w;
+  bf16* y;
+  int n, first;
+};
+__device__ __forceinline__ Segment segment_of(const Rows& p, int block) {
+  const bool b1 = block >= p.first[1], b2 = block >= p.first[2];
+  return {b2 ? p.w[2] : b1 ? p.w[1] : p.w[0], b2 ? p.y[2] : b1 ? p.y[1] : p.y[0],
+          b2 ? p.n[2] : b1 ? p.n[1] : p.n[0], b2 ? p.first[2] : b1 ? p.first[1] : 0};
 }
 
 // A wave takes R rows of W, or with GLU one row of gate and the same of up, and
 // has 512 U columns of each in flight. One row and U = 8 reach the highest rate
 // for one row of x: 14336 x 4096 in 18.6 us (6.3 TB/s) against 23.1 with two rows
-// and U = 2, and 24.2 with two rows and U = 1.
+// and U = 2, and 24.2 with two rows and U = 1; short rows end before 8 are in flight.
+// With two rows of x the loads of x count: two rows of W share them from some 48 MB of
+// W on (10240 x 8192 29.5 us, one row 34.2; 5120 x 13824 24.5 and 30.3), below the
+// waves of one row, twice as many, win (4096 x 4096 9.5 and 8.2, 2048 x 9216 14.0 and 10.4).
 template <int B, int R, int U, bool GLU>
 __global__ __launch_bounds__(256) void gemv_bf16_kernel(const Rows p) {
   static_assert(!GLU || R == 2);
   constexpr int STEP = GLU ? 1 : R;               // rows of output per wave
-  const int seg = segment_of(p, blockIdx.x), K = p.K, N = p.n[seg];
+  const Segment seg = segment_of(p, blockIdx.x);
+  const int K = p.K, N = seg.n;
   const int lane = threadIdx.x & (WAVE_SIZE - 1);
-  const int row0 = ((blockIdx.x - p.first[seg]) * 4 + threadIdx.x / WAVE_SIZE) * STEP;
+  const int row0 = ((blockIdx.x - seg.first) * 4 + threadIdx.x / WAVE_SIZE) * STEP;
   if (row0 >= N) return;
   float acc[R][B];
   const bf16* w[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    w[r] = GLU ? p.w[r] + (long)row0 * K : p.w[seg] + (long)min(row0 + r, N - 1) * K;
+    w[r] = GLU ? p.w[r] + (long)row0 * K : seg.w + (long)min(row0 + r, N - 1) * K;
 #pragma unroll
     for (int b = 0; b < B; ++b) acc[r][b] = 0.f;
   }
@@ -135,22 +150,23 @@ __global__ __launch_bounds__(256) void gemv_bf16_kernel(const Rows p) {
         }
         if (p.res) t[r] += bf2f(p.res[(long)b * N + row0 + r]);
         if (p.yf) p.yf[(long)b * N + row0 + r] = t[r];
-        else p.y[seg][(long)b * N + row0 + r] = f2bf(t[r]);
+        else seg.y[(long)b * N + row0 + r] = f2bf(t[r]);
       }
     }
   }
 }
 
 // A workgroup takes 16 RT rows of W (GLU: 16 of gate and the same 16 of up) and
-// 16 NB rows of x; its waves take every WAVES-th tile of K and add up through LDS
-// at the end, so that N = 1024 fills the chip too. Matrix fragments want one row
-// per lane, memory wants consecutive lanes on consecutive bytes: each wave moves
-// its tiles of W and x with coalesced loads into LDS of its own, with the next
-// DEPTH tiles' loads in flight. No workgroup barrier in the loop.
+// 16 NB rows of x; its waves take a stretch of K each and add up through LDS at the
+// end, so that N = 1024 fills the chip too. (Every WAVES-th tile of K instead: 5 rows,
+// 4096 x 4096 8.7 us against 7.7, 8192 x 8192 26.7 against 23.0.) Matrix fragments
+// want one row per lane, memory wants consecutive lanes on consecutive bytes: each
+// wave moves its tiles of W and x with coalesced loads into LDS of its own, with the
+// next tile's loads in flight (two ahead: the same). No workgroup barrier in the loop.
 constexpr int SK_KC = 128;                        // K per tile
 constexpr int SK_STRIDE = SK_KC * 2 + 16;         // LDS bytes per row
 
-template <int NB, int WAVES, int RT, int DEPTH, bool GLU>
+template <int NB, int WAVES, int RT, bool GLU>
 __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(const Rows p, int B) {
   static_assert(!GLU || RT == 2);
   constexpr int OUT = GLU ? 16 : 16 * RT;         // rows of output per workgroup
@@ -160,8 +176,9 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(const Ro
   __shared__ __attribute__((aligned(16))) char lds[WAVES * TILE > RED ? WAVES * TILE : RED];
   const int lane = threadIdx.x & (WAVE_SIZE - 1), wid = threadIdx.x / WAVE_SIZE;
   const int lo16 = lane & 15, hi4 = lane >> 4;
-  const int seg = segment_of(p, blockIdx.x), K = p.K, N = p.n[seg];
-  const int n0 = (blockIdx.x - p.first[seg]) * OUT;
+  const Segment seg = segment_of(p, blockIdx.x);
+  const int K = p.K, N = seg.n;
+  const int n0 = (blockIdx.x - seg.first) * OUT;
   const bf16* x = p.x;
   if (p.group_n) x += (long)(n0 / p.group_n) * B * K;   // group_n % OUT == 0
   char* wl = lds + wid * TILE;                    // [16 RT][SK_STRIDE]
@@ -172,59 +189,54 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(const Ro
   for (int r = 0; r < RT; ++r)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[r][b] = gemv_f32x4{0.f, 0.f, 0.f, 0.f};
-  const int tiles = (K + SK_KC - 1) / SK_KC;
+  const int tiles = (K + SK_KC - 1) / SK_KC, per = (tiles + WAVES - 1) / WAVES;
+  const int t_lo = wid * per, t_hi = min(t_lo + per, tiles);
 
   // load j covers rows 4j + hi4, 16 bytes per lane at column 8 lo16
-  bf16x8 wr[DEPTH][4 * RT], xr[DEPTH][4 * NB];
-  auto fetch = [&](int t, int d) {
+  bf16x8 wr[4 * RT], xr[4 * NB];
+  auto fetch = [&](int t) {
     const int k = t * SK_KC + lo16 * 8;
     const bool in = k < K;                        // K % 8 == 0: all 8 or none
 #pragma unroll
     for (int j = 0; j < 4 * RT; ++j) {
-      wr[d][j] = bf16x8{};
-      const bf16* w = GLU ? p.w[j / 4] : p.w[seg];
+      wr[j] = bf16x8{};
+      const bf16* w = GLU ? p.w[j / 4] : seg.w;
       const int row = n0 + 4 * (GLU ? j % 4 : j) + hi4;
-      if (in) wr[d][j] = load_stream(w + (long)min(row, N - 1) * K + k);
+      if (in) wr[j] = load_stream(w + (long)min(row, N - 1) * K + k);
     }
 #pragma unroll
     for (int j = 0; j < 4 * NB; ++j) {
-      xr[d][j] = bf16x8{};
+      xr[j] = bf16x8{};
       if (in)
-        xr[d][j] = *reinterpret_cast<const bf16x8*>(x + (long)min(4 * j + hi4, B - 1) * K + k);
+        xr[j] = *reinterpret_cast<const bf16x8*>(x + (long)min(4 * j + hi4, B - 1) * K + k);
     }
   };
+  if (t_lo < t_hi) fetch(t_lo);
+  for (int t = t_lo; t < t_hi; ++t) {
 #pragma unroll
-  for (int d = 0; d < DEPTH; ++d) fetch(wid + d * WAVES, d);
-  for (int t0 = wid; t0 < tiles; t0 += WAVES * DEPTH) {
+    for (int j = 0; j < 4 * RT; ++j)
+      *reinterpret_cast<bf16x8*>(wl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = wr[j];
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      const int t = t0 + d * WAVES;
-      if (t >= tiles) break;
+    for (int j = 0; j < 4 * NB; ++j)
+      *reinterpret_cast<bf16x8*>(xl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = xr[j];
+    __builtin_amdgcn_wave_barrier();
+    if (t + 1 < t_hi) fetch(t + 1);
 #pragma unroll
-      for (int j = 0; j < 4 * RT; ++j)
-        *reinterpret_cast<bf16x8*>(wl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = wr[d][j];
+    for (int kk = 0; kk < SK_KC / 32; ++kk) {
+      const int off = lo16 * SK_STRIDE + kk * 64 + hi4 * 16;
+      gemv_bf16x8 xv[NB];
 #pragma unroll
-      for (int j = 0; j < 4 * NB; ++j)
-        *reinterpret_cast<bf16x8*>(xl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = xr[d][j];
-      __builtin_amdgcn_wave_barrier();
-      fetch(t + WAVES * DEPTH, d);
+      for (int b = 0; b < NB; ++b)
+        xv[b] = *reinterpret_cast<const gemv_bf16x8*>(xl + b * 16 * SK_STRIDE + off);
 #pragma unroll
-      for (int kk = 0; kk < SK_KC / 32; ++kk) {
-        const int off = lo16 * SK_STRIDE + kk * 64 + hi4 * 16;
-        gemv_bf16x8 xv[NB];
+      for (int r = 0; r < RT; ++r) {
+        const gemv_bf16x8 wv = *reinterpret_cast<const gemv_bf16x8*>(wl + r * 16 * SK_STRIDE + off);
 #pragma unroll
         for (int b = 0; b < NB; ++b)
-          xv[b] = *reinterpret_cast<const gemv_bf16x8*>(xl + b * 16 * SK_STRIDE + off);
-#pragma unroll
-        for (int r = 0; r < RT; ++r) {
-          const gemv_bf16x8 wv = *reinterpret_cast<const gemv_bf16x8*>(wl + r * 16 * SK_STRIDE + off);
-#pragma unroll
-          for (int b = 0; b < NB; ++b)
-            acc[r][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, xv[b], acc[r][b], 0, 0, 0);
-        }
+          acc[r][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, xv[b], acc[r][b], 0, 0, 0);
       }
-      __builtin_amdgcn_wave_barrier();            // the tile is overwritten next
     }
+    __builtin_amdgcn_wave_barrier();              // the tile is overwritten next
   }
   __syncthreads();                                // tiles become the reduction buffer
   float* red = reinterpret_cast<float*>(lds);
@@ -254,7 +266,7 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(const Ro
     }
     if (p.res) t += bf2f(p.res[o]);
     if (p.yf) p.yf[o] = t;
-    else p.y[seg][o] = f2bf(t);
+    else seg.y[o] = f2bf(t);
   }
 }
 
@@ -279,35 +291,78 @@ void launch_gemv(Rows p, int segments) {
       <<<dim3(blocks), dim3(256), 0, c10::hip::getCurrentHIPStream()>>>(p);
 }
 
-template <int NB, int WAVES, int RT, int DEPTH, bool GLU = false>
-void launch_skinny(Rows p, int segments, int B) {
+// one or two rows of x
+void gemv_rows(const Rows& p, int segments, int B) {
+  long rows = 0;
+  for (int s = 0; s < segments; ++s) rows += p.n[s];
+  if (B == 1 && p.K > 2048) launch_gemv<1, 1, 8>(p, segments);
+  else if (B == 1) launch_gemv<1, 1, 4>(p, segments);
+  else if (rows * p.K >= (24l << 20)) launch_gemv<2, 2, 1>(p, segments);
+  else launch_gemv<2, 1, 4>(p, segments);
+}
+
+template <int NB, int WAVES, int RT, bool GLU = false>
+void launch_skinny(const Rows& rows, int segments, int B) {
+  Rows p = rows;
   const int blocks = place(p, segments, GLU ? 16 : 16 * RT);
-  gemm_skinny_kernel<NB, WAVES, RT, DEPTH, GLU>
+  gemm_skinny_kernel<NB, WAVES, RT, GLU>
       <<<dim3(blocks), dim3(WAVES * WAVE_SIZE), 0, c10::hip::getCurrentHIPStream()>>>(p, B);
 }
 
-// Up to 16 rows the loads in flight decide: 8 waves, and 2 tiles ahead, for a K
-// that has that many (8 rows, 14336 x 4096: 21.4 us, 23.0 with 1 tile ahead and W
-// through the caches; K < 2048 keeps 4 waves). Above that the x rows of each
-// workgroup weigh as much as its rows of W: 64 rows of W per workgroup once that
-// still leaves 128 workgroups (32 rows, 14336 x 4096: 28.1 us, 16 rows each 34.9;
-// at 4096 x 4096 22.2 against 11.4). A gated pair has 32 rows of W anyway.
+// Workgroups of 16, 32 or 64 rows of W, and 2, 4 or 8 waves in them. What decides is how many
+// tiles of 16 rows the fullest CU gets, with the rows of x that each workgroup loads besides;
+// a workgroup alone on its CU needs all the waves that fit, several share them. Small K has
+// tiles for few waves. Times in us for rows x columns of W, weights from memory:
+//  * up to 16 rows of x: 16 rows of W, 8 waves (4096 x 4096 7.7, 4 waves 9.1; 10240 x 8192 29.6
+//    and 34.7), 4 with more workgroups than two a CU and short rows (9216 x 2048 9.2, 8 waves 9.9);
+//    32 rows between one and one and a half workgroups a CU (5120 x 5120 12.4, 16 rows 13.5; but
+//    8192 x 8192 24.5 and 23.0), and for many rows of x and of W (16 rows, 32000 x 2048 22.8 and 24.8).
+//  * up to 32: 32 rows of W where that gives the fullest CU no more (24 rows, 8192 x 8192 26.6 and
+//    31.5; 21504 x 4096 36.2 and 40.7), else 16 (9216 x 2048 12.5, 32 rows 14.1).
+//  * up to 64: the least sum of tiles and 2/5 (long rows: 3/5) of one a workgroup, out of 16, 32 and
+//    64 rows (48 rows, 9216 x 2048 17.8, 32 rows 19.4; 8192 x 8192 40.6, 16 rows 50.1; 10240 x 8192
+//    55.4, 16 rows 61.0; 32000 x 2048 35.2, 32 rows 41.5).
 void skinny(const Rows& p, int segments, int B, bool glu) {
-  int rows = 0;
-  for (int s = 0; s < segments; ++s) rows += p.n[s];
-  const bool wide = rows >= 8192 && p.group_n % 64 == 0;
+  if (glu) {
+    if (B <= 16) launch_skinny<1, 4, 2, true>(p, segments, B);
+    else if (B <= 32) launch_skinny<2, 4, 2, true>(p, segments, B);
+    else launch_skinny<4, 2, 2, true>(p, segments, B);
+    return;
+  }
+  constexpr int CUS = 256;
+  auto workgroups = [&](int rt) {
+    int n = 0;
+    for (int s = 0; s < segments; ++s) n += (p.n[s] + 16 * rt - 1) / (16 * rt);
+    return n;
+  };
+  auto fullest = [&](int rt) { return (workgroups(rt) + CUS - 1) / CUS; };
+  auto may = [&](int rt) { return p.group_n % (16 * rt) == 0; };
+  const int n1 = workgroups(1);
   if (B <= 16) {
-    if (glu) launch_skinny<1, 4, 2, 1, true>(p, segments, B);
-    else if (p.K >= 2048) launch_skinny<1, 8, 1, 2>(p, segments, B);
-    else launch_skinny<1, 4, 1, 1>(p, segments, B);
+    const bool pairs = may(2) && ((n1 > CUS && n1 <= CUS * 3 / 2) || (B > 8 && n1 >= CUS * 7 / 2));
+    const bool few = p.K <= 512 || (n1 > 2 * CUS && p.K <= 2048);
+    if (pairs && n1 > 2 * CUS) launch_skinny<1, 4, 2>(p, segments, B);
+    else if (pairs) launch_skinny<1, 8, 2>(p, segments, B);
+    else if (few) launch_skinny<1, 4, 1>(p, segments, B);
+    else launch_skinny<1, 8, 1>(p, segments, B);
   } else if (B <= 32) {
-    if (glu) launch_skinny<2, 4, 2, 1, true>(p, segments, B);
-    else if (wide) launch_skinny<2, 4, 4, 1>(p, segments, B);
-    else launch_skinny<2, 8, 1, 1>(p, segments, B);
+    const bool pairs = may(2) && 2 * fullest(2) <= fullest(1);
+    if (pairs && fullest(2) > 1) launch_skinny<2, 4, 2>(p, segments, B);
+    else if (pairs) launch_skinny<2, 8, 2>(p, segments, B);
+    else if (n1 > CUS || p.K <= 512) launch_skinny<2, 4, 1>(p, segments, B);
+    else launch_skinny<2, 8, 1>(p, segments, B);
   } else {
-    if (glu) launch_skinny<4, 2, 2, 1, true>(p, segments, B);
-    else if (wide) launch_skinny<4, 4, 4, 1>(p, segments, B);
-    else launch_skinny<4, 4, 1, 1>(p, segments, B);
+    const int x = p.K > 4096 ? 3 : 2;              // fifths of a tile
+    int best = 1;
+    for (int rt : {2, 4})
+      if (may(rt) && fullest(rt) * (5 * rt + x) < fullest(best) * (5 * best + x)) best = rt;
+    const bool alone = fullest(best) == 1;
+    if (best == 4 && alone) launch_skinny<4, 4, 4>(p, segments, B);
+    else if (best == 4) launch_skinny<4, 2, 4>(p, segments, B);
+    else if (best == 2 && alone) launch_skinny<4, 4, 2>(p, segments, B);
+    else if (best == 2) launch_skinny<4, 2, 2>(p, segments, B);
+    else if (alone) launch_skinny<4, 4, 1>(p, segments, B);
+    else launch_skinny<4, 2, 1>(p, segments, B);
   }
 }
 
@@ -356,8 +411,8 @@ at::Tensor gemv_bf16(const at::Tensor& x, const at::Tensor& w,
     p.bias = data(bc);
   }
   switch (B) {
-    case 1: launch_gemv<1, 1, 8>(p, 1); break;
-    case 2: launch_gemv<2, 1, 4>(p, 1); break;
+    case 1:
+    case 2: gemv_rows(p, 1, B); break;
     case 3: launch_gemv<3, 2, 1>(p, 1); break;
     case 4: launch_gemv<4, 2, 1>(p, 1); break;
     case 8: launch_gemv<8, 2, 1>(p, 1); break;
@@ -418,9 +473,8 @@ std::vector<at::Tensor> decode_rows(const at::Tensor& x, at::TensorList ws, bool
   }
   if (B > 2) skinny(p, segments, (int)B, glu);
   else if (B == 1 && glu) launch_gemv<1, 2, 4, true>(p, 1);
-  else if (B == 1) launch_gemv<1, 1, 8>(p, segments);
-  else if (glu) launch_gemv<2, 2, 4, true>(p, 1);
-  else launch_gemv<2, 1, 4>(p, segments);
+  else if (glu && B == 2) launch_gemv<2, 2, 4, true>(p, 1);
+  else gemv_rows(p, segments, (int)B);
   HIP_CHECK_KERNEL();
   return out;
 }

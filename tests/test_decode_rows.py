@@ -38,6 +38,19 @@ def test_several_weights(B, K, ns, glu):
         check(y, ref)
 
 
+# every split of the rows of W: 16, 32 and 64 a workgroup, alone on a CU or not, the last ones partly empty
+@pytest.mark.parametrize("N", [4090, 5110, 6150, 9210, 10250, 15370, 21510, 32010])
+@pytest.mark.parametrize("B,K", [(1, 2056), (2, 2056), (2, 5000), (8, 264), (8, 520), (16, 2056), (32, 520), (32, 264),
+                                 (64, 520), (33, 4104)])
+def test_every_split_of_the_rows(N, B, K):
+    from automodel_amd.ops._backend import hip_ops
+
+    torch.manual_seed(0)
+    x = torch.randn(B, K, device="cuda").bfloat16()
+    w = torch.randn(N, K, device="cuda").bfloat16() * K ** -0.5
+    check(hip_ops().decode_rows(x, [w])[0], x.double() @ w.double().t())
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 20, 40])
 @pytest.mark.parametrize("K,sizes", [(512, [64, 64, 64]), (2056, [48, 48, 16]), (264, [4096, 4096, 64])])
 def test_groups_and_epilogues(T, K, sizes):
