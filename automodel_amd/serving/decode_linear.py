@@ -131,11 +131,10 @@ def decode_rows(lins: list[nn.Module], x: torch.Tensor,
     ``[silu(a) * b]`` of the two outputs a and b, or of the halves of one layer's.
     None where the kernels don't apply, and nothing is done.
 
-    Up to 32 rows. Alone, the library is faster on wide layers from 17 rows on (32 rows,
-    14336 x 4096: 26 us against 29, 8192 x 8192 31 against 42; 48 rows of the former 26
-    against 35) and slower on narrow ones (32 rows, 1024 x 4096: 12 against 9, 2048 x 2048
-    11 against 6); one launch for several layers with their activation and sum makes up for
-    the difference up to 32."""
+    Up to 32 rows: with them the library is as fast on wide layers and slower on narrow
+    ones (32 rows, 14336 x 4096 26.0 us against 26.4, 8192 x 8192 30.8 and 28.4, 1024 x
+    4096 11.8 and 9.3; only 10240 x 8192 stands out, 38 and 48), with more it is faster on
+    most (48 rows, 14336 x 4096 28.3 and 36.2, 4096 x 4096 13.7 and 16.6)."""
     K = x.shape[-1]
     rows = x.numel() // max(K, 1)
     if not (x.is_cuda and x.dtype == torch.bfloat16 and 1 <= rows <= 32 and K % 8 == 0
