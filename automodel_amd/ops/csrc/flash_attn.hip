@@ -15,7 +15,7 @@
 // accumulators leave too few registers: it spilled and ran at 100 TFLOP/s.
 // Measured (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128: 6.52 -> 2.19 ms,
 // 1006 TFLOP/s; 2 x 4096: 1030 -> 289 us; 2 x 3072, 16 heads (192, 128): 414 -> 120 us;
-// 4 x 2048, 16/8 heads of 64: 154 -> 55 us.
+// 4 x 2048, 16/8 heads of 64: 154 -> 55 us; 2 x 4096, 8 heads of 256: 544 -> 207 us.
 //
 // Varlen: per-token doc_start gates the causal mask to the query's own document; tiles
 // before a block's first document are skipped.
@@ -117,9 +117,7 @@ struct Fwd {
   }
 };
 
-// PIPE: as above. Without (head dim 256, whose accumulators leave no room for a second
-// half tile in flight) scores, softmax and values follow one another.
-template <int DQK, int DV, int WAVES, int OCC, bool PIPE, bool VARLEN>
+template <int DQK, int DV, int WAVES, int OCC, bool VARLEN>
 __global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArgs a) {
   using F = Fwd<DQK, DV, WAVES, VARLEN>;
   constexpr int KT = F::KT, VT = F::VT;
@@ -189,91 +187,68 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void flash_fwd_kernel(const FwdArg
 
   if (t0 < t1) {
     load_k(t0);
-    if constexpr (PIPE) {
-      wait_loads();
-      barrier();
-      if (t0 + 1 < t1) load_k(t0 + 1);
-    }
+    wait_loads();
+    barrier();
+    if (t0 + 1 < t1) load_k(t0 + 1);
     load_v(t0);
   }
-  if constexpr (PIPE) {
-    // A tile that every row of the wave sees whole, with neighbours on both sides: the hot
-    // loop, without a branch but the rescaling. At two waves a SIMD instructions are issued
-    // nearly all the time, so that each one less counts: one loop with all of a tile's cases
-    // kept the output in two sets of registers and moved it between them, and buffers
-    // known when this is compiled are offsets in the reads (29 us of the next figure). 16384, 32/8
-    // heads of 128: 2499 -> 2187 us; 2 x 3072, 16 heads of (192, 128): 168 -> 120.
-    auto steady = [&](int t, auto parity) {
-      constexpr int PARITY = decltype(parity)::value;      // of t; -1: any
-      const unsigned odd = PARITY < 0 ? t % 2 : PARITY, kt = odd * KT, kn = KT - kt;
-      const unsigned vt = 2 * KT + odd * VT, vo = 4 * KT + VT - vt;
-      f.template softmax<false>(s0, t * 64, p0, [&] { f.scores(s1, kt, 1); f.values(p1, vo, 1); });
-      wait_loads();       // K of t + 1, V of t; the buffers of K of t, V of t - 1 are free
-      barrier();
-      load_v(t + 1);
-      load_k(t + 2);
-      f.template softmax<false>(s1, t * 64 + 32, p1, [&] { f.scores(s0, kn, 0); f.values(p0, vt, 0); });
-    };
-    auto general = [&](int t) {
-      const bool live = t >= t0w && t < t1w;
-      const unsigned kt = (t & 1) * KT, kn = KT - kt;
-      const unsigned vt = 2 * KT + (t & 1) * VT, vo = 4 * KT + VT - vt;
-      if (live) {
-        if (t == t0w) f.scores(s0, kt, 0);
-        f.template softmax<true>(s0, t * 64, p0, [&] {
-          f.scores(s1, kt, 1);
-          if (t != t0w) f.values(p1, vo, 1);
-        });
-      }
-      wait_loads();
-      barrier();
-      if (t + 1 < t1) load_v(t + 1);
-      if (t + 2 < t1) load_k(t + 2);
-      if (live) {
-        // (the scores of the tile after a wave's last one are formed and not used)
-        f.template softmax<true>(s1, t * 64 + 32, p1, [&] { f.scores(s0, kn, 0); f.values(p0, vt, 0); });
-        if (t == t1w - 1) f.values(p1, vt, 1);
-      }
-    };
-    // Tiles of the steady kind: [first, end). There is a tile t + 2 for each of them to load:
-    // the buffer of t + 1, which a step reads, has no load in flight.
-    const int first = max(t0w + 1, VARLEN ? (doc_w + 63) / 64 : 0);
-    const int end = min(min(t_diag, a.Skv / 64), min(t1w - 1, t1 - 2));
-    int t = t0;
-    for (; t < min(first, t1) || (!VARLEN && t < end && t % 2); ++t) general(t);
-    // (pairs leave a tile over at either end; the runs of short documents are too short)
-    if constexpr (VARLEN)
-      for (; t < end; ++t) steady(t, std::integral_constant<int, -1>{});
-    else
-      for (; t + 1 < end; t += 2) {
-        steady(t, std::integral_constant<int, 0>{});
-        steady(t + 1, std::integral_constant<int, 1>{});
-      }
-    for (; t < t1; ++t) general(t);
-  } else {
-    for (int t = t0; t < t1; ++t) {
-      const bool live = t >= t0w && t < t1w;
-      const unsigned kt = (t & 1) * KT, vt = 2 * KT + (t & 1) * VT;
-      const bool mask = t >= t_diag || t * 64 + 64 > a.Skv || (VARLEN && t * 64 < doc_w);
-      wait_loads();     // K and V of t; the other buffers are free
-      barrier();
-      if (t + 1 < t1) {
-        load_k(t + 1);
-        load_v(t + 1);
-      }
-      if (live) {
-#pragma unroll 1
-        for (int sub = 0; sub < 2; ++sub) {
-          f.scores(s0, kt, sub);
-          __builtin_amdgcn_sched_barrier(0);
-          if (mask) f.template softmax<true>(s0, t * 64 + 32 * sub, p0, [] {});
-          else f.template softmax<false>(s0, t * 64 + 32 * sub, p0, [] {});
-          __builtin_amdgcn_sched_barrier(0);
-          f.values(p0, vt, sub);
-        }
-      }
+  // A tile that every row of the wave sees whole, with neighbours on both sides: the hot
+  // loop, without a branch but the rescaling. At two waves a SIMD instructions are issued
+  // nearly all the time, so that each one less counts: one loop with all of a tile's cases
+  // kept the output in two sets of registers and moved it between them, and buffers
+  // known when this is compiled are offsets in the reads (29 us of the next figure). 16384, 32/8
+  // heads of 128: 2499 -> 2187 us; 2 x 3072, 16 heads of (192, 128): 168 -> 120.
+  auto steady = [&](int t, auto parity) {
+    constexpr int PARITY = decltype(parity)::value;      // of t; -1: any
+    const unsigned odd = PARITY < 0 ? t % 2 : PARITY, kt = odd * KT, kn = KT - kt;
+    const unsigned vt = 2 * KT + odd * VT, vo = 4 * KT + VT - vt;
+    f.template softmax<false>(s0, t * 64, p0, [&] { f.scores(s1, kt, 1); f.values(p1, vo, 1); });
+    wait_loads();       // K of t + 1, V of t; the buffers of K of t, V of t - 1 are free
+    barrier();
+    load_v(t + 1);
+    load_k(t + 2);
+    f.template softmax<false>(s1, t * 64 + 32, p1, [&] { f.scores(s0, kn, 0); f.values(p0, vt, 0); });
+  };
+  auto general = [&](int t) {
+    const bool live = t >= t0w && t < t1w;
+    const unsigned kt = (t & 1) * KT, kn = KT - kt;
+    const unsigned vt = 2 * KT + (t & 1) * VT, vo = 4 * KT + VT - vt;
+    if (live) {
+      if (t == t0w) f.scores(s0, kt, 0);
+      f.template softmax<true>(s0, t * 64, p0, [&] {
+        f.scores(s1, kt, 1);
+        if (t != t0w) f.values(p1, vo, 1);
+      });
     }
-  }
+    wait_loads();
+    barrier();
+    if (t + 1 < t1) load_v(t + 1);
+    if (t + 2 < t1) load_k(t + 2);
+    if (live) {
+      // (the scores of the tile after a wave's last one are formed and not used)
+      f.template softmax<true>(s1, t * 64 + 32, p1, [&] { f.scores(s0, kn, 0); f.values(p0, vt, 0); });
+      if (t == t1w - 1) f.values(p1, vt, 1);
+    }
+  };
+  // Tiles of the steady kind: [first, end). There is a tile t + 2 for each of them to load:
+  // the buffer of t + 1, which a step reads, has no load in flight.
+  const int first = max(t0w + 1, VARLEN ? (doc_w + 63) / 64 : 0);
+  const int end = min(min(t_diag, a.Skv / 64), min(t1w - 1, t1 - 2));
+  // Pairs leave a tile over at either end: the runs of short documents are too short for
+  // them. With 256 columns of output they spill; one at a time does not (2 x 4096 tokens, 8
+  // heads of 256: 207 us, 494 with scores, softmax and values one after the other, 544 with the
+  // kernel before; without a mask 378, 895 and 558).
+  constexpr bool PAIRS = !VARLEN && DV < 256;
+  int t = t0;
+  for (; t < min(first, t1) || (PAIRS && t < end && t % 2); ++t) general(t);
+  if constexpr (!PAIRS)
+    for (; t < end; ++t) steady(t, std::integral_constant<int, -1>{});
+  else
+    for (; t + 1 < end; t += 2) {
+      steady(t, std::integral_constant<int, 0>{});
+      steady(t + 1, std::integral_constant<int, 1>{});
+    }
+  for (; t < t1; ++t) general(t);
 
   // ---- normalise, then through LDS (the tiles are done with) to whole-row stores. A
   // sink is one more logit in the denominator, without a key.
@@ -317,11 +292,11 @@ std::tuple<at::Tensor, at::Tensor> doc_bounds(const at::Tensor& cu, int64_t tota
   return {start, end};
 }
 
-template <int DQK, int DV, int WAVES, int OCC, bool PIPE, bool VARLEN>
+template <int DQK, int DV, int WAVES, int OCC, bool VARLEN>
 static void launch_fwd(const FwdArgs& a, hipStream_t stream) {
   using F = Fwd<DQK, DV, WAVES, VARLEN>;
   const long blocks = (long)((a.Sq + F::BM - 1) / F::BM) * a.Hq * a.B;
-  hipLaunchKernelGGL((flash_fwd_kernel<DQK, DV, WAVES, OCC, PIPE, VARLEN>), dim3((unsigned)blocks),
+  hipLaunchKernelGGL((flash_fwd_kernel<DQK, DV, WAVES, OCC, VARLEN>), dim3((unsigned)blocks),
                      dim3(64 * WAVES), F::SMEM, stream, a);
   HIP_CHECK_KERNEL();
 }
@@ -368,18 +343,18 @@ std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
   // (120 us; 4 waves at one a SIMD were 1.3 times slower); (192, 192) would spill at two a SIMD (457
   // against 178 us).
   bool done = false;
-#define FA_FWD_CASE(A, C, W, OCC, PIPE)                             \
-  if (!done && Dqk == A && Dv == C) {                               \
-    done = true;                                                    \
-    if (varlen) launch_fwd<A, C, W, OCC, PIPE, true>(a, stream);    \
-    else launch_fwd<A, C, W, OCC, PIPE, false>(a, stream);          \
+#define FA_FWD_CASE(A, C, W, OCC)                             \
+  if (!done && Dqk == A && Dv == C) {                         \
+    done = true;                                              \
+    if (varlen) launch_fwd<A, C, W, OCC, true>(a, stream);    \
+    else launch_fwd<A, C, W, OCC, false>(a, stream);          \
   }
-  FA_FWD_CASE(64, 64, 4, 3, true)
-  FA_FWD_CASE(96, 96, 4, 2, true)
-  FA_FWD_CASE(128, 128, 4, 2, true)
-  FA_FWD_CASE(192, 128, 8, 2, true)
-  FA_FWD_CASE(192, 192, 4, 1, true)
-  FA_FWD_CASE(256, 256, 4, 1, false)
+  FA_FWD_CASE(64, 64, 4, 3)
+  FA_FWD_CASE(96, 96, 4, 2)
+  FA_FWD_CASE(128, 128, 4, 2)
+  FA_FWD_CASE(192, 128, 8, 2)
+  FA_FWD_CASE(192, 192, 4, 1)
+  FA_FWD_CASE(256, 256, 4, 1)
 #undef FA_FWD_CASE
   TORCH_CHECK(done, "flash_attn_fwd: unsupported head dims (Dqk=", Dqk, ", Dv=", Dv,
               "); supported pairs: (64,64),(96,96),(128,128),(192,128),(192,192),(256,256)");

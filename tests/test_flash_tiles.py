@@ -68,7 +68,7 @@ def test_forward(dims, sq, skv, causal, q_start, cuts, scale):
     assert (lse - rlse).abs().max() < 1e-5 * max(1.0, float(rlse.abs().max()))
 
 
-@pytest.mark.parametrize("dims", [(64, 64), (128, 128), (192, 128)])
+@pytest.mark.parametrize("dims", [(64, 64), (128, 128), (192, 128), (256, 256)])
 @pytest.mark.parametrize("s,causal,cuts", [(160, True, None), (544, True, None), (701, False, None),
                                            (832, False, None), (448, True, ()), (1344, True, (40, 1000))])
 def test_last_tiles_without_a_successor(dims, s, causal, cuts):
