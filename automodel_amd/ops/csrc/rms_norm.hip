@@ -2,7 +2,7 @@
 // registers of the lanes that load it (16 bytes each), so that it is read once.
 //
 // Rows of up to 2048 take one wave or a part of one (LPR lanes of ITERS vectors), without
-// barriers; longer ones a workgroup (at 4096 a wave would hold 8 vectors of each operand
+// barriers; longer ones, and those beyond 512 where rows are few, a workgroup (at 4096 a wave would hold 8 vectors of each operand
 // a lane, too few waves to hide the loads: 74 against 44 us). The backward gives a workgroup a stretch of rows and
 // keeps its share of the weight gradient in registers; the shares go to a [blocks, H]
 // buffer and a second kernel adds them up in a fixed order. Atomic adds into one row of H
@@ -249,15 +249,31 @@ __global__ __launch_bounds__(256) void rms_norm_dw_kernel(const float* __restric
   }
 }
 
-// calls f(lanes per row, vectors per lane) for rows of H
+// calls f(lanes per row, vectors per lane) for T rows of H. A row of more than 512 columns
+// takes one wave where that gives the chip enough of them, and the workgroup where there are
+// few: then the row's own chain of two or four loads and sums a lane is the time (us, a
+// wave's row against a workgroup's)
+//                     1 row  64    256   1000  2000  4096
+//   2048, forward     3.0    3.7   3.8   4.2   4.8   6.9
+//                     2.3    2.8   2.8   3.4   4.5   7.0
+//   2048, backward    6.7    7.6   7.9   10.8  14.0  19.2
+//                     4.8    5.4   7.3   15.7  16.9  20.7
+//   768, forward      2.5    2.9   2.9   3.0   3.3   4.1
+//                     2.4    2.7   2.8   3.0   3.6   5.3
+//   768, backward     5.3    5.7   6.0   8.1   9.9   11.1
+//                     4.8    5.2   6.6   12.8  13.5  15.8
+// The lines cross at about as many rows as columns, and in the backward at an eighth of
+// that: a workgroup's share of the weight gradient is a row of sums for each row then.
 template <typename F>
-void by_row_size(int H, F f) {
+void by_row_size(long T, int H, long few, F f) {
   using std::integral_constant;
 #define RMS_CASE(MAX, LPR, ITERS) \
   if (H <= MAX) return f(integral_constant<int, LPR>{}, integral_constant<int, ITERS>{});
   RMS_CASE(128, 16, 1)
   RMS_CASE(256, 32, 1)
   RMS_CASE(512, 64, 1)
+  if (H <= 2048 && T <= few)
+    return f(integral_constant<int, 256>{}, integral_constant<int, 1>{});
   RMS_CASE(1024, 64, 2)
   RMS_CASE(2048, 64, 4)
   RMS_CASE(4096, 256, 2)
@@ -281,7 +297,7 @@ void launch_fwd(const at::Tensor& x, const bf16* delta, bf16* sum, const at::Ten
                 const at::Tensor& y, const at::Tensor& invrms, double eps) {
   const long T = x.size(0);
   const int H = x.size(1);
-  by_row_size(H, [&](auto lpr, auto iters) {
+  by_row_size(T, H, H, [&](auto lpr, auto iters) {
     constexpr int LPR = lpr.value, ITERS = iters.value;
     hipLaunchKernelGGL((rms_norm_fwd_kernel<LPR, ITERS, ADD>), dim3(ceil_div_i(T, 256 / LPR)),
                        dim3(256), 0, c10::hip::getCurrentHIPStream().stream(), data(x), delta, sum,
@@ -348,7 +364,7 @@ std::tuple<at::Tensor, at::Tensor> rms_norm_bwd(const at::Tensor& dy,
   auto dx = at::empty_like(x);
   at::Tensor dw, part;
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  by_row_size(H, [&](auto lpr, auto iters) {
+  by_row_size(T, H, H / 8, [&](auto lpr, auto iters) {
     constexpr int LPR = lpr.value, ITERS = iters.value;
     // enough workgroups to fill the chip; more only add to the sums that are written and
     // read again (8192 x 4096: 52 us with 512, 44 with 1024, 53 with 2048; 6001 x 2048,

@@ -7,6 +7,7 @@ pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(),
 
 
 @pytest.mark.parametrize("T,H", [(1, 8), (5, 128), (67, 136), (9, 256), (300, 512), (33, 520), (7, 1024),
+                                 (1, 520), (96, 768), (97, 768), (769, 768), (64, 2048), (256, 2048), (2040, 2040),
                                  (2051, 2048), (5, 2056), (1100, 4096), (3, 8192), (2, 16384)])
 def test_forward_backward(T, H):
     from automodel_amd.ops._backend import hip_ops
