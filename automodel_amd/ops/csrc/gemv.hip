@@ -79,9 +79,13 @@ __device__ __forceinline__ Segment segment_of(const Rows& p, int block) {
 // has 512 U columns of each in flight. One row and U = 8 reach the highest rate
 // for one row of x: 14336 x 4096 in 18.6 us (6.3 TB/s) against 23.1 with two rows
 // and U = 2, and 24.2 with two rows and U = 1; short rows end before 8 are in flight.
-// With two rows of x the loads of x count: two rows of W share them from some 48 MB of
-// W on (10240 x 8192 29.5 us, one row 34.2; 5120 x 13824 24.5 and 30.3), below the
-// waves of one row, twice as many, win (4096 x 4096 9.5 and 8.2, 2048 x 9216 14.0 and 10.4).
+// With two rows of x the loads of x count: two rows of W share them, and in steps of 512
+// columns (10240 x 8192 30.5 us, one row in steps of 2048 36.7; 5120 x 17408 32.2 and 39.3;
+// 28672 x 3072 0.95 of one row's). Not up to 4096 rows, which leave too few waves (2048 x
+// 14336 21.7 and 14.4, 3072 x 8192 14.3 and 11.6), nor for rows of 2048 or 4096 columns,
+// which the longer steps divide, below some 128 MB (11008 x 4096 20.0 and 19.0, 12288 x 2048
+// 11.6 and 11.1; but 28672 x 4096 41.4 and 43.5, 65536 x 2048 44.1 and 46.0). Weights of
+// less than 24 MB keep one row.
 template <int B, int R, int U, bool GLU>
 __global__ __launch_bounds__(256) void gemv_bf16_kernel(const Rows p) {
   static_assert(!GLU || R == 2);
@@ -297,7 +301,8 @@ void gemv_rows(const Rows& p, int segments, int B) {
   for (int s = 0; s < segments; ++s) rows += p.n[s];
   if (B == 1 && p.K > 2048) launch_gemv<1, 1, 8>(p, segments);
   else if (B == 1) launch_gemv<1, 1, 4>(p, segments);
-  else if (rows * p.K >= (24l << 20)) launch_gemv<2, 2, 1>(p, segments);
+  else if (rows > 4096 && rows * p.K >= (p.K == 2048 || p.K == 4096 ? 64l << 20 : 12l << 20))
+    launch_gemv<2, 2, 1>(p, segments);
   else launch_gemv<2, 1, 4>(p, segments);
 }
 
