@@ -47,6 +47,7 @@ struct Rows {
   bool relu2;                // max(y, 0)^2
   int K;
   int group_n;               // > 0: every group_n rows of w take the next B rows of x
+  bool stretches;            // skinny: a wave has consecutive tiles of K, else every WAVES-th
 };
 
 __device__ __forceinline__ float dot2(const bf16x8& a, const bf16x8& b, int j, float c) {
@@ -161,10 +162,8 @@ __global__ __launch_bounds__(256) void gemv_bf16_kernel(const Rows p) {
 }
 
 // A workgroup takes 16 RT rows of W (GLU: 16 of gate and the same 16 of up) and
-// 16 NB rows of x; its waves take a stretch of K each and add up through LDS at the
-// end, so that N = 1024 fills the chip too. (Every WAVES-th tile of K instead: 5 rows,
-// 4096 x 4096 8.7 us against 7.7, 8192 x 8192 26.7 against 23.0.) Matrix fragments
-// want one row per lane, memory wants consecutive lanes on consecutive bytes: each
+// 16 NB rows of x; its waves take a part of K each and add up through LDS at the
+// end, so that N = 1024 fills the chip too. Matrix fragments want one row per lane, memory wants consecutive lanes on consecutive bytes: each
 // wave moves its tiles of W and x with coalesced loads into LDS of its own, with the
 // next tile's loads in flight (two ahead: the same). No workgroup barrier in the loop.
 constexpr int SK_KC = 128;                        // K per tile
@@ -194,7 +193,8 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(const Ro
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[r][b] = gemv_f32x4{0.f, 0.f, 0.f, 0.f};
   const int tiles = (K + SK_KC - 1) / SK_KC, per = (tiles + WAVES - 1) / WAVES;
-  const int t_lo = wid * per, t_hi = min(t_lo + per, tiles);
+  const int step = p.stretches ? 1 : WAVES;
+  const int t_lo = p.stretches ? wid * per : wid, t_hi = p.stretches ? min(t_lo + per, tiles) : tiles;
 
   // load j covers rows 4j + hi4, 16 bytes per lane at column 8 lo16
   bf16x8 wr[4 * RT], xr[4 * NB];
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(const Ro
     }
   };
   if (t_lo < t_hi) fetch(t_lo);
-  for (int t = t_lo; t < t_hi; ++t) {
+  for (int t = t_lo; t < t_hi; t += step) {
 #pragma unroll
     for (int j = 0; j < 4 * RT; ++j)
       *reinterpret_cast<bf16x8*>(wl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = wr[j];
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_skinny_kernel(const Ro
     for (int j = 0; j < 4 * NB; ++j)
       *reinterpret_cast<bf16x8*>(xl + (4 * j + hi4) * SK_STRIDE + lo16 * 16) = xr[j];
     __builtin_amdgcn_wave_barrier();
-    if (t + 1 < t_hi) fetch(t + 1);
+    if (t + step < t_hi) fetch(t + step);
 #pragma unroll
     for (int kk = 0; kk < SK_KC / 32; ++kk) {
       const int off = lo16 * SK_STRIDE + kk * 64 + hi4 * 16;
@@ -323,11 +323,23 @@ void launch_skinny(const Rows& rows, int segments, int B) {
 //    32 rows between one and one and a half workgroups a CU (5120 x 5120 12.4, 16 rows 13.5; but
 //    8192 x 8192 24.5 and 23.0), and for many rows of x and of W (16 rows, 32000 x 2048 22.8 and 24.8).
 //  * up to 32: 32 rows of W where that gives the fullest CU no more (24 rows, 8192 x 8192 26.6 and
-//    31.5; 21504 x 4096 36.2 and 40.7), else 16 (9216 x 2048 12.5, 32 rows 14.1).
+//    31.5; 21504 x 4096 36.2 and 40.7), else 16 (9216 x 2048 12.5, 32 rows 14.1); 64 for long rows,
+//    many rows of x and a workgroup a CU (32 rows, 9216 x 5120 30.0 and 31.7, 9216 x 8192 43.1 and 46.0).
 //  * up to 64: the least sum of tiles and 2/5 (long rows: 3/5) of one a workgroup, out of 16, 32 and
 //    64 rows (48 rows, 9216 x 2048 17.8, 32 rows 19.4; 8192 x 8192 40.6, 16 rows 50.1; 10240 x 8192
 //    55.4, 16 rows 61.0; 32000 x 2048 35.2, 32 rows 41.5).
-void skinny(const Rows& p, int segments, int B, bool glu) {
+//
+// Waves read neighbouring tiles of K, or a stretch of K each where rows of W lie a multiple of
+// 4 KB apart (8 rows of x, neighbours and stretches: 4096 x 2048 6.6 and 6.0 us, 6144 x 4096
+// 13.0 and 11.1, 6144 x 8192 22.6 and 19.0; but 4096 x 2560 0.97 to 1, 22016 x 5120 the same).
+// Not with more than 4096 columns where a wave's tile has 32 rows of W or more than 32 rows of x
+// (gated, 4096 x 8192 22.1 and 23.3; 64 rows of x, 14336 x 8192 0.92 to 1), nor for few workgroups
+// and more than 16 rows of x (24 rows, 2048 x 4096 8.7 and 9.4).
+void skinny(Rows p, int segments, int B, bool glu) {
+  long n = 0;
+  for (int s = 0; s < segments; ++s) n += p.n[s];
+  p.stretches = p.K % 2048 == 0 && (p.K <= 4096 || !(glu || B > 32)) &&
+                (p.K <= 2048 || n > 3072 || B <= 16 || glu);
   if (glu) {
     if (B <= 16) launch_skinny<1, 4, 2, true>(p, segments, B);
     else if (B <= 32) launch_skinny<2, 4, 2, true>(p, segments, B);
@@ -345,7 +357,7 @@ void skinny(const Rows& p, int segments, int B, bool glu) {
   const int n1 = workgroups(1);
   if (B <= 16) {
     const bool pairs = may(2) && ((n1 > CUS && n1 <= CUS * 3 / 2) || (B > 8 && n1 >= CUS * 7 / 2));
-    const bool few = p.K <= 512 || (n1 > 2 * CUS && p.K <= 2048);
+    const bool few = p.K <= 512 || (n1 > 2 * CUS && p.K < 4096);
     if (pairs && n1 > 2 * CUS) launch_skinny<1, 4, 2>(p, segments, B);
     else if (pairs) launch_skinny<1, 8, 2>(p, segments, B);
     else if (few) launch_skinny<1, 4, 1>(p, segments, B);
@@ -354,10 +366,12 @@ void skinny(const Rows& p, int segments, int B, bool glu) {
     const bool pairs = may(2) && 2 * fullest(2) <= fullest(1);
     if (pairs && fullest(2) > 1) launch_skinny<2, 4, 2>(p, segments, B);
     else if (pairs) launch_skinny<2, 8, 2>(p, segments, B);
+    else if (may(4) && B > 24 && p.K > 4096 && n1 > 2 * CUS && fullest(4) == 1)
+      launch_skinny<2, 4, 4>(p, segments, B);
     else if (n1 > CUS || p.K <= 512) launch_skinny<2, 4, 1>(p, segments, B);
     else launch_skinny<2, 8, 1>(p, segments, B);
   } else {
-    const int x = p.K > 4096 ? 3 : 2;              // fifths of a tile
+    const int x = p.K > 2048 ? 3 : 2;              // fifths of a tile
     int best = 1;
     for (int rt : {2, 4})
       if (may(rt) && fullest(rt) * (5 * rt + x) < fullest(best) * (5 * best + x)) best = rt;
