@@ -163,9 +163,10 @@ __global__ __launch_bounds__(256) void gemv_bf16_kernel(const Rows p) {
 
 // A workgroup takes 16 RT rows of W (GLU: 16 of gate and the same 16 of up) and
 // 16 NB rows of x; its waves take a part of K each and add up through LDS at the
-// end, so that N = 1024 fills the chip too. Matrix fragments want one row per lane, memory wants consecutive lanes on consecutive bytes: each
-// wave moves its tiles of W and x with coalesced loads into LDS of its own, with the
-// next tile's loads in flight (two ahead: the same). No workgroup barrier in the loop.
+// end, so that N = 1024 fills the chip too. Matrix fragments want one row per lane,
+// memory wants consecutive lanes on consecutive bytes: each wave moves its tiles of W
+// and x with coalesced loads into LDS of its own, with the next tile's loads in flight
+// (two ahead: the same). No workgroup barrier in the loop.
 constexpr int SK_KC = 128;                        // K per tile
 constexpr int SK_STRIDE = SK_KC * 2 + 16;         // LDS bytes per row
 

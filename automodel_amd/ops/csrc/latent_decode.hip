@@ -682,7 +682,7 @@ std::tuple<at::Tensor, at::Tensor> latent_decode_attn(const at::Tensor& q, const
   // whole CU. They win from 64 rows on, where splits are long (one head tile and pairs, prep
   // and combine included: 64 rows of 16000 keys, 32 heads 350 and 313 us, 128 heads 1312 and
   // 1076; of 500 keys 45 and 44, 132 and 125), and lose below (32 rows of 2000 keys, 64 heads
-  // 66.8 and 70.3; 1 of 200, 32 heads 15.6 and 18.6), or where their last round leaves more of the
+  // 66.8 and 70.3; 1 of 200, 32 heads 15.6 and 18.6), or where their last pass leaves more of the
   // chip idle (96 rows of 8000, 128 heads, 256 latents: 620 and 712; 128 rows: 918 and 741).
   auto fill = [&](int ht) {
     const int64_t round = 256 * (LDS_MAX / smem_of(ht));
