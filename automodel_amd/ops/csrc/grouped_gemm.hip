@@ -6,7 +6,7 @@
 //                w (gate and up): one sum in the accumulators instead of an addition after
 //   tn (dw)   dw[e, n, k]  = sum_{m of e} g[m, n] x[m, k]
 //
-// One kernel for the three: 8 waves compute BM x 256 of the output, 64 x 64 or 64 x 128
+// grouped_gemm_kernel has the three: 8 waves compute BM x 256 of the output, 64 x 64 or 64 x 128
 // each, over steps of 64 of the summed index. What differs is which index of an
 // operand is contiguous: tiles whose rows are output rows or columns are read by rows,
 // tiles whose rows are the summed index by columns, with the transposing LDS reads
@@ -19,14 +19,20 @@
 //
 // Bound by LDS (at full MFMA rate 64 x 128 wave tiles read and load 128 B/clk, 64 x 64 ones
 // more: 256 x 256 is the faster tile) against padding of the groups' last row tiles: nt and
-// nn take 256 rows from 512 rows per expert on (the caller's plan, ops/grouped_gemm.py, has both
+// nn take 256 rows from 320 rows per expert on (the caller's plan, ops/grouped_gemm.py, has both
 // sides), tn, whose tiles have no padding, always. 4 waves of 64 x 128, one a SIMD, wait for
 // LDS more than they save (128 x 256: 374 against 345 us).
-// Measured, nt / nn / tn, groups as a random choice fills them, before (tn with its transposes)
-// -> now: 65536 rows, 128 experts, 768 x 2048: 515 / 607 / 742 -> 255 / 281 / 286 us; 2048 x 768:
-// 502 / 691 / 757 -> 280 / 262 / 275 us; 18018 rows, 64 experts, 1408 x 2048: 284 / 369 / 403 ->
-// 166 / 166 / 184 us; 16384 rows, 8 experts, 4096 x 2048: 495 / 779 / 639 -> 280 / 307 / 276 us
-// (982 / 895 / 996 TFLOP/s).
+//
+// grouped_tile_kernel: 4 waves of 128 x 128 (gemm_tile.h), for nn's tiles of 256 rows, and for tn
+// from 512 rows per expert on. Its fixed cost per tile is the larger one, with nothing beside it on
+// the CU: tn, 768 x 2048, 128 experts of 512, 640, 1024 and 2048 rows: 336 / 355 / 479 / 876 ->
+// 319 / 333 / 420 / 729 us, but 64 experts of 281 rows, 1408 x 2048: 186 -> 196. (nt has not got
+// it: 1.00 of the time in one shape, 1.05 in another.)
+// Measured, nt / nn / tn, groups as a random choice fills them, without grouped_tile_kernel -> now:
+// 65536 rows, 128 experts, 768 x 2048: 251 / 281 / 275 -> 251 / 250 / 271 us; 2048 x 768:
+// 279 / 259 / 270 -> 279 / 227 / 269 us; 18018 rows, 64 experts, 1408 x 2048: 164 / 163 / 186 us;
+// 16384 rows, 8 experts, 4096 x 2048: 289 / 326 / 272 -> 289 / 260 / 212 us (951 / 1057 / 1297
+// TFLOP/s).
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -34,6 +40,7 @@
 
 #include "common.h"
 #include "flash_tile.h"
+#include "gemm_tile.h"
 #include "ops_api.h"
 
 namespace amd_ops {
@@ -50,7 +57,7 @@ struct GroupedArgs {
   const bf16 *r2, *c2;                 // nn: a second pair, added to the sum
   bf16* out;
   const int *tile_map, *offs, *n_tiles;
-  int n_mtiles, N, K, E;               // tile_map's capacity; w is [E, N, K]
+  int n_mtiles, M, N, K, E;            // tile_map's capacity; rows; w is [E, N, K]
 };
 
 }  // namespace
@@ -187,6 +194,49 @@ __global__ __launch_bounds__(64 * WAVES, 1) void grouped_gemm_kernel(const Group
   }
 }
 
+// nn and tn by 256 x 256 tiles of four waves (gemm_tile.h).
+template <Mode MODE>
+__global__ __launch_bounds__(gt::THREADS, 1) void grouped_tile_kernel(const GroupedArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int nr = (a.N + gt::TILE - 1) / gt::TILE, nc = (a.K + gt::TILE - 1) / gt::TILE;
+  const int total = MODE == TN ? a.E * nr * nc : (a.n_tiles ? a.n_tiles[0] : a.n_mtiles) * nc;
+  const int per = (total + 7) / 8, slot = blockIdx.x >> 3, id = (blockIdx.x & 7) * per + slot;
+  if (slot >= per || id >= total) return;
+  const int c0 = id % nc * gt::TILE;
+  gt::Tile t{};
+  t.cols = a.K - c0;
+  t.c_ld = a.K;
+  bf16* out;
+  if constexpr (MODE == TN) {
+    const int e = id / (nr * nc), r0 = id / nc % nr * gt::TILE, m0 = a.offs[e];
+    t.sum = a.offs[e + 1] - m0;
+    t.rows = a.N - r0;
+    t.r = a.r + (long)m0 * a.N + r0;
+    t.c = a.c + (long)m0 * a.K + c0;
+    t.r_ld = a.N;
+    t.before = m0;
+    t.after = a.M - m0;
+    out = a.out + ((long)e * a.N + r0) * a.K + c0;
+  } else {
+    const int e = a.tile_map[2 * (id / nc)], r0 = a.tile_map[2 * (id / nc) + 1];
+    const long w = (long)e * a.N * a.K + c0;
+    t.sum = t.after = a.N;
+    t.rows = a.offs[e + 1] - r0;
+    t.r_ld = a.N;
+    t.r = a.r + (long)r0 * a.N;
+    t.c = a.c + w;
+    if (a.r2) {
+      t.r2 = a.r2 + (long)r0 * a.N;
+      t.c2 = a.c2 + w;
+    }
+    out = a.out + (long)r0 * a.K + c0;
+  }
+  gt::f32x4_t acc[8][8];
+  if (t.sum > 0) gt::multiply<MODE == TN>(acc, t, smem);
+  else gt::zero(acc);
+  gt::store(acc, smem, out, a.K, t.rows, t.cols);
+}
+
 // Offsets and (expert, first row) tiles of the groups, from counts on the device, so that
 // routing never waits for the host. One workgroup: thread t sums a stretch of experts, a
 // scan over the threads gives every stretch its first row and tile. (A single thread took
@@ -248,19 +298,38 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> build_group_plan(
 
 namespace {
 
-template <Mode MODE, int BM, int BN, int WAVES, int BUFS>
-void launch(const GroupedArgs& a) {
-  constexpr int rt = MODE == TN ? STEP * row_bytes(BM) : BM * row_bytes(STEP);
-  constexpr int ct = MODE != NT ? STEP * row_bytes(BN) : BN * row_bytes(STEP);
-  constexpr int wn = BN * BM / 64 / WAVES;
-  constexpr int smem = std::max(BUFS * (rt + ct), WAVES * 32 * row_bytes(wn));
-  const int nc = ((MODE == NT ? a.N : a.K) + BN - 1) / BN;
-  const long tiles = MODE == TN ? (long)a.E * ((a.N + BM - 1) / BM) * nc : (long)a.n_mtiles * nc;
+// tile: rows of the output's tiles; four: by grouped_tile_kernel
+template <Mode MODE>
+void launch(const GroupedArgs& a, int64_t tile, bool four) {
+  const int nc = ((MODE == NT ? a.N : a.K) + 255) / 256;
+  const long tiles = MODE == TN ? (long)a.E * ((a.N + 255) / 256) * nc : (long)a.n_mtiles * nc;
   TORCH_CHECK(tiles < (1l << 31) - 8, "grouped_gemm: too many tiles");
   // the stretches of the 8 XCDs are rounded up: up to 7 workgroups beyond the tiles
-  hipLaunchKernelGGL((grouped_gemm_kernel<MODE, BM, BN, WAVES, BUFS>), dim3((unsigned)((tiles + 7) / 8 * 8)),
-                     dim3(64 * WAVES), smem, c10::hip::getCurrentHIPStream().stream(), a);
-  HIP_CHECK_KERNEL();
+  const dim3 grid((unsigned)((tiles + 7) / 8 * 8));
+  const auto stream = c10::hip::getCurrentHIPStream().stream();
+  auto eight = [&](auto bm_, auto bufs_) {
+    constexpr int BM = decltype(bm_)::value, BUFS = decltype(bufs_)::value;
+    constexpr int rt = MODE == TN ? STEP * row_bytes(BM) : BM * row_bytes(STEP);
+    constexpr int ct = MODE != NT ? STEP * row_bytes(256) : 256 * row_bytes(STEP);
+    constexpr int smem = std::max(BUFS * (rt + ct), 8 * 32 * row_bytes(BM / 2));
+    hipLaunchKernelGGL((grouped_gemm_kernel<MODE, BM, 256, 8, BUFS>), grid, dim3(512), smem, stream, a);
+  };
+  if constexpr (MODE != NT)
+    if (four) {
+      hipLaunchKernelGGL((grouped_tile_kernel<MODE>), grid, dim3(gt::THREADS), gt::SMEM, stream, a);
+      HIP_CHECK_KERNEL();
+      return;
+    }
+  if constexpr (MODE != TN)
+    if (tile == 128) {
+      eight(std::integral_constant<int, 128>{}, std::integral_constant<int, 3>{});
+      HIP_CHECK_KERNEL();
+      return;
+    }
+  if constexpr (MODE != NN) {
+    eight(std::integral_constant<int, 256>{}, std::integral_constant<int, 2>{});
+    HIP_CHECK_KERNEL();
+  }
 }
 
 GroupedArgs grouped_args(const at::Tensor& r, const at::Tensor& c, at::Tensor& out,
@@ -273,6 +342,7 @@ GroupedArgs grouped_args(const at::Tensor& r, const at::Tensor& c, at::Tensor& o
   a.c = reinterpret_cast<const bf16*>(c.data_ptr());
   a.out = reinterpret_cast<bf16*>(out.data_ptr());
   a.offs = offs.data_ptr<int>();
+  a.M = r.size(0);
   return a;
 }
 
@@ -300,8 +370,7 @@ at::Tensor grouped_gemm_nt(const at::Tensor& x, const at::Tensor& w,
   if (tile_map.size(0) == 0 || x.size(0) == 0) return y;
   auto a = grouped_args(x, w, y, offs);
   set_tiles(a, w, offs, tile_map, n_tiles);
-  if (bm == 256) launch<NT, 256, 256, 8, 2>(a);
-  else launch<NT, 128, 256, 8, 3>(a);
+  launch<NT>(a, bm, false);
   return y;
 }
 
@@ -321,8 +390,7 @@ static at::Tensor nn(const at::Tensor& g, const at::Tensor& w, const at::Tensor*
     a.c2 = b.c;
   }
   set_tiles(a, w, offs, tile_map, n_tiles);
-  if (bm == 256) launch<NN, 256, 256, 8, 2>(a);
-  else launch<NN, 128, 256, 8, 3>(a);
+  launch<NN>(a, bm, bm == 256);
   return dx;
 }
 
@@ -348,7 +416,7 @@ at::Tensor grouped_gemm_tn(const at::Tensor& g, const at::Tensor& x, const at::T
   a.E = E;
   a.N = g.size(1);
   a.K = x.size(1);
-  launch<TN, 256, 256, 8, 2>(a);
+  launch<TN>(a, 256, (int64_t)a.M >= 512l * E);
   return dw;
 }
 

@@ -46,13 +46,13 @@ def tile_rows(rows: int, experts: int) -> int:
     every group is padding for half of it on average, and there are half as many.
     Time of 256 over that of 128, forward and dx together, groups as a random choice
     fills them, at 128, 256, 320, 384, 512 and 1024 rows per expert:
-    128 experts of 768 x 2048: 1.06 1.04 0.99 0.90 0.93 0.90;
-    64 of 1408 x 2048: 1.06 1.05 0.96 0.90 0.93 0.89;
-    8 of 4096 x 2048, few tiles: 1.46 1.24 1.15 1.10 0.90 1.01;
-    32 of 1024 x 1024: 1.38 0.84 0.86 0.86 1.03 1.01.
-    From 512 on it is slower nowhere by more than 3%; below, the sign depends on how
-    the tiles fill the chip."""
-    return 256 if rows >= 512 * experts else 128
+    128 experts of 768 x 2048: 1.09 1.01 0.97 0.88 0.88 0.86;
+    64 of 1408 x 2048: 1.05 0.97 0.94 0.84 0.86 0.83;
+    8 of 4096 x 2048, few tiles: 1.32 1.04 1.03 1.03 0.81 0.91;
+    32 of 1024 x 1024: 1.39 0.84 0.86 0.84 1.02 0.94.
+    From 320 on it is slower nowhere by more than 3%; below, the sign depends on how
+    the tiles fill the chip, and the forward alone is up to 12% slower."""
+    return 256 if rows >= 320 * experts else 128
 
 
 def _loop_gemm_nt(x, w, counts):

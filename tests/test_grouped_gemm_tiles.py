@@ -40,3 +40,36 @@ def test_grouped_gemm(counts, N, K, bm):
               torch.cat([g[s].double() @ w[e].double() for e, s in enumerate(part)]))
         close(ops.grouped_gemm_tn(g, x, offs, E),
               torch.stack([g[s].double().t() @ x[s].double() for s in part]))
+
+
+# rows of 512 per group and more on average: the weight gradients' 256 x 256 tiles of four waves
+@pytest.mark.parametrize("counts,N,K", [
+    ([1600, 0, 31, 513], 384, 640), ([1, 1, 2000], 128, 128), ([512, 512], 256, 1408),
+    ([0, 0, 3000], 128, 384), ([2000, 33, 1], 896, 256), ([1025], 128, 128), ([1535, 1], 128, 128),
+])
+def test_grouped_weight_gradient(counts, N, K):
+    from automodel_amd.ops._backend import hip_ops
+
+    torch.manual_seed(0)
+
+    def close(got, want):       # f32 sums, rounded to bf16 once
+        assert (got.double() - want).norm() <= 2.0 ** -9 * 1.02 * want.norm()
+
+    M, E = sum(counts), len(counts)
+    assert M >= 512 * E
+    g, x = (torch.randn(M, n, device="cuda").bfloat16() for n in (N, K))
+    at = torch.tensor([0, *counts]).cumsum(0).tolist()
+    part = [slice(at[e], at[e + 1]) for e in range(E)]
+    offs = torch.tensor(at, dtype=torch.int32, device="cuda")
+    want = torch.stack([g[s].double().t() @ x[s].double() for s in part])
+    close(hip_ops().grouped_gemm_tn(g, x, offs, E), want)
+    # a group's infinities stay its own
+    for e in range(E):
+        if counts[e]:
+            gi, xi = g.clone(), x.clone()
+            gi[part[e]], xi[part[e]] = float("inf"), float("inf")
+            got = hip_ops().grouped_gemm_tn(gi, xi, offs, E)
+            rest = [i for i in range(E) if i != e]
+            assert not got[e].isfinite().any()
+            if rest and want[rest].norm() > 0:
+                close(got[rest], want[rest])
