@@ -21,6 +21,7 @@ from __future__ import annotations
 import torch
 
 from automodel_amd.ops._backend import hip_ops
+from automodel_amd.ops.linear import input_grad, weight_grad
 
 IGNORE_INDEX = -100
 
@@ -99,9 +100,9 @@ def _chunk_grads(ctx, dloss: torch.Tensor):
             g = h @ weight.t()
             ops.ce_bwd_logits(g, y, lse, d, 0)
         if need_h:
-            dh[rows] = g @ weight
+            dh[rows] = input_grad(g, weight)
         if need_w:
-            part = g.t() @ h
+            part = weight_grad(g, h)
             # sums of three and more parts in float32; of two, rounding their float32 sum
             # once is what a bf16 addition does
             if dw is None:

@@ -22,6 +22,7 @@ import torch.nn as nn
 from automodel_amd.models.common.backend import BackendConfig
 from automodel_amd.ops import attention as attn_mod
 from automodel_amd.ops.attention import _sdpa, flash_attention, sdpa_masked
+from automodel_amd.ops.linear import linear
 from automodel_amd.ops.rms_norm import RMSNorm, add_norm
 from automodel_amd.ops.rope import apply_rope, build_rope_cache
 from automodel_amd.ops.swiglu import swiglu, swiglu_cat
@@ -140,7 +141,7 @@ def _project(backend: BackendConfig, lins: list[nn.Module], x: torch.Tensor) -> 
         ys = decode_rows(lins, x)
         if ys is not None:
             return ys
-    return [lin(x) for lin in lins]
+    return [linear(lin, x) for lin in lins]
 
 
 class LlamaAttention(nn.Module):
@@ -270,8 +271,9 @@ class LlamaMLP(nn.Module):
             if act is not None:
                 return _project(self.backend, [self.down_proj], act[0])[0]
         if self.fused:
-            return self.down_proj(swiglu_cat(self.gate_up_proj(x)))
-        return self.down_proj(swiglu(self.gate_proj(x), self.up_proj(x)))
+            return linear(self.down_proj, swiglu_cat(linear(self.gate_up_proj, x)))
+        return linear(self.down_proj,
+                      swiglu(linear(self.gate_proj, x), linear(self.up_proj, x)))
 
 
 class XIELUActivation(nn.Module):

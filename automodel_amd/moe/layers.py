@@ -14,6 +14,7 @@ import torch.nn as nn
 from automodel_amd.moe.config import MoEConfig
 from automodel_amd.moe.experts import GroupedExperts, check_experts
 from automodel_amd.ops._backend import ops_available
+from automodel_amd.ops.linear import linear
 from automodel_amd.ops.swiglu import swiglu
 
 
@@ -191,7 +192,8 @@ class SharedExpert(nn.Module):
         self.down_proj = nn.Linear(intermediate, hidden_size, bias=False)
 
     def forward(self, x):
-        return self.down_proj(swiglu(self.gate_proj(x), self.up_proj(x)))
+        return linear(self.down_proj,
+                      swiglu(linear(self.gate_proj, x), linear(self.up_proj, x)))
 
 
 _SHARED_STREAMS: dict = {}

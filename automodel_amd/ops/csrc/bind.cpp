@@ -94,6 +94,10 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("grouped_gemm_nn", &amd_ops::grouped_gemm_nn);
   m.def("grouped_gemm_tn(Tensor g, Tensor x, Tensor offs, int E) -> Tensor");
   m.impl("grouped_gemm_tn", &amd_ops::grouped_gemm_tn);
+  m.def("linear_dw(Tensor g, Tensor x) -> Tensor");
+  m.impl("linear_dw", &amd_ops::linear_dw);
+  m.def("linear_dx(Tensor g, Tensor w) -> Tensor");
+  m.impl("linear_dx", &amd_ops::linear_dx);
   m.def("grouped_gemm_nt_fp8(Tensor x8, Tensor w8, Tensor offs, Tensor tile_map, Tensor scale, Tensor? n_tiles=None, int bm=128) -> Tensor");
   m.impl("grouped_gemm_nt_fp8", &amd_ops::grouped_gemm_nt_fp8);
   m.def("route_plan(Tensor indices, Tensor probs, int E) -> (Tensor, Tensor, Tensor, Tensor, Tensor)");

@@ -116,6 +116,8 @@ at::Tensor grouped_gemm_nn(const at::Tensor& g, const at::Tensor& w,
                            const std::optional<at::Tensor>& n_tiles = std::nullopt,
                            int64_t bm = 128);
 at::Tensor grouped_gemm_tn(const at::Tensor& g, const at::Tensor& x, const at::Tensor& offs, int64_t E);
+at::Tensor linear_dw(const at::Tensor& g, const at::Tensor& x);
+at::Tensor linear_dx(const at::Tensor& g, const at::Tensor& w);
 at::Tensor grouped_gemm_nt_fp8(const at::Tensor& x8, const at::Tensor& w8,
                                const at::Tensor& offs, const at::Tensor& tile_map,
                                const at::Tensor& scale,

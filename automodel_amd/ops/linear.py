@@ -1,0 +1,115 @@
+"""``linear(lin, x)``: an ``nn.Linear`` whose gradients run on csrc/linear_grad.hip.
+
+The product itself stays the library's (x w^T is where it is at its best). The two products of
+the backward have the summed index as a row of one operand or both; there the library
+reaches 1.1 to 1.4 PFLOP/s, the kernels 1.5.
+"""
+
+from __future__ import annotations
+
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+from torch.autograd import forward_ad
+from torch.utils import _python_dispatch
+
+from automodel_amd.ops._backend import hip_ops
+
+TILE, CUS = 256, 256
+# below this many products a layer's backward takes the library some 80 us, and an autograd
+# function of Python's costs the host as much as is gained
+MIN_PRODUCTS = 1 << 34
+
+
+def _fills(rows: int, cols: int, share: float) -> bool:
+    """Whether output tiles of 256 x 256 keep that share of the chip's rounds busy."""
+    tiles = -(-rows // TILE) * -(-cols // TILE)
+    return tiles >= share * CUS * -(-tiles // CUS)
+
+
+def weight_grad_wins(T: int, N: int, K: int) -> bool:
+    """Kernel or library for g^T x, g [T, N], x [T, K]. Time of the one over the other's, by the
+    share of the rounds that the tiles fill: 1.0 at 0.67 to 0.81 (10240 x 2560, 2000 to 8192
+    rows: 400 tiles, 0.78, 0.66 to 0.74), 0.83 to 0.95 at 0.75 (6144 x 4096, 384 tiles),
+    1.1 to 1.2 at 0.5, 1.3 to 1.7 at 0.25; 200 to 8192 rows alike."""
+    return T * N * K >= MIN_PRODUCTS and N % 8 == 0 and K % 8 == 0 and _fills(N, K, 0.75)
+
+
+def input_grad_wins(T: int, N: int, K: int) -> bool:
+    """Kernel or library for g w, g [T, N], w [N, K]: 0.85 to 0.91 of the library's time where
+    the tiles fill the rounds, 0.96 to 1.02 at 0.75, 1.0 to 1.2 at 0.5."""
+    return T * N * K >= MIN_PRODUCTS and N % 64 == 0 and K % 8 == 0 and _fills(T, K, 0.875)
+
+
+def _plain(*ts: torch.Tensor) -> bool:
+    return all(t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous()
+               and t.data_ptr() % 16 == 0 for t in ts)
+
+
+def weight_grad(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """g^T x for g [T, N] and x [T, K]."""
+    if weight_grad_wins(*g.shape, x.shape[1]) and _plain(g, x):
+        return hip_ops().linear_dw(g, x)
+    return g.t() @ x
+
+
+def input_grad(g: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """g w for g [T, N] and w [N, K]."""
+    if input_grad_wins(*g.shape, w.shape[1]) and _plain(g, w):
+        return hip_ops().linear_dx(g, w)
+    return g @ w
+
+
+class _Linear(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w):
+        need_x, need_w = ctx.needs_input_grad
+        ctx.save_for_backward(x if need_w else None, w if need_x else None)
+        ctx.shape = x.shape
+        return F.linear(x, w)
+
+    @staticmethod
+    def backward(ctx, g):
+        x, w = ctx.saved_tensors
+        g = g.reshape(-1, g.shape[-1])
+        twice = torch.is_grad_enabled()        # the backward is recorded itself
+        if not twice:
+            g = g.contiguous()
+        dx = dw = None
+        if w is not None:
+            dx = (g @ w if twice else input_grad(g, w)).view(ctx.shape)
+        if x is not None:
+            x = x.reshape(-1, x.shape[-1])
+            dw = g.t() @ x if twice else weight_grad(g, x)
+        return dx, dw
+
+
+def _unseen(lin: nn.Linear) -> bool:
+    """No hook sees the module's call or its gradients, and nothing follows the operations
+    (transforms, forward-mode derivatives, tracing, dispatch modes) but autograd."""
+    every = nn.modules.module
+    return not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks
+                or lin._backward_pre_hooks or every._global_forward_hooks
+                or every._global_forward_pre_hooks or every._global_backward_hooks
+                or every._global_backward_pre_hooks or torch.compiler.is_compiling()
+                or torch.jit.is_tracing() or torch.is_autocast_enabled("cuda")
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or forward_ad._current_level >= 0
+                or _python_dispatch._get_current_dispatch_mode() is not None)
+
+
+def linear(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``lin(x)``. Plain bf16 layers without a bias on the GPU that are large enough take the
+    kernels in their backward, everything else is the module's call."""
+    if (type(lin) is nn.Linear and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda
+            and x.dtype == torch.bfloat16 and torch.is_grad_enabled() and lin.bias is None):
+        w = lin.weight
+        if (type(w) is nn.Parameter and w.dim() == 2 and x.shape[-1:] == w.shape[1:]
+                and w.dtype == x.dtype and w.device == x.device and x.numel() > 0):
+            N, K = w.shape
+            T = x.numel() // K
+            if (((x.requires_grad and input_grad_wins(T, N, K))
+                 or (w.requires_grad and weight_grad_wins(T, N, K)))
+                    and "forward" not in lin.__dict__ and _unseen(lin)):
+                return _Linear.apply(x, w)
+    return lin(x)

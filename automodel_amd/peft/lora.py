@@ -16,6 +16,8 @@ from dataclasses import dataclass, field
 import torch
 import torch.nn as nn
 
+from automodel_amd.ops.linear import linear
+
 
 @dataclass
 class PeftConfig:
@@ -116,7 +118,7 @@ class LinearLoRA(nn.Module):
             y = torch.nn.functional.linear(x, w, self.base.bias)
             return y
         wa, wb = self.lora_A.weight, self.lora_B.weight
-        y = self.base(x)
+        y = linear(self.base, x)
         if (x.is_cuda and x.dtype == torch.bfloat16 and not self.training_dropout()
                 and wa.shape[0] in (32, 64) and wa.shape[1] % 64 == 0
                 and wb.shape[0] % 64 == 0 and wa.dtype == y.dtype == torch.bfloat16

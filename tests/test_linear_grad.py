@@ -1,0 +1,158 @@
+"""Gradients of linear layers on 256 x 256 tiles: edges of the tiles and of the summed index, and
+which calls of a layer come to them."""
+
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from automodel_amd.ops import linear as L
+
+gpu = pytest.mark.gpu
+cuda = pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+
+
+def close(got, want):
+    # f32 sums, rounded to bf16 once: 8 bits, so half a unit is at most 2^-8 of a value (results of 64
+    # elements come to 0.54 of that, large ones to 0.42). The f32 sums of up to 4096 products are
+    # off by 1e-6 of the result's size, which 2% of it covers
+    assert got.shape == want.shape
+    assert (got.double() - want).norm() <= 2.0 ** -8 * 1.02 * want.norm()
+
+
+def rand(*shape):
+    return torch.randn(*shape, device="cuda").bfloat16()
+
+
+@gpu
+@cuda
+@pytest.mark.parametrize("T", [1, 7, 31, 32, 33, 63, 64, 65, 95, 97, 130, 1001])
+@pytest.mark.parametrize("N,K", [(8, 8), (256, 512), (264, 248), (1000, 136)])
+def test_weight_gradient(T, N, K):
+    from automodel_amd.ops._backend import hip_ops
+
+    torch.manual_seed(T)
+    g, x = rand(T, N), rand(T, K)
+    close(hip_ops().linear_dw(g, x), g.double().t() @ x.double())
+
+
+@gpu
+@cuda
+@pytest.mark.parametrize("T", [1, 8, 255, 256, 257, 1001])
+@pytest.mark.parametrize("N,K", [(64, 8), (128, 512), (192, 248), (320, 1000), (1024, 136)])
+def test_input_gradient(T, N, K):
+    from automodel_amd.ops._backend import hip_ops
+
+    torch.manual_seed(T)
+    g, w = rand(T, N), rand(N, K)
+    close(hip_ops().linear_dx(g, w), g.double() @ w.double())
+
+
+@gpu
+@cuda
+def test_refusals():
+    from automodel_amd.ops._backend import hip_ops
+
+    ops = hip_ops()
+    for bad in (lambda: ops.linear_dw(rand(4, 12), rand(4, 8)), lambda: ops.linear_dw(rand(4, 8), rand(5, 8)),
+                lambda: ops.linear_dw(rand(4, 8).float(), rand(4, 8)), lambda: ops.linear_dw(rand(8, 4).t(), rand(4, 8)),
+                lambda: ops.linear_dx(rand(4, 32), rand(32, 8)), lambda: ops.linear_dx(rand(4, 64), rand(64, 12)),
+                lambda: ops.linear_dx(rand(4, 64), rand(64, 8).cpu())):
+        with pytest.raises(RuntimeError):
+            bad()
+
+
+@gpu
+@cuda
+@pytest.mark.parametrize("T,N,K,dw,dx", [
+    (1040, 4096, 4096, True, False), (4095, 1088, 4096, False, True), (2048, 4096, 4096, True, False),
+    (4096, 4096, 4096, True, True), (1000, 4096, 4096, False, False), (4096, 4100, 4096, False, False),
+])
+@pytest.mark.parametrize("train_x,train_w", [(True, True), (True, False), (False, True)])
+def test_layer(monkeypatch, T, N, K, dw, dx, train_x, train_w):
+    torch.manual_seed(0)
+    lin = nn.Linear(K, N, bias=False, device="cuda", dtype=torch.bfloat16).requires_grad_(train_w)
+    x = rand(1, T, K).requires_grad_(train_x)
+    g = rand(1, T, N)
+    assert L.weight_grad_wins(T, N, K) == dw and L.input_grad_wins(T, N, K) == dx
+    y = L.linear(lin, x)
+    own = (dw and train_w) or (dx and train_x)
+    assert ("_Linear" in type(y.grad_fn).__name__) == own
+    assert torch.equal(y, lin(x))
+    inputs = [t for t in (x, lin.weight) if t.requires_grad]
+    got = dict(zip(map(id, inputs), torch.autograd.grad(y, inputs, g, retain_graph=True)))
+    if train_x:
+        close(got[id(x)][0], g[0].double() @ lin.weight.double())
+    if train_w:
+        close(got[id(lin.weight)], g[0].double().t() @ x[0].double())
+    if own and train_x and train_w:       # gradients of gradients, as F.linear has them
+        twice = []
+        for z in (y, F.linear(x, lin.weight)):
+            first = torch.autograd.grad(z, inputs, g, create_graph=True)
+            twice.append(torch.autograd.grad(sum((t.float() ** 2).sum() for t in first), inputs))
+        for a, b in zip(*twice):
+            assert torch.equal(a, b)
+
+
+@gpu
+@cuda
+def test_calls_that_stay_the_module(monkeypatch):
+    T, N, K = 4096, 4096, 4096
+    x = rand(T, K).requires_grad_()
+
+    def own(lin, x=x):
+        return "_Linear" in type(L.linear(lin, x).grad_fn).__name__
+
+    def make(**kw):
+        return nn.Linear(K, N, device="cuda", dtype=torch.bfloat16, **{"bias": False, **kw})
+
+    assert own(make())
+    assert not own(make(bias=True))
+    assert own(make(), x.view(2, -1, K)) and not own(make(), x[:100])
+    for hook in ("register_forward_hook", "register_forward_pre_hook", "register_full_backward_hook",
+                 "register_full_backward_pre_hook"):
+        lin, seen = make(), []
+        handle = getattr(lin, hook)(lambda *a: seen.append(1) and None)
+        L.linear(lin, x).sum().backward()
+        assert seen == [1]
+        handle.remove()
+        assert own(lin)
+
+    class Other(nn.Linear):
+        pass
+
+    assert not own(Other(K, N, bias=False, device="cuda", dtype=torch.bfloat16))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not own(make())
+    with torch.no_grad():
+        assert L.linear(make(), x).grad_fn is None
+    from torch.utils.flop_counter import FlopCounterMode
+
+    lin = make()
+    with FlopCounterMode(display=False) as count:
+        L.linear(lin, x).sum().backward()
+    assert count.get_total_flops() == 6 * T * N * K
+    import torch.autograd.forward_ad as fwd
+
+    with fwd.dual_level():
+        y = L.linear(lin, fwd.make_dual(x.detach().requires_grad_(), torch.ones_like(x)))
+        close(fwd.unpack_dual(y).tangent, torch.ones_like(x).double() @ lin.weight.double().t())
+    out = torch.func.vmap(lambda t: L.linear(lin, t))(x.detach().view(4, -1, K).requires_grad_())
+    assert out.shape == (4, T // 4, N)
+
+
+def test_layers_elsewhere():
+    lin, seen = nn.Linear(16, 8, bias=False), []
+    lin.register_forward_hook(lambda *a: seen.append(1))
+    x = torch.randn(3, 16, requires_grad=True)
+    assert torch.equal(L.linear(lin, x), F.linear(x, lin.weight)) and seen == [1]
+    assert torch.equal(L.weight_grad(x, x), x.t() @ x) and torch.equal(L.input_grad(x, lin.weight.t()), x @ lin.weight.t())
+
+
+def test_rule():
+    # the chip's 256 workgroups per round: whole, three quarters and half rounds
+    assert L.weight_grad_wins(8192, 4096, 4096) and L.weight_grad_wins(8192, 6144, 4096)
+    assert not L.weight_grad_wins(8192, 2048, 4096) and not L.weight_grad_wins(64, 4096, 4096)
+    assert not L.weight_grad_wins(8192, 4100, 4096) and not L.weight_grad_wins(8192, 4096, 4092)
+    assert L.input_grad_wins(8192, 6144, 4096) and not L.input_grad_wins(6001, 4096, 4096)
+    assert not L.input_grad_wins(8192, 6176, 4096) and not L.input_grad_wins(8192, 4096, 4100)
