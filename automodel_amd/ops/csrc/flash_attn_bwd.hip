@@ -15,14 +15,13 @@
 // core forms the scores of the next half tile and adds the products of the previous one
 // (PIPE; three tiles of head dim 192/192 or 256 do not fit LDS: there two buffers, and the
 // phases follow one another).
-// dK/dV is bound by waits that nothing fills: its accumulators and operands leave one wave a
-// SIMD (matrix cores 39% busy, instructions issued 46% of the cycles, at 16384 x 128); dQ, two
-// waves a SIMD, by the matrix cores (66%) and LDS reads (32 rows per wave: 128 B/clk at full
-// MFMA rate).
+// dK/dV for values of 128 columns has a kernel of its own with its instructions in a given
+// order (flash_dkv.h). The others' is bound by waits that nothing fills: its accumulators and
+// operands leave one wave a SIMD. dQ, two waves a SIMD, is bound by the matrix cores (66% busy at
+// 16384 x 128) and LDS reads (32 rows per wave: 128 B/clk at full MFMA rate).
 // Measured, dK/dV + dQ + stats (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128:
-// 21.25 -> 7.90 ms (4932 + 2811 us); 2 x 4096: 2960 -> 1150 us; 2 x 3072, 16 heads (192, 128):
-// 1725 -> 489 us; 4 x 2048, 16/8 heads of 64: 616 -> 176 us; 2 x 4096, 16/8 heads of 256:
-// 5.99 -> 1.35 ms.
+// 8.04 -> 6.33 ms (dK/dV 5.45 -> 3.75); 2 x 4096: 1069 -> 870 us; 2 x 3001, 16 heads (192, 128):
+// 457 -> 396 us; 4 x 2048, 16/8 heads of 64: 176 us; 2 x 4096, 16/8 heads of 256: 1.35 ms.
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -82,6 +81,14 @@ struct BwdArgs {
   float scale;
   bool causal;
 };
+
+}  // namespace amd_ops
+
+#include "flash_dkv.h"
+
+namespace amd_ops {
+
+using namespace fa;
 
 template <int D>
 __device__ __forceinline__ void load_row_frags(bf16x8_t (&f)[D / 16], const bf16* row) {
@@ -437,6 +444,18 @@ static void launch_dkv(const BwdArgs& a, hipStream_t stream) {
   HIP_CHECK_KERNEL();
 }
 
+template <int DQK, int DV>
+static void launch_dkv_ordered(const BwdArgs& a, hipStream_t stream) {
+  const dim3 grid((unsigned)((long)((a.Skv + 127) / 128) * a.Hk * a.B));
+  if (a.doc_end)
+    hipLaunchKernelGGL((bwd_dkv_ordered_kernel<DQK, DV, true, BwdArgs>), grid, dim3(256),
+                       (DkvTile<DQK, DV>::SMEM), stream, a);
+  else
+    hipLaunchKernelGGL((bwd_dkv_ordered_kernel<DQK, DV, false, BwdArgs>), grid, dim3(256),
+                       (DkvTile<DQK, DV>::SMEM), stream, a);
+  HIP_CHECK_KERNEL();
+}
+
 template <int DQK, int DV, int WAVES, int OCC, bool PIPE>
 static void launch_dq(const BwdArgs& a, hipStream_t stream) {
   const long blocks = (long)((a.Sq + WAVES * 32 - 1) / (WAVES * 32)) * a.Hq * a.B;
@@ -489,15 +508,16 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
   const bf16* op = reinterpret_cast<const bf16*>(o.data_ptr());
 
   // Waves per SIMD and pipelining by what fits the registers and LDS; dK/dV need one wave a
-  // SIMD from head dim 96 on (at two a SIMD it spills: 1620 against 680 us at 2 x 4096, 32/8
-  // heads of 128). dQ of 128/128 at two waves a SIMD overlaps as well without the third K
+  // SIMD from head dim 96 on (at two a SIMD it spills), and for values of 128 columns there is
+  // the ordered kernel, whose tiles fit LDS. dQ of 128/128 at two waves a SIMD overlaps as well without the third K
   // buffer (379 against 392 us); (192, 128) would spill there (461 against 203 us).
   bool done = false;
 #define FA_BWD_CASE(A, C, KV_OCC, KV_PIPE, Q_OCC, Q_PIPE)                                 \
   if (!done && Dqk == A && Dv == C) {                                                     \
     done = true;                                                                          \
     launch_stats<C>(a, op, lse.data_ptr<float>(), stats.data_ptr<float>(), stream);       \
-    launch_dkv<A, C, 4, KV_OCC, KV_PIPE>(a, stream);                                      \
+    if constexpr (C == 128) launch_dkv_ordered<A, C>(a, stream);                          \
+    else launch_dkv<A, C, 4, KV_OCC, KV_PIPE>(a, stream);                                 \
     launch_dq<A, C, 4, Q_OCC, Q_PIPE>(a, stream);                                         \
   }
   FA_BWD_CASE(64, 64, 2, true, 2, true)
@@ -534,8 +554,7 @@ __global__ void mfma_probe_kernel(const bf16* a, const bf16* b, float* d) {
 
 // ---- ds_read_b64_tr_b16 layout probe: fill LDS with a linear pattern and
 // dump what each lane receives for reads at stride-8B lane addresses.
-// Guide T10: the gather is hardware-defined; verify on silicon before
-// building kernels on it (cdna_hip_programming.md §5.4 rule 27).
+// The gather is the hardware's: this shows what the kernels above rely on.
 __global__ void tr16_probe_kernel(const bf16* __restrict__ in, float* __restrict__ out,
                                   int n) {
   __shared__ __attribute__((aligned(16))) bf16 lds[2048];

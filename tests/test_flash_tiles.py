@@ -119,6 +119,36 @@ def test_backward(dims, sq, skv, causal, q_start, cuts, scale):
         assert (g.float() - r).norm() / r.norm() < BWD, name
 
 
+# dK and dV walk the tiles of all heads of a group from the last one on, four (128) or three
+# (192, 128) buffers in turn: fewer tiles than buffers, several rounds of them, short last tiles,
+# groups of one head and of four
+@pytest.mark.parametrize("dims", [(128, 128), (192, 128)])
+@pytest.mark.parametrize("heads", [(2, 2), (8, 2)])
+@pytest.mark.parametrize("sq,skv,causal,q_start,cuts", [
+    (64, 64, False, 0, None), (65, 65, True, 0, None), (200, 333, False, 0, None),
+    (1000, 1000, True, 0, None), (700, 1211, True, 511, None), (1088, 1088, True, 0, (300, 301, 650, 1000)),
+])
+def test_key_gradients_over_many_tiles(dims, heads, sq, skv, causal, q_start, cuts):
+    torch.manual_seed(0)
+    B = 2 if cuts is None else 1
+    q = torch.randn(B, sq, heads[0], dims[0], device="cuda").bfloat16()
+    k = torch.randn(B, skv, heads[1], dims[0], device="cuda").bfloat16()
+    v = torch.randn(B, skv, heads[1], dims[1], device="cuda").bfloat16()
+    do = torch.randn(B, sq, heads[0], dims[1], device="cuda").bfloat16()
+    scale = dims[0] ** -0.5
+    start, end = (None, None) if cuts is None else _docs(cuts, skv)
+    from automodel_amd.ops.attention import _FlashAttnHip
+
+    run = lambda: _grads(lambda *t: _FlashAttnHip.apply(*t, causal, scale, q_start, start, end), (q, k, v), do)
+    got = run()
+    ref = _grads(lambda *t: _reference(*t, causal, q_start, start, scale)[0],
+                 (q.float(), k.float(), v.float()), do.float())
+    for name, g, r in zip(("dq", "dk", "dv"), got, ref):
+        assert (g.float() - r).norm() / r.norm() < BWD, name
+    for first, again in zip(got, run()):        # the same bits
+        assert torch.equal(first, again)
+
+
 def test_document_bounds():
     from automodel_amd.ops.attention import doc_bounds_from_cu
 
