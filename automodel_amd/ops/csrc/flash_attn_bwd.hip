@@ -15,13 +15,13 @@
 // core forms the scores of the next half tile and adds the products of the previous one
 // (PIPE; three tiles of head dim 192/192 or 256 do not fit LDS: there two buffers, and the
 // phases follow one another).
-// dK/dV for values of 128 columns has a kernel of its own with its instructions in a given
-// order (flash_dkv.h). The others' is bound by waits that nothing fills: its accumulators and
-// operands leave one wave a SIMD. dQ, two waves a SIMD, is bound by the matrix cores (66% busy at
-// 16384 x 128) and LDS reads (32 rows per wave: 128 B/clk at full MFMA rate).
+// For values of 128 columns dK/dV, and dQ of long walks, have kernels of their own with their
+// instructions in a given order (flash_dkv.h, flash_dq.h). The others' dK/dV is bound by waits that
+// nothing fills: its accumulators and operands leave one wave a SIMD. dQ here, two waves a SIMD, is
+// bound by the matrix cores and LDS reads (32 rows per wave: 128 B/clk at full MFMA rate).
 // Measured, dK/dV + dQ + stats (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128:
-// 8.04 -> 6.33 ms (dK/dV 5.45 -> 3.75); 2 x 4096: 1069 -> 870 us; 2 x 3001, 16 heads (192, 128):
-// 457 -> 396 us; 4 x 2048, 16/8 heads of 64: 176 us; 2 x 4096, 16/8 heads of 256: 1.35 ms.
+// 8.04 -> 5.80 ms (dK/dV 5.45 -> 3.75, dQ 2.76 -> 2.3); 2 x 4096: 1069 -> 801 us; 2 x 3001, 16 heads
+// (192, 128): 457 -> 320 us; 4 x 2048, 16/8 heads of 64: 176 us; 2 x 4096, 16/8 heads of 256: 1.35 ms.
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -85,6 +85,7 @@ struct BwdArgs {
 }  // namespace amd_ops
 
 #include "flash_dkv.h"
+#include "flash_dq.h"
 
 namespace amd_ops {
 
@@ -422,6 +423,28 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void bwd_dq_kernel(const BwdArgs a
                   a.dq + (((long)b * a.Sq + q0) * a.Hq + h) * DQK, (long)a.Hq * DQK, a.Sq - q0);
 }
 
+// Which of the two for values of 128 columns. The ordered kernel has half the workgroups, one on a CU,
+// and more to do before its first product: it takes long walks, for 128 / 128 enough of them to fill
+// the chip. Whole backward, this one over the other: (192, 128): 0.85 at 2 x 3001 x 16 heads, 0.95 at 1024 to
+// 4096 x 8 to 16 heads, 1.0 to 1.02 at 512, 1.05 at 200; 128 / 128: 0.92 at 2 x 4096 x 32 heads, 0.96 at
+// 2 x 3001 x 16 (384 workgroups), with 256 of them 1.02 causal and 0.94 without a mask (2048 x 32 heads),
+// with 128 1.04 (4096 x 8 heads). Packed documents are short walks: dQ of 6001 tokens in 9 of them,
+// 16/8 heads: 77 us, 100 with the ordered kernel.
+template <int DQK, int DV>
+static bool dq_ordered(const BwdArgs& a) {
+  const long blocks = (long)((a.Sq + DqTile<DQK, DV>::BM - 1) / DqTile<DQK, DV>::BM) * a.Hq * a.B;
+  return !a.doc_start && a.Skv >= 1024 && (DQK == 192 || blocks >= (a.causal ? 384 : 256));
+}
+
+template <int DQK, int DV>
+static void launch_dq_ordered(const BwdArgs& a, hipStream_t stream) {
+  using T = DqTile<DQK, DV>;
+  hipLaunchKernelGGL((bwd_dq_ordered_kernel<DQK, DV, BwdArgs>),
+                     dim3((unsigned)((long)((a.Sq + T::BM - 1) / T::BM) * a.Hq * a.B)), dim3(256), T::SMEM,
+                     stream, a);
+  HIP_CHECK_KERNEL();
+}
+
 template <int DV>
 static void launch_stats(const BwdArgs& a, const bf16* o, const float* lse, float* stats,
                          hipStream_t stream) {
@@ -518,7 +541,12 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
     launch_stats<C>(a, op, lse.data_ptr<float>(), stats.data_ptr<float>(), stream);       \
     if constexpr (C == 128) launch_dkv_ordered<A, C>(a, stream);                          \
     else launch_dkv<A, C, 4, KV_OCC, KV_PIPE>(a, stream);                                 \
-    launch_dq<A, C, 4, Q_OCC, Q_PIPE>(a, stream);                                         \
+    bool ordered = false;                                                                 \
+    if constexpr (C == 128) {                                                             \
+      ordered = dq_ordered<A, C>(a);                                                      \
+      if (ordered) launch_dq_ordered<A, C>(a, stream);                                    \
+    }                                                                                     \
+    if (!ordered) launch_dq<A, C, 4, Q_OCC, Q_PIPE>(a, stream);                           \
   }
   FA_BWD_CASE(64, 64, 2, true, 2, true)
   FA_BWD_CASE(96, 96, 1, true, 2, true)

@@ -26,40 +26,10 @@
 // and conflicts in the reads of rows); 2 x 3001, 16 heads (192, 128): 283 -> 203 us.
 #pragma once
 
-#include "flash_tile.h"
-#include "gemm_tile.h"
+#include "flash_ordered.h"
 
 namespace amd_ops {
 namespace fa {
-
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-
-// The compiler does not know what these are (see gt::mfma): their results are read, and their
-// operands written by vector instructions, at least 16 MFMAs away.
-__device__ __forceinline__ void mfma_first(f32x4_t& d, bf16x8_t a, bf16x8_t b) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "a"(b));
-}
-__device__ __forceinline__ void mfma_first(f32x4_t& d, bf16x8_t a, bf16x8_t b, f32x4_t c) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %3" : "=&v"(d) : "v"(a), "a"(b), "v"(c));
-}
-__device__ __forceinline__ void mfma_next(f32x4_t& d, bf16x8_t a, bf16x8_t b) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "a"(b));
-}
-
-// the value is formed here, and not where the compiler would rather have it
-template <class T>
-__device__ __forceinline__ void here(T& x) { asm volatile("" : "+v"(x)); }
-
-// f(0), ..., f(N - 1) with compile-time arguments
-template <class F, int... I>
-__device__ __forceinline__ void unrolled_(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void unrolled(F&& f) {
-  unrolled_(f, std::make_integer_sequence<int, N>{});
-}
 
 template <int DQK, int DV>
 struct DkvTile {
@@ -69,12 +39,6 @@ struct DkvTile {
   // fragments of a step: rows of Q and dO, columns of dO and Q
   static constexpr int F1 = DQK / 16, F2 = F1 + DV / 16, F3 = F2 + DV / 16, F = F3 + DQK / 16;
   static_assert(DQK % 64 == 0 && DV % 64 == 0 && SMEM <= 160 * 1024, "whole tiles, 8 places for operands");
-  // The 16-byte slot of a row's chunk c is c ^ swz(row): no conflicts between the 32 bytes of 8 rows
-  // that meet in a read of columns, nor between the 16 lanes that meet in a read of rows, which are
-  // 8 rows' chunk c and the other 8 rows' chunk c ^ 1 (lanes 0-3, 12-15, 20-27 and so on).
-  static __device__ __forceinline__ int swz(int bytes, int row) {
-    return bytes % 256 == 0 ? (row & 7) << 1 : (row & 6);
-  }
 };
 
 template <int DQK, int DV, bool VARLEN, class Args>
@@ -139,12 +103,12 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_ordered_kernel(const Args a) {
 #pragma unroll
       for (int h = 0; h < DQK / 32; ++h) {
         const int c = (4 * h + wid) * 64 + lane, row = c / (DQK / 8), slot = c % (DQK / 8);
-        qoff[h] = (unsigned)min(row, have - 1) * (unsigned)(a.Hq * T::QR) + ((slot ^ T::swz(T::QR, row)) << 4);
+        qoff[h] = (unsigned)min(row, have - 1) * (unsigned)(a.Hq * T::QR) + ((slot ^ place(T::QR, row)) << 4);
       }
 #pragma unroll
       for (int h = 0; h < DV / 32; ++h) {
         const int c = (4 * h + wid) * 64 + lane, row = c / (DV / 8), slot = c % (DV / 8);
-        ooff[h] = (unsigned)min(row, have - 1) * (unsigned)(a.Hq * T::OR) + ((slot ^ T::swz(T::OR, row)) << 4);
+        ooff[h] = (unsigned)min(row, have - 1) * (unsigned)(a.Hq * T::OR) + ((slot ^ place(T::OR, row)) << 4);
       }
     };
     auto advance = [&]() {
@@ -188,16 +152,16 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_ordered_kernel(const Args a) {
     unsigned qr[DQK / 32], orow[DV / 32], oc[DV / 16], qc[DQK / 16];
     const int crow = 4 * g + (i16 >> 2), piece = (i16 & 3) >> 1;
 #pragma unroll
-    for (int s = 0; s < DQK / 32; ++s) qr[s] = lds + i16 * T::QR + (((4 * s + g) ^ T::swz(T::QR, i16)) << 4);
+    for (int s = 0; s < DQK / 32; ++s) qr[s] = lds + i16 * T::QR + (((4 * s + g) ^ place(T::QR, i16)) << 4);
 #pragma unroll
     for (int s = 0; s < DV / 32; ++s)
-      orow[s] = lds + QT + i16 * T::OR + (((4 * s + g) ^ T::swz(T::OR, i16)) << 4);
+      orow[s] = lds + QT + i16 * T::OR + (((4 * s + g) ^ place(T::OR, i16)) << 4);
 #pragma unroll
     for (int t = 0; t < DV / 16; ++t)
-      oc[t] = lds + QT + crow * T::OR + (((2 * t + piece) ^ T::swz(T::OR, crow)) << 4) + (i16 & 1) * 8;
+      oc[t] = lds + QT + crow * T::OR + (((2 * t + piece) ^ place(T::OR, crow)) << 4) + (i16 & 1) * 8;
 #pragma unroll
     for (int t = 0; t < DQK / 16; ++t)
-      qc[t] = lds + crow * T::QR + (((2 * t + piece) ^ T::swz(T::QR, crow)) << 4) + (i16 & 1) * 8;
+      qc[t] = lds + crow * T::QR + (((2 * t + piece) ^ place(T::QR, crow)) << 4) + (i16 & 1) * 8;
     unsigned sw = lds + QT + T::OT + 16 * g;     // statistics of the tile at hand
     unsigned nw = sw;                            // and of the tile whose rows are read
     typedef __attribute__((address_space(3))) f32x4_t* stat_ptr;
@@ -408,7 +372,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_ordered_kernel(const Args a) {
         bf16x4_t w;
 #pragma unroll
         for (int r = 0; r < 4; ++r) w[r] = (__bf16)(acc[t][k][r] * scale);
-        const int row = k * 16 + i16, ch = (2 * t + (g >> 1)) ^ T::swz(D * 2, row);
+        const int row = k * 16 + i16, ch = (2 * t + (g >> 1)) ^ place(D * 2, row);
         *reinterpret_cast<bf16x4_t*>(mine + row * D * 2 + (ch << 4) + (g & 1) * 8) = w;
       }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // a wave reads what it wrote itself
@@ -416,7 +380,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_ordered_kernel(const Args a) {
       const int row = c / CH, ch = c % CH;
       if (kv0 + row < a.Skv)
         *reinterpret_cast<uint4*>(dst + (long)row * a.Hk * D + ch * 8) =
-            *reinterpret_cast<const uint4*>(mine + row * D * 2 + ((ch ^ T::swz(D * 2, row)) << 4));
+            *reinterpret_cast<const uint4*>(mine + row * D * 2 + ((ch ^ place(D * 2, row)) << 4));
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };

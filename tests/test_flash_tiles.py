@@ -149,6 +149,33 @@ def test_key_gradients_over_many_tiles(dims, heads, sq, skv, causal, q_start, cu
         assert torch.equal(first, again)
 
 
+# dQ of long walks, three buffers in turn: workgroups of 256 (192 for keys of 192) rows of which the last
+# is short, short last key tiles, a diagonal that ends some waves of a workgroup early
+@pytest.mark.parametrize("dims", [(128, 128), (192, 128)])
+@pytest.mark.parametrize("B,heads,sq,skv,causal,q_start", [
+    (4, (32, 32), 257, 1024, False, 0), (4, (48, 16), 300, 1100, True, 800), (4, (32, 32), 200, 1281, True, 1081),
+    (3, (32, 8), 1030, 1030, True, 0), (1, (16, 16), 1, 1024, True, 1023),
+])
+def test_query_gradients_of_long_walks(dims, B, heads, sq, skv, causal, q_start):
+    torch.manual_seed(0)
+    q = torch.randn(B, sq, heads[0], dims[0], device="cuda").bfloat16()
+    k = torch.randn(B, skv, heads[1], dims[0], device="cuda").bfloat16()
+    v = torch.randn(B, skv, heads[1], dims[1], device="cuda").bfloat16()
+    do = torch.randn(B, sq, heads[0], dims[1], device="cuda").bfloat16()
+    scale = dims[0] ** -0.5
+    from automodel_amd.ops.attention import _FlashAttnHip
+
+    run = lambda: _grads(lambda *t: _FlashAttnHip.apply(*t, causal, scale, q_start, None, None), (q, k, v), do)
+    got = run()
+    for b in range(B):              # (the reference holds a score for every pair)
+        ref = _grads(lambda *t: _reference(*t, causal, q_start, None, scale)[0],
+                     [t[b : b + 1].float() for t in (q, k, v)], do[b : b + 1].float())
+        for name, g, r in zip(("dq", "dk", "dv"), got, ref):
+            assert (g[b : b + 1].float() - r).norm() / r.norm() < BWD, name
+    for first, again in zip(got, run()):        # the same bits
+        assert torch.equal(first, again)
+
+
 def test_document_bounds():
     from automodel_amd.ops.attention import doc_bounds_from_cu
 
