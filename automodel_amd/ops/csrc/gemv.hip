@@ -23,32 +23,10 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_stream.h"
 #include "ops_api.h"
 
 namespace amd_ops {
-
-typedef __bf16 gemv_bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 gemv_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float gemv_f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int MAX_SEGMENTS = 3;
-
-// What a launch computes: weights [n[s], K] whose blocks begin at first[s]. With a
-// gated product, w[0] and w[1] are gate and up and there is one output.
-struct Rows {
-  const bf16* x;
-  const bf16* w[MAX_SEGMENTS];
-  bf16* y[MAX_SEGMENTS];
-  int n[MAX_SEGMENTS];
-  int first[MAX_SEGMENTS];   // INT_MAX: no such segment
-  const bf16* bias;          // of a single weight
-  float* yf;                 // of a single weight: float32 output instead of y[0]
-  const bf16* res;           // of a single weight: added to y
-  bool relu2;                // max(y, 0)^2
-  int K;
-  int group_n;               // > 0: every group_n rows of w take the next B rows of x
-  bool stretches;            // skinny: a wave has consecutive tiles of K, else every WAVES-th
-};
 
 __device__ __forceinline__ float dot2(const bf16x8& a, const bf16x8& b, int j, float c) {
   const gemv_bf16x8 av = __builtin_bit_cast(gemv_bf16x8, a), bv = __builtin_bit_cast(gemv_bf16x8, b);
@@ -59,21 +37,6 @@ __device__ __forceinline__ float dot2(const bf16x8& a, const bf16x8& b, int j, f
 __device__ __forceinline__ bf16x8 load_stream(const bf16* p) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   return __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)));
-}
-
-__device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.f + __expf(-g)) * u; }
-
-// The segment of a block, by selection: an index into the arguments would be one more load
-// in the chain that every launch begins with.
-struct Segment {
-  const bf16* w;
-  bf16* y;
-  int n, first;
-};
-__device__ __forceinline__ Segment segment_of(const Rows& p, int block) {
-  const bool b1 = block >= p.first[1], b2 = block >= p.first[2];
-  return {b2 ? p.w[2] : b1 ? p.w[1] : p.w[0], b2 ? p.y[2] : b1 ? p.y[1] : p.y[0],
-          b2 ? p.n[2] : b1 ? p.n[1] : p.n[0], b2 ? p.first[2] : b1 ? p.first[1] : 0};
 }
 
 // A wave takes R rows of W, or with GLU one row of gate and the same of up, and
@@ -315,6 +278,74 @@ void launch_skinny(const Rows& rows, int segments, int B) {
       <<<dim3(blocks), dim3(WAVES * WAVE_SIZE), 0, c10::hip::getCurrentHIPStream()>>>(p, B);
 }
 
+template <int R, int D, int WAVES, bool GLU>
+void launch_stream(const Rows& rows, int segments, int B) {
+  Rows p = rows;
+  auto go = [&](auto xr) {
+    using S = Stream<R, decltype(xr)::value, D, WAVES, GLU>;
+    const int blocks = place(p, segments, S::OUT);
+    gemm_stream_kernel<R, decltype(xr)::value, D, WAVES, GLU>
+        <<<dim3(blocks), dim3(WAVES * WAVE_SIZE), S::SMEM, c10::hip::getCurrentHIPStream()>>>(p, B);
+  };
+  if (B <= 8) return go(std::integral_constant<int, 8>{});
+  go(std::integral_constant<int, 16>{});
+}
+
+// Rows of W a workgroup: the least of (rows + x) times the workgroups of the fullest CU, where x
+// stands for the loads of x and the workgroup's beginning and end; of more than one a CU, as far as
+// the others fill in for it, x counts otherwise and the fullest for 0.7. In us, 8 and 16 rows of
+// x, rows x columns of W:
+//  * 8 rows of W: 2048 x 4096 5.3 and 6.1, 16 rows 6.2 and 7.1
+//  * 24: 5120 x 4096 8.8 and 9.8, 16 rows 11.0 and 12.5, 32 rows 9.4 and 10.5
+//  * 32: 7168 x 14336 32.5 and 35.0, 16 rows 35.0 and 40.2
+//  * 40: 10240 x 8192 26.8 and 27.3, 24 rows 27.7 and 30.2, 64 rows 30.3 and 31.7
+//  * 56: 28672 x 4096 36.8 and 37.1, 32 rows 37.8 and 39.2
+// No multiples of 16 above 16 for rows of a multiple of 16 KB, whose channels they crowd (8192 x 8192,
+// 32 rows 25.6 and 26.0, 16 rows 21.5 and 23.8); nor many rows where rows of W are short, which leaves
+// too few waves (28672 x 1024, 16 rows 11.1 and 12.5, 64 rows 12.0 and 12.6; 18944 x 1024, 8.3 and
+// 9.4, 40 rows 10.4 and 11.3).
+// The ring: 8 waves where one workgroup has the CU to itself and rows are long (4096 x 4096 7.3 us,
+// 4 waves 7.8; 4096 x 2048 6.2, 4 waves 4.9), else 4; two slots, one from 48 rows (gate and up
+// of 14336 x 4096, 56 rows and 16 of x: 36.3 us, two slots 37.3) and where 32 rows have many workgroups
+// (28672 x 4096, 16 rows of x: 39.2 and 42.8).
+template <bool GLU>
+void stream(const Rows& p, int segments, int B) {
+  constexpr int CUS = 256;
+  const int x = B <= 8 ? 6 : 8, x_more = B <= 8 ? 4 : 12;
+  int best = 0, fullest = 0;
+  float least = 0.f;
+  for (int r : {8, 16, 24, 32, 40, 48, 56, 64}) {
+    const int out = GLU ? r / 2 : r;
+    if (r > 16 && ((p.group_n % out != 0) || (p.K % 8192 == 0 && r % 16 == 0) ||
+                   (r > 32 && p.K <= (B <= 8 ? 2048 : 1024))))
+      continue;
+    long blocks = 0;
+    for (int s = 0; s < segments; ++s) blocks += (p.n[s] + out - 1) / out;
+    const long full = (blocks + CUS - 1) / CUS;
+    float cost = (float)full * (r + x);
+    if (full > 1) cost = 0.7f * cost + 0.3f * ((float)blocks / CUS) * (r + x_more);
+    if (best && cost >= least) continue;
+    best = r;
+    least = cost;
+    fullest = (int)std::min(full, 1l << 20);
+  }
+  switch (best) {
+    case 8: return launch_stream<8, 3, 8, GLU>(p, segments, B);
+    case 16:
+      if (fullest == 1 && p.K >= 3072) return launch_stream<16, 2, 8, GLU>(p, segments, B);
+      if (fullest > 2 && p.K <= 2048) return launch_stream<16, 1, 4, GLU>(p, segments, B);
+      return launch_stream<16, 2, 4, GLU>(p, segments, B);
+    case 24: return launch_stream<24, 2, 4, GLU>(p, segments, B);
+    case 32:
+      if (fullest > 2) return launch_stream<32, 1, 4, GLU>(p, segments, B);
+      return launch_stream<32, 2, 4, GLU>(p, segments, B);
+    case 40: return launch_stream<40, 2, 4, GLU>(p, segments, B);
+    case 48: return launch_stream<48, 1, 4, GLU>(p, segments, B);
+    case 56: return launch_stream<56, 1, 4, GLU>(p, segments, B);
+    default: return launch_stream<64, 1, 4, GLU>(p, segments, B);
+  }
+}
+
 // Workgroups of 16, 32 or 64 rows of W, and 2, 4 or 8 waves in them. What decides is how many
 // tiles of 16 rows the fullest CU gets, with the rows of x that each workgroup loads besides;
 // a workgroup alone on its CU needs all the waves that fit, several share them. Small K has
@@ -339,6 +370,9 @@ void launch_skinny(const Rows& rows, int segments, int B) {
 void skinny(Rows p, int segments, int B, bool glu) {
   long n = 0;
   for (int s = 0; s < segments; ++s) n += p.n[s];
+  bool streams = B <= 16 && p.K % 128 == 0 && p.K < 1 << 25 && (uintptr_t)p.x % 16 == 0;
+  for (int s = 0; s < (glu ? 2 : segments); ++s) streams &= (uintptr_t)p.w[s] % 16 == 0;
+  if (streams) return glu ? stream<true>(p, segments, B) : stream<false>(p, segments, B);
   p.stretches = p.K % 2048 == 0 && (p.K <= 4096 || !(glu || B > 32)) &&
                 (p.K <= 2048 || n > 3072 || B <= 16 || glu);
   if (glu) {
