@@ -11,8 +11,8 @@
 // through exp, the matrix core forms the scores of i + 1 and the values of i - 1. Two waves
 // a SIMD, or two workgroups a CU, fill what one wave leaves. Bound by instruction issue (at
 // (128, 128) 96% of the cycles, the matrix core busy 45% and LDS 23% of them, before whole
-// tiles had a loop of their own). 64 rows per wave would halve the LDS reads, but the
-// accumulators leave too few registers: it spilled and ran at 100 TFLOP/s.
+// tiles had a loop of their own). Long walks of (128, 128) and (192, 128) without documents
+// have the kernel of flash_fwd.h.
 // Measured (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128: 6.52 -> 2.19 ms,
 // 1006 TFLOP/s; 2 x 4096: 1030 -> 289 us; 2 x 3072, 16 heads (192, 128): 414 -> 120 us;
 // 4 x 2048, 16/8 heads of 64: 154 -> 55 us; 2 x 4096, 8 heads of 256: 544 -> 207 us.
@@ -25,6 +25,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include "common.h"
+#include "flash_fwd.h"
 #include "flash_tile.h"
 #include "ops_api.h"
 
@@ -301,6 +302,55 @@ static void launch_fwd(const FwdArgs& a, hipStream_t stream) {
   HIP_CHECK_KERNEL();
 }
 
+template <int DQK, int DV, int N>
+static void launch_fwd_ordered(const FwdArgs& a, hipStream_t stream) {
+  using T = FwdTile<DQK, DV, N>;
+  const long blocks = (long)((a.Sq + T::BM - 1) / T::BM) * a.Hq * a.B;
+  hipLaunchKernelGGL((flash_fwd_ordered_kernel<DQK, DV, N, FwdArgs>), dim3((unsigned)blocks), dim3(256), T::SMEM,
+                     stream, a);
+  HIP_CHECK_KERNEL();
+}
+
+// Sixteens of rows a wave of the kernel in a given order, or 0: the one above. Times in us, the kernel above
+// first; batch x length, heads.
+//
+// (128, 128): a workgroup has 256 rows and a CU, against 128 and half of one. Without a mask it wants
+// full rounds of workgroups (1 x 8192, 8: 264 and 228; 8 x 1024, 32: 179 and 156; 2 x 1024, 32: 42.5 and
+// 42.3; but 1 x 5000, 32, two and a half rounds: 406 and 424; 4 x 512, 32: 27.5 and 28.6). With a causal
+// one, whose last tiles are wasted on most waves, long rows, and two rounds (1 x 8000, 16: 277 and 251;
+// 1 x 16384, 32: 2020 and 1843; but 2 x 6000, 16: 294 and 304; 1 x 8192, 8: 183 and 228).
+template <int N>
+static long ordered_blocks(const FwdArgs& a) { return (long)((a.Sq + 64 * N - 1) / (64 * N)) * a.Hq * a.B; }
+
+static int ordered_rows_128(const FwdArgs& a) {
+  const long blocks = ordered_blocks<4>(a), rounds = (blocks + 255) / 256;
+  if (a.causal) return a.Skv >= 8000 && blocks >= 512 ? 4 : 0;
+  return a.Skv >= 1024 && 8 * blocks >= 7 * 256 * rounds ? 4 : 0;
+}
+
+// (192, 128): 4 sixteens against 3, which take 0.77 of the time of 4: by rounds of workgroups without a
+// mask (2 x 3001, 16: 164 against 201; 2 x 2048, 16: 111 against 77), with a causal one by the longest
+// workgroup or all of them, what is more (2 x 3001, 16: 98 against 103; 1 x 8192, 16: 325 against 292).
+// The kernel above has 8 waves for 256 rows: it stays for short rows (1 x 100, 4: 9.1 and 12.8; without a
+// mask 4 x 512, 32: 32.7 and 33.9), and, where each workgroup has few tiles and wasted ones among them,
+// with a causal mask (16 x 1500, 32: 560 and 593; 2 x 1024, 32: 44.2 and 47.6; but 1 x 1024, 32, one
+// round: 41.5 and 34.6; 2 x 2048, 16: 72 and 57; 2 x 4096, 32: 356 and 338).
+static int ordered_rows_192(const FwdArgs& a) {
+  const long b4 = ordered_blocks<4>(a), b3 = ordered_blocks<3>(a);
+  if (!a.causal) {
+    if ((b3 + 255) / 256 * 0.77 < (double)((b4 + 255) / 256)) return a.Skv >= 512 ? 3 : 0;
+    return a.Skv >= 1024 ? 4 : 0;
+  }
+  const double longest = std::min<long>((long)a.q_start + a.Sq, a.Skv);
+  auto cost = [&](long blocks, int rows) {
+    const double first = std::min<long>((long)a.q_start + rows, a.Skv);
+    return std::max(longest, (double)blocks * (longest + first) / 512);
+  };
+  const double c4 = cost(b4, 256), c3 = cost(b3, 192) * 0.77;
+  if (a.Skv >= 3000) return c3 < c4 ? 3 : 4;
+  return (a.Skv >= 512 && b3 <= 256) || (a.Skv >= 2048 && c3 < 0.9 * c4) ? 3 : 0;
+}
+
 std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
     const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, double scale,
     bool causal, int64_t q_start, const std::optional<at::Tensor>& doc_start,
@@ -343,6 +393,13 @@ std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
   // (120 us; 4 waves at one a SIMD were 1.3 times slower); (192, 192) would spill at two a SIMD (457
   // against 178 us).
   bool done = false;
+  if (!varlen && Dv == 128 && (Dqk == 128 || Dqk == 192)) {
+    const int n = Dqk == 128 ? ordered_rows_128(a) : ordered_rows_192(a);
+    done = n > 0;
+    if (n > 0 && Dqk == 128) launch_fwd_ordered<128, 128, 4>(a, stream);
+    else if (n == 4) launch_fwd_ordered<192, 128, 4>(a, stream);
+    else if (n == 3) launch_fwd_ordered<192, 128, 3>(a, stream);
+  }
 #define FA_FWD_CASE(A, C, W, OCC)                             \
   if (!done && Dqk == A && Dv == C) {                         \
     done = true;                                              \

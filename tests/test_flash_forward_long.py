@@ -1,0 +1,88 @@
+"""The attention forward of long walks: ends of rows and keys, rows that see keys from the middle on,
+sinks, negative scales, and scores that leave what the first keys' maximum allows."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(q, k, v, scale, causal, q_start=0, sink=None):
+    from automodel_amd.ops._backend import hip_ops
+
+    out, lse = hip_ops().flash_attn_fwd(q, k, v, scale, causal, q_start, None, sink)
+    B, S, H, _ = q.shape
+    n, rep = k.shape[1], H // k.shape[2]
+    g = torch.Generator().manual_seed(1)
+    some = torch.randint(S, (96,), generator=g).tolist()
+    rows = torch.tensor(sorted({0, 1, S // 2, S - 2, S - 1, *some})).cuda().clamp(0, S - 1)
+    for b, h in {(0, 0), (B - 1, H - 1), (0, H // 2)}:
+        x, y = k[b, :, h // rep].double(), v[b, :, h // rep].double()
+        s = q[b, rows, h].double() @ x.t() * scale
+        if causal:
+            s = s.masked_fill(torch.arange(n, device="cuda") > (rows + q_start)[:, None], float("-inf"))
+        most = s.amax(-1, keepdim=True)
+        p = (s - most).exp()
+        total = p.sum(-1, keepdim=True)
+        if sink is not None:
+            total = total + (sink[h].double() - most).exp()
+        p = p / total
+        # the weights rounded once to bf16 and the output too: half a step of 8 significant bits,
+        # up to 2^-8 of the value, each. A float32 score is 2^-24 a
+        # product off its absolute sum, scale * log2(e) and the difference to the maximum once each
+        # of the score itself; so much relative to a weight is the error of all of them
+        of_score = (2.0**-24 * abs(scale) * (q.shape[-1] * (q[b, rows, h].double().abs() @ x.abs().t()))
+                    ).amax(-1, keepdim=True) + 2.0**-22 * s.masked_fill(p == 0, 0).abs().amax(-1, keepdim=True)
+        want, absolute = p @ y, p @ y.abs()
+        bound = (2.0**-8 + 2 * of_score + 2.0**-16) * absolute * 1.02 + 2.0**-8 * want.abs() + 1e-30
+        err = (out[b, rows, h].double() - want).abs()
+        assert (err <= bound).all(), (err / bound).max()
+        ref = (most + total.log()).squeeze(-1)
+        assert ((lse[b, h, rows].double() - ref).abs() <= 2 * of_score.squeeze(-1) + 2.0**-16
+                + 2.0**-22 * ref.abs()).all()
+
+
+def _inputs(B, S, n, H, K, D, seed=0):
+    g = torch.Generator("cuda").manual_seed(seed)
+    return tuple(torch.randn(B, m, h, d, generator=g, device="cuda").bfloat16()
+                 for m, h, d in ((S, H, D), (n, K, D), (n, K, 128)))
+
+
+@pytest.mark.parametrize("B,S,n,H,K,D,causal,start", [
+    (2, 1024, 1024, 32, 8, 128, False, 0),
+    (2, 997, 1500, 32, 8, 128, False, 0),
+    (64, 1, 1025, 4, 2, 128, False, 0),        # one row a workgroup
+    (1, 8000, 8000, 16, 4, 128, True, 0),
+    (1, 8001, 8003, 16, 4, 128, True, 2),
+    (1, 512, 512, 8, 8, 192, True, 0),         # 3 sixteens of rows
+    (2, 577, 577, 8, 8, 192, True, 0),
+    (1, 191, 1300, 8, 8, 192, True, 700),
+    (1, 600, 777, 16, 16, 192, False, 0),
+    (2, 3001, 3001, 16, 16, 192, True, 0),
+    (1, 8192, 8192, 16, 16, 192, True, 0),     # 4 of them
+    (2, 2047, 2050, 16, 16, 192, False, 0),
+])
+def test_long_walks(B, S, n, H, K, D, causal, start):
+    q, k, v = _inputs(B, S, n, H, K, D)
+    _check(q, k, v, D**-0.5, causal, start)
+
+
+@pytest.mark.parametrize("D,n,H", [(192, 700, 8), (128, 1100, 64)])
+def test_sink_and_negative_scale(D, n, H):
+    q, k, v = _inputs(1, n, n, H, H, D, 2)
+    _check(q, k, v, -0.3, False, sink=torch.randn(H, device="cuda").bfloat16() * 4)
+    _check(q, k, v, -0.3, D == 192, sink=torch.randn(H, device="cuda").bfloat16() * 4)
+
+
+@pytest.mark.parametrize("D,H", [(192, 8), (128, 64)])
+@pytest.mark.parametrize("kind", ["ramp", "late", "early", "first"])
+def test_scores_far_above_the_first_ones(D, H, kind):
+    n = 1024
+    q, k, v = _inputs(1, n, n, H, H, D, 3)
+    at = torch.arange(n, device="cuda")[:, None, None]
+    factor = {"ramp": at / 16.0, "late": torch.where(at == 1000, 200.0, 1.0),
+              "early": torch.where(at == 40, 200.0, 1.0), "first": torch.where(at == 3, 200.0, 1.0)}[kind]
+    k = (k.float() * factor).bfloat16()
+    _check(q, k, v, D**-0.5, False)
+    if D == 192:
+        _check(q, k, v, D**-0.5, True)
