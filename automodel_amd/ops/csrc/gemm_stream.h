@@ -9,6 +9,7 @@
 #pragma once
 
 #include "common.h"
+#include "lds_load.h"
 
 namespace amd_ops {
 
@@ -69,11 +70,6 @@ struct Stream {
   static_assert(SMEM <= 160 * 1024);
 };
 
-template <int LEFT>
-__device__ __forceinline__ void wait_loads() {
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(LEFT) : "memory");
-}
-
 // K % 128 == 0; x and W on 16 bytes; 128 K below 2^32
 template <int R, int XR, int D, int WAVES, bool GLU>
 __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_stream_kernel(const Rows p, int B) {
@@ -110,17 +106,12 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_stream_kernel(const Ro
   const char* w1 = GLU ? reinterpret_cast<const char*>(p.w[1] + (long)n0 * K) + at0 : nullptr;
 
   char* ring = stream_lds + wid * D * S::SLOT;
-  const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+  const unsigned lds = fa::lds_address(ring);
   auto fetch = [&](unsigned to) {
 #pragma unroll
     for (int j = 0; j < S::LOADS; ++j) {
-      if (j < R / 4)
-        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
-                     :: "s"(to), "v"(off[j]), "s"(GLU && j >= R / 8 ? w1 : w0), "n"(j * 1024)
-                     : "memory", "m0", "scc");
-      else
-        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     :: "s"(to), "v"(off[j]), "s"(xp), "n"(j * 1024) : "memory", "m0", "scc");
+      if (j < R / 4) fa::load_lds16_once(to + j * 1024, GLU && j >= R / 8 ? w1 : w0, off[j]);
+      else fa::load_lds16(to + j * 1024, xp, off[j]);
     }
     const long on = (++turn == count ? 1 - count : 1) * 256l;
     w0 += on;
@@ -137,9 +128,9 @@ __global__ __launch_bounds__(WAVES * WAVE_SIZE) void gemm_stream_kernel(const Ro
   int slot = 0;
   for (int i = 0; i < count; ++i) {
     const int left = count - 1 - i;               // tiles after this one; up to D - 1 are in flight
-    if (D == 1 || left == 0) wait_loads<0>();
-    else if (D == 2 || left == 1) wait_loads<S::LOADS>();
-    else wait_loads<2 * S::LOADS>();
+    if (D == 1 || left == 0) fa::wait_loads<0>();
+    else if (D == 2 || left == 1) fa::wait_loads<S::LOADS>();
+    else fa::wait_loads<2 * S::LOADS>();
     const char* at = ring + slot * S::SLOT;
     gemv_bf16x8 xv[4], wv[4][S::RT];
 #pragma unroll

@@ -50,10 +50,9 @@ __device__ __forceinline__ void mfma(f32x4_t& d, bf16x8_t a, bf16x8_t b) {
 }
 __device__ __forceinline__ void settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
-// 16 bytes a lane to the LDS address lds + to, a constant
+// 16 bytes a lane to the LDS address lds + to
 __device__ __forceinline__ void load_lds(unsigned lds, int to, unsigned off, const char* base) {
-  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds), "v"(off), "s"(base), "n"(to) : "memory", "m0", "scc");
+  fa::load_lds16(lds + to, base, off);
 }
 
 // What a block multiplies: pointers to the tile's first row and column and the sum's

@@ -19,6 +19,11 @@ __device__ __forceinline__ void load_lds16(unsigned lds, const void* base, unsig
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :: "s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
+// the same of data that is read once: it leaves no trace in the caches
+__device__ __forceinline__ void load_lds16_once(unsigned lds, const void* base, unsigned off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+               :: "s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
 // the same from an address of the lane's own
 __device__ __forceinline__ void load_lds16(unsigned lds, const void* mine) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
