@@ -101,7 +101,9 @@ def _unseen(lin: nn.Linear) -> bool:
 def linear(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """``lin(x)``. Plain bf16 layers without a bias on the GPU that are large enough take the
     kernels in their backward, everything else is the module's call."""
-    if (type(lin) is nn.Linear and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda
+    # (the size first: small layers are bound by the host)
+    if (type(lin) is nn.Linear and x.numel() * lin.out_features >= MIN_PRODUCTS
+            and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda
             and x.dtype == torch.bfloat16 and torch.is_grad_enabled() and lin.bias is None):
         w = lin.weight
         if (type(w) is nn.Parameter and w.dim() == 2 and x.shape[-1:] == w.shape[1:]
