@@ -13,9 +13,9 @@
 // (128, 128) 96% of the cycles, the matrix core busy 45% and LDS 23% of them, before whole
 // tiles had a loop of their own). Long walks of (128, 128) and (192, 128) without documents
 // have the kernel of flash_fwd.h.
-// Measured (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128: 6.52 -> 2.19 ms,
-// 1006 TFLOP/s; 2 x 4096: 1030 -> 289 us; 2 x 3072, 16 heads (192, 128): 414 -> 120 us;
-// 4 x 2048, 16/8 heads of 64: 154 -> 55 us; 2 x 4096, 8 heads of 256: 544 -> 207 us.
+// Measured (causal, bf16, before -> now): 1 x 16384, 32/8 heads of 128: 6.52 -> 2.02 ms,
+// 1090 TFLOP/s (there flash_fwd.h takes 1.84); 2 x 4096: 1030 -> 289 us; 2 x 3072, 16 heads
+// (192, 128): 414 -> 120 us; 4 x 2048, 16/8 heads of 64: 154 -> 55 us; 2 x 4096, 8 heads of 256: 544 -> 207 us.
 //
 // Varlen: per-token doc_start gates the causal mask to the query's own document; tiles
 // before a block's first document are skipped.

@@ -5,7 +5,7 @@
 // wave takes a row of W and its lanes run along K; above that the matrix cores
 // take 16 rows of W against 16 rows of x per instruction, since a dot product
 // per row of x would cost more than the load (4 rows, 14336 x 4096: 27 us against
-// 21 us). Weight loads leave no trace in the caches (nontemporal): a model's weights are gone
+// 21 us), to 16 rows with the kernel of gemm_stream.h where K % 128 == 0. Weight loads leave no trace in the caches (nontemporal): a model's weights are gone
 // from them before its next step (5 rows, 2048 x 2048: 4.7 us, 5.0 through the caches). Weights of
 // a model that the last-level cache could hold pay for it (16 rows, 1024 x 4096: 7.7 and 6.2).
 //
@@ -350,7 +350,7 @@ void stream(const Rows& p, int segments, int B) {
 // tiles of 16 rows the fullest CU gets, with the rows of x that each workgroup loads besides;
 // a workgroup alone on its CU needs all the waves that fit, several share them. Small K has
 // tiles for few waves. Times in us for rows x columns of W, weights from memory:
-//  * up to 16 rows of x: 16 rows of W, 8 waves (4096 x 4096 7.7, 4 waves 9.1; 10240 x 8192 29.6
+//  * up to 16 rows of x (K % 128 != 0 or not on 16 bytes): 16 rows of W, 8 waves (4096 x 4096 7.7, 4 waves 9.1; 10240 x 8192 29.6
 //    and 34.7), 4 with more workgroups than two a CU and short rows (9216 x 2048 9.2, 8 waves 9.9);
 //    32 rows between one and one and a half workgroups a CU (5120 x 5120 12.4, 16 rows 13.5; but
 //    8192 x 8192 24.5 and 23.0), and for many rows of x and of W (16 rows, 32000 x 2048 22.8 and 24.8).
@@ -361,7 +361,7 @@ void stream(const Rows& p, int segments, int B) {
 //    64 rows (48 rows, 9216 x 2048 17.8, 32 rows 19.4; 8192 x 8192 40.6, 16 rows 50.1; 10240 x 8192
 //    55.4, 16 rows 61.0; 32000 x 2048 35.2, 32 rows 41.5).
 //
-// Waves read neighbouring tiles of K, or a stretch of K each where rows of W lie a multiple of
+// Waves of this kernel read neighbouring tiles of K, or a stretch of K each where rows of W lie a multiple of
 // 4 KB apart (8 rows of x, neighbours and stretches: 4096 x 2048 6.6 and 6.0 us, 6144 x 4096
 // 13.0 and 11.1, 6144 x 8192 22.6 and 19.0; but 4096 x 2560 0.97 to 1, 22016 x 5120 the same).
 // Not with more than 4096 columns where a wave's tile has 32 rows of W or more than 32 rows of x
