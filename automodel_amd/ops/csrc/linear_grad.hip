@@ -56,7 +56,8 @@ at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t c
               "linear_grad: contiguous bf16 operands on one GPU");
   TORCH_CHECK((uintptr_t)r.data_ptr() % 16 == 0 && (uintptr_t)c.data_ptr() % 16 == 0,
               "linear_grad: operands at multiples of 16 bytes");
-  TORCH_CHECK(std::max({rows, cols, sum}) < (1l << 24), "linear_grad: sizes below 2^24");
+  // a tile's addresses are 32 bits: 256 rows of 2^23
+  TORCH_CHECK(std::max({rows, cols, sum}) < (1l << 23), "linear_grad: sizes below 2^23");
   const c10::DeviceGuard guard(r.device());
   auto out = at::empty({rows, cols}, r.options());
   if (out.numel() == 0) return out;

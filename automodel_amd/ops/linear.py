@@ -19,6 +19,8 @@ TILE, CUS = 256, 256
 # below this many products a layer's backward takes the library some 80 us, and an autograd
 # function of Python's costs the host as much as is gained
 MIN_PRODUCTS = 1 << 34
+# the kernels' addresses within a tile are 32 bits
+MAX_SIZE = 1 << 23
 
 
 def _fills(rows: int, cols: int, share: float) -> bool:
@@ -32,13 +34,15 @@ def weight_grad_wins(T: int, N: int, K: int) -> bool:
     share of the rounds that the tiles fill: 1.0 at 0.67 to 0.81 (10240 x 2560, 2000 to 8192
     rows: 400 tiles, 0.78, 0.66 to 0.74), 0.83 to 0.95 at 0.75 (6144 x 4096, 384 tiles),
     1.1 to 1.2 at 0.5, 1.3 to 1.7 at 0.25; 200 to 8192 rows alike."""
-    return T * N * K >= MIN_PRODUCTS and N % 8 == 0 and K % 8 == 0 and _fills(N, K, 0.75)
+    return (max(T, N, K) < MAX_SIZE and T * N * K >= MIN_PRODUCTS and N % 8 == 0 and K % 8 == 0
+            and _fills(N, K, 0.75))
 
 
 def input_grad_wins(T: int, N: int, K: int) -> bool:
     """Kernel or library for g w, g [T, N], w [N, K]: 0.85 to 0.91 of the library's time where
     the tiles fill the rounds, 0.96 to 1.02 at 0.75, 1.0 to 1.2 at 0.5."""
-    return T * N * K >= MIN_PRODUCTS and N % 64 == 0 and K % 8 == 0 and _fills(T, K, 0.875)
+    return (max(T, N, K) < MAX_SIZE and T * N * K >= MIN_PRODUCTS and N % 64 == 0 and K % 8 == 0
+            and _fills(T, K, 0.875))
 
 
 def _plain(*ts: torch.Tensor) -> bool:

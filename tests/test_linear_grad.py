@@ -156,3 +156,9 @@ def test_rule():
     assert not L.weight_grad_wins(8192, 4100, 4096) and not L.weight_grad_wins(8192, 4096, 4092)
     assert L.input_grad_wins(8192, 6144, 4096) and not L.input_grad_wins(6001, 4096, 4096)
     assert not L.input_grad_wins(8192, 6176, 4096) and not L.input_grad_wins(8192, 4096, 4100)
+
+
+def test_sizes_beyond_the_kernels_addresses():
+    for T, N, K in ((1 << 23, 4096, 4096), (8192, 1 << 23, 4096), (8192, 4096, 1 << 23)):
+        assert not L.weight_grad_wins(T, N, K) and not L.input_grad_wins(T, N, K)
+    assert L.weight_grad_wins((1 << 23) - 1, 4096, 4096) and L.input_grad_wins(8192, (1 << 23) - 64, 4096)
