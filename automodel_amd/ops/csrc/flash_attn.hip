@@ -318,11 +318,13 @@ static void launch_fwd_ordered(const FwdArgs& a, hipStream_t stream) {
 // full rounds of workgroups (1 x 8192, 8: 264 and 228; 8 x 1024, 32: 179 and 156; 2 x 1024, 32: 42.5 and
 // 42.3; but 1 x 5000, 32, two and a half rounds: 406 and 424; 4 x 512, 32: 27.5 and 28.6). With a causal
 // one, whose last tiles are wasted on most waves, long rows, and two rounds (1 x 8000, 16: 277 and 251;
-// 1 x 16384, 32: 2020 and 1843; but 2 x 6000, 16: 294 and 304; 1 x 8192, 8: 183 and 228).
+// 1 x 16384, 32: 2020 and 1843; but 2 x 6000, 16: 294 and 304; 1 x 8192, 8: 183 and 228). Few queries
+// leave its waves empty rows (8 x 64 of 4096 keys, 32: 102 and 134).
 template <int N>
 static long ordered_blocks(const FwdArgs& a) { return (long)((a.Sq + 64 * N - 1) / (64 * N)) * a.Hq * a.B; }
 
 static int ordered_rows_128(const FwdArgs& a) {
+  if (a.Sq < 1024) return 0;
   const long blocks = ordered_blocks<4>(a), rounds = (blocks + 255) / 256;
   if (a.causal) return a.Skv >= 8000 && blocks >= 512 ? 4 : 0;
   return a.Skv >= 1024 && 8 * blocks >= 7 * 256 * rounds ? 4 : 0;
@@ -334,8 +336,10 @@ static int ordered_rows_128(const FwdArgs& a) {
 // The kernel above has 8 waves for 256 rows: it stays for short rows (1 x 100, 4: 9.1 and 12.8; without a
 // mask 4 x 512, 32: 32.7 and 33.9), and, where each workgroup has few tiles and wasted ones among them,
 // with a causal mask (16 x 1500, 32: 560 and 593; 2 x 1024, 32: 44.2 and 47.6; but 1 x 1024, 32, one
-// round: 41.5 and 34.6; 2 x 2048, 16: 72 and 57; 2 x 4096, 32: 356 and 338).
+// round: 41.5 and 34.6; 2 x 2048, 16: 72 and 57; 2 x 4096, 32: 356 and 338); and for fewer queries than a
+// workgroup's (8 x 64 of 4096 keys, 32: 119 and 129; 1 x 192 of 8192, 16: 239 and 189).
 static int ordered_rows_192(const FwdArgs& a) {
+  if (a.Sq < 192) return 0;
   const long b4 = ordered_blocks<4>(a), b3 = ordered_blocks<3>(a);
   if (!a.causal) {
     if ((b3 + 255) / 256 * 0.77 < (double)((b4 + 255) / 256)) return a.Skv >= 512 ? 3 : 0;

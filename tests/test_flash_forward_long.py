@@ -51,12 +51,13 @@ def _inputs(B, S, n, H, K, D, seed=0):
 @pytest.mark.parametrize("B,S,n,H,K,D,causal,start", [
     (2, 1024, 1024, 32, 8, 128, False, 0),
     (2, 997, 1500, 32, 8, 128, False, 0),
-    (64, 1, 1025, 4, 2, 128, False, 0),        # one row a workgroup
+    (64, 1025, 1025, 4, 2, 128, False, 0),     # one row in the last workgroups
     (1, 8000, 8000, 16, 4, 128, True, 0),
     (1, 8001, 8003, 16, 4, 128, True, 2),
     (1, 512, 512, 8, 8, 192, True, 0),         # 3 sixteens of rows
     (2, 577, 577, 8, 8, 192, True, 0),
-    (1, 191, 1300, 8, 8, 192, True, 700),
+    (1, 193, 1300, 8, 8, 192, True, 700),
+    (1, 191, 1300, 8, 8, 192, True, 700),      # (the other kernel)
     (1, 600, 777, 16, 16, 192, False, 0),
     (2, 3001, 3001, 16, 16, 192, True, 0),
     (1, 8192, 8192, 16, 16, 192, True, 0),     # 4 of them
