@@ -433,7 +433,14 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void bwd_dq_kernel(const BwdArgs a
 template <int DQK, int DV>
 static bool dq_ordered(const BwdArgs& a) {
   const long blocks = (long)((a.Sq + DqTile<DQK, DV>::BM - 1) / DqTile<DQK, DV>::BM) * a.Hq * a.B;
-  return !a.doc_start && a.Skv >= 1024 && (DQK == 192 || blocks >= (a.causal ? 384 : 256));
+  return !a.doc_start && a.Skv >= 1024 && a.Sq >= DqTile<DQK, DV>::BM && (DQK == 192 || blocks >= (a.causal ? 384 : 256));
+}
+
+// The ordered dK/dV of 128 columns, but for walks of a few tiles of queries, where what a workgroup does
+// before and after them counts (whole backward, this one over the other, keys 2048 to 4096: 1.09
+// and 1.12 at 16 and 64 queries of 8 x 32 heads, 1.04 and 1.07 at 100 of 16 x 16, the same at 192).
+static bool dkv_ordered(const BwdArgs& a) {
+  return a.doc_end || (long)a.Sq * (a.Hq / a.Hk) >= 192;
 }
 
 template <int DQK, int DV>
@@ -532,16 +539,20 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
 
   // Waves per SIMD and pipelining by what fits the registers and LDS; dK/dV need one wave a
   // SIMD from head dim 96 on (at two a SIMD it spills), and for values of 128 columns there is
-  // the ordered kernel, whose tiles fit LDS. dQ of 128/128 at two waves a SIMD overlaps as well without the third K
+  // the ordered kernel, whose tiles fit LDS, for all but the shortest walks. dQ of 128/128 at two waves a SIMD overlaps as well without the third K
   // buffer (379 against 392 us); (192, 128) would spill there (461 against 203 us).
   bool done = false;
 #define FA_BWD_CASE(A, C, KV_OCC, KV_PIPE, Q_OCC, Q_PIPE)                                 \
   if (!done && Dqk == A && Dv == C) {                                                     \
     done = true;                                                                          \
     launch_stats<C>(a, op, lse.data_ptr<float>(), stats.data_ptr<float>(), stream);       \
-    if constexpr (C == 128) launch_dkv_ordered<A, C>(a, stream);                          \
-    else launch_dkv<A, C, 4, KV_OCC, KV_PIPE>(a, stream);                                 \
     bool ordered = false;                                                                 \
+    if constexpr (C == 128) {                                                             \
+      ordered = dkv_ordered(a);                                                           \
+      if (ordered) launch_dkv_ordered<A, C>(a, stream);                                   \
+    }                                                                                     \
+    if (!ordered) launch_dkv<A, C, 4, KV_OCC, KV_PIPE>(a, stream);                        \
+    ordered = false;                                                                      \
     if constexpr (C == 128) {                                                             \
       ordered = dq_ordered<A, C>(a);                                                      \
       if (ordered) launch_dq_ordered<A, C>(a, stream);                                    \
