@@ -303,7 +303,7 @@ void launch_stream(const Rows& rows, int segments, int B) {
 // No multiples of 16 above 16 for rows of a multiple of 16 KB, whose channels they crowd (8192 x 8192,
 // 32 rows 25.6 and 26.0, 16 rows 21.5 and 23.8); nor many rows where rows of W are short, which leaves
 // too few waves (28672 x 1024, 16 rows 11.1 and 12.5, 64 rows 12.0 and 12.6; 18944 x 1024, 8.3 and
-// 9.4, 40 rows 10.4 and 11.3).
+// 9.4, 40 rows 10.4 and 11.3; 16 rows of x, 16384 x 128, 16 rows 3.3, 32 rows 4.8).
 // The ring: 8 waves where one workgroup has the CU to itself and rows are long (4096 x 4096 7.3 us,
 // 4 waves 7.8; 4096 x 2048 6.2, 4 waves 4.9), else 4; two slots, one from 48 rows (gate and up
 // of 14336 x 4096, 56 rows and 16 of x: 36.3 us, two slots 37.3) and where 32 rows have many workgroups
@@ -317,7 +317,7 @@ void stream(const Rows& p, int segments, int B) {
   for (int r : {8, 16, 24, 32, 40, 48, 56, 64}) {
     const int out = GLU ? r / 2 : r;
     if (r > 16 && ((p.group_n % out != 0) || (p.K % 8192 == 0 && r % 16 == 0) ||
-                   (r > 32 && p.K <= (B <= 8 ? 2048 : 1024))))
+                   p.K < 1024 || (r > 32 && p.K <= (B <= 8 ? 2048 : 1024))))
       continue;
     long blocks = 0;
     for (int s = 0; s < segments; ++s) blocks += (p.n[s] + out - 1) / out;
