@@ -90,13 +90,12 @@ class _Linear(torch.autograd.Function):
 
 def _unseen(lin: nn.Linear) -> bool:
     """No hook sees the module's call or its gradients, and nothing follows the operations
-    (transforms, forward-mode derivatives, tracing, dispatch modes) but autograd."""
+    (transforms, forward-mode derivatives, dispatch modes) but autograd."""
     every = nn.modules.module
     return not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks
                 or lin._backward_pre_hooks or every._global_forward_hooks
                 or every._global_forward_pre_hooks or every._global_backward_hooks
-                or every._global_backward_pre_hooks or torch.compiler.is_compiling()
-                or torch.jit.is_tracing() or torch.is_autocast_enabled("cuda")
+                or every._global_backward_pre_hooks or torch.is_autocast_enabled("cuda")
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or forward_ad._current_level >= 0
                 or _python_dispatch._get_current_dispatch_mode() is not None)
@@ -105,10 +104,12 @@ def _unseen(lin: nn.Linear) -> bool:
 def linear(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """``lin(x)``. Plain bf16 layers without a bias on the GPU that are large enough take the
     kernels in their backward, everything else is the module's call."""
-    # (the size first: small layers are bound by the host)
-    if (type(lin) is nn.Linear and x.numel() * lin.out_features >= MIN_PRODUCTS
-            and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda
-            and x.dtype == torch.bfloat16 and torch.is_grad_enabled() and lin.bias is None):
+    # Traced calls first: a size that is looked at there becomes a condition of what was traced.
+    # Then the size: small layers are bound by the host.
+    if (not torch.compiler.is_compiling() and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda
+            and x.dtype == torch.bfloat16 and not torch.jit.is_tracing() and type(lin) is nn.Linear
+            and x.numel() * lin.out_features >= MIN_PRODUCTS
+            and torch.is_grad_enabled() and lin.bias is None):
         w = lin.weight
         if (type(w) is nn.Parameter and w.dim() == 2 and x.shape[-1:] == w.shape[1:]
                 and w.dtype == x.dtype and w.device == x.device and x.numel() > 0):

@@ -1,0 +1,64 @@
+"""Layers whose linears may take kernels of their own, exported, compiled and scripted: the number of
+rows stays free, as torch's own layers have it."""
+
+import pytest
+import torch
+import torch.nn as nn
+from torch._dynamo.testing import CompileCounter
+from torch.export import Dim, export
+
+from automodel_amd.models.common.backend import BackendConfig
+from automodel_amd.models.llama.model import LlamaConfig, LlamaForCausalLM, LlamaMLP
+from automodel_amd.moe.layers import SharedExpert
+from automodel_amd.ops import linear as ops_linear
+from automodel_amd.peft.lora import LinearLoRA
+
+
+def _config(**kw):
+    return LlamaConfig(**{**dict(vocab_size=64, hidden_size=32, intermediate_size=64, num_hidden_layers=1,
+                                 num_attention_heads=2, num_key_value_heads=2, head_dim=16,
+                                 max_position_embeddings=8192), **kw})
+
+
+def _layer(kind, width, inter):
+    if kind == "shared":
+        return SharedExpert(width, inter)
+    if kind == "mlp":
+        return LlamaMLP(_config(hidden_size=width, intermediate_size=inter), BackendConfig())
+    return LinearLoRA(nn.Linear(width, inter, bias=False), 4, 8.0)
+
+
+@pytest.mark.parametrize("kind", ["shared", "mlp", "lora"])
+@pytest.mark.parametrize("strict", [False, True])
+@pytest.mark.parametrize("dim", [Dim("t"), Dim("t", max=4096), Dim.AUTO], ids=["free", "bounded", "auto"])
+def test_export_leaves_the_rows_free(kind, strict, dim):
+    layer = _layer(kind, 16, 32)
+    program = export(layer, (torch.randn(8, 16),), dynamic_shapes=(({0: dim}),), strict=strict)
+    (bounds,) = program.range_constraints.values()
+    assert bounds.upper >= 4096 and (dim is not Dim.AUTO or bounds.upper > 1 << 40)
+    x = torch.randn(700, 16)
+    assert torch.equal(program.module()(x), layer(x))
+
+
+@pytest.mark.parametrize("strict", [False, True])
+def test_export_of_a_model(monkeypatch, strict):
+    monkeypatch.setattr(ops_linear, "MIN_PRODUCTS", 1 << 16)      # 32 rows of the MLP
+    model = LlamaForCausalLM(_config(), backend=BackendConfig().for_cpu())
+    ids = torch.zeros(1, 8, dtype=torch.long)
+    program = export(model, (ids,), dynamic_shapes=({1: Dim("s", max=4096)},), strict=strict)
+    assert max(b.upper for b in program.range_constraints.values()) >= 4096
+    ids = torch.randint(64, (1, 100))
+    torch.testing.assert_close(program.module()(ids), model(ids))
+
+
+@pytest.mark.parametrize("kind", ["shared", "mlp", "lora"])
+@pytest.mark.parametrize("dynamic,graphs", [(True, 1), (None, 2)])
+def test_compiled_once_for_all_lengths(kind, dynamic, graphs):
+    torch._dynamo.reset()
+    # 16 and 2400 rows lie on both sides of MIN_PRODUCTS
+    layer, count = _layer(kind, 512, 14336), CompileCounter()
+    compiled = torch.compile(layer, backend=count, dynamic=dynamic)
+    for rows in (8, 16, 100, 1200, 2400):
+        x = torch.randn(rows, 512)
+        torch.testing.assert_close(compiled(x), layer(x))
+    assert count.frame_count == graphs
