@@ -192,8 +192,11 @@ class SharedExpert(nn.Module):
         self.down_proj = nn.Linear(intermediate, hidden_size, bias=False)
 
     def forward(self, x):
-        return linear(self.down_proj,
-                      swiglu(linear(self.gate_proj, x), linear(self.up_proj, x)))
+        if torch.jit.is_scripting():          # (a module is no argument there)
+            return self.down_proj(swiglu(self.gate_proj(x), self.up_proj(x)))
+        else:
+            return linear(self.down_proj,
+                          swiglu(linear(self.gate_proj, x), linear(self.up_proj, x)))
 
 
 _SHARED_STREAMS: dict = {}

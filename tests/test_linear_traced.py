@@ -62,3 +62,8 @@ def test_compiled_once_for_all_lengths(kind, dynamic, graphs):
         x = torch.randn(rows, 512)
         torch.testing.assert_close(compiled(x), layer(x))
     assert count.frame_count == graphs
+
+
+def test_script():
+    layer, x = SharedExpert(16, 32), torch.randn(3, 16)
+    assert torch.equal(torch.jit.script(layer)(x), layer(x))
