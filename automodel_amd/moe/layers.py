@@ -13,7 +13,7 @@ import torch.nn as nn
 
 from automodel_amd.moe.config import MoEConfig
 from automodel_amd.moe.experts import GroupedExperts, check_experts
-from automodel_amd.ops._backend import ops_available
+from automodel_amd.ops._backend import followed, ops_available
 from automodel_amd.ops.linear import linear
 from automodel_amd.ops.swiglu import swiglu
 
@@ -22,11 +22,8 @@ def _device_op(name: str, t: torch.Tensor):
     """The kernel of that name for an ordinary GPU tensor in an eager call, else None: traced,
     transformed and mode-wrapped calls stay with torch's own operations, which those can see
     into, and so does a build of the inference kernels alone."""
-    if not (t.is_cuda and type(t) in (torch.Tensor, nn.Parameter)
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and not torch._C._are_functorch_transforms_active()
-            and torch.autograd.forward_ad._current_level < 0
-            and not torch._C._len_torch_dispatch_stack() and ops_available()):
+    if not (t.is_cuda and type(t) in (torch.Tensor, nn.Parameter) and not followed()
+            and ops_available()):
         return None
     return getattr(torch.ops.amd_ops, name, None)
 

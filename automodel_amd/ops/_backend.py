@@ -55,3 +55,13 @@ def hip_ops():
     """Return the torch.ops.amd_ops namespace, loading the extension first."""
     require_ops()
     return torch.ops.amd_ops
+
+
+def followed() -> bool:
+    """Whether something besides autograd follows the operations: tracing, a transform,
+    forward-mode derivatives or a dispatch mode, which see into torch's own operations but not
+    into the kernels."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() > 0)

@@ -10,10 +10,8 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
-from torch.autograd import forward_ad
-from torch.utils import _python_dispatch
 
-from automodel_amd.ops._backend import hip_ops
+from automodel_amd.ops._backend import followed, hip_ops
 
 TILE, CUS = 256, 256
 # below this many products a layer's backward takes the library some 80 us, and an autograd
@@ -45,21 +43,31 @@ def input_grad_wins(T: int, N: int, K: int) -> bool:
             and _fills(T, K, 0.875))
 
 
+def _ordinary(*ts: torch.Tensor) -> bool:
+    """No subclass, and no batch of gradients (autograd.grad's is_grads_batched has tensors of
+    its own, without memory to point to)."""
+    return all(type(t) in (torch.Tensor, nn.Parameter)
+               and not torch._C._functorch.is_legacy_batchedtensor(t) for t in ts)
+
+
 def _plain(*ts: torch.Tensor) -> bool:
     return all(t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous()
                and t.data_ptr() % 16 == 0 for t in ts)
 
 
 def weight_grad(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """g^T x for g [T, N] and x [T, K]."""
-    if weight_grad_wins(*g.shape, x.shape[1]) and _plain(g, x):
+    """g^T x for g [T, N] and x [T, K]. Called in backward passes, which may be followed where
+    their forward was not: batched gradients, a mode around the backward alone."""
+    if (not followed() and _ordinary(g, x) and weight_grad_wins(*g.shape, x.shape[1])
+            and _plain(g, x)):
         return hip_ops().linear_dw(g, x)
     return g.t() @ x
 
 
 def input_grad(g: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """g w for g [T, N] and w [N, K]."""
-    if input_grad_wins(*g.shape, w.shape[1]) and _plain(g, w):
+    if (not followed() and _ordinary(g, w) and input_grad_wins(*g.shape, w.shape[1])
+            and _plain(g, w)):
         return hip_ops().linear_dx(g, w)
     return g @ w
 
@@ -89,16 +97,14 @@ class _Linear(torch.autograd.Function):
 
 
 def _unseen(lin: nn.Linear) -> bool:
-    """No hook sees the module's call or its gradients, and nothing follows the operations
-    (transforms, forward-mode derivatives, dispatch modes) but autograd."""
+    """No hook sees the module's call or its gradients, and nothing follows the operations but
+    autograd."""
     every = nn.modules.module
     return not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks
                 or lin._backward_pre_hooks or every._global_forward_hooks
                 or every._global_forward_pre_hooks or every._global_backward_hooks
                 or every._global_backward_pre_hooks or torch.is_autocast_enabled("cuda")
-                or torch._C._functorch.peek_interpreter_stack() is not None
-                or forward_ad._current_level >= 0
-                or _python_dispatch._get_current_dispatch_mode() is not None)
+                or followed())
 
 
 def linear(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:

@@ -141,6 +141,66 @@ def test_calls_that_stay_the_module(monkeypatch):
     assert out.shape == (4, T // 4, N)
 
 
+@gpu
+@cuda
+def test_backward_that_is_followed():
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from automodel_amd.loss.linear_ce import fused_linear_cross_entropy
+
+    T, N, K = 4096, 4096, 4096
+    torch.manual_seed(0)
+    lin = nn.Linear(K, N, bias=False, device="cuda", dtype=torch.bfloat16)
+    x, g = rand(T, K).requires_grad_(), rand(2, T, N)
+    y = L.linear(lin, x)
+    assert "_Linear" in type(y.grad_fn).__name__
+    with FlopCounterMode(display=False) as count:       # around the backward alone
+        torch.autograd.grad(y, (x, lin.weight), g[0], retain_graph=True)
+    assert count.get_total_flops() == 4 * T * N * K
+    dx, dw = torch.autograd.grad(y, (x, lin.weight), g, is_grads_batched=True)
+    for i in range(2):
+        close(dx[i], g[i].double() @ lin.weight.double())
+        close(dw[i], g[i].double().t() @ x.double())
+    # the head: logits are kept, so that its backward has two products
+    h, labels = rand(T, 2048).requires_grad_(), torch.randint(16384, (T,), device="cuda")
+    head = rand(16384, 2048).requires_grad_()
+    loss = fused_linear_cross_entropy(h, head, labels)
+    with FlopCounterMode(display=False) as count:
+        loss.backward()
+    assert count.get_total_flops() == 4 * T * 16384 * 2048
+
+
+def test_backward_that_is_followed_elsewhere(monkeypatch):
+    # which products a backward takes, with the kernels' part played by Python
+    from torch.utils.flop_counter import FlopCounterMode
+
+    class Kernels:
+        calls = 0
+
+        def linear_dw(self, g, x):
+            Kernels.calls += 1
+            return g.t() @ x
+
+        def linear_dx(self, g, w):
+            Kernels.calls += 1
+            return g @ w
+
+    monkeypatch.setattr(L, "hip_ops", Kernels)
+    monkeypatch.setattr(L, "_plain", lambda *ts: all(t.data_ptr() for t in ts))
+    for rule in ("weight_grad_wins", "input_grad_wins"):
+        monkeypatch.setattr(L, rule, lambda *sizes: True)
+    x, w, g = torch.randn(5, 16, requires_grad=True), torch.randn(8, 16, requires_grad=True), torch.randn(2, 5, 8)
+    y = L._Linear.apply(x, w)
+    one = torch.autograd.grad(y, (x, w), g[0], retain_graph=True)
+    assert Kernels.calls == 2
+    both = torch.autograd.grad(y, (x, w), g, is_grads_batched=True, retain_graph=True)
+    for a, b in zip(one, both):
+        torch.testing.assert_close(a, b[0])
+    with FlopCounterMode(display=False) as count:
+        torch.autograd.grad(y, (x, w), g[0])
+    assert Kernels.calls == 2 and count.get_total_flops() == 4 * 5 * 8 * 16
+
+
 def test_layers_elsewhere():
     lin, seen = nn.Linear(16, 8, bias=False), []
     lin.register_forward_hook(lambda *a: seen.append(1))
