@@ -11,7 +11,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from automodel_amd.ops._backend import followed, hip_ops
+from automodel_amd.ops._backend import followed, hip_ops, ops_available
 
 TILE, CUS = 256, 256
 # below this many products a layer's backward takes the library some 80 us, and an autograd
@@ -107,6 +107,11 @@ def _unseen(lin: nn.Linear) -> bool:
                 or followed())
 
 
+def _built() -> bool:
+    """The kernels may be missing: nothing is built, or the inference kernels alone."""
+    return ops_available() and getattr(torch.ops.amd_ops, "linear_dw", None) is not None
+
+
 def linear(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """``lin(x)``. Plain bf16 layers without a bias on the GPU that are large enough take the
     kernels in their backward, everything else is the module's call."""
@@ -123,6 +128,6 @@ def linear(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
             T = x.numel() // K
             if (((x.requires_grad and input_grad_wins(T, N, K))
                  or (w.requires_grad and weight_grad_wins(T, N, K)))
-                    and "forward" not in lin.__dict__ and _unseen(lin)):
+                    and "forward" not in lin.__dict__ and _unseen(lin) and _built()):
                 return _Linear.apply(x, w)
     return lin(x)

@@ -143,6 +143,25 @@ def test_calls_that_stay_the_module(monkeypatch):
 
 @gpu
 @cuda
+def test_without_the_kernels(monkeypatch):
+    lin = nn.Linear(4096, 4096, bias=False, device="cuda", dtype=torch.bfloat16)
+    x = rand(4096, 4096).requires_grad_()
+    monkeypatch.setattr(L, "_built", lambda: False)
+    assert "_Linear" not in type(L.linear(lin, x).grad_fn).__name__
+
+
+def test_what_is_built(monkeypatch):
+    inference = type("Inference", (), {"flash_attn_fwd": None})()
+    monkeypatch.setattr(torch.ops, "amd_ops", inference, raising=False)
+    for found in (False, True):
+        monkeypatch.setattr(L, "ops_available", lambda: found)
+        assert not L._built()
+    inference.linear_dw = lambda *a: None
+    assert L._built()
+
+
+@gpu
+@cuda
 def test_backward_that_is_followed():
     from torch.utils.flop_counter import FlopCounterMode
 
