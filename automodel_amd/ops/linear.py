@@ -10,6 +10,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from automodel_amd.ops._backend import followed, hip_ops, ops_available
 
@@ -96,6 +97,13 @@ class _Linear(torch.autograd.Function):
         return dx, dw
 
 
+def _functions_followed() -> bool:
+    """Whether a mode may put something else in a function's place. (The mode of a default device
+    only touches factories.)"""
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+               for i in range(torch._C._len_torch_function_stack()))
+
+
 def _unseen(lin: nn.Linear) -> bool:
     """No hook sees the module's call or its gradients, and nothing follows the operations but
     autograd."""
@@ -104,7 +112,7 @@ def _unseen(lin: nn.Linear) -> bool:
                 or lin._backward_pre_hooks or every._global_forward_hooks
                 or every._global_forward_pre_hooks or every._global_backward_hooks
                 or every._global_backward_pre_hooks or torch.is_autocast_enabled("cuda")
-                or followed())
+                or followed() or _functions_followed())
 
 
 def _built() -> bool:

@@ -150,6 +150,39 @@ def test_without_the_kernels(monkeypatch):
     assert "_Linear" not in type(L.linear(lin, x).grad_fn).__name__
 
 
+class _Halved(torch.overrides.TorchFunctionMode):
+    """Linears with half the weight, as a mode for rounded weights would put them in place."""
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        if func is F.linear:
+            args = (args[0], args[1] * 0.5)
+        return func(*args, **(kwargs or {}))
+
+
+def test_function_modes():
+    lin = nn.Linear(16, 8, bias=False)
+    assert L._unseen(lin)
+    with torch.device("cpu"):
+        assert L._unseen(lin)
+        with _Halved():
+            assert not L._unseen(lin)
+    assert L._unseen(lin)
+
+
+@gpu
+@cuda
+def test_a_mode_in_the_place_of_linears():
+    lin = nn.Linear(4096, 4096, bias=False, device="cuda", dtype=torch.bfloat16)
+    x, g = rand(4096, 4096).requires_grad_(), rand(4096, 4096)
+    with _Halved():
+        y = L.linear(lin, x)
+    dx, dw = torch.autograd.grad(y, (x, lin.weight), g)
+    close(dx, g.double() @ lin.weight.double() * 0.5)
+    close(dw, g.double().t() @ x.double() * 0.5)
+    with torch.device("cuda"):
+        assert "_Linear" in type(L.linear(lin, x).grad_fn).__name__
+
+
 def test_what_is_built(monkeypatch):
     inference = type("Inference", (), {"flash_attn_fwd": None})()
     monkeypatch.setattr(torch.ops, "amd_ops", inference, raising=False)
