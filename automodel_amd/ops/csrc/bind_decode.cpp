@@ -19,6 +19,8 @@ TORCH_LIBRARY_FRAGMENT(amd_ops, m) {
   m.def(
       "gemm_skinny_bf16(Tensor x, Tensor w, bool relu2, bool out_f32, int group_n=0) -> Tensor");
   m.impl("gemm_skinny_bf16", &amd_ops::gemm_skinny_bf16);
+  m.def("decode_rows_shape(int[] n, int K, int B, bool glu=False, int group_n=0) -> (int, int, int)");
+  m.impl("decode_rows_shape", &amd_ops::decode_rows_shape);
   m.def(
       "decode_rows(Tensor x, Tensor[] ws, bool glu=False, bool relu2=False, "
       "Tensor? residual=None) -> Tensor[]");

@@ -295,51 +295,80 @@ void launch_stream(const Rows& rows, int segments, int B) {
 // stands for the loads of x and the workgroup's beginning and end; of more than one a CU, as far as
 // the others fill in for it, x counts otherwise and the fullest for 0.7. In us, 8 and 16 rows of
 // x, rows x columns of W:
-//  * 8 rows of W: 2048 x 4096 5.3 and 6.1, 16 rows 6.2 and 7.1
+//  * 8 rows of W, one workgroup a CU: 2048 x 4096 5.3 and 6.1, 16 rows 6.2 and 7.1; but its ring has the CU
+//    to itself (4224 x 768, 3 a CU: 5.9, 24 rows 3.7), and its waves want a tile each (1232 x 128,
+//    16 rows in 4 waves 2.4, 2.5)
 //  * 24: 5120 x 4096 8.8 and 9.8, 16 rows 11.0 and 12.5, 32 rows 9.4 and 10.5
 //  * 32: 7168 x 14336 32.5 and 35.0, 16 rows 35.0 and 40.2
 //  * 40: 10240 x 8192 26.8 and 27.3, 24 rows 27.7 and 30.2, 64 rows 30.3 and 31.7
 //  * 56: 28672 x 4096 36.8 and 37.1, 32 rows 37.8 and 39.2
 // No multiples of 16 above 16 for rows of a multiple of 16 KB, whose channels they crowd (8192 x 8192,
 // 32 rows 25.6 and 26.0, 16 rows 21.5 and 23.8); nor many rows where rows of W are short, which leaves
-// too few waves (28672 x 1024, 16 rows 11.1 and 12.5, 64 rows 12.0 and 12.6; 18944 x 1024, 8.3 and
-// 9.4, 40 rows 10.4 and 11.3; 16 rows of x, 16384 x 128, 16 rows 3.3, 32 rows 4.8).
+// too few waves (28672 x 1024, 16 rows 11.1 and 12.5, 64 rows 12.0 and 12.6; 12032 x 1280, 9 rows of x:
+// 48 rows 8.4, 24 rows 7.4).
 // The ring: 8 waves where one workgroup has the CU to itself and rows are long (4096 x 4096 7.3 us,
 // 4 waves 7.8; 4096 x 2048 6.2, 4 waves 4.9), else 4; two slots, one from 48 rows (gate and up
-// of 14336 x 4096, 56 rows and 16 of x: 36.3 us, two slots 37.3) and where 32 rows have many workgroups
-// (28672 x 4096, 16 rows of x: 39.2 and 42.8).
-template <bool GLU>
-void stream(const Rows& p, int segments, int B) {
+// of 14336 x 4096, 56 rows and 16 of x: 36.3 us, two slots 37.3), and of more than one workgroup a CU also
+// where that lets them share it: 40 rows (28864 x 3072 33.4 us, one slot 31.6; 50352 x 2560, 16 rows of
+// x: 48.9 and 43.5), 24 and 32 of short rows (16384 x 512, 9 rows of x: 32 rows in one slot 5.2, in two 6.4), 32
+// with many workgroups (28672 x 4096, 16 rows of x: 39.2 and 42.8).
+// Against the kernel above, of 1850 shapes and numbers of rows, 128 x 128 to 151936 x 1024 and more columns, one
+// or several weights: 0.86 of its time in the mean, in 14 more than 1.03, 1.06 at most.
+struct StreamShape {
+  int rows, slots, waves;
+};
+
+StreamShape stream_shape(const int* n, int segments, int K, int B, bool glu, int group_n) {
   constexpr int CUS = 256;
   const int x = B <= 8 ? 6 : 8, x_more = B <= 8 ? 4 : 12;
-  int best = 0, fullest = 0;
+  int best = 0;
+  bool alone = true, many = false;
   float least = 0.f;
   for (int r : {8, 16, 24, 32, 40, 48, 56, 64}) {
-    const int out = GLU ? r / 2 : r;
-    if (r > 16 && ((p.group_n % out != 0) || (p.K % 8192 == 0 && r % 16 == 0) ||
-                   p.K < 1024 || (r > 32 && p.K <= (B <= 8 ? 2048 : 1024))))
-      continue;
+    const int out = glu ? r / 2 : r;
+    if (r > 16 && (group_n % out != 0 || (K % 8192 == 0 && r % 16 == 0))) continue;
+    if (r > 32 && K <= (B <= 8 ? 2048 : 1536)) continue;
     long blocks = 0;
-    for (int s = 0; s < segments; ++s) blocks += (p.n[s] + out - 1) / out;
+    for (int s = 0; s < segments; ++s) blocks += (n[s] + out - 1) / out;
     const long full = (blocks + CUS - 1) / CUS;
+    if (r == 8 && (full > 1 || K <= 512)) continue;
     float cost = (float)full * (r + x);
     if (full > 1) cost = 0.7f * cost + 0.3f * ((float)blocks / CUS) * (r + x_more);
     if (best && cost >= least) continue;
     best = r;
     least = cost;
-    fullest = (int)std::min(full, 1l << 20);
+    alone = full == 1;
+    many = full > 2;
   }
+  const bool share = !alone && K <= 2048;
   switch (best) {
+    case 8: return {8, 3, 8};
+    case 16: return {16, many && K <= 2048 ? 1 : 2, alone && K >= 3072 ? 8 : 4};
+    case 24: return {24, share ? 1 : 2, 4};
+    case 32: return {32, share || many ? 1 : 2, 4};
+    case 40: return {40, alone ? 2 : 1, 4};
+    default: return {best, 1, 4};
+  }
+}
+
+template <bool GLU>
+void stream(const Rows& p, int segments, int B) {
+  const StreamShape s = stream_shape(p.n, segments, p.K, B, GLU, p.group_n);
+  switch (s.rows) {
     case 8: return launch_stream<8, 3, 8, GLU>(p, segments, B);
     case 16:
-      if (fullest == 1 && p.K >= 3072) return launch_stream<16, 2, 8, GLU>(p, segments, B);
-      if (fullest > 2 && p.K <= 2048) return launch_stream<16, 1, 4, GLU>(p, segments, B);
+      if (s.waves == 8) return launch_stream<16, 2, 8, GLU>(p, segments, B);
+      if (s.slots == 1) return launch_stream<16, 1, 4, GLU>(p, segments, B);
       return launch_stream<16, 2, 4, GLU>(p, segments, B);
-    case 24: return launch_stream<24, 2, 4, GLU>(p, segments, B);
+    case 24:
+      if (s.slots == 1) return launch_stream<24, 1, 4, GLU>(p, segments, B);
+      return launch_stream<24, 2, 4, GLU>(p, segments, B);
     case 32:
-      if (fullest > 2) return launch_stream<32, 1, 4, GLU>(p, segments, B);
+      if (s.slots == 1) return launch_stream<32, 1, 4, GLU>(p, segments, B);
       return launch_stream<32, 2, 4, GLU>(p, segments, B);
-    case 40: return launch_stream<40, 2, 4, GLU>(p, segments, B);
+    case 40:
+      if (s.slots == 1) return launch_stream<40, 1, 4, GLU>(p, segments, B);
+      return launch_stream<40, 2, 4, GLU>(p, segments, B);
     case 48: return launch_stream<48, 1, 4, GLU>(p, segments, B);
     case 56: return launch_stream<56, 1, 4, GLU>(p, segments, B);
     default: return launch_stream<64, 1, 4, GLU>(p, segments, B);
@@ -447,6 +476,21 @@ std::pair<Rows, at::Tensor> single(const char* name, const at::Tensor& x, const 
 }
 
 }  // namespace
+
+// which streamed kernel a call of these sizes takes, for the tests
+std::tuple<int64_t, int64_t, int64_t> decode_rows_shape(at::IntArrayRef n, int64_t K, int64_t B, bool glu,
+                                                        int64_t group_n) {
+  TORCH_CHECK(n.size() >= 1 && n.size() <= MAX_SEGMENTS && B >= 3 && B <= 16 && K >= 128 && K % 128 == 0 &&
+                  K < 1 << 25 && group_n >= 0 && group_n % 16 == 0,
+              "decode_rows_shape: 1 to 3 weights, 3 to 16 rows, K in 128s");
+  int sizes[MAX_SEGMENTS] = {};
+  for (size_t s = 0; s < n.size(); ++s) {
+    TORCH_CHECK(n[s] >= 1 && n[s] < INT_MAX / 2, "decode_rows_shape: rows of a weight");
+    sizes[s] = (int)n[s];
+  }
+  const StreamShape s = stream_shape(sizes, (int)n.size(), (int)K, (int)B, glu, (int)group_n);
+  return {s.rows, s.slots, s.waves};
+}
 
 // group_n > 0: x holds several [B, K] inputs one after another, and every
 // group_n rows of w take the next one.

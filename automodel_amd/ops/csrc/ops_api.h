@@ -89,6 +89,9 @@ std::tuple<at::Tensor, at::Tensor> doc_bounds(const at::Tensor& cu, int64_t tota
 at::Tensor kv_decode_attn(const at::Tensor& q, const at::Tensor& k_new, const at::Tensor& v_new,
                           at::Tensor k_cache, at::Tensor v_cache, int64_t pos,
                           const std::optional<at::Tensor>& pos_dev, double scale);
+// rows of W a workgroup, slots of its rings and waves that 3 to 16 rows of x take (see gemv.hip)
+std::tuple<int64_t, int64_t, int64_t> decode_rows_shape(at::IntArrayRef n, int64_t K, int64_t B, bool glu,
+                                                        int64_t group_n);
 at::Tensor gemm_skinny_bf16(const at::Tensor& x, const at::Tensor& w, bool relu2, bool out_f32,
                             int64_t group_n = 0);
 std::vector<at::Tensor> decode_rows(const at::Tensor& x, at::TensorList ws, bool glu = false,

@@ -1,0 +1,25 @@
+"""Which kernel a call takes, by its sizes alone."""
+
+import pytest
+
+from automodel_amd.ops._backend import hip_ops, ops_available
+
+pytestmark = pytest.mark.skipif(not ops_available(), reason="the library is not built")
+
+
+@pytest.mark.parametrize("b", [3, 8, 9, 16])
+def test_few_row_linears(b):
+    def shape(n, k, glu=False):
+        return hip_ops().decode_rows_shape([n], k, b, glu)
+
+    # 8 rows of W in a ring that has the CU to itself: one workgroup a CU, a tile of K for each wave
+    assert shape(2048, 4096)[0] == shape(1024, 4096, True)[0] == 8
+    for n, k in ((4224, 768), (2049, 1024), (1232, 512), (17, 128)):
+        assert shape(n, k)[0] > 8 and shape(n // 2 + 1, k, True)[0] > 8
+    # several workgroups a CU share it: one slot where two leave no room, or where rows are short
+    assert shape(28864, 3072)[:2] in ((40, 1), (48, 1), (56, 1), (64, 1))
+    for n in (14400, 16384, 40960):
+        for k in (512, 1024, 2048):
+            assert shape(n, k)[1] == 1
+    # rows of few columns leave no tiles for the waves of many rows of W
+    assert shape(12032, 1280)[0] <= 32
