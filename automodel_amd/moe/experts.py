@@ -203,7 +203,8 @@ class GroupedExperts(nn.Module):
                     bm = 256 if (self.intermediate_size % 256 == 0
                                  and self.hidden_size % 256 == 0) else 128
                 else:
-                    bm = tile_rows(x_perm.shape[0], self.n_experts)
+                    bm = tile_rows(x_perm.shape[0], self.n_experts, self.intermediate_size,
+                                   self.hidden_size)
                 plan = (*make_group_plan(counts, x_perm.shape[0], bm), bm)
                 cl = counts
             else:

@@ -19,8 +19,8 @@
 //
 // Bound by LDS (at full MFMA rate 64 x 128 wave tiles read and load 128 B/clk, 64 x 64 ones
 // more: 256 x 256 is the faster tile) against padding of the groups' last row tiles: nt and
-// nn take 256 rows from 320 rows per expert on (the caller's plan, ops/grouped_gemm.py, has both
-// sides), tn, whose tiles have no padding, always. 4 waves of 64 x 128, one a SIMD, wait for
+// nn take 256 rows from 512 rows per expert on, from 320 where such tiles fill the chip (the caller's
+// plan, ops/grouped_gemm.py, has both sides), tn, whose tiles have no padding, always. 4 waves of 64 x 128, one a SIMD, wait for
 // LDS more than they save (128 x 256: 374 against 345 us).
 //
 // grouped_tile_kernel: 4 waves of 128 x 128 (gemm_tile.h), for nn's tiles of 256 rows, and for tn

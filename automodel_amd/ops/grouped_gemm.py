@@ -41,18 +41,25 @@ def make_group_plan(counts: torch.Tensor, M: int, bm: int = 128):
     return hip_ops().build_group_plan(counts.to(torch.int32), M, bm)
 
 
-def tile_rows(rows: int, experts: int) -> int:
-    """Row tile of the bf16 kernels: 256 is the faster tile, but the last one of
-    every group is padding for half of it on average, and there are half as many.
-    Time of 256 over that of 128, forward and dx together, groups as a random choice
-    fills them, at 128, 256, 320, 384, 512 and 1024 rows per expert:
-    128 experts of 768 x 2048: 1.09 1.01 0.97 0.88 0.88 0.86;
-    64 of 1408 x 2048: 1.05 0.97 0.94 0.84 0.86 0.83;
-    8 of 4096 x 2048, few tiles: 1.32 1.04 1.03 1.03 0.81 0.91;
-    32 of 1024 x 1024: 1.39 0.84 0.86 0.84 1.02 0.94.
-    From 320 on it is slower nowhere by more than 3%; below, the sign depends on how
-    the tiles fill the chip, and the forward alone is up to 12% slower."""
-    return 256 if rows >= 320 * experts else 128
+def tile_rows(rows: int, experts: int, *widths: int) -> int:
+    """Row tile of the bf16 kernels for products of those widths (the columns of their
+    outputs): 256 is the faster tile, but the last one of every group is padding for half of it on
+    average, and there are half as many. From 512 rows per expert on 256.
+
+    From 320 on where its tiles fill the chip, one workgroup a CU: within one round of them, and
+    beyond some three. Time of 256 over that of 128, groups as a random choice fills them, 110
+    shapes of 4 to 128 experts, 320 to 511 rows each, by the number of tiles:
+    16 to 150: 1.18 to 1.61 (the forward of 8 experts of 2048 x 4096 1.58, their input gradient 0.77);
+    150 to 256: 0.68 to 0.89;
+    260 to 560, part of a second round or third: 0.66 to 1.38;
+    700 on: 0.68 to 0.98, but 1.01 and 1.08 where the sum of an input gradient is 512.
+    It holds for the forward (nt) and the input gradient (nn) alike, so that a forward alone is not
+    slower either."""
+    if rows >= 512 * experts or rows < 320 * experts:
+        return 256 if rows >= 512 * experts else 128
+    row_tiles = rows / 256 + experts / 2
+    tiles = [row_tiles * -(-w // 256) for w in widths]
+    return 256 if all(150 <= t <= 256 or t >= 700 for t in tiles) else 128
 
 
 def _loop_gemm_nt(x, w, counts):
@@ -123,7 +130,7 @@ def grouped_linear(x_perm: torch.Tensor, w: torch.Tensor, counts,
     bm = 128
     if hip_eligible:
         if torch.is_tensor(counts) and counts.is_cuda:
-            bm = tile_rows(x_perm.shape[0], w.shape[0])
+            bm = tile_rows(x_perm.shape[0], *w.shape)
             offs, tile_map, n_tiles = make_group_plan(counts, x_perm.shape[0], bm)
         else:
             cl = counts.tolist() if torch.is_tensor(counts) else list(counts)

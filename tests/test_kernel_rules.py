@@ -23,3 +23,16 @@ def test_few_row_linears(b):
             assert shape(n, k)[1] == 1
     # rows of few columns leave no tiles for the waves of many rows of W
     assert shape(12032, 1280)[0] <= 32
+
+
+@pytest.mark.parametrize("rows", [320, 384, 511])
+def test_row_tiles_of_experts(rows):
+    from automodel_amd.ops.grouped_gemm import tile_rows
+
+    # the larger tile where it fills the chip with both products of a layer, else from 512 rows on
+    for experts, inter, hidden, large in ((8, 2048, 4096, False), (4, 4096, 4096, rows == 511), (16, 768, 2048, False),
+                                          (8, 14336, 4096, rows != 511), (64, 1408, 2048, rows > 330),
+                                          (128, 768, 2048, rows > 330), (128, 2048, 2048, True)):
+        assert tile_rows(rows * experts, experts, inter, hidden) == (256 if large else 128)
+        assert tile_rows(319 * experts, experts, inter, hidden) == 128
+        assert tile_rows(512 * experts, experts, inter, hidden) == 256
