@@ -100,34 +100,34 @@ def _pad_head(t: torch.Tensor, target: int) -> torch.Tensor:
 class _FlashAttnHip(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, causal: bool, scale: float, q_start: int,
-                doc_start=None, doc_end=None):
+                doc_start=None, doc_end=None, docs: int = 0):
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         o, lse = hip_ops().flash_attn_fwd(q, k, v, scale, causal, q_start, doc_start)
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.causal, ctx.scale, ctx.q_start = causal, scale, q_start
-        ctx.docs = (doc_start, doc_end)
+        ctx.docs = (doc_start, doc_end, docs)
         return o
 
     @staticmethod
     def backward(ctx, do):
         q, k, v, o, lse = ctx.saved_tensors
-        ds, de = ctx.docs
         dq, dk, dv = hip_ops().flash_attn_bwd(
             do.contiguous(), q, k, v, o, lse, ctx.scale, ctx.causal, ctx.q_start,
-            ds, de,
+            *ctx.docs,
         )
-        return dq, dk, dv, None, None, None, None, None
+        return dq, dk, dv, None, None, None, None, None, None
 
 
-def _flash_hip(q, k, v, causal, scale, q_start, doc_start=None, doc_end=None):
+def _flash_hip(q, k, v, causal, scale, q_start, doc_start=None, doc_end=None, docs=0):
     """Dispatch to the HIP kernel, zero-padding head dims to a supported
     kernel pair — pad/slice sit outside the Function so autograd routes
-    gradients through them. The kernels take any sequence lengths."""
+    gradients through them. The kernels take any sequence lengths. ``docs``: how many
+    documents there are, as far as the host knows; short ones have another backward."""
     dqk, dv = q.shape[-1], v.shape[-1]
     tq, tv = _target_dims(dqk, dv)
     if tq != dqk or tv != dv:
         q, k, v = _pad_head(q, tq), _pad_head(k, tq), _pad_head(v, tv)
-    o = _FlashAttnHip.apply(q, k, v, causal, scale, q_start, doc_start, doc_end)
+    o = _FlashAttnHip.apply(q, k, v, causal, scale, q_start, doc_start, doc_end, docs)
     return o[..., :dv] if tv != dv else o
 
 
@@ -182,7 +182,7 @@ def flash_attention_varlen(q, k, v, cu_seqlens: torch.Tensor, scale: float | Non
     scale = scale if scale is not None else 1.0 / math.sqrt(q.shape[-1])
     if backend == "hip" and q.is_cuda:
         ds, de = doc_bounds_from_cu(cu_seqlens.to(q.device), q.shape[1])
-        return _flash_hip(q, k, v, True, scale, 0, ds, de)
+        return _flash_hip(q, k, v, True, scale, 0, ds, de, cu_seqlens.numel() - 1)
     from automodel_amd.datasets.llm.packed_sequence import block_causal_mask
 
     mask = block_causal_mask(cu_seqlens.cpu(), q.shape[1]).to(q.device)

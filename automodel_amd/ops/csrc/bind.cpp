@@ -48,8 +48,11 @@ TORCH_LIBRARY(amd_ops, m) {
   m.def(
       "flash_attn_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, "
       "float scale, bool causal, int q_start=0, Tensor? doc_start=None, "
-      "Tensor? doc_end=None) -> (Tensor, Tensor, Tensor)");
+      "Tensor? doc_end=None, int docs=0) -> (Tensor, Tensor, Tensor)");
   m.impl("flash_attn_bwd", &amd_ops::flash_attn_bwd);
+  m.def("flash_attn_bwd_ordered(int B, int Sq, int Skv, int Hq, int Hk, int Dqk, int Dv, bool causal, "
+        "int docs=0) -> (bool, bool)");
+  m.impl("flash_attn_bwd_ordered", &amd_ops::flash_attn_bwd_ordered);
 
   m.def("mfma_probe(Tensor a, Tensor b) -> Tensor");
   m.impl("mfma_probe", &amd_ops::mfma_probe);

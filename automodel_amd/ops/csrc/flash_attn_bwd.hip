@@ -27,6 +27,8 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 
+#include <climits>
+
 #include "common.h"
 #include "flash_tile.h"
 #include "ops_api.h"
@@ -76,7 +78,7 @@ struct BwdArgs {
   const float* stats;              // two planes of B * Hq * sp
   bf16 *dq, *dk, *dv;
   const int *doc_start, *doc_end;
-  int B, Sq, Skv, Hq, Hk, q_start, sp;
+  int B, Sq, Skv, Hq, Hk, q_start, sp, docs;
   long plane;
   float scale;
   bool causal;
@@ -439,10 +441,15 @@ static bool dq_ordered(const BwdArgs& a) {
 // The ordered dK/dV of 128 columns, but for walks of a few tiles of queries, where what a workgroup does
 // before and after them counts (whole backward, this one over the other, keys 2048 to 4096: 1.09
 // and 1.12 at 16 and 64 queries of 8 x 32 heads, 1.04 and 1.07 at 100 of 16 x 16, the same at 192).
-// Packed rows have it whatever their documents' lengths, which the host does not know (8192 tokens,
-// 32 heads, documents of 64 on average 254 and 265 us, of 200 310 and 312, of 700 487 and 461).
+// Of packed rows the walk is a document's, on average, times the heads of a group. (128, 128), 8192
+// tokens, 32 / 32 heads: 1.04 at 64 and 100 tokens a document, 1.01 at 200, 0.99 at 256, 0.93 at 700; 16384, 16 / 16:
+// 1.05, 1.04, 1.01, 0.99, 0.95; 32 / 8 heads: 1.01, 0.99, 0.98, 0.98, 0.99. (192, 128), 8192, 32: 1.03,
+// 1.01, 0.98, 0.96, 0.90; 4096, 32: 1.02, 1.02, 0.99, 0.98, 0.91.
+template <int DQK>
 static bool dkv_ordered(const BwdArgs& a) {
-  return a.doc_end || (long)a.Sq * (a.Hq / a.Hk) >= 192;
+  const long G = a.Hq / a.Hk;
+  if (a.doc_end) return a.docs <= 0 || a.Skv * G >= (DQK == 128 ? 256l : 192l) * a.docs;
+  return a.Sq * G >= 192;
 }
 
 template <int DQK, int DV>
@@ -504,7 +511,7 @@ static void launch_dq(const BwdArgs& a, hipStream_t stream) {
 std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
     const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
     const at::Tensor& o, const at::Tensor& lse, double scale, bool causal, int64_t q_start,
-    const std::optional<at::Tensor>& doc_start, const std::optional<at::Tensor>& doc_end) {
+    const std::optional<at::Tensor>& doc_start, const std::optional<at::Tensor>& doc_end, int64_t docs) {
   const int B = q.size(0), Sq = q.size(1), Hq = q.size(2), Dqk = q.size(3);
   const int Skv = k.size(1), Hk = k.size(2), Dv = v.size(3);
   TORCH_CHECK(q.is_contiguous() && k.is_contiguous() && v.is_contiguous() && o.is_contiguous() &&
@@ -535,6 +542,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
   a.plane = (long)B * Hq * a.sp;
   a.scale = (float)scale;
   a.causal = causal;
+  a.docs = (int)std::min<int64_t>(docs, INT_MAX);
   auto stats = at::empty({2, B, Hq, a.sp}, q.options().dtype(at::kFloat));
   a.stats = stats.data_ptr<float>();
   const bf16* op = reinterpret_cast<const bf16*>(o.data_ptr());
@@ -550,7 +558,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
     launch_stats<C>(a, op, lse.data_ptr<float>(), stats.data_ptr<float>(), stream);       \
     bool ordered = false;                                                                 \
     if constexpr (C == 128) {                                                             \
-      ordered = dkv_ordered(a);                                                           \
+      ordered = dkv_ordered<A>(a);                                                        \
       if (ordered) launch_dkv_ordered<A, C>(a, stream);                                   \
     }                                                                                     \
     if (!ordered) launch_dkv<A, C, 4, KV_OCC, KV_PIPE>(a, stream);                        \
@@ -570,6 +578,21 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
 #undef FA_BWD_CASE
   TORCH_CHECK(done, "flash_attn_bwd: unsupported head dims (Dqk=", Dqk, ", Dv=", Dv, ")");
   return {dq, dk, dv};
+}
+
+std::tuple<bool, bool> flash_attn_bwd_ordered(int64_t B, int64_t Sq, int64_t Skv, int64_t Hq, int64_t Hk,
+                                              int64_t Dqk, int64_t Dv, bool causal, int64_t docs) {
+  TORCH_CHECK(std::min({B, Sq, Skv, Hq, Hk}) >= 1 && std::max({B, Sq, Skv, Hq, Hk, docs}) <= INT_MAX && Hq % Hk == 0,
+              "flash_attn_bwd_ordered: sizes");
+  if (Dv != 128 || (Dqk != 128 && Dqk != 192)) return {false, false};
+  const int here = 0;
+  BwdArgs a{};
+  a.B = (int)B; a.Sq = (int)Sq; a.Skv = (int)Skv; a.Hq = (int)Hq; a.Hk = (int)Hk;
+  a.causal = causal;
+  if (docs) a.doc_start = a.doc_end = &here;       // (that there are some is all that is asked)
+  a.docs = (int)std::max<int64_t>(docs, 0);
+  if (Dqk == 128) return {dkv_ordered<128>(a), dq_ordered<128, 128>(a)};
+  return {dkv_ordered<192>(a), dq_ordered<192, 128>(a)};
 }
 
 // ---- MFMA layout self-test: d[32,32] = a[32,16] @ b[16,32] via one mfma.

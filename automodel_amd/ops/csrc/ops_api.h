@@ -38,12 +38,16 @@ std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
     bool causal, int64_t q_start,
     const std::optional<at::Tensor>& doc_start = std::nullopt,
     const std::optional<at::Tensor>& sink = std::nullopt);
+// whether dK/dV and dQ of such a call have the kernels in a given order; docs: documents of a packed row,
+// 0: rows of their own, -1: documents, but not known how many
+std::tuple<bool, bool> flash_attn_bwd_ordered(int64_t B, int64_t Sq, int64_t Skv, int64_t Hq, int64_t Hk,
+                                              int64_t Dqk, int64_t Dv, bool causal, int64_t docs);
 std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
     const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
     const at::Tensor& o, const at::Tensor& lse, double scale, bool causal,
     int64_t q_start,
     const std::optional<at::Tensor>& doc_start = std::nullopt,
-    const std::optional<at::Tensor>& doc_end = std::nullopt);
+    const std::optional<at::Tensor>& doc_end = std::nullopt, int64_t docs = 0);
 
 at::Tensor mfma_probe(const at::Tensor& a, const at::Tensor& b);
 at::Tensor tr16_probe(const at::Tensor& pattern);

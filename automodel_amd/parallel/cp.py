@@ -192,7 +192,7 @@ def cp_blockdiag_attention(q, k, v, cu_seqlens: torch.Tensor,
         outs = []
         for slot, g in ((0, g0), (1, g1)):
             qc = q.narrow(1, slot * C, C)
-            outs.append(_flash_hip(qc, kg, vg, True, scale, g * C, ds, de))
+            outs.append(_flash_hip(qc, kg, vg, True, scale, g * C, ds, de, cu_seqlens.numel() - 1))
         return torch.cat(outs, dim=1)
 
     bounds = cu_seqlens.to(dev)[1:-1]

@@ -176,6 +176,30 @@ def test_query_gradients_of_long_walks(dims, B, heads, sq, skv, causal, q_start)
         assert torch.equal(first, again)
 
 
+# packed rows of short documents have another backward where their number is known
+@pytest.mark.parametrize("dims", [(128, 128), (192, 128)])
+@pytest.mark.parametrize("heads,sq,q_start,step", [((4, 2), 640, 0, 64), ((4, 4), 333, 0, 37), ((2, 2), 256, 256, 31)])
+def test_short_documents(dims, heads, sq, q_start, step):
+    from automodel_amd.ops._backend import hip_ops
+    from automodel_amd.ops.attention import _FlashAttnHip
+
+    torch.manual_seed(0)
+    skv = sq + q_start
+    cuts = tuple(range(step, skv, step))
+    start, end = _docs(cuts, skv)
+    q = torch.randn(1, sq, heads[0], dims[0], device="cuda").bfloat16()
+    k = torch.randn(1, skv, heads[1], dims[0], device="cuda").bfloat16()
+    v = torch.randn(1, skv, heads[1], dims[1], device="cuda").bfloat16()
+    do = torch.randn(1, sq, heads[0], dims[1], device="cuda").bfloat16()
+    scale, docs = dims[0] ** -0.5, len(cuts) + 1
+    assert not hip_ops().flash_attn_bwd_ordered(1, sq, skv, *heads, *dims, True, docs)[0]
+    got = _grads(lambda *t: _FlashAttnHip.apply(*t, True, scale, q_start, start, end, docs), (q, k, v), do)
+    ref = _grads(lambda *t: _reference(*t, True, q_start, start, scale)[0],
+                 (q.float(), k.float(), v.float()), do.float())
+    for name, g, r in zip(("dq", "dk", "dv"), got, ref):
+        assert (g.float() - r).norm() / r.norm() < BWD, name
+
+
 def test_document_bounds():
     from automodel_amd.ops.attention import doc_bounds_from_cu
 

@@ -36,3 +36,21 @@ def test_row_tiles_of_experts(rows):
         assert tile_rows(rows * experts, experts, inter, hidden) == (256 if large else 128)
         assert tile_rows(319 * experts, experts, inter, hidden) == 128
         assert tile_rows(512 * experts, experts, inter, hidden) == 256
+
+
+def test_attention_backward():
+    def ordered(*sizes, causal=True, docs=0):
+        return hip_ops().flash_attn_bwd_ordered(*sizes, causal, docs)
+
+    for dims, tokens in (((128, 128), 256), ((192, 128), 192)):
+        # short documents have the kernels before, for the heads of a group together; long ones, and
+        # an unknown number of them, the ordered dK/dV; dQ of documents is never ordered
+        for heads, group in ((32, 1), (8, 4)):
+            most = 8192 * group // tokens
+            assert ordered(1, 8192, 8192, 32, heads, *dims, docs=most) == (True, False)
+            assert ordered(1, 8192, 8192, 32, heads, *dims, docs=most + 1) == (False, False)
+        assert ordered(1, 8192, 8192, 32, 32, *dims, docs=-1) == (True, False)
+        # few queries; long walks
+        assert ordered(8, 64, 4096, 32, 32, *dims, causal=False) == (False, False)
+        assert ordered(8, 4096, 4096, 32, 32, *dims) == (True, True)
+    assert ordered(8, 4096, 4096, 32, 32, 64, 64) == ordered(8, 4096, 4096, 32, 32, 256, 256) == (False, False)
