@@ -240,37 +240,35 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_ordered_kernel(const Args a) {
         }
         // P and dS: 64 operations, 16 multiplications and additions with their exponentials,
         // then 16 products with the roundings
-        unrolled<64>([&](auto i_) __attribute__((always_inline)) {
+        spread<m, 2 * F, 64>([&](auto i_) __attribute__((always_inline)) {
           constexpr int i = decltype(i_)::value;
-          if constexpr (i * 2 * F / 64 == m) {
-            constexpr int v = i % 32 / 2, q = v / 8, kk = v / 4 % 2, r = v % 4;
-            if constexpr (i < 32) {
-              float y = s[SUB][q][kk][r];
-              if constexpr (i % 2 == 0) y = fmaf(y, c, -l2[q][r]);
-              else y = __builtin_amdgcn_exp2f(y);
-              here(y);
-              s[SUB][q][kk][r] = y;
-              if (i == 31 && mask) {
+          constexpr int v = i % 32 / 2, q = v / 8, kk = v / 4 % 2, r = v % 4;
+          if constexpr (i < 32) {
+            float y = s[SUB][q][kk][r];
+            if constexpr (i % 2 == 0) y = fmaf(y, c, -l2[q][r]);
+            else y = __builtin_amdgcn_exp2f(y);
+            here(y);
+            s[SUB][q][kk][r] = y;
+            if (i == 31 && mask) {
 #pragma unroll
-                for (int z = 0; z < 16; ++z) {
-                  const int zq = z / 8, zk = z / 4 % 2, zr = z % 4;
-                  const int qq = qpos + SUB * 32 + zq * 16 + 4 * g + zr;
-                  if ((a.causal && kv0 + 16 * zk + i16 > qq) || (VARLEN && qq >= kend[zk]))
-                    s[SUB][zq][zk][zr] = 0.f;
-                }
+              for (int z = 0; z < 16; ++z) {
+                const int zq = z / 8, zk = z / 4 % 2, zr = z % 4;
+                const int qq = qpos + SUB * 32 + zq * 16 + 4 * g + zr;
+                if ((a.causal && kv0 + 16 * zk + i16 > qq) || (VARLEN && qq >= kend[zk]))
+                  s[SUB][zq][zk][zr] = 0.f;
               }
-            } else if constexpr (i % 2 == 0) {
-              float y = dp[SUB][q][kk][r] * s[SUB][q][kk][r];
-              here(y);
-              dp[SUB][q][kk][r] = y;
-            } else {
-              typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-              constexpr int w = v / 2, wq = w / 4, wk = w / 2 % 2, wr = w % 2;
-              const auto& from = v % 2 == 0 ? s[SUB][wq][wk] : dp[SUB][wq][wk];
-              unsigned y = __builtin_bit_cast(unsigned, bf16x2_t{(__bf16)from[2 * wr], (__bf16)from[2 * wr + 1]});
-              here(y);
-              (v % 2 == 0 ? p : e)[SUB][wk][wq * 2 + wr] = y;
             }
+          } else if constexpr (i % 2 == 0) {
+            float y = dp[SUB][q][kk][r] * s[SUB][q][kk][r];
+            here(y);
+            dp[SUB][q][kk][r] = y;
+          } else {
+            typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+            constexpr int w = v / 2, wq = w / 4, wk = w / 2 % 2, wr = w % 2;
+            const auto& from = v % 2 == 0 ? s[SUB][wq][wk] : dp[SUB][wq][wk];
+            unsigned y = __builtin_bit_cast(unsigned, bf16x2_t{(__bf16)from[2 * wr], (__bf16)from[2 * wr + 1]});
+            here(y);
+            (v % 2 == 0 ? p : e)[SUB][wk][wq * 2 + wr] = y;
           }
         });
         // statistics: delta of the rows that are read; log-sum-exp of the next step's P

@@ -200,37 +200,35 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_ordered_kernel(const Args a) {
         // 28 N operations: multiplications and additions with their exponentials, then products
         // with the roundings
         constexpr int E = 8 * N, OPS = E * 7 / 2;
-        unrolled<OPS>([&](auto i_) __attribute__((always_inline)) {
+        spread<m, SLOTS, OPS>([&](auto i_) __attribute__((always_inline)) {
           constexpr int i = decltype(i_)::value;
-          if constexpr (i * SLOTS / OPS == m) {
-            if constexpr (i < 2 * E) {
-              constexpr int v = i / 2, k = v / (4 * N), q = v / 4 % N, r = v % 4;
-              float y = s[SUB][k][q][r];
-              if constexpr (i % 2 == 0) y = fmaf(y, c, -l2[q]);
-              else y = __builtin_amdgcn_exp2f(y);
-              here(y);
-              s[SUB][k][q][r] = y;
-              if (i == 2 * E - 1 && mask) {
+          if constexpr (i < 2 * E) {
+            constexpr int v = i / 2, k = v / (4 * N), q = v / 4 % N, r = v % 4;
+            float y = s[SUB][k][q][r];
+            if constexpr (i % 2 == 0) y = fmaf(y, c, -l2[q]);
+            else y = __builtin_amdgcn_exp2f(y);
+            here(y);
+            s[SUB][k][q][r] = y;
+            if (i == 2 * E - 1 && mask) {
 #pragma unroll
-                for (int z = 0; z < E; ++z) {
-                  const int zk = z / (4 * N), zq = z / 4 % N, zr = z % 4;
-                  const int key = t * 64 + SUB * 32 + zk * 16 + 4 * g + zr;
-                  if ((a.causal && key > qpos + 16 * zq) || key >= a.Skv)
-                    s[SUB][zk][zq][zr] = 0.f;
-                }
+              for (int z = 0; z < E; ++z) {
+                const int zk = z / (4 * N), zq = z / 4 % N, zr = z % 4;
+                const int key = t * 64 + SUB * 32 + zk * 16 + 4 * g + zr;
+                if ((a.causal && key > qpos + 16 * zq) || key >= a.Skv)
+                  s[SUB][zk][zq][zr] = 0.f;
               }
+            }
+          } else {
+            constexpr int j = i - 2 * E, w = j / 3, k = w / (2 * N), q = w / 2 % N, r = w % 2 * 2;   // pair w
+            if constexpr (j % 3 < 2) {
+              float y = dp[k][q][r + j % 3] * s[SUB][k][q][r + j % 3];
+              here(y);
+              dp[k][q][r + j % 3] = y;
             } else {
-              constexpr int j = i - 2 * E, w = j / 3, k = w / (2 * N), q = w / 2 % N, r = w % 2 * 2;   // pair w
-              if constexpr (j % 3 < 2) {
-                float y = dp[k][q][r + j % 3] * s[SUB][k][q][r + j % 3];
-                here(y);
-                dp[k][q][r + j % 3] = y;
-              } else {
-                typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-                unsigned y = __builtin_bit_cast(unsigned, bf16x2_t{(__bf16)dp[k][q][r], (__bf16)dp[k][q][r + 1]});
-                here(y);
-                e[SUB][q][k * 2 + r / 2] = y;
-              }
+              typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+              unsigned y = __builtin_bit_cast(unsigned, bf16x2_t{(__bf16)dp[k][q][r], (__bf16)dp[k][q][r + 1]});
+              here(y);
+              e[SUB][q][k * 2 + r / 2] = y;
             }
           }
         });

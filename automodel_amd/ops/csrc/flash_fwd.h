@@ -36,10 +36,9 @@ struct FwdTile {
   static_assert(F % 2 == 0 && RING <= F1 && SMEM <= 160 * 1024 && BM * VR <= SMEM, "places, tiles; the result in them");
   static_assert((DQK / 32 + DV / 16) * N * 4 <= 256, "Q and the output in AGPRs");
 
-  // The slot of operation i behind the MFMAs. By threes: multiply and add of a score, exponential of the
+  // Operations behind the MFMAs, but the last two. By threes: multiply and add of a score, exponential of the
   // one before, sum with the one before that; then the roundings.
   static constexpr int E = 8 * N, EXPS = 3 * (E + 2), OPS = EXPS + E / 2;
-  static constexpr int slot(int i) { return i * (N * F - 2) / OPS; }
 };
 
 __device__ __forceinline__ unsigned pair(float a, float b) {
@@ -241,30 +240,28 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_ordered_kernel(const Args a)
         }
         if constexpr (m == N * F1 + 4)
           if (mask) hide(s[O], key0);
-        unrolled<T::OPS>([&](auto i_) __attribute__((always_inline)) {
+        spread<m, SLOTS - 2, T::OPS>([&](auto i_) __attribute__((always_inline)) {
           constexpr int i = decltype(i_)::value, E = T::E;
-          if constexpr (T::slot(i) == m) {
-            constexpr int v = i / 3 - i % 3, k = v / (4 * N), q = v / 4 % N, r = v % 4;
-            if constexpr (i < T::EXPS) {
-              if constexpr (v >= 0 && v < E) {
-                if constexpr (i % 3 == 2) {
-                  if constexpr (k == 0 && r == 0) ls[q] = s[SUB][k][q][r];
-                  else ls[q] += s[SUB][k][q][r];
-                  here(ls[q]);
-                } else {
-                  float y = s[SUB][k][q][r];
-                  if constexpr (i % 3 == 0) y = fmaf(y, c, -mc[q]);
-                  else y = __builtin_amdgcn_exp2f(y);
-                  here(y);
-                  s[SUB][k][q][r] = y;
-                }
+          constexpr int v = i / 3 - i % 3, k = v / (4 * N), q = v / 4 % N, r = v % 4;
+          if constexpr (i < T::EXPS) {
+            if constexpr (v >= 0 && v < E) {
+              if constexpr (i % 3 == 2) {
+                if constexpr (k == 0 && r == 0) ls[q] = s[SUB][k][q][r];
+                else ls[q] += s[SUB][k][q][r];
+                here(ls[q]);
+              } else {
+                float y = s[SUB][k][q][r];
+                if constexpr (i % 3 == 0) y = fmaf(y, c, -mc[q]);
+                else y = __builtin_amdgcn_exp2f(y);
+                here(y);
+                s[SUB][k][q][r] = y;
               }
-            } else {
-              constexpr int w = i - T::EXPS, wk = w / (2 * N), wq = w / 2 % N, wr = w % 2 * 2;   // pair w
-              unsigned y = pair(s[SUB][wk][wq][wr], s[SUB][wk][wq][wr + 1]);
-              here(y);
-              e[SUB][wq][wk * 2 + wr / 2] = y;
             }
+          } else {
+            constexpr int w = i - T::EXPS, wk = w / (2 * N), wq = w / 2 % N, wr = w % 2 * 2;   // pair w
+            unsigned y = pair(s[SUB][wk][wq][wr], s[SUB][wk][wq][wr + 1]);
+            here(y);
+            e[SUB][wq][wk * 2 + wr / 2] = y;
           }
         });
         if constexpr (SUB == 0) {

@@ -36,14 +36,23 @@ __device__ __forceinline__ void mfma_next_v(f32x4_t& d, bf16x8_t a, bf16x8_t b) 
 template <class T>
 __device__ __forceinline__ void here(T& x) { asm volatile("" : "+v"(x)); }
 
-// f(0), ..., f(N - 1) with compile-time arguments
-template <class F, int... I>
+// f(FROM), ..., f(FROM + N - 1) with compile-time arguments
+template <int FROM, class F, int... I>
 __device__ __forceinline__ void unrolled_(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
+  (f(std::integral_constant<int, FROM + I>{}), ...);
 }
-template <int N, class F>
+template <int N, int FROM = 0, class F>
 __device__ __forceinline__ void unrolled(F&& f) {
-  unrolled_(f, std::make_integer_sequence<int, N>{});
+  unrolled_<FROM>(f, std::make_integer_sequence<int, N>{});
+}
+
+// OPS operations spread over SLOTS slots, operation i in slot i SLOTS / OPS: f(i) for those of slot M. (Only
+// these are expanded: a test of each operation in each slot took three quarters of the compile time.)
+template <int M, int SLOTS, int OPS, class F>
+__device__ __forceinline__ void spread(F&& f) {
+  constexpr int from = (M * OPS + SLOTS - 1) / SLOTS, to = ((M + 1) * OPS + SLOTS - 1) / SLOTS;
+  constexpr int first = from < OPS ? from : OPS, end = to < OPS ? to : OPS;
+  unrolled<end - first, first>(f);
 }
 
 // The 16-byte slot of a row's chunk c is c ^ place(row): no conflicts between the 32 bytes of 8 rows
