@@ -11,6 +11,9 @@ TORCH_LIBRARY_FRAGMENT(amd_ops, m) {
       "flash_attn_fwd(Tensor q, Tensor k, Tensor v, float scale, bool causal, "
       "int q_start=0, Tensor? doc_start=None, Tensor? sink=None) -> (Tensor, Tensor)");
   m.impl("flash_attn_fwd", &amd_ops::flash_attn_fwd);
+  m.def("flash_attn_fwd_ordered(int B, int Sq, int Skv, int Hq, int Hk, int Dqk, int Dv, bool causal, "
+        "int q_start=0) -> int");
+  m.impl("flash_attn_fwd_ordered", &amd_ops::flash_attn_fwd_ordered);
 
   m.def(
       "gemv_bf16(Tensor x, Tensor w, Tensor? bias, bool relu2=False, bool out_f32=False, "

@@ -24,6 +24,8 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 
+#include <climits>
+
 #include "common.h"
 #include "flash_fwd.h"
 #include "flash_tile.h"
@@ -311,6 +313,9 @@ static void launch_fwd_ordered(const FwdArgs& a, hipStream_t stream) {
   HIP_CHECK_KERNEL();
 }
 
+template <int N>
+static long ordered_blocks(const FwdArgs& a) { return (long)((a.Sq + 64 * N - 1) / (64 * N)) * a.Hq * a.B; }
+
 // Sixteens of rows a wave of the kernel in a given order, or 0: the one above. Times in us, the kernel above
 // first; batch x length, heads.
 //
@@ -320,9 +325,6 @@ static void launch_fwd_ordered(const FwdArgs& a, hipStream_t stream) {
 // one, whose last tiles are wasted on most waves, long rows, and two rounds (1 x 8000, 16: 277 and 251;
 // 1 x 16384, 32: 2020 and 1843; but 2 x 6000, 16: 294 and 304; 1 x 8192, 8: 183 and 228). Few queries
 // leave its waves empty rows (8 x 64 of 4096 keys, 32: 102 and 134).
-template <int N>
-static long ordered_blocks(const FwdArgs& a) { return (long)((a.Sq + 64 * N - 1) / (64 * N)) * a.Hq * a.B; }
-
 static int ordered_rows_128(const FwdArgs& a) {
   if (a.Sq < 1024) return 0;
   const long blocks = ordered_blocks<4>(a), rounds = (blocks + 255) / 256;
@@ -353,6 +355,22 @@ static int ordered_rows_192(const FwdArgs& a) {
   const double c4 = cost(b4, 256), c3 = cost(b3, 192) * 0.77;
   if (a.Skv >= 3000) return c3 < c4 ? 3 : 4;
   return (a.Skv >= 512 && b3 <= 256) || (a.Skv >= 2048 && c3 < 0.9 * c4) ? 3 : 0;
+}
+
+// of any dims, without documents
+static int ordered_rows(const FwdArgs& a, int Dqk, int Dv) {
+  if (Dv != 128 || (Dqk != 128 && Dqk != 192)) return 0;
+  return Dqk == 128 ? ordered_rows_128(a) : ordered_rows_192(a);
+}
+
+int64_t flash_attn_fwd_ordered(int64_t B, int64_t Sq, int64_t Skv, int64_t Hq, int64_t Hk, int64_t Dqk, int64_t Dv,
+                               bool causal, int64_t q_start) {
+  TORCH_CHECK(std::min({B, Sq, Skv, Hq, Hk}) >= 1 && std::max({B, Sq, Skv, Hq, Hk, q_start}) <= INT_MAX &&
+                  Hq % Hk == 0 && q_start >= 0, "flash_attn_fwd_ordered: sizes");
+  FwdArgs a{};
+  a.B = (int)B; a.Sq = (int)Sq; a.Skv = (int)Skv; a.Hq = (int)Hq; a.Hk = (int)Hk; a.q_start = (int)q_start;
+  a.causal = causal;
+  return ordered_rows(a, (int)Dqk, (int)Dv);
 }
 
 std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
@@ -397,12 +415,11 @@ std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
   // (120 us; 4 waves at one a SIMD were 1.3 times slower); (192, 192) would spill at two a SIMD (457
   // against 178 us).
   bool done = false;
-  if (!varlen && Dv == 128 && (Dqk == 128 || Dqk == 192)) {
-    const int n = Dqk == 128 ? ordered_rows_128(a) : ordered_rows_192(a);
-    done = n > 0;
-    if (n > 0 && Dqk == 128) launch_fwd_ordered<128, 128, 4>(a, stream);
+  if (const int n = varlen ? 0 : ordered_rows(a, Dqk, Dv); n > 0) {
+    done = true;
+    if (Dqk == 128) launch_fwd_ordered<128, 128, 4>(a, stream);
     else if (n == 4) launch_fwd_ordered<192, 128, 4>(a, stream);
-    else if (n == 3) launch_fwd_ordered<192, 128, 3>(a, stream);
+    else launch_fwd_ordered<192, 128, 3>(a, stream);
   }
 #define FA_FWD_CASE(A, C, W, OCC)                             \
   if (!done && Dqk == A && Dv == C) {                         \

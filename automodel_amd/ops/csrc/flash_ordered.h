@@ -12,8 +12,9 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
 // Products into vector registers, of an operand from LDS and one that stays in AGPRs. The compiler does
-// not know what these are (see gt::mfma): their results are read, and their operands written
-// by vector instructions, at least 16 MFMAs away.
+// not know what these are (see gt::mfma). Their operands are written by vector instructions at least 16
+// MFMAs away. Their results are read by those at least 5 MFMAs of 16 cycles later (the closest is `hide` in
+// flash_fwd.h), or after gt::settle.
 __device__ __forceinline__ void mfma_first(f32x4_t& d, bf16x8_t a, bf16x8_t b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "a"(b));
 }

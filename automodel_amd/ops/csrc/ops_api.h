@@ -93,6 +93,9 @@ std::tuple<at::Tensor, at::Tensor> doc_bounds(const at::Tensor& cu, int64_t tota
 at::Tensor kv_decode_attn(const at::Tensor& q, const at::Tensor& k_new, const at::Tensor& v_new,
                           at::Tensor k_cache, at::Tensor v_cache, int64_t pos,
                           const std::optional<at::Tensor>& pos_dev, double scale);
+// sixteens of rows a wave of the kernel in a given order, for a forward without documents; 0: the other one
+int64_t flash_attn_fwd_ordered(int64_t B, int64_t Sq, int64_t Skv, int64_t Hq, int64_t Hk, int64_t Dqk, int64_t Dv,
+                               bool causal, int64_t q_start);
 // rows of W a workgroup, slots of its rings and waves that 3 to 16 rows of x take (see gemv.hip)
 std::tuple<int64_t, int64_t, int64_t> decode_rows_shape(at::IntArrayRef n, int64_t K, int64_t B, bool glu,
                                                         int64_t group_n);

@@ -222,6 +222,35 @@ def test_backward_that_is_followed():
     assert count.get_total_flops() == 4 * T * 16384 * 2048
 
 
+@gpu
+@cuda
+@pytest.mark.parametrize("kept", ["hooks", "cpu", "checkpoint", "reentrant"])
+def test_what_is_kept_for_the_backward(kept):
+    from torch.utils.checkpoint import checkpoint
+
+    T, N, K = 4096, 4096, 4096
+    torch.manual_seed(0)
+    lin = nn.Linear(K, N, bias=False, device="cuda", dtype=torch.bfloat16)
+    x, g, seen = rand(T, K).requires_grad_(), rand(T, N), []
+    if kept == "hooks":
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t.shape) or t, lambda t: t):
+            y = L.linear(lin, x)
+        assert sorted(seen) == sorted([x.shape, lin.weight.shape])
+    elif kept == "cpu":
+        with torch.autograd.graph.save_on_cpu():
+            y = L.linear(lin, x)
+    else:
+        y = checkpoint(lambda t: L.linear(lin, t), x, use_reentrant=kept == "reentrant")
+    (y * g).sum().backward()
+    close(x.grad, g.double() @ lin.weight.double())
+    close(lin.weight.grad, g.double().t() @ x.double())
+    z = L.linear(lin, x)
+    with torch.no_grad():
+        lin.weight.mul_(2)                       # what the backward needs is gone, as with F.linear
+    with pytest.raises(RuntimeError, match="modified by an inplace"):
+        z.sum().backward()
+
+
 def test_backward_that_is_followed_elsewhere(monkeypatch):
     # which products a backward takes, with the kernels' part played by Python
     from torch.utils.flop_counter import FlopCounterMode
