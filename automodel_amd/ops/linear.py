@@ -126,7 +126,7 @@ def linear(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
     # Traced calls first: a size that is looked at there becomes a condition of what was traced.
     # Then the size: small layers are bound by the host.
     if (not torch.compiler.is_compiling() and type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda
-            and x.dtype == torch.bfloat16 and not torch.jit.is_tracing() and type(lin) is nn.Linear
+            and x.dtype == torch.bfloat16 and not torch._C._is_tracing() and type(lin) is nn.Linear
             and x.numel() * lin.out_features >= MIN_PRODUCTS
             and torch.is_grad_enabled() and lin.bias is None):
         w = lin.weight
