@@ -1,7 +1,7 @@
 """Causal (flash-style) attention: CDNA4 HIP kernel + sdpa/eager references.
 
 Replaces the reference's TE DotProductAttention / flash-attn / FlexAttention
-backends (SURVEY §2.9 #10-#12) with one in-tree HIP flash kernel
+backends with one in-tree HIP flash kernel
 (csrc/flash_attn.hip): BSHD layout, GQA, online softmax, MFMA 32x32 tiles,
 LDS-staged K/V, fused backward (dKV kv-parallel + dQ q-parallel kernels).
 
@@ -174,8 +174,8 @@ def flash_attention_varlen(q, k, v, cu_seqlens: torch.Tensor, scale: float | Non
 
     GPU path: ONE kernel launch per batch — per-token doc bounds gate the
     causal mask inside the HIP kernel and clip KV-tile ranges per block
-    (replaces the round-1 per-document launch loop with its host-side
-    cu_seqlens.tolist() sync; reference THD runtime thd_utils.py:85).
+    (a launch per document would wait for cu_seqlens on the host; reference
+    THD runtime thd_utils.py:85).
     CPU path: one sdpa call with a dense block-causal mask.
     """
     assert q.shape[0] == 1, "varlen expects a packed THD batch [1, T, H, D]"

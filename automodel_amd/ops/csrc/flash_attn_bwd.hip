@@ -548,9 +548,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
   const bf16* op = reinterpret_cast<const bf16*>(o.data_ptr());
 
   // Waves per SIMD and pipelining by what fits the registers and LDS; dK/dV need one wave a
-  // SIMD from head dim 96 on (at two a SIMD it spills), and for values of 128 columns there is
-  // the ordered kernel, whose tiles fit LDS, for all but the shortest walks. dQ of 128/128 at two waves a SIMD overlaps as well without the third K
-  // buffer (379 against 392 us); (192, 128) would spill there (461 against 203 us).
+  // SIMD from head dim 96 on (at two a SIMD it spills); values of 128 columns have the ordered kernel for
+  // all but the shortest walks. dQ of 128/128 at two waves a SIMD overlaps as well without the third
+  // K buffer (379 against 392 us); (192, 128) would spill there (461 against 203 us).
   bool done = false;
 #define FA_BWD_CASE(A, C, KV_OCC, KV_PIPE, Q_OCC, Q_PIPE)                                 \
   if (!done && Dqk == A && Dv == C) {                                                     \

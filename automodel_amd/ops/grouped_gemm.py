@@ -7,11 +7,11 @@ grouped dx (NN) and dw (TN) kernels — no per-expert loop, no atomics.
 
 With ``counts`` as a DEVICE int tensor the (offs, tile_map, n_tiles) plan is
 built by a device kernel (build_group_plan) so the hot path never syncs the
-routing counts to the host (the round-1 counts.tolist() cost one device sync
-per MoE layer per direction).
+routing counts to the host (a counts.tolist() costs one device sync per MoE
+layer per direction).
 
 Replaces the reference's grouped_gemm / torch._grouped_mm expert backends
-(nemo_automodel/components/moe/experts.py:656, SURVEY §2.9 #14).
+(nemo_automodel/components/moe/experts.py:656).
 """
 
 from __future__ import annotations
@@ -93,8 +93,7 @@ class _GroupedLinear(torch.autograd.Function):
         x, w = ctx.saved_tensors
         g = g.contiguous()
         offs, tile_map, n_tiles = ctx.plan
-        # single-kernel grouped backward; dw's TN
-        # kernel needs N%128 and K%128
+        # single-kernel grouped backward; dw's TN kernel needs N%128 and K%128
         if ctx.use_hip and w.shape[1] % 128 == 0 and w.shape[2] % 128 == 0:
             ops = hip_ops()
             dx = ops.grouped_gemm_nn(g, w.contiguous(), offs, tile_map, n_tiles, ctx.bm)
@@ -175,7 +174,7 @@ def grouped_linear_pair(x_perm, w1, w2, counts, plan):
 
 
 # ===========================================================================
-# fp8 grouped forward (SURVEY §2.5 MXFP8-grouped equivalent): tensorwise
+# fp8 grouped forward (the reference has MXFP8 groups): tensorwise
 # delayed scaling exactly like quantization/fp8.py Float8Linear — the step's
 # activation scale comes from LAST step's recorded amax (margin 1.25x), the
 # whole expert stack shares one cached e4m3 cast refreshed when the

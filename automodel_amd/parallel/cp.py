@@ -1,6 +1,6 @@
 """Context parallelism: zigzag sequence sharding + all-gather-KV attention.
 
-Reference behavior (SURVEY §2.4 CP rows): the reference ships five CP
+Reference behavior: the reference ships five CP
 mechanisms; the canonical MI355X one here is all-gather KV over the cp group
 (RCCL all-gather over xGMI — for a single node the 7 direct links make one
 large all-gather cheaper than per-step ring P2P) with zigzag (2-chunk
@@ -169,8 +169,7 @@ def cp_blockdiag_attention(q, k, v, cu_seqlens: torch.Tensor,
     cuts documents.
 
     GPU path: the native varlen flash kernel with per-token doc bounds and
-    ``q_start`` — O(T) metadata, no dense mask, one launch per chunk
-    (round-1 materialized an O(S_local x T) mask).
+    ``q_start`` — O(T) metadata, no dense mask, one launch per chunk.
     CPU path keeps the dense-mask sdpa reference (parity tests)."""
     import math
 
@@ -210,8 +209,7 @@ def cp_blockdiag_attention(q, k, v, cu_seqlens: torch.Tensor,
 
 # ===========================================================================
 # Ring-P2P KV context parallelism (reference's ring exchange strategy,
-# context_parallel/exchange.py ring mode; VERDICT r1 §2.4: "no ring-P2P KV
-# rotate"). Peak KV memory is O(S/P) per step instead of the all-gather
+# context_parallel/exchange.py ring mode). Peak KV memory is O(S/P) per step instead of the all-gather
 # path's O(S): each rank's zigzag KV block rotates around the cp ring
 # (P2P isend/irecv — on xGMI these ride the direct per-pair links), and
 # attention partials merge by online softmax in fp32. Backward makes the
