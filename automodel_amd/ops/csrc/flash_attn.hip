@@ -320,8 +320,9 @@ static long ordered_blocks(const FwdArgs& a) { return (long)((a.Sq + 64 * N - 1)
 // first; batch x length, heads.
 //
 // (128, 128): a workgroup has 256 rows and a CU, against 128 and half of one. Without a mask it wants
-// full rounds of workgroups (1 x 8192, 8: 264 and 228; 8 x 1024, 32: 179 and 156; 2 x 1024, 32: 42.5 and
-// 42.3; but 1 x 5000, 32, two and a half rounds: 406 and 424; 4 x 512, 32: 27.5 and 28.6). With a causal
+// full rounds of workgroups, counted in rows, as the last workgroup of a sequence may be nearly empty (1 x 8192,
+// 8: 264 and 228; 8 x 1024, 32: 179 and 156; 2 x 1024, 32: 42.5 and 42.3; but 1 x 5000, 32, two and a half
+// rounds: 406 and 424; 1672, 128 in all, 0.82 of four: 222 and 250; 4 x 512, 32: 27.5 and 28.6). With a causal
 // one, whose last tiles are wasted on most waves, long rows, and two rounds (1 x 8000, 16: 277 and 251;
 // 1 x 16384, 32: 2020 and 1843; but 2 x 6000, 16: 294 and 304; 1 x 8192, 8: 183 and 228). Few queries
 // leave its waves empty rows (8 x 64 of 4096 keys, 32: 102 and 134).
@@ -329,7 +330,7 @@ static int ordered_rows_128(const FwdArgs& a) {
   if (a.Sq < 1024) return 0;
   const long blocks = ordered_blocks<4>(a), rounds = (blocks + 255) / 256;
   if (a.causal) return a.Skv >= 8000 && blocks >= 512 ? 4 : 0;
-  return a.Skv >= 1024 && 8 * blocks >= 7 * 256 * rounds ? 4 : 0;
+  return a.Skv >= 1024 && (double)a.Sq * a.Hq * a.B >= 0.85 * 65536 * rounds ? 4 : 0;
 }
 
 // (192, 128): 4 sixteens against 3, which take 0.77 of the time of 4: by rounds of workgroups without a
@@ -348,9 +349,15 @@ static int ordered_rows_192(const FwdArgs& a) {
     return a.Skv >= 1024 ? 4 : 0;
   }
   const double longest = std::min<long>((long)a.q_start + a.Sq, a.Skv);
+  // the workgroups in the order of their lengths, the longest first: the two that follow one another on
+  // a CU are about as long together everywhere, and of an odd number of rounds the last one begins with its
+  // longest (3465, 32 in all: 608 workgroups of 192 rows, 170 us, 150 the kernel above, 149 in fours)
   auto cost = [&](long blocks, int rows) {
-    const double first = std::min<long>((long)a.q_start + rows, a.Skv);
-    return std::max(longest, (double)blocks * (longest + first) / 512);
+    const double first = std::min<long>((long)a.q_start + rows, a.Skv), all = blocks * (longest + first) / 2;
+    const long k = (blocks + 255) / 256, pairs = k / 2 * 2;
+    if (k == 1) return longest;
+    const double before = pairs * (256. * pairs - 1) / 2 + (k > pairs ? 256. * pairs : 0.);
+    return std::max({longest, all / 256, k * longest - (longest - first) * before / (blocks - 1)});
   };
   const double c4 = cost(b4, 256), c3 = cost(b3, 192) * 0.77;
   if (a.Skv >= 3000) return c3 < c4 ? 3 : 4;

@@ -54,3 +54,16 @@ def test_attention_backward():
         assert ordered(8, 64, 4096, 32, 32, *dims, causal=False) == (False, False)
         assert ordered(8, 4096, 4096, 32, 32, *dims) == (True, True)
     assert ordered(8, 4096, 4096, 32, 32, 64, 64) == ordered(8, 4096, 4096, 32, 32, 256, 256) == (False, False)
+
+
+def test_attention_forward():
+    def rows(S, heads, d, causal, B=1):
+        return hip_ops().flash_attn_fwd_ordered(B, S, S, heads, heads, d, 128, causal)
+
+    # without a mask full rounds of workgroups of 256 rows, counted in rows: 7 x 256 for 1672 are not
+    assert rows(1024, 64, 128, False) == rows(7103, 8, 128, False) == 4
+    assert rows(1672, 128, 128, False) == rows(1672, 32, 128, False, 4) == rows(5000, 32, 128, False) == 0
+    # with one: the last of three rounds begins with its longest workgroup
+    assert rows(3001, 32, 192, True) == 3 and rows(3465, 32, 192, True) == 4
+    assert rows(2048, 32, 192, True) == 3 and rows(2048, 48, 192, True) == 0
+    assert rows(8192, 16, 192, True) == 4 and rows(16384, 32, 128, True) == 4 and rows(6000, 32, 128, True) == 0
