@@ -56,7 +56,7 @@ def _adapter_grads(ctx, g, x2, wa, wb, t):
     """(g, dA, dB, dt, A^T), dt the gradient of t, on csrc/lora_grad.hip, the last two with zeros behind the rank;
     A^T None where the backward is followed or recorded itself, or the kernels do not take the tensors."""
     g = g.contiguous()
-    if (ctx.turned and not torch.is_grad_enabled() and not followed() and _ordinary(g, x2, wa, wb, t)
+    if (ctx.turned and g.shape[0] > 0 and not torch.is_grad_enabled() and not followed() and _ordinary(g, x2, wa, wb, t)
             and _plain(g, x2, wa, wb, t) and max(*g.shape, x2.shape[1]) < MAX_SIZE):
         from automodel_amd.ops._backend import hip_ops
 

@@ -83,7 +83,7 @@ def test_input_grad_with_an_extra_product(T, N, K, R):
 
 @pytest.mark.parametrize("rank", [8, 32, 48])
 @pytest.mark.parametrize("T,K,N,need_x", [(2048, 2048, 2560, True), (2048, 2048, 2560, False), (64, 128, 192, True),
-                                          (8, 64, 64, True)])
+                                          (8, 64, 64, True), (0, 128, 192, True)])
 def test_adapted_layer(T, K, N, need_x, rank):
     from automodel_amd.peft.lora import LinearLoRA
 

@@ -79,3 +79,11 @@ def test_once_and_twice(kernels, kind, rank):
                                               materialize_grads=True))
         for u, v in zip(*second):
             torch.testing.assert_close(u, v)
+
+
+@pytest.mark.parametrize("rank", [8, 32])
+@pytest.mark.parametrize("kind", ["linear", "fused"])
+def test_no_rows(kernels, kind, rank):
+    x, w, a, b, g = layer(0, rank)
+    for d, of in zip(torch.autograd.grad(kinds(x, w, a, b)[kind](), (x, a, b), g), (x, a, b)):
+        assert d.shape == of.shape and not d.any()
