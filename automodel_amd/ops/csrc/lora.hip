@@ -367,7 +367,8 @@ at::Tensor sgmv_fused_fwd(const at::Tensor& x, const at::Tensor& A, const at::Te
   return out;
 }
 
-// t = scale x A^T [M, r rounded up to 32] with zeros behind r, and t^T, M rounded up to 64, with zeros behind M
+// t = scale x A^T [M, r rounded up to 32] with zeros behind r, and t^T, M rounded up to 64, with zeros behind M; x and A
+// at multiples of 16 bytes
 void lora_down(const at::Tensor& x, const at::Tensor& A, at::Tensor* t, at::Tensor* turned, double scale) {
   const long M = x.size(0), pitch = (M + 63) / 64 * 64, blocks = ((turned ? pitch : M) + DOWN - 1) / DOWN;
   // (a grid has 2^32 threads; a lane's offsets of 64 rows are 32 bits)
@@ -413,9 +414,11 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> forward(const std::optional<at::T
   TORCH_CHECK(blocks < (1l << 24), "lora_apply: too many rows");
   auto stream = c10::hip::getCurrentHIPStream().stream();
   const bf16* yp = y ? reinterpret_cast<const bf16*>(y->data_ptr()) : nullptr;
+  // lora_down's loads take whole pieces of 16 bytes; a view into a larger buffer may lie anywhere
+  const auto whole = [](const at::Tensor& v) { return (uintptr_t)v.data_ptr() % 16 ? v.clone() : v; };
   auto run = [&](auto rank) {
     constexpr int RANK = rank.value;
-    lora_down(x, A, &t, turn ? &turned : nullptr, 1.);
+    lora_down(whole(x), whole(A), &t, turn ? &turned : nullptr, 1.);
     hipLaunchKernelGGL((lora_up_kernel<RANK>), dim3((unsigned)blocks), dim3(256), 0, stream, yp,
                        reinterpret_cast<const bf16*>(t.data_ptr()),
                        reinterpret_cast<const bf16*>(B.data_ptr()),

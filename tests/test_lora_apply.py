@@ -25,6 +25,22 @@ def test_lora_apply(M, H, O, R, with_y):
     assert (out.double() - ref).norm() <= 2.0 ** -9 * 1.05 * ref.norm()
 
 
+@pytest.mark.parametrize("at", [1, 2, 3, 4])
+def test_operands_anywhere_in_a_buffer(at):
+    from automodel_amd.ops._backend import hip_ops
+
+    def moved(v):
+        return torch.cat([v.new_zeros(at), v.flatten()])[at:].view(v.shape)
+
+    torch.manual_seed(0)
+    x, A = torch.randn(40, 192, device="cuda").bfloat16(), torch.randn(32, 192, device="cuda").bfloat16()
+    B, y = torch.randn(64, 32, device="cuda").bfloat16(), torch.randn(40, 64, device="cuda").bfloat16()
+    want = hip_ops().lora_forward(y, x, A, B, 0.5)
+    for args in ((y, moved(x), A, B), (y, x, moved(A), B), (y, moved(x), moved(A), B)):
+        assert all(torch.equal(a, b) for a, b in zip(hip_ops().lora_forward(*args, 0.5), want))
+        assert torch.equal(hip_ops().lora_apply(*args, 0.5)[0], want[0])
+
+
 def test_more_rows_than_a_grid_is_high():
     from automodel_amd.ops._backend import hip_ops
 
