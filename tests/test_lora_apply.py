@@ -118,3 +118,23 @@ def test_adapted_layer(T, K, N, need_x, rank):
         for v, ref in zip(grads, (dt.t() @ xd, 2.0 * gd.t() @ (xd @ a.t()), gd @ w + dt @ a)):
             # t and dt are rounded to bf16, some results a few times more
             assert (v.double().view(ref.shape) - ref).norm() <= 2.0 ** -8 * ref.norm()
+
+
+@pytest.mark.parametrize("rank", [8, 32, 40])
+def test_infinite_rows(rank):
+    """They are infinite, and not NaN, where all signs agree, as the modules have them."""
+    from automodel_amd.peft.lora import LinearLoRA
+
+    torch.manual_seed(0)
+    lin = LinearLoRA(torch.nn.Linear(128, 64, bias=False), rank, 2.0 * rank).to("cuda", torch.bfloat16)
+    with torch.no_grad():
+        for p in lin.parameters():
+            p.copy_(torch.rand(p.shape) + 0.1)
+    x, g = (torch.randn(16, n, device="cuda").bfloat16() for n in (128, 64))
+    x[3, 70], x[5, 1], g[2, 7], g[9, 63] = float("inf"), -float("inf"), float("inf"), -float("inf")
+    x.requires_grad_()
+    y = lin(x)
+    dx, = torch.autograd.grad(y, x, g)
+    for got, rows in ((y, (3, 5)), (dx, (2, 9))):
+        assert (got[rows[0]] == float("inf")).all() and (got[rows[1]] == -float("inf")).all()
+        assert got.isfinite().all(1).sum() == 14
