@@ -104,7 +104,7 @@ class _LoRALinear(torch.autograd.Function):
 
             dx = hip_ops().linear_dx_extra(g, w, dt, a_t)
         else:
-            dx = g @ w + dt @ wa
+            dx = g @ w + dt[:, :wa.shape[0]] @ wa
         return dx, None, da, db, None
 
 

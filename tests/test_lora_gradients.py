@@ -87,3 +87,15 @@ def test_no_rows(kernels, kind, rank):
     x, w, a, b, g = layer(0, rank)
     for d, of in zip(torch.autograd.grad(kinds(x, w, a, b)[kind](), (x, a, b), g), (x, a, b)):
         assert d.shape == of.shape and not d.any()
+
+
+@pytest.mark.parametrize("rank", [8, 40])
+def test_a_weight_that_came_back_in_another_form(kernels, monkeypatch, rank):
+    x, w, a, b, g = layer(10, rank)
+    make = kinds(x, w, a, b)
+    plain = lora._plain
+    monkeypatch.setattr(lora, "_plain", lambda *ts: all(t.shape != w.shape for t in ts) and plain(*ts))
+    got, want = (torch.autograd.grad(make[k](), (x, a, b), g) for k in ("linear", "torch"))
+    assert kernels.calls == 1
+    for u, v in zip(got, want):
+        torch.testing.assert_close(u, v)
