@@ -401,8 +401,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> forward(const std::optional<at::T
   TORCH_CHECK(A.dim() == 2 && B.dim() == 2 && A.size(1) == H && B.size(1) == r, "shape mismatch");
   TORCH_CHECK(A.scalar_type() == at::kBFloat16 && B.scalar_type() == at::kBFloat16 && A.is_contiguous() &&
                   B.is_contiguous(), "lora_apply: A [r,H], B [O,r] bf16");
-  TORCH_CHECK((turn ? r >= 8 && r <= 64 && r % 8 == 0 : r == R) && H % 64 == 0 && O % 64 == 0,
-              "lora: r in {32, 64} (lora_forward: a multiple of 8 up to 64), H%64==0, O%64==0");
+  TORCH_CHECK(r >= 8 && r <= 64 && r % 8 == 0 && H % 64 == 0 && O % 64 == 0,
+              "lora: r a multiple of 8 up to 64, H%64==0, O%64==0");
   if (y)
     TORCH_CHECK(y->is_cuda() && y->dim() == 2 && y->size(0) == M && y->size(1) == O && y->is_contiguous() &&
                     y->scalar_type() == at::kBFloat16, "lora_apply: y [M,O] bf16");
@@ -434,7 +434,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> forward(const std::optional<at::T
 
 }  // namespace
 
-// -> (y + scale * (x A^T) B^T, x A^T)
+// r a multiple of 8 up to 64 -> (y + scale * (x A^T) B^T, x A^T [M, r rounded up to 32] with zeros behind r)
 std::tuple<at::Tensor, at::Tensor> lora_apply(const std::optional<at::Tensor>& y, const at::Tensor& x,
                                               const at::Tensor& A, const at::Tensor& B, double scale) {
   const auto r = forward(y, x, A, B, scale, false);
@@ -450,6 +450,7 @@ std::tuple<at::Tensor, at::Tensor> lora_forward(const at::Tensor& y, const at::T
 
 at::Tensor lora_fused_fwd(const at::Tensor& x, const at::Tensor& A, const at::Tensor& B,
                           double scale) {
+  TORCH_CHECK(A.dim() == 2 && (A.size(0) == 32 || A.size(0) == 64), "lora_fused_fwd: r in {32, 64}");
   return std::get<0>(lora_apply(std::nullopt, x.contiguous(), A.contiguous(), B.contiguous(), scale));
 }
 

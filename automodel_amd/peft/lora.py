@@ -42,12 +42,13 @@ class PeftConfig:
         return cls(**{k: (list(v) if k == "target_modules" else v) for k, v in d.items()})
 
 
-def _adapter_forward(ctx, y, x2, wa, wb, scale):
-    """The sum, and what the backward needs of t = x A^T: t^T for the kernels, t where something else follows."""
+def _adapter_forward(ctx, y, x2, wa, wb, scale, recorded):
+    """The sum, and what the backward needs of t = x A^T: t^T for the kernels, t where something else follows, or
+    nothing (``recorded``: whether there is a backward; a function's own forward cannot tell)."""
     from automodel_amd.ops._backend import hip_ops
 
     ctx.scale = scale
-    ctx.turned = wa.shape[0] not in (32, 64) or (any(ctx.needs_input_grad) and not followed())
+    ctx.turned = recorded and any(ctx.needs_input_grad) and not followed()
     op = hip_ops().lora_forward if ctx.turned else hip_ops().lora_apply
     return op(y, x2, wa.contiguous(), wb.contiguous(), scale)
 
@@ -63,8 +64,8 @@ def _adapter_grads(ctx, g, x2, wa, wb, t):
         return (g, *hip_ops().lora_grads(g, x2, wa, wb, t, ctx.scale))
     if torch.is_grad_enabled():        # the backward is recorded itself, and t is no constant to it
         t = x2 @ wa.t()
-    elif ctx.turned:
-        t = t[:wa.shape[0], :x2.shape[0]].t()
+    else:
+        t = t[:wa.shape[0], :x2.shape[0]].t() if ctx.turned else t[:, :wa.shape[0]]
     dt = ((g @ wb) * ctx.scale).to(x2.dtype)
     return g, (dt.t() @ x2).to(wa.dtype), ((g.t() @ t) * ctx.scale).to(wb.dtype), dt, None
 
@@ -74,8 +75,8 @@ class _FusedLoRAFn(torch.autograd.Function):
     lora_forward_kernel): one pass over y, the sum rounded once."""
 
     @staticmethod
-    def forward(ctx, y, x2, wa, wb, scale):
-        out, t = _adapter_forward(ctx, y, x2, wa, wb, scale)
+    def forward(ctx, y, x2, wa, wb, scale, recorded=True):
+        out, t = _adapter_forward(ctx, y, x2, wa, wb, scale, recorded)
         ctx.save_for_backward(x2, wa, wb, t)
         return out
 
@@ -83,7 +84,7 @@ class _FusedLoRAFn(torch.autograd.Function):
     def backward(ctx, g):
         x2, wa, wb, t = ctx.saved_tensors
         g, da, db, dt, _ = _adapter_grads(ctx, g, x2, wa, wb, t)
-        return g, dt[:, :wa.shape[0]] @ wa if ctx.needs_input_grad[1] else None, da, db, None
+        return g, dt[:, :wa.shape[0]] @ wa if ctx.needs_input_grad[1] else None, da, db, None, None
 
 
 class _LoRALinear(torch.autograd.Function):
@@ -91,7 +92,7 @@ class _LoRALinear(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x2, w, wa, wb, scale):
-        out, t = _adapter_forward(ctx, F.linear(x2, w), x2, wa, wb, scale)
+        out, t = _adapter_forward(ctx, F.linear(x2, w), x2, wa, wb, scale, True)
         ctx.save_for_backward(x2, w, wa, wb, t)
         return out
 
@@ -173,7 +174,7 @@ class LinearLoRA(nn.Module):
         if fused and y.dtype == torch.bfloat16:
             x2 = x.reshape(-1, x.shape[-1]).contiguous()
             y2 = y.reshape(-1, wb.shape[0]).contiguous()
-            return _FusedLoRAFn.apply(y2, x2, wa, wb, self.scale).view(y.shape)
+            return _FusedLoRAFn.apply(y2, x2, wa, wb, self.scale, torch.is_grad_enabled()).view(y.shape)
         return y + self.lora_B(self.lora_A(self.dropout(x))) * self.scale
 
     def _fills_up(self, wa: torch.Tensor, wb: torch.Tensor) -> bool:

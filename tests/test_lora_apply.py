@@ -73,6 +73,7 @@ def test_adapter_grads(M, H, O, R):
     A0[:R], B0[:, :R] = A, B                    # what is filled up with zeros
     out2, t = hip_ops().lora_apply(y, x, A0, B0, 0.5)
     assert torch.equal(out, out2) and torch.equal(tt[:, :M], t.t()) and not tt[:, M:].any()
+    assert all(torch.equal(a, b) for a, b in zip(hip_ops().lora_apply(y, x, A, B, 0.5), (out, t)))
     da, db, dt, a_t = hip_ops().lora_grads(g, x, A, B, tt, 0.5)
     assert torch.equal(a_t, A0.t()) and not dt[:, R:].any()
     t, dt = t[:, :R], dt[:, :R]

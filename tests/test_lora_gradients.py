@@ -18,13 +18,14 @@ class Kernels:
         return 32 if r <= 32 else 64
 
     def lora_apply(self, y, x, A, B, scale):
+        Kernels.turned = False
         t = x @ A.t()
-        return y + scale * t @ B.t(), t
+        return y + scale * t @ B.t(), F.pad(t, (0, self._filled(A.shape[0]) - A.shape[0]))
 
     def lora_forward(self, y, x, A, B, scale):
-        M, r = x.shape[0], A.shape[0]
         out, t = self.lora_apply(y, x, A, B, scale)
-        return out, F.pad(t.t(), (0, -M % 64, 0, self._filled(r) - r))
+        Kernels.turned = True
+        return out, F.pad(t.t(), (0, -x.shape[0] % 64))
 
     def lora_grads(self, g, x, A, B, tt, scale):
         Kernels.calls += 1
@@ -96,5 +97,27 @@ def test_a_weight_that_came_back_in_another_form(kernels, monkeypatch, rank):
     monkeypatch.setattr(lora, "_plain", lambda *ts: all(t.data_ptr() != w.data_ptr() for t in ts))
     got, want = (torch.autograd.grad(make[k](), (x, a, b), g) for k in ("linear", "torch"))
     assert kernels.calls == 1
+    for u, v in zip(got, want):
+        torch.testing.assert_close(u, v)
+
+
+@pytest.mark.parametrize("rank", [8, 32])
+def test_what_is_kept(kernels, rank):
+    """t^T only for a backward by the kernels; a followed forward keeps t for torch's products."""
+    x, w, a, b, g = layer(10, rank)
+    y = F.linear(x, w).detach()
+    run = lambda: lora._FusedLoRAFn.apply(y, x, a, b, 0.5, torch.is_grad_enabled())
+    with torch.no_grad():
+        out = run()
+        assert not kernels.turned
+    assert torch.equal(run(), out) and kernels.turned
+    from torch.utils.flop_counter import FlopCounterMode
+
+    make = kinds(x, w, a, b)
+    with FlopCounterMode(display=False):
+        z = make["fused"]()
+    assert not kernels.turned
+    got, want = (torch.autograd.grad(v, (x, a, b), g) for v in (z, make["torch"]()))
+    assert kernels.calls == 0
     for u, v in zip(got, want):
         torch.testing.assert_close(u, v)
