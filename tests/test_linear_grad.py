@@ -106,7 +106,7 @@ def test_layer_of_cut_tiles(T, N, K):
     x, g = rand(T, K).requires_grad_(), rand(T, N)
     assert L.weight_grad_cut(T, N, K) and L.input_grad_cut(T, N, K)
     y = L.linear(lin, x)
-    assert "_Cut" in type(y.grad_fn).__name__ and torch.equal(y, lin(x))
+    assert "_Linear" in type(y.grad_fn).__name__ and torch.equal(y, lin(x))
     dx, dw = torch.autograd.grad(y, (x, lin.weight), g)
     close(dx, g.double() @ lin.weight.double())
     close(dw, g.double().t() @ x.double())
@@ -131,6 +131,7 @@ def test_refusals():
 @pytest.mark.parametrize("T,N,K,dw,dx", [
     (1040, 4096, 4096, True, False), (4095, 1088, 4096, False, True), (2048, 4096, 4096, True, False),
     (4096, 4096, 4096, True, True), (1000, 4096, 4096, False, False), (4096, 4100, 4096, False, False),
+    (300, 4096, 4096, False, False), (16384, 192, 4096, False, False), (200, 8192, 8192, False, False),
 ])
 @pytest.mark.parametrize("train_x,train_w", [(True, True), (True, False), (False, True)])
 def test_layer(monkeypatch, T, N, K, dw, dx, train_x, train_w):
@@ -140,7 +141,9 @@ def test_layer(monkeypatch, T, N, K, dw, dx, train_x, train_w):
     g = rand(1, T, N)
     assert L.weight_grad_wins(T, N, K) == dw and L.input_grad_wins(T, N, K) == dx
     y = L.linear(lin, x)
-    own = (dw and train_w) or (dx and train_x)
+    # whole tiles, or cut ones of sizes from 256 on and 2^33 products
+    cut = min(T, N, K) >= 256 and T * N * K >= 1 << 33 and N % 64 == 0
+    own = (dw or cut) and train_w or (dx or cut) and train_x
     assert ("_Linear" in type(y.grad_fn).__name__) == own
     assert torch.equal(y, lin(x))
     inputs = [t for t in (x, lin.weight) if t.requires_grad]
@@ -160,8 +163,8 @@ def test_layer(monkeypatch, T, N, K, dw, dx, train_x, train_w):
 
 @gpu
 @cuda
-def test_calls_that_stay_the_module(monkeypatch):
-    T, N, K = 4096, 4096, 4096
+@pytest.mark.parametrize("T,N,K", [(4096, 4096, 4096), (2000, 2816, 2048)])        # whole tiles, and cut ones
+def test_calls_that_stay_the_module(monkeypatch, T, N, K):
     x = rand(T, K).requires_grad_()
 
     def own(lin, x=x):
@@ -207,9 +210,11 @@ def test_calls_that_stay_the_module(monkeypatch):
 
 @gpu
 @cuda
-def test_without_the_kernels(monkeypatch):
+@pytest.mark.parametrize("rows", [4096, 1000])
+def test_without_the_kernels(monkeypatch, rows):
     lin = nn.Linear(4096, 4096, bias=False, device="cuda", dtype=torch.bfloat16)
-    x = rand(4096, 4096).requires_grad_()
+    x = rand(rows, 4096).requires_grad_()
+    assert "_Linear" in type(L.linear(lin, x).grad_fn).__name__
     monkeypatch.setattr(L, "_built", lambda: False)
     assert "_Linear" not in type(L.linear(lin, x).grad_fn).__name__
 
