@@ -142,8 +142,6 @@ TORCH_LIBRARY(amd_ops, m) {
       "grouped_gemm_nn2(Tensor g1, Tensor w1, Tensor g2, Tensor w2, Tensor offs, Tensor tile_map, "
       "Tensor? n_tiles=None, int bm=128) -> Tensor");
   m.impl("grouped_gemm_nn2", &amd_ops::grouped_gemm_nn2);
-  m.def("permute_gather(Tensor x, Tensor src) -> Tensor");
-  m.impl("permute_gather", &amd_ops::permute_gather);
   m.def("unpermute_combine(Tensor yp, Tensor pos, Tensor probs) -> Tensor");
   m.impl("unpermute_combine", &amd_ops::unpermute_combine);
   m.def("permute_rows(Tensor x, Tensor pos) -> Tensor");

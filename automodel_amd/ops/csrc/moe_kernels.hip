@@ -2,10 +2,11 @@
 // The bf16 grouped GEMM is in grouped_gemm.hip.
 //   route_topk / expert_load: the router's choice of experts and how often each was chosen.
 //   route_plan: token replicas sorted by expert (stable counting sort), on the device.
-//   permute_gather / unpermute_combine: gather token replicas into expert-
-//     sorted order and combine top-k outputs with routing probs without
-//     materializing the repeat_interleave copy; combine_bwd: the gradients of both
-//     factors in one pass.
+//   route_weights: the chosen experts' weights, and the gradient of the router's logits.
+//   permute_rows / unpermute_combine: write a token's copies to their places in expert-
+//     sorted order, and combine top-k outputs with routing probs, without
+//     materializing the repeat_interleave copy; unpermute_sum: the copies' gradient;
+//     combine_bwd: the gradients of both factors in one pass.
 
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -477,16 +478,6 @@ std::tuple<at::Tensor, at::Tensor> combine_bwd(const at::Tensor& g, const at::Te
 }
 
 // ---- fused permute / unpermute -------------------------------------------
-// gather: y[i, :] = x[src[i], :]
-__global__ void permute_gather_kernel(const bf16* __restrict__ x, bf16* __restrict__ y,
-                                      const int* __restrict__ src, int H, long M) {
-  const long i = blockIdx.x;
-  const bf16* xr = x + (long)src[i] * H;
-  bf16* yr = y + i * (long)H;
-  for (int c = threadIdx.x * 8; c < H; c += blockDim.x * 8)
-    *reinterpret_cast<bf16x8*>(yr + c) = *reinterpret_cast<const bf16x8*>(xr + c);
-}
-
 // y[pos[t, k]] = x[t] for all k: a token's row is read once and its copies' stores go out together, instead of a
 // workgroup for each copy (65536 rows of 2048 columns: 74 us, now 47)
 template <int KS>
@@ -541,20 +532,6 @@ __global__ void unpermute_combine_kernel(const bf16* __restrict__ yp,
     for (int j = 0; j < 8; ++j) o.v[j] = f2bf(accv[j]);
     *reinterpret_cast<bf16x8*>(orow + c) = o;
   }
-}
-
-at::Tensor permute_gather(const at::Tensor& x, const at::Tensor& src) {
-  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.size(1) % 8 == 0,
-              "permute_gather: bf16 [T,H], H%8==0");
-  const long M = src.size(0);
-  const int H = x.size(1);
-  auto y = at::empty({M, (long)H}, x.options());
-  auto stream = c10::hip::getCurrentHIPStream();
-  hipLaunchKernelGGL(permute_gather_kernel, dim3(M), dim3(std::min(256, H / 8)), 0,
-                     stream.stream(), reinterpret_cast<const bf16*>(x.data_ptr()),
-                     reinterpret_cast<bf16*>(y.data_ptr()), src.data_ptr<int>(), H, M);
-  HIP_CHECK_KERNEL();
-  return y;
 }
 
 // x [T, H], pos [T, K]: the place of each token's copies, every place once -> [T * K, H]

@@ -196,7 +196,6 @@ std::tuple<at::Tensor, at::Tensor> combine_bwd(const at::Tensor& g, const at::Te
 at::Tensor grouped_gemm_nn2(const at::Tensor& g1, const at::Tensor& w1, const at::Tensor& g2,
                             const at::Tensor& w2, const at::Tensor& offs, const at::Tensor& tile_map,
                             const std::optional<at::Tensor>& n_tiles, int64_t bm);
-at::Tensor permute_gather(const at::Tensor& x, const at::Tensor& src);
 at::Tensor unpermute_combine(const at::Tensor& yp, const at::Tensor& pos,
                              const at::Tensor& probs);
 

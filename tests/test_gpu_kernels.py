@@ -247,12 +247,12 @@ def test_permute_kernels_parity():
     torch.manual_seed(0)
     T, H, K = 64, 256, 2
     x = torch.randn(T, H, device="cuda", dtype=torch.bfloat16)
-    src = torch.randint(0, T, (T * K,), device="cuda", dtype=torch.int32)
-    y = hip_ops().permute_gather(x, src)
-    assert torch.equal(y, x[src.long()])
+    pos = torch.randperm(T * K, device="cuda", dtype=torch.int32)
+    y = hip_ops().permute_rows(x, pos.view(T, K))
+    src = pos.long().argsort() // K
+    assert torch.equal(y, x[src])
 
     yp = torch.randn(T * K, H, device="cuda", dtype=torch.bfloat16)
-    pos = torch.randperm(T * K, device="cuda", dtype=torch.int32)
     probs = torch.rand(T, K, device="cuda", dtype=torch.float32)
     out = hip_ops().unpermute_combine(yp, pos, probs)
     ref = (yp[pos.long()].view(T, K, H).float() * probs[:, :, None]).sum(1)
