@@ -478,27 +478,34 @@ std::tuple<at::Tensor, at::Tensor> combine_bwd(const at::Tensor& g, const at::Te
 }
 
 // ---- fused permute / unpermute -------------------------------------------
+// A token's choices in groups of 8, of which the last has TAIL (1 to 8): f(first of the group, constant of its size).
+// The loads or stores of a group are expanded and go out together, whatever the number of choices.
+template <int TAIL, typename F>
+__device__ __forceinline__ void choice_groups(int topk, F&& f) {
+  int k = 0;
+  for (; k + TAIL < topk; k += 8) f(k, std::integral_constant<int, 8>{});
+  f(k, std::integral_constant<int, TAIL>{});
+}
+
 // y[pos[t, k]] = x[t] for all k: a token's row is read once and its copies' stores go out together, instead of a
-// workgroup for each copy (65536 rows of 2048 columns: 74 us, now 47)
-template <int KS>
+// workgroup for each copy (65536 rows of 2048 columns, 8 a token: 74 us, now 47; one by one 5 and 9 a token were 69 and 58,
+// now 60 and 48)
+template <int TAIL>
 __global__ void permute_rows_kernel(const bf16* __restrict__ x, bf16* __restrict__ y, const int* __restrict__ pos, int H,
                                     int topk) {
   const long t = blockIdx.x;
-  const int* at = pos + t * (KS ? KS : topk);
+  const int* at = pos + t * topk;
   for (int c = threadIdx.x * 8; c < H; c += blockDim.x * 8) {
     const bf16x8 v = *reinterpret_cast<const bf16x8*>(x + t * H + c);
-    if constexpr (KS > 0) {
+    choice_groups<TAIL>(topk, [&](int k0, auto n) __attribute__((always_inline)) {
 #pragma unroll
-      for (int k = 0; k < KS; ++k) *reinterpret_cast<bf16x8*>(y + (long)at[k] * H + c) = v;
-    } else {
-      for (int k = 0; k < topk; ++k) *reinterpret_cast<bf16x8*>(y + (long)at[k] * H + c) = v;
-    }
+      for (int k = 0; k < decltype(n)::value; ++k) *reinterpret_cast<bf16x8*>(y + (long)at[k0 + k] * H + c) = v;
+    });
   }
 }
 
-// combine: out[t, :] = sum_k probs[t, k] * yp[pos[t*K + k], :], or without probs the sum alone. KS > 0: so many
-// terms, whose loads are issued together.
-template <int KS>
+// combine: out[t, :] = sum_k probs[t, k] * yp[pos[t*K + k], :], or without probs the sum alone
+template <int TAIL>
 __global__ void unpermute_combine_kernel(const bf16* __restrict__ yp,
                                          bf16* __restrict__ out,
                                          const int* __restrict__ pos,
@@ -508,29 +515,38 @@ __global__ void unpermute_combine_kernel(const bf16* __restrict__ yp,
   bf16* orow = out + t * (long)H;
   for (int c = threadIdx.x * 8; c < H; c += blockDim.x * 8) {
     float accv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if constexpr (KS > 0) {
-      bf16x8 v[KS];
+    choice_groups<TAIL>(topk, [&](int k0, auto n) __attribute__((always_inline)) {
+      constexpr int N = decltype(n)::value;
+      const long at = t * topk + k0;
+      bf16x8 v[N];
 #pragma unroll
-      for (int k = 0; k < KS; ++k) v[k] = *reinterpret_cast<const bf16x8*>(yp + (long)pos[t * KS + k] * H + c);
+      for (int k = 0; k < N; ++k) v[k] = *reinterpret_cast<const bf16x8*>(yp + (long)pos[at + k] * H + c);
 #pragma unroll
-      for (int k = 0; k < KS; ++k) {
-        const float p = probs ? probs[t * KS + k] : 1.f;
+      for (int k = 0; k < N; ++k) {
+        const float p = probs ? probs[at + k] : 1.f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) accv[j] += p * bf2f(v[k].v[j]);
       }
-    } else {
-      for (int k = 0; k < topk; ++k) {
-        const float p = probs ? probs[t * topk + k] : 1.f;
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(
-            yp + (long)pos[t * topk + k] * H + c);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) accv[j] += p * bf2f(v.v[j]);
-      }
-    }
+    });
     bf16x8 o;
 #pragma unroll
     for (int j = 0; j < 8; ++j) o.v[j] = f2bf(accv[j]);
     *reinterpret_cast<bf16x8*>(orow + c) = o;
+  }
+}
+
+// f(constant of the last group's size)
+template <typename F>
+static void with_tail(int topk, F&& f) {
+  switch ((topk - 1) % 8) {
+    case 0: return f(std::integral_constant<int, 1>{});
+    case 1: return f(std::integral_constant<int, 2>{});
+    case 2: return f(std::integral_constant<int, 3>{});
+    case 3: return f(std::integral_constant<int, 4>{});
+    case 4: return f(std::integral_constant<int, 5>{});
+    case 5: return f(std::integral_constant<int, 6>{});
+    case 6: return f(std::integral_constant<int, 7>{});
+    default: return f(std::integral_constant<int, 8>{});
   }
 }
 
@@ -543,16 +559,11 @@ at::Tensor permute_rows(const at::Tensor& x, const at::Tensor& pos) {
   const int H = x.size(1), topk = pos.size(1);
   auto y = at::empty({T * topk, (long)H}, x.options());
   if (y.numel() == 0) return y;
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(T), dim3(std::min(256, H / 8)), 0, c10::hip::getCurrentHIPStream().stream(),
-                       reinterpret_cast<const bf16*>(x.data_ptr()), reinterpret_cast<bf16*>(y.data_ptr()),
-                       pos.data_ptr<int>(), H, topk);
-  };
-  if (topk == 2) launch(permute_rows_kernel<2>);
-  else if (topk == 4) launch(permute_rows_kernel<4>);
-  else if (topk == 6) launch(permute_rows_kernel<6>);
-  else if (topk == 8) launch(permute_rows_kernel<8>);
-  else launch(permute_rows_kernel<0>);
+  with_tail(topk, [&](auto tail) {
+    hipLaunchKernelGGL((permute_rows_kernel<decltype(tail)::value>), dim3(T), dim3(std::min(256, H / 8)), 0,
+                       c10::hip::getCurrentHIPStream().stream(), reinterpret_cast<const bf16*>(x.data_ptr()),
+                       reinterpret_cast<bf16*>(y.data_ptr()), pos.data_ptr<int>(), H, topk);
+  });
   HIP_CHECK_KERNEL();
   return y;
 }
@@ -561,16 +572,12 @@ static at::Tensor combine(const at::Tensor& yp, const int* pos, const float* pro
   const int H = yp.size(1);
   auto out = at::empty({T, (long)H}, yp.options());
   if (T == 0) return out;
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(T), dim3(std::min(256, H / 8)), 0, c10::hip::getCurrentHIPStream().stream(),
-                       reinterpret_cast<const bf16*>(yp.data_ptr()), reinterpret_cast<bf16*>(out.data_ptr()), pos, probs,
-                       H, topk, T);
-  };
-  if (topk == 2) launch(unpermute_combine_kernel<2>);
-  else if (topk == 4) launch(unpermute_combine_kernel<4>);
-  else if (topk == 6) launch(unpermute_combine_kernel<6>);
-  else if (topk == 8) launch(unpermute_combine_kernel<8>);
-  else launch(unpermute_combine_kernel<0>);
+  if (topk == 0) return out.zero_();
+  with_tail(topk, [&](auto tail) {
+    hipLaunchKernelGGL((unpermute_combine_kernel<decltype(tail)::value>), dim3(T), dim3(std::min(256, H / 8)), 0,
+                       c10::hip::getCurrentHIPStream().stream(), reinterpret_cast<const bf16*>(yp.data_ptr()),
+                       reinterpret_cast<bf16*>(out.data_ptr()), pos, probs, H, topk, T);
+  });
   HIP_CHECK_KERNEL();
   return out;
 }

@@ -234,7 +234,8 @@ def test_gate_of_both_kinds(options, monkeypatch):
         assert (a.float() - b.float()).norm() <= 2.0 ** -8 * b.float().norm()
 
 
-@pytest.mark.parametrize("T,K,H", [(1, 1, 8), (37, 3, 520), (100, 8, 2048), (65, 6, 264), (9, 2, 4096), (20, 4, 16)])
+@pytest.mark.parametrize("T,K,H", [(1, 1, 8), (37, 3, 520), (100, 8, 2048), (65, 6, 264), (9, 2, 4096), (20, 4, 16),
+                                   (33, 5, 264), (17, 7, 128), (12, 9, 64), (5, 16, 40)])
 def test_copies_combine_and_sum(T, K, H):
     from automodel_amd.ops._backend import hip_ops
 
