@@ -70,6 +70,11 @@ def _adapter_grads(ctx, g, x2, wa, wb, t):
     return g, (dt.t() @ x2).to(wa.dtype), ((g.t() @ t) * ctx.scale).to(wb.dtype), dt, None
 
 
+def _of_rank(dt, wa):
+    """Its columns without the zeros behind the rank. (Slices of everything have no batching rule.)"""
+    return dt if dt.shape[1] == wa.shape[0] else dt[:, :wa.shape[0]]
+
+
 class _FusedLoRAFn(torch.autograd.Function):
     """y + (x @ A^T) @ B^T * scale (csrc/lora.hip; reference _peft/lora_kernel.py
     lora_forward_kernel): one pass over y, the sum rounded once."""
@@ -84,7 +89,7 @@ class _FusedLoRAFn(torch.autograd.Function):
     def backward(ctx, g):
         x2, wa, wb, t = ctx.saved_tensors
         g, da, db, dt, _ = _adapter_grads(ctx, g, x2, wa, wb, t)
-        return g, dt[:, :wa.shape[0]] @ wa if ctx.needs_input_grad[1] else None, da, db, None, None
+        return g, _of_rank(dt, wa) @ wa if ctx.needs_input_grad[1] else None, da, db, None, None
 
 
 class _LoRALinear(torch.autograd.Function):
@@ -105,7 +110,7 @@ class _LoRALinear(torch.autograd.Function):
 
             dx = hip_ops().linear_dx_extra(g, w, dt, a_t)
         else:
-            dx = g @ w + dt[:, :wa.shape[0]] @ wa
+            dx = g @ w + _of_rank(dt, wa) @ wa
         return dx, None, da, db, None
 
 

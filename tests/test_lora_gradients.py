@@ -121,3 +121,14 @@ def test_what_is_kept(kernels, rank):
     assert kernels.calls == 0
     for u, v in zip(got, want):
         torch.testing.assert_close(u, v)
+
+
+@pytest.mark.parametrize("rank", [8, 32])
+@pytest.mark.parametrize("kind", ["linear", "fused"])
+def test_batched(kernels, kind, rank):
+    x, w, a, b, g = layer(10, rank)
+    make, gs = kinds(x, w, a, b), torch.stack([g, g.flip(0)])
+    got, want = (torch.autograd.grad(make[k](), (x, a, b), gs, is_grads_batched=True) for k in (kind, "torch"))
+    assert kernels.calls == 0
+    for u, v in zip(got, want):
+        torch.testing.assert_close(u, v)
