@@ -516,9 +516,9 @@ static bool dkv_ordered(const BwdArgs& a) {
 // a tile takes, how many workgroups a CU has, and the memory's rate: the longest walk or all of them on all
 // CUs, 4 tiles' time for a workgroup's beginning and end, and the adding. Of packed rows the lengths are not
 // known here: cuts at random have their longest document at about (ln n + 0.6) of the mean, and half their
-// tokens lie in documents of twice that. Whole backward, cut over uncut, 204 shapes of 100 to 16000 queries:
-// 0.78 in the mean, 0.28 (1 x 2048, 8/2 heads of 256) to 1.02, one at 1.05; 48 of packed rows 0.80, 0.33 to
-// 1.0. Always the best of 1, 2, 3, 4, 6 and 8 parts would be 1.2% faster.
+// tokens lie in documents of twice that. Whole backward, cut over uncut, 198 shapes of 100 to 16000 queries:
+// 0.79 in the mean, 0.27 (1 x 2048, 8/2 heads of 256) to 1.0; 48 of packed rows 0.81, 0.33 to
+// 1.0. Always the best of 1, 2, 3, 4, 6 and 8 parts would be 1.4% faster.
 static int dkv_parts(const BwdArgs& a, int dqk, int dv) {
   if (a.doc_end && a.docs <= 0) return 1;
   const bool two = dqk == 64;                            // workgroups a CU

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(gt::THREADS, 1) void linear_grad_kernel(const Args 
 }
 
 // us that tiles of `height` rows and sums in `parts` take. A pair of steps of a tile of 32 n rows takes a + b
-// n, a little more where all CUs are at work (the card's power); fitted to 119 shapes of either product and 5
+// n, a little more where all CUs are at work (the card's power); fitted to 114 shapes of either product and 5
 // heights (1, 2, 3, 4, 6 and 8 parts for two of them): off by 7% (rms), and the choice by it by 0.5% from the
 // best one.
 inline float predicted(bool dw, long rows, long cols, long sum, int height, int parts) {

@@ -3,8 +3,9 @@
 Reference behavior: nemo_automodel/components/_peft/lora.py:45-570
 (PeftConfig, LinearLoRA with frozen base + A/B adapters, wildcard
 target_modules matching, apply_lora_to_linear_modules freezes the base model).
-The fused SGMV HIP kernels (reference _peft/lora_kernel.py) are a later
-optimization; the adapter math here is two small GEMMs riding hipBLASLt.
+The adapters' products run on csrc/lora.hip and lora_grad.hip (reference
+_peft/lora_kernel.py) for bf16 layers on the GPU of ranks in 8s up to 64, else on the
+library's.
 """
 
 from __future__ import annotations
