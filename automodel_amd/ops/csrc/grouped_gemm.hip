@@ -249,30 +249,44 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> build_group_plan(
 namespace {
 
 // Rows of grouped_tile_kernel's tiles at most, or 0 where grouped_gemm_kernel is the faster one; M rows in E
-// groups, weights [E, N, K]. 540 shapes each of nt, nn and tn (4 to 128 groups filled at random, 16 to 2000 rows
-// each, 512 x 1024 to 4096 x 2048) take 0.86, 0.86 and 0.90 of the time where the rule has the tiles; a few are up
-// to 1.09. What decides is how many rows an expert's weights serve and whether the tiles fill the chip's rounds:
+// groups, weights [E, N, K]. 9210 shapes each of nt, nn and tn (2 to 512 groups of 16 to 2000 rows on average,
+// filled at random or unequally, widths and sums of 128 to 4096) take 0.87, 0.81 and 0.84 of the time where the
+// rule has the tiles; 1% of these more than 1.05, 1.24 at most. What decides is how many rows an
+// expert's weights serve, whether the tiles fill the chip's rounds, and what a tile costs beside its products:
 //   tn      from 320 rows a group on (0.75 to 1.01); from 128 on with two rounds of tiles (0.81 to 1.02; with
-//           fewer 1.0 to 1.2)
-//   nt, nn  from 512 rows on, tiles of 128 for up to half a round (0.65 to 1.0); from 128 rows on with 168 to
-//           256 tiles of 256 rows (0.55 to 0.87); from 256 (nt) with 360 and more (0.8 to 1.0). Between them is a
-//           short second round (1.0 to 1.15), below them are idle CUs (1.1 to 1.5)
-//   nn      also otherwise from 80 rows on, tiles of 128 (0.8 to 1.07; sums of 512, 1.05 to 1.16, left out)
+//           fewer 1.0 to 1.2). Not with 128 columns, half of a tile's (1.07 in the mean, to 1.48)
+//   nt, nn  from 512 rows on, tiles of 128 for up to half a round (0.65 to 1.0); from 200 rows on (nn with sums from 768
+//           on: 128) with 168 to 256 tiles of 256 rows (0.55 to 0.9); from 256 (nt) with 360 and more (0.8 to 1.0).
+//           Between them is a short second round (1.0 to 1.15), below them are idle CUs (1.1 to 1.5)
+//   nn      also otherwise from 80 rows on, tiles of 128 (0.8 to 1.05): sums from 1024 on (768: 1.0 to 1.2), and with
+//           128 columns from 2048 on
+//   nt, nn  no sums below 512 and no 128 columns with more tiles than half a round (sums of 128 1.14 in the mean, to 2.06;
+//           of 256 1.05, to 1.8; 128 columns 1.07 to 1.13, to 2.0): a tile's beginning and stores are most of it,
+//           and the other kernel's workgroups overlap them. With fewer tiles sums from 256 on (0.83 to 0.96)
+//   any     of small weights, up to 2^20, no more than 256 groups, and more than 128 from 320 rows on: every workgroup
+//           sorts all groups (256 of 130 to 200 rows: nt 1.14, nn 1.02, tn 0.96; 512: 1.16, 1.18, 1.02; but with
+//           weights of 1408 x 2048 and more 0.9, 0.8 and 0.85)
 template <Mode MODE>
 int tile_cap(long M, long E, long N, long K) {
   const long cols = MODE == NT ? N : K, sum = MODE == NT ? K : N, rows = M / std::max(E, 1l);
-  // the table of groups, 32-bit addresses within a tile, sums of as many steps as are loaded ahead
-  if (E < 1 || E > MAX_GROUPS || std::max(N, K) >= (1 << 23) || (MODE != TN && sum < 4 * gt::STEP)) return 0;
+  // the table of groups, 32-bit addresses within a tile
+  if (E < 1 || E > MAX_GROUPS || std::max(N, K) >= (1 << 23)) return 0;
+  if (E > 128 && N * K <= (1l << 20) && (E > 256 || rows < 320)) return 0;
   const long nc = (cols + gt::TILE - 1) / gt::TILE;
-  if (MODE == TN) return rows >= 320 || (rows >= 128 && E * ((N + gt::TILE - 1) / gt::TILE) * nc >= 512) ? 256 : 0;
+  if (MODE == TN) {
+    if (K < 256 && N >= 256) return 0;
+    return rows >= 320 || (rows >= 128 && E * ((N + gt::TILE - 1) / gt::TILE) * nc >= 512) ? 256 : 0;
+  }
   // parts of groups that are not all of one size
   const auto parts = [&](long pct) { return (M * pct / 100 + E * 256 - 1) / (E * 256); };
   const long tiles = E * nc * (parts(95) + parts(101) + parts(107)) / 3;
-  if (rows >= 512) return tiles <= 128 ? 128 : 256;
+  const bool few = tiles <= 128, long_sum = sum >= 512, wide = cols >= 256;
+  if (sum < 256 || (few ? !long_sum && !wide : !long_sum || !wide)) return 0;
+  if (rows >= 512) return few ? 128 : 256;
   const bool fills = (tiles >= 168 && tiles <= 256) || tiles >= 360;
-  if (MODE == NT) return rows >= (tiles >= 360 ? 256 : 128) && fills ? 256 : 0;
-  if (rows >= 128 && fills) return 256;
-  return rows >= (tiles < 168 ? 80 : 128) && (sum > 512 || tiles >= 168) ? 128 : 0;
+  if (MODE == NT) return rows >= (tiles >= 360 ? 256 : 200) && fills ? 256 : 0;
+  if (rows >= (sum >= 768 ? 128 : 200) && fills) return 256;
+  return rows >= (tiles < 168 ? 80 : 128) && sum >= (wide ? 1024 : 2048) ? 128 : 0;
 }
 
 // by grouped_tile_kernel, or by grouped_gemm_kernel with tiles of `tile` rows

@@ -81,11 +81,12 @@ UNEVEN = [1, 129, 160, 161, 0, 193, 225, 256, 257, 300, 33, 400, 513, 1030, 3000
 # Tiles of 4 to 8 times 32 rows, dealt to workgroups that stay: tall and short ones, one part and several, fewer tiles than
 # workgroups and more, tables of more than a wave's groups and more groups than they hold
 @pytest.mark.parametrize("counts,N,K,caps", [
-    (UNEVEN, 384, 640, (128, 256, 256)), (UNEVEN, 128, 192, (128, None, None)), ([700], 256, 128, (128, 128, 256)),
-    (UNEVEN, 3456, 128, (256, 128, 256)), (UNEVEN, 128, 3456, (128, 256, 256)),
-    ([1600, 0, 31, 513], 3456, 256, (256, 128, 256)), ([512] * 6 + [3000], 1408, 1408, (256, 256, 256)),
-    ([130, 250, 200, 255] * 16, 768, 768, (256, 256, 256)), ([90, 110] * 20, 768, 256, (0, 128, 0)),
-    ([40, 1000] * 150, 128, 128, (256, 256, 256)), ([512] * 513, 128, 128, (0, 0, 0)),
+    (UNEVEN, 640, 640, (256, 256, 256)), (UNEVEN, 128, 576, (128, None, None)), ([700], 512, 256, (128, 128, 256)),
+    (UNEVEN, 3456, 512, (256, 128, 256)), (UNEVEN, 512, 3456, (128, 256, 256)), (UNEVEN, 128, 3456, (128, 0, 256)),
+    ([1600, 0, 31, 513], 3456, 512, (256, 128, 256)), ([512] * 6 + [3000], 1408, 1408, (256, 256, 256)),
+    ([130, 250, 200, 255] * 16, 768, 768, (256, 256, 256)), ([90, 110] * 20, 1024, 256, (0, 128, 0)),
+    ([40, 1000] * 120, 512, 512, (256, 256, 256)), ([30, 990] * 150, 1152, 1024, (256, 256, 256)),
+    ([40] * 513, 1152, 1024, (0, 0, 0)),
 ])
 def test_tiles_of_unequal_heights(counts, N, K, caps):
     from automodel_amd.ops._backend import hip_ops
@@ -130,8 +131,9 @@ def test_more_tiles_than_are_dealt_out():
 
     ops = hip_ops()
     torch.manual_seed(2)
-    M, N, K = 65000, 16384, 128            # 254 x 64 tiles, more than 48 for each of 256 workgroups
+    M, N, K = 65000, 16384, 512            # 254 x 64 tiles, more than 48 for each of 256 workgroups
     x, w = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(1, N, K, device="cuda").bfloat16()
+    assert ops.grouped_gemm_cap(0, M, 1, N, K) == 256
     plan = ops.build_group_plan(torch.tensor([M], dtype=torch.int32, device="cuda"), M, 256)
     got = ops.grouped_gemm_nt(x, w, *plan, 256)
     rows = torch.cat([torch.randperm(M, device="cuda")[:1000], torch.tensor([0, M - 1], device="cuda")])
@@ -139,3 +141,17 @@ def test_more_tiles_than_are_dealt_out():
     assert (got[rows].double() - want).norm() <= 2.0 ** -9 * 1.02 * want.norm()
     for i in range(0, M, 8192):            # every tile is there
         assert (got[i:i + 8192].abs().amax(1) > 0).all()
+
+
+@pytest.mark.parametrize("E,rows,N,K,caps", [
+    (64, 1000, 128, 2048, (0, 0, 256)), (64, 1000, 2048, 128, (0, 0, 0)),       # half a tile's columns
+    (64, 1000, 384, 2048, (256, 0, 256)), (64, 1000, 2048, 384, (0, 256, 256)),     # short sums
+    (8, 700, 1024, 256, (128, 128, 256)), (8, 700, 256, 128, (0, 0, 0)),        # in few tiles
+    (256, 191, 512, 256, (0, 0, 0)), (256, 400, 512, 512, (256, 256, 256)),     # many groups
+    (400, 400, 512, 512, (0, 0, 0)), (400, 300, 1408, 2048, (256, 256, 256)), (513, 400, 1408, 2048, (0, 0, 0)),
+    (64, 150, 768, 2048, (0, 256, 256)), (64, 100, 768, 1024, (0, 0, 0)),       # few rows
+])
+def test_rule(E, rows, N, K, caps):
+    from automodel_amd.ops._backend import hip_ops
+
+    assert tuple(hip_ops().grouped_gemm_cap(m, E * rows, E, N, K) for m in range(3)) == caps
