@@ -11,7 +11,8 @@
 // out by how long they take (grouped_tiles.h).
 //
 // grouped_gemm_kernel has them for few rows, where a step's time is that of the weights' reads and more
-// workgroups of less LDS read more at a time: 8 waves compute BM x 256 of the output, 64 x 64 or 64 x 128 each,
+// workgroups of less LDS read more at a time, and for short sums and few columns, where a tile's beginning and end
+// are most of it: 8 waves compute BM x 256 of the output, 64 x 64 or 64 x 128 each,
 // over steps of 64 of the summed index. What differs is which index of an operand is contiguous: tiles whose
 // rows are output rows or columns are read by rows, tiles whose rows are the summed index by columns, with the
 // transposing LDS reads (flash_tile.h). So dw takes g and x as they are, and dx takes w as it is. Direct loads

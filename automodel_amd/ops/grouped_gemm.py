@@ -43,8 +43,8 @@ def make_group_plan(counts: torch.Tensor, M: int, bm: int = 128):
 
 def tile_rows(rows: int, experts: int, *widths: int) -> int:
     """Row tile of the plan for products of those widths (the columns of their outputs), which the kernels of
-    one tile a workgroup follow: the fp8 products, and bf16 ones of groups too short for the kernel that cuts
-    its tiles itself (csrc/grouped_gemm.hip has that rule). 256 is the faster tile, but the last one of every
+    one tile a workgroup follow: the fp8 products, and bf16 ones of groups, sums or widths too short for the kernel
+    that cuts its tiles itself (csrc/grouped_gemm.hip has that rule). 256 is the faster tile, but the last one of every
     group is padding for half of it on average, and there are half as many. From 512 rows per expert on 256.
 
     From 320 on where its tiles fill the chip, one workgroup a CU: within one round of them, and
