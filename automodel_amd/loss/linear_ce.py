@@ -21,7 +21,7 @@ from __future__ import annotations
 import torch
 
 from automodel_amd.ops._backend import hip_ops
-from automodel_amd.ops.linear import input_grad, weight_grad
+from automodel_amd.ops.linear import input_grad, product, weight_grad
 
 IGNORE_INDEX = -100
 
@@ -97,7 +97,7 @@ def _chunk_grads(ctx, dloss: torch.Tensor):
         if i < len(kept):                      # stays as it is: the graph may be run again
             g = ops.ce_grad_logits(kept[i], y, lse, d, 0)
         else:
-            g = h @ weight.t()
+            g = product(h, weight)
             ops.ce_bwd_logits(g, y, lse, d, 0)
         if need_h:
             dh[rows] = input_grad(g, weight)
@@ -125,11 +125,10 @@ class _HybridLinearCE(torch.autograd.Function):
         T, H = hidden.shape
         loss_sum = torch.zeros(1, dtype=torch.float32, device=hidden.device)
         lse_all = torch.empty(T, dtype=torch.float32, device=hidden.device)
-        wt = weight.t()
         n_kept = _kept_chunks(T, H, weight.shape[0], chunk_size) if keep else 0
         kept = []
         for i, s in enumerate(range(0, T, chunk_size)):
-            logits = hidden[s : s + chunk_size] @ wt
+            logits = product(hidden[s : s + chunk_size], weight)
             lse, _ = ops.ce_fwd_logits(logits, labels[s : s + chunk_size], loss_sum)
             lse_all[s : s + chunk_size] = lse
             if i < n_kept:

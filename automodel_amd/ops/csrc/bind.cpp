@@ -114,6 +114,14 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("grouped_gemm_cap", &amd_ops::grouped_gemm_cap);
   m.def("grouped_gemm_tn(Tensor g, Tensor x, Tensor offs, int E) -> Tensor");
   m.impl("grouped_gemm_tn", &amd_ops::grouped_gemm_tn);
+  m.def("small_nt(Tensor x, Tensor w) -> Tensor");
+  m.impl("small_nt", &amd_ops::small_nt);
+  m.def("small_nn(Tensor g, Tensor w) -> Tensor");
+  m.impl("small_nn", &amd_ops::small_nn);
+  m.def("small_tn(Tensor g, Tensor x) -> Tensor");
+  m.impl("small_tn", &amd_ops::small_tn);
+  m.def("small_cut(int rows, int cols, int sum) -> (int, int)", &amd_ops::small_cut);
+  m.def("linear_small(Tensor x, Tensor w) -> Tensor", &amd_ops::linear_small);
   m.def("linear_dw(Tensor g, Tensor x) -> Tensor");
   m.impl("linear_dw", &amd_ops::linear_dw);
   m.def("linear_grad_cut(bool dw, int T, int N, int K) -> int[]");

@@ -170,6 +170,12 @@ at::Tensor grouped_gemm_nn(const at::Tensor& g, const at::Tensor& w,
                            int64_t bm = 128);
 int64_t grouped_gemm_cap(int64_t mode, int64_t M, int64_t E, int64_t N, int64_t K);
 at::Tensor grouped_gemm_tn(const at::Tensor& g, const at::Tensor& x, const at::Tensor& offs, int64_t E);
+at::Tensor small_nt(const at::Tensor& x, const at::Tensor& w);
+at::Tensor small_nn(const at::Tensor& g, const at::Tensor& w);
+at::Tensor small_tn(const at::Tensor& g, const at::Tensor& x);
+bool small_takes(int64_t T, int64_t N, int64_t K);
+std::tuple<int64_t, int64_t> small_cut(int64_t rows, int64_t cols, int64_t sum);
+at::Tensor linear_small(const at::Tensor& x, const at::Tensor& w);
 at::Tensor linear_dw(const at::Tensor& g, const at::Tensor& x);
 std::vector<int64_t> linear_grad_cut(bool dw, int64_t T, int64_t N, int64_t K);
 at::Tensor linear_dx(const at::Tensor& g, const at::Tensor& w);

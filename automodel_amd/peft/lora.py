@@ -16,10 +16,18 @@ from dataclasses import dataclass, field
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from automodel_amd.ops._backend import followed
-from automodel_amd.ops.linear import MAX_SIZE, _built, _ordinary, _plain, _unseen, input_grad_takes, linear
+from automodel_amd.ops.linear import (
+    MAX_SIZE,
+    _built,
+    _ordinary,
+    _plain,
+    _unseen,
+    input_grad_takes,
+    linear,
+    product,
+)
 
 
 @dataclass
@@ -98,7 +106,7 @@ class _LoRALinear(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x2, w, wa, wb, scale):
-        out, t = _adapter_forward(ctx, F.linear(x2, w), x2, wa, wb, scale, True)
+        out, t = _adapter_forward(ctx, product(x2, w), x2, wa, wb, scale, True)
         ctx.save_for_backward(x2, w, wa, wb, t)
         return out
 
