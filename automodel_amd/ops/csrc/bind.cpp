@@ -31,6 +31,8 @@ TORCH_LIBRARY(amd_ops, m) {
 
   m.def("swiglu_fwd(Tensor g, Tensor u) -> Tensor");
   m.impl("swiglu_fwd", &amd_ops::swiglu_fwd);
+  m.def("swiglu_rows_bwd(Tensor dh, Tensor g, Tensor u, Tensor p, Tensor order) -> (Tensor, Tensor, Tensor, Tensor)");
+  m.impl("swiglu_rows_bwd", &amd_ops::swiglu_rows_bwd);
   m.def("swiglu_bwd(Tensor dy, Tensor g, Tensor u) -> (Tensor, Tensor)");
   m.impl("swiglu_bwd", &amd_ops::swiglu_bwd);
   m.def("swiglu_cat_fwd(Tensor gu) -> Tensor");

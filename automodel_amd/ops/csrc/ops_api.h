@@ -28,6 +28,9 @@ at::Tensor rope_join(const at::Tensor& dq, const at::Tensor& dk, const at::Tenso
 at::Tensor swiglu_fwd(const at::Tensor& g, const at::Tensor& u);
 at::Tensor swiglu_cat_fwd(const at::Tensor& gu);
 at::Tensor swiglu_cat_bwd(const at::Tensor& dy, const at::Tensor& gu);
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> swiglu_rows_bwd(const at::Tensor& dh, const at::Tensor& g,
+                                                                           const at::Tensor& u, const at::Tensor& p,
+                                                                           const at::Tensor& order);
 std::tuple<at::Tensor, at::Tensor> swiglu_bwd(const at::Tensor& dy, const at::Tensor& g,
                                               const at::Tensor& u);
 
