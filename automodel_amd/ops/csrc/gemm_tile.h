@@ -31,9 +31,10 @@
 // bytes. Otherwise two steps together, [256][64], twice: whole 128-byte lines are loaded (with 64 bytes per
 // step 1340 against 1490 TFLOP/s, 8192 x 28672 x 4096); 16-byte pieces permuted by row for the 16 rows that
 // meet in a read. Where both are loaded so (x w^T), a pair's place is filled again as soon as its second step
-// is in registers, a third of a step after that began: there a barrier, and from there on the loads, which have
-// until the middle of the next pair's second step then (loads a step later and waited for half a step earlier:
-// 248 against 224 us, 65536 rows, 2048 x 768).
+// is in registers, a third of a step after that began: there a barrier, and from there on the loads, evenly over what
+// is left of the pair. They are waited for in the middle of the next pair's second step. The even spread is worth more
+// than a late wait: all loads in the two thirds of a step after the barrier 1406 us, over twice as much 1303, to the
+// pair's end 1282 (8192 rows, 4096 -> 28672; of zeros, where the card's power is not the bound, 1302, 1142, 1042).
 #pragma once
 
 #include <algorithm>
@@ -309,16 +310,17 @@ struct Run {
     // Step P of a pair. Loads of the buffers' next contents, in this order:
     //   TN: four of rows and four of columns, for the step four on
     //   NN: P 0: four of columns, for the step four on; P 1: eight of rows, for the pair two on, and four of columns
-    //   NT: P 0, when the rows' and columns' fragments are read (MID): eight of both, for the pair two on
-    // Waits: what is read next has landed. So many loads are later, and in a tile's first pair the last tile's stores
-    // are, 16 at least (loads and stores are counted in the order of their issue).
+    //   NT: from P 0 on, when the rows' and columns' fragments are read (MID): eight of both, for the pair two on
+    // Waits: what is read next has landed. So many loads are later (NT: of the 16 those before the middle of P 1), and
+    // in a tile's first pair the last tile's stores are, 16 at least (loads and stores are counted in the order of
+    // their issue).
     constexpr int RR = RC ? 2 : 1, CR = CC ? 2 : 1, READS = NR * RR + 8 * CR, S = NR * 8;
     auto step = [&](auto p_, auto first_) __attribute__((always_inline)) {
       constexpr int P = decltype(p_)::value;
       constexpr bool FIRST = decltype(first_)::value;
-      constexpr int LATER = (NN && P == 1 ? 8 : 16) + (FIRST ? 16 : 0);
       constexpr int DENSE = READS > 3 * S / 8 ? READS : 3 * S / 8;
-      constexpr int MID = P == 1 || !NT ? S : DENSE + 4;
+      constexpr int MID = DENSE + 4, OVER = 2 * S - MID;       // NT: slots of a pair that loads are spread over
+      constexpr int LATER = (NT ? ((S + S / 2 - MID) * 16 + OVER - 1) / OVER : NN && P == 1 ? 8 : 16) + (FIRST ? 16 : 0);
       // slots of the reads
       constexpr int FROM = NT && P == 1 ? S / 2 : 0, TO = TN || NN || P == 1 ? S : DENSE;
       if constexpr (!NT) {
@@ -328,7 +330,7 @@ struct Run {
       __builtin_amdgcn_sched_barrier(0);
       fa::unrolled<S>([&](auto m_) __attribute__((always_inline)) {
         constexpr int m = decltype(m_)::value, i = m / 8, j = m % 8;
-        if constexpr (m == MID) fa::barrier();
+        if constexpr (NT && P == 0 && m == MID) fa::barrier();
         if constexpr (NT && P == 1 && m == FROM) {
           fa::wait_loads<LATER>();
           fa::barrier();
@@ -345,8 +347,8 @@ struct Run {
             if constexpr (P == 0 && part > 0) move(f);
           });
         if constexpr (NT) {
-          if constexpr (m >= MID)
-            fa::spread<m - MID, S - MID, 16>([&](auto l_) __attribute__((always_inline)) {
+          if constexpr (P * S + m >= MID)
+            fa::spread<P * S + m - MID, OVER, 16>([&](auto l_) __attribute__((always_inline)) {
               constexpr int l = decltype(l_)::value / 2, odd = decltype(l_)::value % 2;
               if constexpr (odd) load_lds(cur, l * 4096, R.off[l], R.base, R.num);
               else load_lds(cur, HALF + l * 4096, C.off[l], C.base, C.num);
