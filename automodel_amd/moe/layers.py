@@ -241,12 +241,13 @@ class SharedExpert(nn.Module):
         self.up_proj = nn.Linear(hidden_size, intermediate, bias=False)
         self.down_proj = nn.Linear(intermediate, hidden_size, bias=False)
 
-    def forward(self, x):
+    def forward(self, x, beside: bool = False):
+        """``beside``: on a stream of its own beside the routed experts."""
         if torch.jit.is_scripting():          # (a module is no argument there)
             return self.down_proj(swiglu(self.gate_proj(x), self.up_proj(x)))
         else:
-            return linear(self.down_proj,
-                          swiglu(linear(self.gate_proj, x), linear(self.up_proj, x)))
+            return linear(self.down_proj, swiglu(linear(self.gate_proj, x, beside), linear(self.up_proj, x, beside)),
+                          beside)
 
 
 _SHARED_STREAMS: dict = {}
@@ -300,7 +301,8 @@ class MoE(nn.Module):
             ss = _shared_stream(xf.device)
             ss.wait_stream(torch.cuda.current_stream())
             with torch.cuda.stream(ss):
-                shared = self.shared_experts(xf)
+                own = type(self.shared_experts) is SharedExpert
+                shared = self.shared_experts(xf, beside=True) if own else self.shared_experts(xf)
                 if getattr(self, "shared_expert_gate", None) is not None:
                     shared = torch.sigmoid(self.shared_expert_gate(xf)) * shared
             y = self.experts(xf, probs, indices, **known)

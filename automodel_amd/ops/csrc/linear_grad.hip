@@ -1,16 +1,17 @@
-// Gradients of y = x w^T in bf16 with f32 accumulation (gfx950), by the tiles of gemm_tile.h:
+// y = x w^T and its gradients in bf16 with f32 accumulation (gfx950), by the tiles of gemm_tile.h:
 //
+//   linear_y    y[t, n]  = sum_k x[t, k] w[n, k]
 //   linear_dw   dw[n, k] = sum_t g[t, n] x[t, k]
 //   linear_dx   dx[t, k] = sum_n g[t, n] w[n, k]
 //
-// Both take their operands as they are.
+// All take their operands as they are.
 //
 // The chip has 256 workgroups, and most layers have not so many tiles of 256 x 256, or a few more (2048 x 2048:
 // 64; 6144 x 4096: 384). So tiles have 128 to 256 rows, and a sum can be cut into parts, each a tile of its own
 // in 32 bits, which `add_parts_kernel` adds up in their order: what takes least by `predicted`. Against 256
 // rows and whole sums, us: dw of 8192 tokens, 2048 x 2048 141 -> 70 (128 rows, 2 parts), 2816 x 2048 141 -> 95
 // (256 rows, 2 parts), 6144 x 4096 317 -> 289 (192 rows); dx of 1001 tokens, 6144 x 1536 104 -> 30 (128 rows, 4
-// parts). The library: 86, 127, 343, 56.
+// parts). The library: 86, 127, 343, 56. (x w^T has measurements of its own in linear_out.hip.)
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(256) void add_parts_kernel(const Args a) {
   }
 }
 
-template <bool DW>
+template <lg::Form FORM>
 at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t cols, int64_t sum,
                const at::Tensor* r2 = nullptr, const at::Tensor* c2 = nullptr) {
   TORCH_CHECK(r.is_cuda() && r.device() == c.device() && r.is_contiguous() && c.is_contiguous() &&
@@ -73,7 +74,7 @@ at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t c
     a.c2 = reinterpret_cast<const bf16*>(c2->data_ptr());
     a.rank = (int)r2->size(1);
   }
-  cut(DW, a);
+  cut(FORM, a);
   const long tiles = lg::tiles_of(a);
   TORCH_CHECK(tiles * 32 < (1l << 31), "linear_grad: too many tiles");
   at::Tensor part;
@@ -85,13 +86,15 @@ at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t c
   const long blocks = std::min((tiles * a.parts + 7) / 8 * 8, gt::workgroups());
   const auto stream = c10::hip::getCurrentHIPStream().stream();
   const auto launch = [&](auto short_, auto parts_) {
-    hipLaunchKernelGGL((lg::linear_grad_kernel<DW, decltype(short_)::value, decltype(parts_)::value>), dim3((unsigned)blocks),
+    hipLaunchKernelGGL((lg::linear_tile_kernel<FORM, decltype(short_)::value, decltype(parts_)::value>), dim3((unsigned)blocks),
                        dim3(gt::THREADS), gt::SMEM, stream, a);
     HIP_CHECK_KERNEL();
   };
   using Yes = std::true_type;
   using No = std::false_type;
-  if constexpr (DW) {
+  if constexpr (FORM == lg::Y) {
+    lg::launch_out(a, (unsigned)blocks, stream);
+  } else if constexpr (FORM == lg::DW) {
     if (a.parts > 1) launch(Yes{}, Yes{});
     else launch(Yes{}, No{});
   } else {
@@ -112,14 +115,14 @@ at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t c
 at::Tensor linear_dw(const at::Tensor& g, const at::Tensor& x) {
   TORCH_CHECK(g.dim() == 2 && x.dim() == 2 && g.size(0) == x.size(0), "linear_dw: g [T, N], x [T, K]");
   TORCH_CHECK(g.size(0) > 0 && g.size(1) % 8 == 0 && x.size(1) % 8 == 0, "linear_dw: rows, N%8 == 0, K%8 == 0");
-  return run<true>(g, x, g.size(1), x.size(1), g.size(0));
+  return run<lg::DW>(g, x, g.size(1), x.size(1), g.size(0));
 }
 
 at::Tensor linear_dx(const at::Tensor& g, const at::Tensor& w) {
   TORCH_CHECK(g.dim() == 2 && w.dim() == 2 && g.size(1) == w.size(0), "linear_dx: g [T, N], w [N, K]");
   TORCH_CHECK(w.size(0) > 0 && w.size(0) % (2 * gt::STEP) == 0 && w.size(1) % 8 == 0,
               "linear_dx: N%64 == 0, K%8 == 0");
-  return run<false>(g, w, g.size(0), w.size(1), w.size(0));
+  return run<lg::DX>(g, w, g.size(0), w.size(1), w.size(0));
 }
 
 // the same and t A for t [T, r], A^T [K, r]
@@ -132,16 +135,33 @@ at::Tensor linear_dx_extra(const at::Tensor& g, const at::Tensor& w, const at::T
                     e->size(1) == t.size(1) && (uintptr_t)e->data_ptr() % 16 == 0, "linear_dx: t [T, r], A^T [K, r]");
   TORCH_CHECK(t.size(1) >= 32 && t.size(1) % 32 == 0 && t.size(0) == g.size(0) && a_t.size(0) == w.size(1),
               "linear_dx: t [T, r], A^T [K, r], r % 32 == 0");
-  return run<false>(g, w, g.size(0), w.size(1), w.size(0), &t, &a_t);
+  return run<lg::DX>(g, w, g.size(0), w.size(1), w.size(0), &t, &a_t);
 }
 
-// {rows of a tile, parts of the sum} for linear_dw (of T rows, [N, K]) or linear_dx
+at::Tensor linear_y(const at::Tensor& x, const at::Tensor& w) {
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "linear_y: x [T, K], w [N, K]");
+  TORCH_CHECK(w.size(1) >= 4 * gt::STEP && w.size(1) % (2 * gt::STEP) == 0 && w.size(0) % 8 == 0,
+              "linear_y: K%64 == 0 and 128 or more, N%8 == 0");
+  return run<lg::Y>(x, w, x.size(0), w.size(0), w.size(1));
+}
+
+// {rows of a tile, parts of the sum} for linear_y of T rows, [N, K]
+std::vector<int64_t> linear_y_cut(int64_t T, int64_t N, int64_t K) {
+  Args a{};
+  a.rows = T;
+  a.cols = N;
+  a.sum = K;
+  cut(lg::Y, a);
+  return {a.height, a.parts};
+}
+
+// the same for linear_dw (of T rows, [N, K]) or linear_dx
 std::vector<int64_t> linear_grad_cut(bool dw, int64_t T, int64_t N, int64_t K) {
   Args a{};
   a.rows = dw ? N : T;
   a.cols = K;
   a.sum = dw ? T : N;
-  cut(dw, a);
+  cut(dw ? lg::DW : lg::DX, a);
   return {a.height, a.parts};
 }
 

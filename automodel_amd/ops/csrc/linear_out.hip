@@ -1,0 +1,26 @@
+// Launches of y = x w^T by the tiles of gemm_tile.h (linear_grad.hip has the rest). The library's tiles of 256 x 256
+// are as fast where they fill the chip's rounds and the sum is short, and leave CUs idle otherwise: here tiles and sums
+// are cut as the gradients' are. us, library -> here, bf16 of unit variance, the weights not in a cache:
+//   511 x 14336 -> 4096 92 -> 67 (256 rows, 8 parts), 1001 x 21504 -> 4096 240 -> 150, 3003 x 2048 -> 2816 43 -> 34,
+//   6001 x 4096 -> 4096 156 -> 143, 24000 x 4096 -> 14336 1977 -> 1913; 8192 x 4096 -> 28672 1264 and 1282.
+// ops/linear.py (output_own) has the rule and what it was fitted to.
+#include <ATen/ATen.h>
+
+#include "common.h"
+#include "linear_tiles.h"
+
+namespace amd_ops {
+namespace lg {
+
+void launch_out(const Args& a, unsigned blocks, hipStream_t stream) {
+  const auto launch = [&](auto parts_) {
+    hipLaunchKernelGGL((linear_tile_kernel<Y, false, decltype(parts_)::value>), dim3(blocks), dim3(gt::THREADS), gt::SMEM,
+                       stream, a);
+    HIP_CHECK_KERNEL();
+  };
+  if (a.parts > 1) launch(std::true_type{});
+  else launch(std::false_type{});
+}
+
+}  // namespace lg
+}  // namespace amd_ops

@@ -1,5 +1,5 @@
-// Tiles of the gradients of y = x w^T (linear_grad.hip, lora_grad.hip): their order, and how they and their sums
-// are cut.
+// Tiles of y = x w^T and its gradients (linear_grad.hip, linear_out.hip, lora_grad.hip): their order, and how they
+// and their sums are cut.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -9,6 +9,8 @@
 
 namespace amd_ops {
 namespace lg {
+
+enum Form { Y, DX, DW };
 
 struct Args {
   const bf16 *r, *c;
@@ -31,7 +33,7 @@ __device__ __forceinline__ void place(int i, int nr, int nc, int height, int& r0
 }
 
 // Blocks are dealt to the 8 XCDs in contiguous stretches of the tile list, one part after another.
-template <bool DW, bool EXTRA = false>
+template <Form F, bool EXTRA = false>
 struct Tiles {
   const Args& a;
   const int nc, nr, stride;
@@ -56,8 +58,8 @@ struct Tiles {
     t.rows = min(a.rows - r0, a.height);
     t.cols = a.cols - c0;
     t.sum = min(a.sum - from, a.per);
-    t.r = DW ? a.r + (long)from * a.rows + r0 : a.r + (long)r0 * a.sum + from;
-    t.c = a.c + (long)from * a.cols + c0;
+    t.r = F == DW ? a.r + (long)from * a.rows + r0 : a.r + (long)r0 * a.sum + from;
+    t.c = F == Y ? a.c + (long)c0 * a.sum + from : a.c + (long)from * a.cols + c0;
     t.out = a.out + (long)r0 * a.cols + c0;
     t.part = a.part + (long)u * a.height * gt::TILE;
     if (EXTRA && s == 0) {
@@ -70,24 +72,26 @@ struct Tiles {
 };
 
 // SHORT, PARTS, EXTRA: gemm_tile.h
-template <bool DW, bool SHORT, bool PARTS, bool EXTRA = false>
-__global__ __launch_bounds__(gt::THREADS, 1) void linear_grad_kernel(const Args a) {
+template <Form F, bool SHORT, bool PARTS, bool EXTRA = false>
+__global__ __launch_bounds__(gt::THREADS, 1) void linear_tile_kernel(const Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  Tiles<DW, EXTRA> tiles(a);
-  const gt::Shape shape{2u * (DW ? a.rows : a.sum), 2u * a.cols, 2u * a.cols};
-  gt::Run<DW, true, Tiles<DW, EXTRA>, SHORT, PARTS, EXTRA>(tiles, shape, smem)();
+  Tiles<F, EXTRA> tiles(a);
+  const gt::Shape shape{2u * (F == DW ? a.rows : a.sum), 2u * (F == Y ? a.sum : a.cols), 2u * a.cols};
+  gt::Run<F == DW, F != Y, Tiles<F, EXTRA>, SHORT, PARTS, EXTRA>(tiles, shape, smem)();
 }
 
 // us that tiles of `height` rows and sums in `parts` take. A pair of steps of a tile of 32 n rows takes a + b
-// n, a little more where all CUs are at work (the card's power); fitted to 114 shapes of either product and 5
+// n, a little more where all CUs are at work (the card's power); fitted to 114 shapes of either gradient and 5
 // heights (1, 2, 3, 4, 6 and 8 parts for two of them): off by 7% (rms), and the choice by it by 0.5% from the
-// best one.
-inline float predicted(bool dw, long rows, long cols, long sum, int height, int parts) {
+// best one. x w^T: fitted to the three or four best by it of 1917 shapes of 100 to 24000 rows; off by 10%, the choice
+// by 1.3%.
+inline float predicted(Form form, long rows, long cols, long sum, int height, int parts) {
   struct Fit {
     float start, a, b, a_all, b_all, tile, add, add_mb;
   };
-  const Fit f = dw ? Fit{5.8f, .104f, .103f, .196f, .141f, 2.36f, 2.6f, .92f}
-                   : Fit{5.6f, .044f, .109f, .136f, .146f, 1.78f, 4.6f, .88f};
+  const Fit f = form == DW   ? Fit{5.8f, .104f, .103f, .196f, .141f, 2.36f, 2.6f, .92f}
+                : form == DX ? Fit{5.6f, .044f, .109f, .136f, .146f, 1.78f, 4.6f, .88f}
+                             : Fit{2.6f, .387f, .0415f, .314f, .1364f, 3.13f, 6.f, .86f};
   const long tiles = (rows + height - 1) / height * ((cols + gt::TILE - 1) / gt::TILE) * parts;
   const float pairs = (sum + 64 * parts - 1) / (64 * parts), n = height / 32;
   const auto round = [&](float busy) {
@@ -98,7 +102,7 @@ inline float predicted(bool dw, long rows, long cols, long sum, int height, int 
   return parts == 1 ? t : t + f.add + f.add_mb * 1e-6f * rows * cols * parts;
 }
 
-inline void cut(bool dw, Args& a) {
+inline void cut(Form form, Args& a) {
   float least = 0.f;
   a.height = 0;
   for (const int parts : {1, 2, 3, 4, 6, 8}) {
@@ -106,7 +110,7 @@ inline void cut(bool dw, Args& a) {
     // each has 4 pairs of steps or more, the last one 2
     if (parts > 1 && (per < 256 || a.sum - (parts - 1) * per < 128)) continue;
     for (int height = 128; height <= gt::TILE; height += 32) {
-      const float t = predicted(dw, a.rows, a.cols, a.sum, height, parts);
+      const float t = predicted(form, a.rows, a.cols, a.sum, height, parts);
       if (a.height && t >= least) continue;
       least = t;
       a.height = height;
@@ -120,8 +124,9 @@ inline long tiles_of(const Args& a) {
   return ((long)(a.rows + a.height - 1) / a.height) * ((a.cols + gt::TILE - 1) / gt::TILE);
 }
 
-// linear_dx with an EXTRA product (lora_grad.hip)
+// linear_dx with an EXTRA product (lora_grad.hip); linear_y, with one or without (linear_out.hip)
 void launch_extra(const Args& a, unsigned blocks, hipStream_t stream);
+void launch_out(const Args& a, unsigned blocks, hipStream_t stream);
 
 }  // namespace lg
 }  // namespace amd_ops

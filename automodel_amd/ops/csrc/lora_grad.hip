@@ -24,7 +24,7 @@ namespace lg {
 
 void launch_extra(const Args& a, unsigned blocks, hipStream_t stream) {
   const auto launch = [&](auto short_, auto parts_) {
-    hipLaunchKernelGGL((linear_grad_kernel<false, decltype(short_)::value, decltype(parts_)::value, true>), dim3(blocks),
+    hipLaunchKernelGGL((linear_tile_kernel<DX, decltype(short_)::value, decltype(parts_)::value, true>), dim3(blocks),
                        dim3(gt::THREADS), gt::SMEM, stream, a);
     HIP_CHECK_KERNEL();
   };

@@ -14,6 +14,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from automodel_amd.ops.linear import inferred
+
 _PAD_TO = {5: 8, 6: 8, 7: 8, 9: 16, 10: 16, 11: 16, 12: 16, 13: 16, 14: 16, 15: 16}
 
 
@@ -49,8 +51,9 @@ def project(lin: nn.Module, x: torch.Tensor, relu2: bool = False,
     to bf16 on the way out of the accumulator).
 
     Inference on the GPU: up to 2 bf16 rows take the GEMV, up to 64 the skinny
-    MFMA GEMM, both with fused epilogues; more take the library GEMM. Wrapped
-    layers (adapters) and autograd take the module itself."""
+    MFMA GEMM, both with fused epilogues; more take the faster one of the kernels of
+    ops/linear.py and the library's GEMM. Wrapped layers (adapters) and autograd take the
+    module itself."""
     from automodel_amd.ops import residual_norm as rn
 
     if type(lin) not in (nn.Linear, DecodeLinear) or lin.bias is not None or not rn.use_hip(x):
@@ -69,7 +72,8 @@ def project(lin: nn.Module, x: torch.Tensor, relu2: bool = False,
     if out_f32 and x.dtype == torch.bfloat16:
         y = torch.mm(x, w.t(), out_dtype=torch.float32)
     else:
-        y = F.linear(x, w)
+        y = inferred(x, w)
+        y = F.linear(x, w) if y is None else y
     return rn.relu2(y) if relu2 else y
 
 
@@ -194,7 +198,8 @@ class DecodeLinear(nn.Linear):
             lead = x.shape[:-1]
             y = gemv_bf16(x.reshape(-1, x.shape[-1]), self.weight, self.bias)
             return y.reshape(*lead, self.out_features)
-        return F.linear(x, self.weight, self.bias)
+        y = inferred(x, self.weight) if self.bias is None else None
+        return F.linear(x, self.weight, self.bias) if y is None else y
 
 
 def swap_linears_for_decode(model: nn.Module) -> int:
