@@ -97,6 +97,8 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("lora_apply", &amd_ops::lora_apply);
   m.def("lora_forward(Tensor y, Tensor x, Tensor A, Tensor B, float scale) -> (Tensor, Tensor)");
   m.impl("lora_forward", &amd_ops::lora_forward);
+  m.def("lora_linear(Tensor x, Tensor w, Tensor A, Tensor B, float scale) -> (Tensor, Tensor)");
+  m.impl("lora_linear", &amd_ops::lora_linear);
   m.def("lora_grads(Tensor g, Tensor x, Tensor A, Tensor B, Tensor tt, float scale) -> (Tensor, Tensor, Tensor, Tensor)");
   m.impl("lora_grads", &amd_ops::lora_grads);
   m.def("linear_dx_extra(Tensor g, Tensor w, Tensor t, Tensor a_t) -> Tensor");

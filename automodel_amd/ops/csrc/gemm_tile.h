@@ -115,7 +115,7 @@ __device__ __forceinline__ int lane_here() {
 struct Tile {
   const bf16 *r, *c;
   const bf16 *r2, *c2;         // a second pair, added to the sum, or null
-  int rank;                    // EXTRA: how long a row of theirs is, a multiple of 32
+  int rank, rank_c;            // EXTRA: how long a row of r2 is, a multiple of 32, and of c2, one of 8: zeros behind it
   int rows, cols;              // of the output, from the tile's first on
   int sum;                     // a multiple of 64 unless both operands are COLS
   bf16* out;
@@ -230,7 +230,7 @@ struct Operand {
 // first() and next() are their numbers, or negative; get(number) is the tile; loaded() is called once, while
 // the first tile's operands come.
 // PARTS: tiles of sums that are added up later, 32 bits in the order of the accumulators.
-// EXTRA: the second pair is [rows][rank] and [columns][rank], short rows that are loaded as fragments behind the
+// EXTRA: the second pair is [rows][rank] and [columns][rank_c], short rows that are loaded as fragments behind the
 // sum. They come from the L2, and with them the wave waits for the next tile's loads (8192 rows, a sum of 4096,
 // 4096 columns: 192 us without, 190 with it).
 template <bool RC, bool CC, class Tiles, bool SHORT = RC && CC, bool PARTS = false, bool EXTRA = false>
@@ -416,7 +416,8 @@ struct Run {
         rx[i] = *reinterpret_cast<const bf16x8_t*>(r2 + min(r0 + i * 16, t.rows - 1) * t.rank + k);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        cx[j] = *reinterpret_cast<const bf16x8_t*>(c2 + min(c0 + j * 16, t.cols - 1) * t.rank + k);
+        cx[j] = k + g * 8 < t.rank_c ? *reinterpret_cast<const bf16x8_t*>(c2 + min(c0 + j * 16, t.cols - 1) * t.rank_c + k)
+                                     : bf16x8_t{};
 #pragma unroll
       for (int i = 0; i < NR; ++i)
 #pragma unroll

@@ -68,11 +68,12 @@ at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t c
   auto out = at::empty({rows, cols}, r.options());
   if (out.numel() == 0) return out;
   Args a{reinterpret_cast<const bf16*>(r.data_ptr()), reinterpret_cast<const bf16*>(c.data_ptr()),
-         reinterpret_cast<bf16*>(out.data_ptr()), nullptr, (int)rows, (int)cols, (int)sum, 0, 0, 0, nullptr, nullptr, 0};
+         reinterpret_cast<bf16*>(out.data_ptr()), nullptr, (int)rows, (int)cols, (int)sum, 0, 0, 0, nullptr, nullptr, 0, 0};
   if (r2) {
     a.r2 = reinterpret_cast<const bf16*>(r2->data_ptr());
     a.c2 = reinterpret_cast<const bf16*>(c2->data_ptr());
     a.rank = (int)r2->size(1);
+    a.rank_c = (int)c2->size(1);
   }
   cut(FORM, a);
   const long tiles = lg::tiles_of(a);
@@ -143,6 +144,29 @@ at::Tensor linear_y(const at::Tensor& x, const at::Tensor& w) {
   TORCH_CHECK(w.size(1) >= 4 * gt::STEP && w.size(1) % (2 * gt::STEP) == 0 && w.size(0) % 8 == 0,
               "linear_y: K%64 == 0 and 128 or more, N%8 == 0");
   return run<lg::Y>(x, w, x.size(0), w.size(0), w.size(1));
+}
+
+// x w^T + scale (x A^T) B^T, A [r, K], B [N, r], r a multiple of 8 up to 64: B's product behind the sums, one rounding. ->
+// {it, (x A^T)^T [r rounded up to 32, T to 64] with zeros behind both, which lora_grads reads}. Against the product by
+// the faster of kernel and library and lora_forward's pass over it: 1840 shapes of 100 to 8200 rows 0.88 of their time in
+// the mean, 0.82 from 2^31 products on; 8192 rows, 4096 -> 28672 1547 -> 1344 us, 4096 -> 6144 349 -> 301, 14336 -> 4096
+// 734 -> 700. 200 shapes are above 1.02, up to 1.2, of some 25 us, where the host is the bound and has a launch less.
+std::tuple<at::Tensor, at::Tensor> lora_linear(const at::Tensor& x, const at::Tensor& w, const at::Tensor& A,
+                                               const at::Tensor& B, double scale) {
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && A.dim() == 2 && B.dim() == 2 && x.size(1) == w.size(1),
+              "lora_linear: x [T, K], w [N, K]");
+  const int64_t T = x.size(0), N = w.size(0), K = w.size(1), r = A.size(0);
+  TORCH_CHECK(T > 0 && K >= 4 * gt::STEP && K % (2 * gt::STEP) == 0 && N % 64 == 0 && r >= 8 && r <= 64 && r % 8 == 0 &&
+                  A.size(1) == K && B.size(0) == N && B.size(1) == r,
+              "lora_linear: rows, K%64 == 0 and 128 or more, N%64 == 0, A [r, K], B [N, r], r a multiple of 8 up to 64");
+  for (const at::Tensor* t : {&x, &w, &A, &B})
+    TORCH_CHECK(t->is_cuda() && t->device() == x.device() && t->scalar_type() == at::kBFloat16 && t->is_contiguous() &&
+                    (uintptr_t)t->data_ptr() % 16 == 0, "lora_linear: bf16, whole, at multiples of 16 bytes");
+  const c10::DeviceGuard guard(x.device());
+  const int64_t R = r <= 32 ? 32 : 64;
+  auto t = at::empty({T, R}, x.options()), turned = at::empty({R, (T + 63) / 64 * 64}, x.options());
+  lora_down(x, A, r, &t, &turned, scale, 1.);
+  return {run<lg::Y>(x, w, T, N, K, &t, &B), turned};
 }
 
 // {rows of a tile, parts of the sum} for linear_y of T rows, [N, K]

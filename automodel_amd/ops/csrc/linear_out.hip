@@ -13,13 +13,15 @@ namespace amd_ops {
 namespace lg {
 
 void launch_out(const Args& a, unsigned blocks, hipStream_t stream) {
-  const auto launch = [&](auto parts_) {
-    hipLaunchKernelGGL((linear_tile_kernel<Y, false, decltype(parts_)::value>), dim3(blocks), dim3(gt::THREADS), gt::SMEM,
-                       stream, a);
+  const auto launch = [&](auto parts_, auto extra_) {
+    hipLaunchKernelGGL((linear_tile_kernel<Y, false, decltype(parts_)::value, decltype(extra_)::value>), dim3(blocks),
+                       dim3(gt::THREADS), gt::SMEM, stream, a);
     HIP_CHECK_KERNEL();
   };
-  if (a.parts > 1) launch(std::true_type{});
-  else launch(std::false_type{});
+  using Yes = std::true_type;
+  using No = std::false_type;
+  if (a.parts > 1) a.rank ? launch(Yes{}, Yes{}) : launch(Yes{}, No{});
+  else a.rank ? launch(No{}, Yes{}) : launch(No{}, No{});
 }
 
 }  // namespace lg

@@ -18,8 +18,8 @@ struct Args {
   float* part;                         // [part][tile][height][256], in the order of the accumulators
   int rows, cols, sum;
   int height, parts, per;              // rows of a tile; parts of the sum, and how much of it each but the last has
-  const bf16 *r2, *c2;                 // EXTRA: [rows][rank] and [cols][rank], whose product is added
-  int rank;
+  const bf16 *r2, *c2;                 // EXTRA: [rows][rank] and [cols][rank_c], whose product is added
+  int rank, rank_c;
 };
 
 // The tiles' order is down 4 row tiles, then on to the next column tile: the 32 tiles of an XCD at a time read
@@ -64,8 +64,9 @@ struct Tiles {
     t.part = a.part + (long)u * a.height * gt::TILE;
     if (EXTRA && s == 0) {
       t.r2 = a.r2 + (long)r0 * a.rank;
-      t.c2 = a.c2 + (long)c0 * a.rank;
+      t.c2 = a.c2 + (long)c0 * a.rank_c;
       t.rank = a.rank;
+      t.rank_c = a.rank_c;
     }
     return t;
   }

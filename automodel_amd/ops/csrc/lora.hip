@@ -36,13 +36,13 @@ struct Down {
   bf16 *t, *turned;          // turned: or null
   long M, pitch;
   int H, r;                  // r: rows of A, R at most; columns of t behind them are zeros, whatever x is
-  float scale;
+  float scale, scale_turned;
 };
 
 constexpr int DOWN = 32;     // rows of a workgroup
 
 // t[M, R] = scale x[M, H] A[R, H]^T, and, where they are wanted, its columns as rows of M rounded up to 64
-// (`pitch`), zeros behind M. Bound by reading x: 32 rows a workgroup, so that 8192 rows fill the chip, and its waves
+// (`pitch`), zeros behind M, by a scale of their own. Bound by reading x: 32 rows a workgroup, so that 8192 rows fill the chip, and its waves
 // take a quarter of H each, 64 columns a step: their own stretches of x and of A (from the L2) come straight to
 // their own LDS, three steps ahead (R 64: two), with no barrier in the loop. 8192 x 28672 90 us, 8192 x 4096 14.
 // (Fragments straight from memory, four of each in flight: 158, 3.0 TB/s, and 23.)
@@ -122,14 +122,14 @@ __global__ __launch_bounds__(256, 1) void lora_down_kernel(const Down a) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) red[wid][i * 16 + g * 4 + v][j * 16 + l16] = acc[i][j][v];
   __syncthreads();
-  auto sum = [&](int m, int r) {                       // (0 x infinity is none)
-    return r < a.r ? (red[0][m][r] + red[1][m][r] + red[2][m][r] + red[3][m][r]) * a.scale : 0.f;
+  auto sum = [&](int m, int r, float scale) {          // (0 x infinity is none)
+    return r < a.r ? (red[0][m][r] + red[1][m][r] + red[2][m][r] + red[3][m][r]) * scale : 0.f;
   };
   for (int e = threadIdx.x; e < DOWN * R; e += 256)
-    if (e / R < have) a.t[m0 * R + e] = f2bf(sum(e / R, e % R));
+    if (e / R < have) a.t[m0 * R + e] = f2bf(sum(e / R, e % R, a.scale));
   if (!a.turned) return;
   for (int e = threadIdx.x; e < DOWN * R; e += 256)
-    a.turned[e / DOWN * a.pitch + m0 + e % DOWN] = f2bf(e % DOWN < have ? sum(e % DOWN, e / DOWN) : 0.f);
+    a.turned[e / DOWN * a.pitch + m0 + e % DOWN] = f2bf(e % DOWN < have ? sum(e % DOWN, e / DOWN, a.scale_turned) : 0.f);
 }
 
 // out[M, O] = y + scale * t[M, R] B[O, R]^T (without y: the product alone). Bound by y and
@@ -369,15 +369,16 @@ at::Tensor sgmv_fused_fwd(const at::Tensor& x, const at::Tensor& A, const at::Te
   return out;
 }
 
-// t = scale x A^T [M, r rounded up to 32] of A's first r rows, with zeros behind r, and t^T, M rounded up to 64, with zeros
-// behind M; x and A at multiples of 16 bytes
-void lora_down(const at::Tensor& x, const at::Tensor& A, int64_t r, at::Tensor* t, at::Tensor* turned, double scale) {
+// t = scale x A^T [M, r rounded up to 32] of A's first r rows, with zeros behind r, and scale_turned (x A^T)^T, M rounded up
+// to 64, with zeros behind M; x and A at multiples of 16 bytes
+void lora_down(const at::Tensor& x, const at::Tensor& A, int64_t r, at::Tensor* t, at::Tensor* turned, double scale,
+               double scale_turned) {
   const long M = x.size(0), pitch = (M + 63) / 64 * 64, blocks = ((turned ? pitch : M) + DOWN - 1) / DOWN;
   // (a grid has 2^32 threads; a lane's offsets of 64 rows are 32 bits)
   TORCH_CHECK(blocks < 1l << 24 && x.size(1) < 1l << 25, "lora: too many rows or columns");
   const Down a{reinterpret_cast<const bf16*>(x.data_ptr()), reinterpret_cast<const bf16*>(A.data_ptr()),
                reinterpret_cast<bf16*>(t->data_ptr()), turned ? reinterpret_cast<bf16*>(turned->data_ptr()) : nullptr, M,
-               pitch, (int)x.size(1), (int)r, (float)scale};
+               pitch, (int)x.size(1), (int)r, (float)scale, (float)scale_turned};
   const auto launch = [&](auto rank) {
     constexpr int RANK = rank.value, smem = 4 * (RANK == 32 ? 4 : 3) * (DOWN / 8 + RANK / 8) * 1024;
     hipLaunchKernelGGL((lora_down_kernel<RANK>), dim3((unsigned)blocks), dim3(256), smem,
@@ -420,7 +421,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> forward(const std::optional<at::T
   const auto whole = [](const at::Tensor& v) { return (uintptr_t)v.data_ptr() % 16 ? v.clone() : v; };
   auto run = [&](auto rank) {
     constexpr int RANK = rank.value;
-    lora_down(whole(x), whole(A), r, &t, turn ? &turned : nullptr, 1.);
+    lora_down(whole(x), whole(A), r, &t, turn ? &turned : nullptr, 1., 1.);
     hipLaunchKernelGGL((lora_up_kernel<RANK>), dim3((unsigned)blocks), dim3(256), 0, stream, yp,
                        reinterpret_cast<const bf16*>(t.data_ptr()),
                        reinterpret_cast<const bf16*>(B.data_ptr()),

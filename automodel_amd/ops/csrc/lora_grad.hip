@@ -224,7 +224,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> lora_grads(const at::
                        (int)r);
     HIP_CHECK_KERNEL();
     outer<RANK, false>(g, tt, dB, scale, stream);
-    lora_down(g, Bt, r, &dt, &dtt, scale);
+    lora_down(g, Bt, r, &dt, &dtt, scale, scale);
     outer<RANK, true>(x, dtt, dA, 1., stream);
   };
   if (R == 32) run(std::integral_constant<int, 32>{});

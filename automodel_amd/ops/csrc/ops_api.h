@@ -92,7 +92,10 @@ std::tuple<at::Tensor, at::Tensor> lora_apply(const std::optional<at::Tensor>& y
                                               const at::Tensor& A, const at::Tensor& B, double scale);
 std::tuple<at::Tensor, at::Tensor> lora_forward(const at::Tensor& y, const at::Tensor& x, const at::Tensor& A,
                                                 const at::Tensor& B, double scale);
-void lora_down(const at::Tensor& x, const at::Tensor& A, int64_t r, at::Tensor* t, at::Tensor* turned, double scale);
+void lora_down(const at::Tensor& x, const at::Tensor& A, int64_t r, at::Tensor* t, at::Tensor* turned, double scale,
+               double scale_turned);
+std::tuple<at::Tensor, at::Tensor> lora_linear(const at::Tensor& x, const at::Tensor& w, const at::Tensor& A,
+                                               const at::Tensor& B, double scale);
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> lora_grads(const at::Tensor& g, const at::Tensor& x,
                                                                       const at::Tensor& A, const at::Tensor& B,
                                                                       const at::Tensor& tt, double scale);

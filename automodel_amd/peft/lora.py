@@ -102,11 +102,19 @@ class _FusedLoRAFn(torch.autograd.Function):
 
 
 class _LoRALinear(torch.autograd.Function):
-    """x w^T + (x @ A^T) @ B^T * scale, w frozen: the gradient of x is one product."""
+    """x w^T + (x @ A^T) @ B^T * scale, w frozen: one product, and so is the gradient of x."""
 
     @staticmethod
     def forward(ctx, x2, w, wa, wb, scale):
-        out, t = _adapter_forward(ctx, product(x2, w), x2, wa, wb, scale, True)
+        sizes = (x2.shape[0], *w.shape)
+        if (x2.shape[0] > 0 and max(sizes) < MAX_SIZE and w.shape[1] >= 128 and not followed()
+                and _ordinary(x2, w, wa, wb) and _plain(x2, w, wa, wb)):
+            from automodel_amd.ops._backend import hip_ops
+
+            ctx.scale, ctx.turned = scale, True
+            out, t = hip_ops().lora_linear(x2, w, wa, wb, scale)
+        else:
+            out, t = _adapter_forward(ctx, product(x2, w), x2, wa, wb, scale, True)
         ctx.save_for_backward(x2, w, wa, wb, t)
         return out
 
