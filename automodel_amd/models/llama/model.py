@@ -24,7 +24,7 @@ from automodel_amd.ops import attention as attn_mod
 from automodel_amd.ops.attention import _sdpa, flash_attention, sdpa_masked
 from automodel_amd.ops.linear import linear
 from automodel_amd.ops.rms_norm import RMSNorm, add_norm
-from automodel_amd.ops.rope import apply_rope, build_rope_cache, split_rope
+from automodel_amd.ops.rope import apply_rope, build_rope_cache, split_rope, token_rows
 from automodel_amd.ops.swiglu import swiglu, swiglu_cat
 from automodel_amd.parallel.cp import active_cp, cp_blockdiag_attention, cp_flash_attention
 from automodel_amd.serving.decode_linear import decode_rows, plain_linears, unobserved
@@ -409,11 +409,16 @@ class LlamaModel(nn.Module):
         self.register_buffer("rope_sin", sin, persistent=False)
 
     def forward(self, input_ids: torch.Tensor, position_ids: torch.Tensor | None = None) -> torch.Tensor:
-        x = self.embed_tokens(input_ids)
+        begun = None
+        if position_ids is not None and active_kv_cache() is not None:
+            begun = token_rows(self.embed_tokens, input_ids, position_ids[0], self.rope_cos, self.rope_sin)
+        x = self.embed_tokens(input_ids) if begun is None else begun[0]
         if self.cfg.embedding_multiplier != 1.0:
             x = x * self.cfg.embedding_multiplier
         S = input_ids.shape[1]
-        if position_ids is None:
+        if begun is not None:
+            cos, sin = begun[1:]
+        elif position_ids is None:
             cos, sin = self.rope_cos[:S], self.rope_sin[:S]
         else:
             cos, sin = self.rope_cos[position_ids[0]], self.rope_sin[position_ids[0]]

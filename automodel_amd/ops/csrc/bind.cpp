@@ -26,6 +26,8 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("rope_fwd", &amd_ops::rope_fwd);
   m.def("rope_split(Tensor qkv, Tensor cos, Tensor sin, int heads, int kv_heads) -> (Tensor, Tensor, Tensor)");
   m.impl("rope_split", &amd_ops::rope_split);
+  m.def("token_rows(Tensor ids, Tensor table, Tensor pos, Tensor cos, Tensor sin) -> (Tensor, Tensor, Tensor)");
+  m.impl("token_rows", &amd_ops::token_rows);
   m.def("rope_join(Tensor dq, Tensor dk, Tensor dv, Tensor cos, Tensor sin) -> Tensor");
   m.impl("rope_join", &amd_ops::rope_join);
 

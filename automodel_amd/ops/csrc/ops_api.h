@@ -22,6 +22,9 @@ std::tuple<at::Tensor, at::Tensor> rope_fwd(const at::Tensor& q, const at::Tenso
 
 std::tuple<at::Tensor, at::Tensor, at::Tensor> rope_split(const at::Tensor& qkv, const at::Tensor& cosb,
                                                           const at::Tensor& sinb, int64_t Hq, int64_t Hk);
+std::tuple<at::Tensor, at::Tensor, at::Tensor> token_rows(const at::Tensor& ids, const at::Tensor& table,
+                                                          const at::Tensor& pos, const at::Tensor& cos,
+                                                          const at::Tensor& sin);
 at::Tensor rope_join(const at::Tensor& dq, const at::Tensor& dk, const at::Tensor& dv, const at::Tensor& cosb,
                      const at::Tensor& sinb);
 

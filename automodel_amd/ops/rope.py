@@ -10,9 +10,10 @@ shape [S, head_dim] (half-table duplicated, fp32).
 from __future__ import annotations
 
 import torch
+import torch.nn as nn
 
-from automodel_amd.ops._backend import followed, hip_ops
-from automodel_amd.ops.linear import _ordinary
+from automodel_amd.ops._backend import followed, hip_ops, ops_available
+from automodel_amd.ops.linear import _functions_followed, _ordinary, _unseen
 
 
 def build_rope_cache(
@@ -169,6 +170,25 @@ def split_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, heads: i
             and qkv.data_ptr() % 16 == 0 and cos.data_ptr() % 16 == 0 and sin.data_ptr() % 16 == 0):
         return None
     return _RopeSplit.apply(qkv, cos, sin, heads, kv_heads)
+
+
+def token_rows(embed: nn.Module, ids: torch.Tensor, pos: torch.Tensor, cos: torch.Tensor,
+               sin: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None:
+    """``embed(ids)``, and ``cos[pos]`` and ``sin[pos]`` as float32, in one launch, for a decode step; None where the
+    kernel does not take that, and nothing is done."""
+    if (followed() or torch.is_grad_enabled() or not ids.is_cuda or type(embed) is not nn.Embedding
+            or embed.max_norm is not None or "forward" in embed.__dict__):
+        return None
+    table = embed.weight
+    if not (_ordinary(ids, pos, cos, sin, table) and table.dtype == torch.bfloat16 and table.shape[1] % 8 == 0
+            and ids.dtype == pos.dtype == torch.int64 and pos.dim() == 1 and 0 < ids.numel() <= 64 and 0 < len(pos) <= 64
+            and cos.dim() == 2 and cos.dtype == sin.dtype and cos.dtype in (torch.bfloat16, torch.float32)
+            and cos.shape == sin.shape and cos.numel() > 0 and table.numel() > 0 and table.data_ptr() % 16 == 0
+            and all(t.device == ids.device and t.is_contiguous() for t in (ids, pos, cos, sin, table))
+            and not _functions_followed() and _unseen(embed) and ops_available()):
+        return None
+    op = getattr(torch.ops.amd_ops, "token_rows", None)          # not in the inference kernels alone
+    return None if op is None else op(ids, table, pos, cos, sin)
 
 
 def apply_rope(

@@ -64,6 +64,8 @@ class DecodeSession:
         self.cache = make_cache(model, max_batch, max_len, static)
         self.device = next(model.parameters()).device
         self.live: list[int] = []
+        # a step's position is a view of these: an arange of its own is a launch
+        self.places = None if self.cache.ragged else torch.arange(max_len, device=self.device)
 
     @torch.no_grad()
     def prefill(self, prompts: Sequence[Sequence[int]],
@@ -113,7 +115,10 @@ class DecodeSession:
                 return logits
             if handles != self.live:
                 raise ValueError("a dense K/V cache moves its whole batch on")
-            pos = torch.arange(cache.pos, cache.pos + 1, device=self.device).unsqueeze(0)
+            if cache.pos < len(self.places):
+                pos = self.places[cache.pos:cache.pos + 1].unsqueeze(0)
+            else:
+                pos = torch.arange(cache.pos, cache.pos + 1, device=self.device).unsqueeze(0)
             logits = self.model(tokens.reshape(-1, 1), position_ids=pos)[:, -1]
             cache.advance(1)
             return logits
