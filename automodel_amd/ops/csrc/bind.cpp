@@ -128,7 +128,7 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("small_tn", &amd_ops::small_tn);
   m.def("small_cut(int rows, int cols, int sum) -> (int, int)", &amd_ops::small_cut);
   m.def("linear_small(Tensor x, Tensor w) -> Tensor", &amd_ops::linear_small);
-  m.def("linear_y(Tensor x, Tensor w) -> Tensor");
+  m.def("linear_y(Tensor x, Tensor w, bool relu2=False) -> Tensor");
   m.impl("linear_y", &amd_ops::linear_y);
   m.def("linear_y_cut(int T, int N, int K) -> int[]");
   m.impl("linear_y_cut", &amd_ops::linear_y_cut);

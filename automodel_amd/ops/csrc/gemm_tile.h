@@ -104,6 +104,12 @@ __device__ __forceinline__ void load_lds(unsigned lds, int to, unsigned off, con
                :: "s"(lds + to), "v"(off), "s"(rsrc) : "memory", "m0");
 }
 
+// max(x, 0)^2; NaN stays
+__device__ __forceinline__ float relu2(float x) {
+  const float y = x < 0.f ? 0.f : x;
+  return y * y;
+}
+
 // the lane, formed anew: what follows from it is not kept in registers over the whole kernel
 __device__ __forceinline__ int lane_here() {
   int lane = threadIdx.x & 63;
@@ -230,10 +236,11 @@ struct Operand {
 // first() and next() are their numbers, or negative; get(number) is the tile; loaded() is called once, while
 // the first tile's operands come.
 // PARTS: tiles of sums that are added up later, 32 bits in the order of the accumulators.
+// RELU2: the results are max(sum, 0)^2.
 // EXTRA: the second pair is [rows][rank] and [columns][rank_c], short rows that are loaded as fragments behind the
 // sum. They come from the L2, and with them the wave waits for the next tile's loads (8192 rows, a sum of 4096,
 // 4096 columns: 192 us without, 190 with it).
-template <bool RC, bool CC, class Tiles, bool SHORT = RC && CC, bool PARTS = false, bool EXTRA = false>
+template <bool RC, bool CC, class Tiles, bool SHORT = RC && CC, bool PARTS = false, bool EXTRA = false, bool RELU2 = false>
 struct Run {
   static constexpr bool TN = RC && CC, NN = !RC && CC, NT = !CC;
   Tiles& tiles;
@@ -454,7 +461,7 @@ struct Run {
       for (int j = 0; j < 8; ++j) {
         bf16x4_t w;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) w[r] = (__bf16)acc[decltype(i_)::value][j][r];
+        for (int r = 0; r < 4; ++r) w[r] = (__bf16)(RELU2 ? relu2(acc[decltype(i_)::value][j][r]) : acc[decltype(i_)::value][j][r]);
         *reinterpret_cast<bf16x4_t*>(mine + i16 * 256 + (((2 * j + (g >> 1)) ^ i16) << 4) + (g & 1) * 8) = w;
       }
       asm volatile("" ::: "memory");

@@ -49,14 +49,14 @@ __global__ __launch_bounds__(256) void add_parts_kernel(const Args a) {
     if (row >= rows || col >= a.cols) continue;
     fa::bf16x4_t o;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = (__bf16)s[e];
+    for (int e = 0; e < 4; ++e) o[e] = (__bf16)(a.relu2 ? gt::relu2(s[e]) : s[e]);
     *reinterpret_cast<fa::bf16x4_t*>(a.out + (long)(r0 + row) * a.cols + col) = o;
   }
 }
 
 template <lg::Form FORM>
 at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t cols, int64_t sum,
-               const at::Tensor* r2 = nullptr, const at::Tensor* c2 = nullptr) {
+               const at::Tensor* r2 = nullptr, const at::Tensor* c2 = nullptr, bool relu2 = false) {
   TORCH_CHECK(r.is_cuda() && r.device() == c.device() && r.is_contiguous() && c.is_contiguous() &&
                   r.scalar_type() == at::kBFloat16 && c.scalar_type() == at::kBFloat16,
               "linear_grad: contiguous bf16 operands on one GPU");
@@ -68,7 +68,7 @@ at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t c
   auto out = at::empty({rows, cols}, r.options());
   if (out.numel() == 0) return out;
   Args a{reinterpret_cast<const bf16*>(r.data_ptr()), reinterpret_cast<const bf16*>(c.data_ptr()),
-         reinterpret_cast<bf16*>(out.data_ptr()), nullptr, (int)rows, (int)cols, (int)sum, 0, 0, 0, nullptr, nullptr, 0, 0};
+         reinterpret_cast<bf16*>(out.data_ptr()), nullptr, (int)rows, (int)cols, (int)sum, 0, 0, 0, nullptr, nullptr, 0, 0, relu2};
   if (r2) {
     a.r2 = reinterpret_cast<const bf16*>(r2->data_ptr());
     a.c2 = reinterpret_cast<const bf16*>(c2->data_ptr());
@@ -139,11 +139,12 @@ at::Tensor linear_dx_extra(const at::Tensor& g, const at::Tensor& w, const at::T
   return run<lg::DX>(g, w, g.size(0), w.size(1), w.size(0), &t, &a_t);
 }
 
-at::Tensor linear_y(const at::Tensor& x, const at::Tensor& w) {
+// x w^T, or max(x w^T, 0)^2 of the unrounded sums
+at::Tensor linear_y(const at::Tensor& x, const at::Tensor& w, bool relu2) {
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "linear_y: x [T, K], w [N, K]");
   TORCH_CHECK(w.size(1) >= 4 * gt::STEP && w.size(1) % (2 * gt::STEP) == 0 && w.size(0) % 8 == 0,
               "linear_y: K%64 == 0 and 128 or more, N%8 == 0");
-  return run<lg::Y>(x, w, x.size(0), w.size(0), w.size(1));
+  return run<lg::Y>(x, w, x.size(0), w.size(0), w.size(1), nullptr, nullptr, relu2);
 }
 
 // x w^T + scale (x A^T) B^T, A [r, K], B [N, r], r a multiple of 8 up to 64: B's product behind the sums, one rounding. ->

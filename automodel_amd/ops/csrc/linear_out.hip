@@ -3,7 +3,9 @@
 // are cut as the gradients' are. us, library -> here, bf16 of unit variance, the weights not in a cache:
 //   511 x 14336 -> 4096 92 -> 67 (256 rows, 8 parts), 1001 x 21504 -> 4096 240 -> 150, 3003 x 2048 -> 2816 43 -> 34,
 //   6001 x 4096 -> 4096 156 -> 143, 24000 x 4096 -> 14336 1977 -> 1913; 8192 x 4096 -> 28672 1264 and 1282.
-// ops/linear.py (output_own) has the rule and what it was fitted to.
+// The squared ReLU of a feed-forward layer's inner results is formed on the way out (6600 x 4096 -> 21504: a pass of 92 us
+// less, of some 800). ops/linear.py (output_own, squared_own) has the rules and what they were
+// fitted to.
 #include <ATen/ATen.h>
 
 #include "common.h"
@@ -13,15 +15,16 @@ namespace amd_ops {
 namespace lg {
 
 void launch_out(const Args& a, unsigned blocks, hipStream_t stream) {
-  const auto launch = [&](auto parts_, auto extra_) {
-    hipLaunchKernelGGL((linear_tile_kernel<Y, false, decltype(parts_)::value, decltype(extra_)::value>), dim3(blocks),
-                       dim3(gt::THREADS), gt::SMEM, stream, a);
+  const auto launch = [&](auto parts_, auto extra_, auto relu2_) {
+    hipLaunchKernelGGL((linear_tile_kernel<Y, false, decltype(parts_)::value, decltype(extra_)::value, decltype(relu2_)::value>),
+                       dim3(blocks), dim3(gt::THREADS), gt::SMEM, stream, a);
     HIP_CHECK_KERNEL();
   };
   using Yes = std::true_type;
   using No = std::false_type;
-  if (a.parts > 1) a.rank ? launch(Yes{}, Yes{}) : launch(Yes{}, No{});
-  else a.rank ? launch(No{}, Yes{}) : launch(No{}, No{});
+  if (a.parts > 1) a.rank ? launch(Yes{}, Yes{}, No{}) : launch(Yes{}, No{}, No{});
+  else if (a.relu2) launch(No{}, No{}, Yes{});
+  else a.rank ? launch(No{}, Yes{}, No{}) : launch(No{}, No{}, No{});
 }
 
 }  // namespace lg

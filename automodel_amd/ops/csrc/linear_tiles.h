@@ -20,6 +20,7 @@ struct Args {
   int height, parts, per;              // rows of a tile; parts of the sum, and how much of it each but the last has
   const bf16 *r2, *c2;                 // EXTRA: [rows][rank] and [cols][rank_c], whose product is added
   int rank, rank_c;
+  bool relu2;                          // Y: max(sum, 0)^2
 };
 
 // The tiles' order is down 4 row tiles, then on to the next column tile: the 32 tiles of an XCD at a time read
@@ -72,13 +73,13 @@ struct Tiles {
   }
 };
 
-// SHORT, PARTS, EXTRA: gemm_tile.h
-template <Form F, bool SHORT, bool PARTS, bool EXTRA = false>
+// SHORT, PARTS, EXTRA, RELU2: gemm_tile.h
+template <Form F, bool SHORT, bool PARTS, bool EXTRA = false, bool RELU2 = false>
 __global__ __launch_bounds__(gt::THREADS, 1) void linear_tile_kernel(const Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   Tiles<F, EXTRA> tiles(a);
   const gt::Shape shape{2u * (F == DW ? a.rows : a.sum), 2u * (F == Y ? a.sum : a.cols), 2u * a.cols};
-  gt::Run<F == DW, F != Y, Tiles<F, EXTRA>, SHORT, PARTS, EXTRA>(tiles, shape, smem)();
+  gt::Run<F == DW, F != Y, Tiles<F, EXTRA>, SHORT, PARTS, EXTRA, RELU2>(tiles, shape, smem)();
 }
 
 // us that tiles of `height` rows and sums in `parts` take. A pair of steps of a tile of 32 n rows takes a + b

@@ -14,7 +14,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from automodel_amd.ops.linear import inferred
+from automodel_amd.ops.linear import inferred, squared_own
 
 _PAD_TO = {5: 8, 6: 8, 7: 8, 9: 16, 10: 16, 11: 16, 12: 16, 13: 16, 14: 16, 15: 16}
 
@@ -72,7 +72,10 @@ def project(lin: nn.Module, x: torch.Tensor, relu2: bool = False,
     if out_f32 and x.dtype == torch.bfloat16:
         y = torch.mm(x, w.t(), out_dtype=torch.float32)
     else:
-        y = inferred(x, w)
+        squared = relu2 and squared_own(x.shape[0], *w.shape)
+        y = inferred(x, w, squared)
+        if squared and y is not None:
+            return y
         y = F.linear(x, w) if y is None else y
     return rn.relu2(y) if relu2 else y
 

@@ -37,7 +37,22 @@ def test_products(T, N, K, parts):
     x, w = rand(T, K), rand(N, K)
     height, cut = hip_ops().linear_y_cut(T, N, K)
     assert 128 <= height <= 256 and height % 32 == 0 and (parts is None or (cut > 1) == parts)
-    close(hip_ops().linear_y(x, w), x.double() @ w.double().t(), K)
+    want = x.double() @ w.double().t()
+    close(hip_ops().linear_y(x, w), want, K)
+    close(hip_ops().linear_y(x, w, True), want.relu().square(), K)
+
+
+@gpu
+@cuda
+def test_squares_of_strange_sums():
+    from automodel_amd.ops._backend import hip_ops
+
+    for K in (128, 8256):
+        x, w = torch.zeros(300, K, device="cuda").bfloat16(), rand(520, K).abs()
+        x[1, 3], x[2, 5], x[3, 7], x[4, 9] = float("inf"), -float("inf"), float("nan"), -1e30
+        y = hip_ops().linear_y(x, w, True)
+        assert (y[1] == float("inf")).all() and (y[2] == 0).all() and y[3].isnan().all() and (y[4] == 0).all()
+        assert (y[[0, 5, 299]] == 0).all()
 
 
 @gpu
@@ -98,7 +113,11 @@ def test_calls_without_gradients(T, N, K):
             assert torch.equal(y, want) and not y.requires_grad
         assert torch.equal(L.linear(lin, x[None]), want[None])
         assert torch.equal(L.linear(lin, x, beside=True), F.linear(x, lin.weight))
-        assert torch.equal(project(lin, x, relu2=True), F.relu(want.float()).square().bfloat16())
+        squares = project(lin, x, relu2=True)
+        if L.small(T, N, K):                       # a pass of its own, over rounded results
+            assert torch.equal(squares, F.relu(want.float()).square().bfloat16())
+        else:
+            close(squares, (x.double() @ lin.weight.double().t()).relu().square(), K)
         # what the kernels do not take is the library's, as before
         strange = (rand(T, 2 * K)[:, ::2], rand(T * K + 1)[1:].view(T, K), rand(K, T).t(), rand(1, K).expand(T, K))
         for v in strange:
