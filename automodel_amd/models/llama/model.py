@@ -27,7 +27,7 @@ from automodel_amd.ops.rms_norm import RMSNorm, add_norm
 from automodel_amd.ops.rope import apply_rope, build_rope_cache, split_rope, token_rows
 from automodel_amd.ops.swiglu import swiglu, swiglu_cat
 from automodel_amd.parallel.cp import active_cp, cp_blockdiag_attention, cp_flash_attention
-from automodel_amd.serving.decode_linear import decode_rows, plain_linears, unobserved
+from automodel_amd.serving.decode_linear import decode_rows, glu_rows, plain_linears, unobserved
 from automodel_amd.utils.kv_cache import KVCache, StaticKVCache, active_kv_cache, maybe_update_kv
 
 
@@ -277,6 +277,9 @@ class LlamaMLP(nn.Module):
             act = decode_rows(lins, x, glu=True)
             if act is not None:
                 return _project(self.backend, [self.down_proj], act[0])[0]
+            act = glu_rows(lins, x)
+            if act is not None:
+                return linear(self.down_proj, act)
         if self.fused:
             return linear(self.down_proj, swiglu_cat(linear(self.gate_up_proj, x)))
         return linear(self.down_proj,

@@ -130,6 +130,8 @@ TORCH_LIBRARY(amd_ops, m) {
   m.def("linear_small(Tensor x, Tensor w) -> Tensor", &amd_ops::linear_small);
   m.def("linear_y(Tensor x, Tensor w, bool relu2=False) -> Tensor");
   m.impl("linear_y", &amd_ops::linear_y);
+  m.def("linear_glu(Tensor x, Tensor w, Tensor up) -> Tensor");
+  m.impl("linear_glu", &amd_ops::linear_glu);
   m.def("linear_y_cut(int T, int N, int K) -> int[]");
   m.impl("linear_y_cut", &amd_ops::linear_y_cut);
   m.def("linear_dw(Tensor g, Tensor x) -> Tensor");

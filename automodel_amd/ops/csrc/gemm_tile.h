@@ -120,6 +120,7 @@ __device__ __forceinline__ int lane_here() {
 // What is multiplied: pointers to the tile's first row and column and the sum's first element.
 struct Tile {
   const bf16 *r, *c;
+  const bf16* up;              // GLU: the second matrix of columns
   const bf16 *r2, *c2;         // a second pair, added to the sum, or null
   int rank, rank_c;            // EXTRA: how long a row of r2 is, a multiple of 32, and of c2, one of 8: zeros behind it
   int rows, cols;              // of the output, from the tile's first on
@@ -136,8 +137,9 @@ struct Shape {
   unsigned r, c, out;
 };
 
-// SHORT: the sum may end within what is loaded
-template <bool COLS, bool SHORT>
+// SHORT: the sum may end within what is loaded. TWO: 16 rows of one matrix, 16 of the other, 128 of each; the first two
+// waves load the one's, the others the other's.
+template <bool COLS, bool SHORT, bool TWO = false>
 struct Operand {
   static constexpr int N = COLS ? 4 : 8;       // loads of a wave: for a step, or for a pair
   static constexpr int W = COLS ? 8 : 2;
@@ -157,8 +159,8 @@ struct Operand {
         const int row = 8 * h + 2 * wid + (lane >> 5);
         off[h] = row * ld + ((lane & 31) ^ (place(row) << 1)) * 16;
       } else {
-        const int row = (4 * h + wid) * 8 + (lane >> 3);
-        off[h] = row * ld + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+        const int row = (4 * h + wid) * 8 + (lane >> 3), from = TWO ? h * 16 + (row & 15) : row;
+        off[h] = from * ld + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
       }
     }
   }
@@ -168,7 +170,7 @@ struct Operand {
   __device__ __forceinline__ void aim(const bf16* p, int edge, int sum) {
     base = reinterpret_cast<const char*>(p);
     left = sum;
-    all = COLS ? ld - 2 * edge : min(edge, TILE) * ld;
+    all = COLS ? ld - 2 * edge : min(edge, TWO ? TILE / 2 : TILE) * ld;
     count();
   }
   __device__ __forceinline__ void count() {
@@ -237,10 +239,12 @@ struct Operand {
 // the first tile's operands come.
 // PARTS: tiles of sums that are added up later, 32 bits in the order of the accumulators.
 // RELU2: the results are max(sum, 0)^2.
+// GLU: the columns are 16 of one matrix and 16 of another, in turn, so that a lane has the sums of both for its column;
+// the results, half as many, are silu(one) other.
 // EXTRA: the second pair is [rows][rank] and [columns][rank_c], short rows that are loaded as fragments behind the
 // sum. They come from the L2, and with them the wave waits for the next tile's loads (8192 rows, a sum of 4096,
 // 4096 columns: 192 us without, 190 with it).
-template <bool RC, bool CC, class Tiles, bool SHORT = RC && CC, bool PARTS = false, bool EXTRA = false, bool RELU2 = false>
+template <bool RC, bool CC, class Tiles, bool SHORT = RC && CC, bool PARTS = false, bool EXTRA = false, bool RELU2 = false, bool GLU = false>
 struct Run {
   static constexpr bool TN = RC && CC, NN = !RC && CC, NT = !CC;
   Tiles& tiles;
@@ -249,7 +253,7 @@ struct Run {
   unsigned lds, cur, oth;      // buffers' addresses: of the pair at hand, of the other
   int by, wid;
   Operand<RC, SHORT> R;
-  Operand<CC, SHORT> C;
+  Operand<CC, SHORT, GLU> C;
 
   __device__ __forceinline__ Run(Tiles& t, const Shape& sh, char* s) : tiles(t), smem(s), shape(sh) {
     wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -264,7 +268,7 @@ struct Run {
   // where the loads go on: at a tile, at its second pair of operands before pair `at` + 2, or at the next tile
   __device__ __forceinline__ void aim(const Tile& t) {
     R.aim(t.r, t.rows, t.sum);
-    C.aim(t.c, t.cols, t.sum);
+    C.aim(GLU && wid >> 1 ? t.up : t.c, t.cols, t.sum);
   }
   __device__ __forceinline__ void go_on(const Tile& t, const Tile& u, int n, int& at) {
     if (NN && !EXTRA && t.r2 && at != n - 2) {
@@ -319,7 +323,7 @@ struct Run {
     //   NN: P 0: four of columns, for the step four on; P 1: eight of rows, for the pair two on, and four of columns
     //   NT: from P 0 on, when the rows' and columns' fragments are read (MID): eight of both, for the pair two on
     // Waits: what is read next has landed. So many loads are later (NT: of the 16 those before the middle of P 1), and
-    // in a tile's first pair the last tile's stores are, 16 at least (loads and stores are counted in the order of
+    // in a tile's first pair the last tile's stores are, 16 at least, of GLU 8 (loads and stores are counted in the order of
     // their issue).
     constexpr int RR = RC ? 2 : 1, CR = CC ? 2 : 1, READS = NR * RR + 8 * CR, S = NR * 8;
     auto step = [&](auto p_, auto first_) __attribute__((always_inline)) {
@@ -327,7 +331,7 @@ struct Run {
       constexpr bool FIRST = decltype(first_)::value;
       constexpr int DENSE = READS > 3 * S / 8 ? READS : 3 * S / 8;
       constexpr int MID = DENSE + 4, OVER = 2 * S - MID;       // NT: slots of a pair that loads are spread over
-      constexpr int LATER = (NT ? ((S + S / 2 - MID) * 16 + OVER - 1) / OVER : NN && P == 1 ? 8 : 16) + (FIRST ? 16 : 0);
+      constexpr int LATER = (NT ? ((S + S / 2 - MID) * 16 + OVER - 1) / OVER : NN && P == 1 ? 8 : 16) + (FIRST ? (GLU ? 8 : 16) : 0);
       // slots of the reads
       constexpr int FROM = NT && P == 1 ? S / 2 : 0, TO = TN || NN || P == 1 ? S : DENSE;
       if constexpr (!NT) {
@@ -406,6 +410,7 @@ struct Run {
     if constexpr (EXTRA) extra<NR>(acc, t);
     settle();
     if constexpr (PARTS) keep<NR>(acc, t);
+    else if constexpr (GLU) store_glu<NR>(acc, t);
     else store<NR>(acc, t);
   }
 
@@ -480,6 +485,47 @@ struct Run {
         const int row = r0 + i * 16 + 4 * k + g;
         const unsigned o = row * shape.out + (c0 + i16 * 8) * 2;
         __builtin_amdgcn_raw_buffer_store_b128(v[k], rsrc, row < t.rows && i16 < chunks ? o : 0xfffffff0u, 0, 0);
+      }
+    });
+    asm volatile("" ::: "memory");
+  }
+
+  // The same of silu(acc[i][2 j]) acc[i][2 j + 1], 64 columns a wave: 2 NR stores.
+  template <int NR>
+  __device__ __forceinline__ void store_glu(const f32x4_t (&acc)[NR][8], const Tile& t) {
+    const int lane = lane_here(), i16 = lane & 15, g = lane >> 4;
+    char* mine = smem + STAGE + wid * 4096;
+    const int c0 = (wid & 1) * 64, chunks = min(t.cols - c0, 64) / 8, r0 = (wid >> 1) * (NR * 16);
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(t.out, 0, 0xffffff00, 0x00027000);
+    auto put = [&](auto i_) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        bf16x4_t w;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float a = acc[decltype(i_)::value][2 * j][r];
+          w[r] = (__bf16)(a * __builtin_amdgcn_rcpf(1.f + __expf(-a)) * acc[decltype(i_)::value][2 * j + 1][r]);
+        }
+        *reinterpret_cast<bf16x4_t*>(mine + i16 * 128 + (((2 * j + (g >> 1)) ^ (i16 >> 1)) << 4) + (g & 1) * 8) = w;
+      }
+      asm volatile("" ::: "memory");
+    };
+    put(std::integral_constant<int, 0>{});
+    fa::unrolled<NR>([&](auto i_) __attribute__((always_inline)) {
+      constexpr int i = decltype(i_)::value;
+      u32x4_t v[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int row = 8 * k + (lane >> 3);
+        v[k] = *reinterpret_cast<const u32x4_t*>(mine + row * 128 + (((lane & 7) ^ (row >> 1)) << 4));
+      }
+      asm volatile("" ::: "memory");
+      if constexpr (i + 1 < NR) put(std::integral_constant<int, i + 1>{});
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int row = r0 + i * 16 + 8 * k + (lane >> 3);
+        const unsigned o = row * shape.out + (c0 + (lane & 7) * 8) * 2;
+        __builtin_amdgcn_raw_buffer_store_b128(v[k], rsrc, row < t.rows && (lane & 7) < chunks ? o : 0xfffffff0u, 0, 0);
       }
     });
     asm volatile("" ::: "memory");

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256) void add_parts_kernel(const Args a) {
 
 template <lg::Form FORM>
 at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t cols, int64_t sum,
-               const at::Tensor* r2 = nullptr, const at::Tensor* c2 = nullptr, bool relu2 = false) {
+               const at::Tensor* r2 = nullptr, const at::Tensor* c2 = nullptr, bool relu2 = false, const at::Tensor* up = nullptr) {
   TORCH_CHECK(r.is_cuda() && r.device() == c.device() && r.is_contiguous() && c.is_contiguous() &&
                   r.scalar_type() == at::kBFloat16 && c.scalar_type() == at::kBFloat16,
               "linear_grad: contiguous bf16 operands on one GPU");
@@ -65,10 +65,11 @@ at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t c
   // a tile's addresses are 32 bits: 256 rows of 2^23
   TORCH_CHECK(std::max({rows, cols, sum}) < (1l << 23), "linear_grad: sizes below 2^23");
   const c10::DeviceGuard guard(r.device());
-  auto out = at::empty({rows, cols}, r.options());
+  auto out = at::empty({rows, FORM == lg::GLU ? cols / 2 : cols}, r.options());
   if (out.numel() == 0) return out;
   Args a{reinterpret_cast<const bf16*>(r.data_ptr()), reinterpret_cast<const bf16*>(c.data_ptr()),
-         reinterpret_cast<bf16*>(out.data_ptr()), nullptr, (int)rows, (int)cols, (int)sum, 0, 0, 0, nullptr, nullptr, 0, 0, relu2};
+         reinterpret_cast<bf16*>(out.data_ptr()), nullptr, (int)rows, (int)cols, (int)sum, 0, 0, 0, nullptr, nullptr, 0, 0, relu2,
+         up ? reinterpret_cast<const bf16*>(up->data_ptr()) : nullptr};
   if (r2) {
     a.r2 = reinterpret_cast<const bf16*>(r2->data_ptr());
     a.c2 = reinterpret_cast<const bf16*>(c2->data_ptr());
@@ -95,6 +96,8 @@ at::Tensor run(const at::Tensor& r, const at::Tensor& c, int64_t rows, int64_t c
   using No = std::false_type;
   if constexpr (FORM == lg::Y) {
     lg::launch_out(a, (unsigned)blocks, stream);
+  } else if constexpr (FORM == lg::GLU) {
+    lg::launch_glu(a, (unsigned)blocks, stream);
   } else if constexpr (FORM == lg::DW) {
     if (a.parts > 1) launch(Yes{}, Yes{});
     else launch(Yes{}, No{});
@@ -145,6 +148,17 @@ at::Tensor linear_y(const at::Tensor& x, const at::Tensor& w, bool relu2) {
   TORCH_CHECK(w.size(1) >= 4 * gt::STEP && w.size(1) % (2 * gt::STEP) == 0 && w.size(0) % 8 == 0,
               "linear_y: K%64 == 0 and 128 or more, N%8 == 0");
   return run<lg::Y>(x, w, x.size(0), w.size(0), w.size(1), nullptr, nullptr, relu2);
+}
+
+// silu(x w^T) (x up^T) of the unrounded sums
+at::Tensor linear_glu(const at::Tensor& x, const at::Tensor& w, const at::Tensor& up) {
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) && up.sizes() == w.sizes(),
+              "linear_glu: x [T, K], w and up [I, K]");
+  TORCH_CHECK(w.size(1) >= 4 * gt::STEP && w.size(1) % (2 * gt::STEP) == 0 && w.size(0) % 8 == 0 && w.size(0) < (1l << 22),
+              "linear_glu: K%64 == 0 and 128 or more, I%8 == 0");
+  TORCH_CHECK(up.device() == x.device() && up.is_contiguous() && up.scalar_type() == at::kBFloat16 &&
+                  (uintptr_t)up.data_ptr() % 16 == 0, "linear_glu: up as w");
+  return run<lg::GLU>(x, w, x.size(0), 2 * w.size(0), w.size(1), nullptr, nullptr, false, &up);
 }
 
 // x w^T + scale (x A^T) B^T, A [r, K], B [N, r], r a multiple of 8 up to 64: B's product behind the sums, one rounding. ->

@@ -10,7 +10,7 @@
 namespace amd_ops {
 namespace lg {
 
-enum Form { Y, DX, DW };
+enum Form { Y, DX, DW, GLU };
 
 struct Args {
   const bf16 *r, *c;
@@ -21,6 +21,7 @@ struct Args {
   const bf16 *r2, *c2;                 // EXTRA: [rows][rank] and [cols][rank_c], whose product is added
   int rank, rank_c;
   bool relu2;                          // Y: max(sum, 0)^2
+  const bf16* up;                      // GLU: c is [cols / 2][sum], and so is this
 };
 
 // The tiles' order is down 4 row tiles, then on to the next column tile: the 32 tiles of an XCD at a time read
@@ -62,6 +63,12 @@ struct Tiles {
     t.r = F == DW ? a.r + (long)from * a.rows + r0 : a.r + (long)r0 * a.sum + from;
     t.c = F == Y ? a.c + (long)c0 * a.sum + from : a.c + (long)from * a.cols + c0;
     t.out = a.out + (long)r0 * a.cols + c0;
+    if constexpr (F == GLU) {
+      t.cols = (a.cols - c0) / 2;
+      t.c = a.c + (long)(c0 / 2) * a.sum;
+      t.up = a.up + (long)(c0 / 2) * a.sum;
+      t.out = a.out + (long)r0 * (a.cols / 2) + c0 / 2;
+    }
     t.part = a.part + (long)u * a.height * gt::TILE;
     if (EXTRA && s == 0) {
       t.r2 = a.r2 + (long)r0 * a.rank;
@@ -78,8 +85,9 @@ template <Form F, bool SHORT, bool PARTS, bool EXTRA = false, bool RELU2 = false
 __global__ __launch_bounds__(gt::THREADS, 1) void linear_tile_kernel(const Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   Tiles<F, EXTRA> tiles(a);
-  const gt::Shape shape{2u * (F == DW ? a.rows : a.sum), 2u * (F == Y ? a.sum : a.cols), 2u * a.cols};
-  gt::Run<F == DW, F != Y, Tiles<F, EXTRA>, SHORT, PARTS, EXTRA, RELU2>(tiles, shape, smem)();
+  const gt::Shape shape{2u * (F == DW ? a.rows : a.sum), 2u * (F == Y || F == GLU ? a.sum : a.cols),
+                        F == GLU ? (unsigned)a.cols : 2u * a.cols};
+  gt::Run<F == DW, F == DW || F == DX, Tiles<F, EXTRA>, SHORT, PARTS, EXTRA, RELU2, F == GLU>(tiles, shape, smem)();
 }
 
 // us that tiles of `height` rows and sums in `parts` take. A pair of steps of a tile of 32 n rows takes a + b
@@ -104,13 +112,14 @@ inline float predicted(Form form, long rows, long cols, long sum, int height, in
   return parts == 1 ? t : t + f.add + f.add_mb * 1e-6f * rows * cols * parts;
 }
 
+// (GLU: sums are whole)
 inline void cut(Form form, Args& a) {
   float least = 0.f;
   a.height = 0;
   for (const int parts : {1, 2, 3, 4, 6, 8}) {
     const int per = (a.sum + 64 * parts - 1) / (64 * parts) * 64;
     // each has 4 pairs of steps or more, the last one 2
-    if (parts > 1 && (per < 256 || a.sum - (parts - 1) * per < 128)) continue;
+    if (parts > 1 && (form == GLU || per < 256 || a.sum - (parts - 1) * per < 128)) continue;
     for (int height = 128; height <= gt::TILE; height += 32) {
       const float t = predicted(form, a.rows, a.cols, a.sum, height, parts);
       if (a.height && t >= least) continue;
@@ -126,9 +135,10 @@ inline long tiles_of(const Args& a) {
   return ((long)(a.rows + a.height - 1) / a.height) * ((a.cols + gt::TILE - 1) / gt::TILE);
 }
 
-// linear_dx with an EXTRA product (lora_grad.hip); linear_y, with one or without (linear_out.hip)
+// linear_dx with an EXTRA product (lora_grad.hip); linear_y, with one or without, and linear_glu (linear_out.hip)
 void launch_extra(const Args& a, unsigned blocks, hipStream_t stream);
 void launch_out(const Args& a, unsigned blocks, hipStream_t stream);
+void launch_glu(const Args& a, unsigned blocks, hipStream_t stream);
 
 }  // namespace lg
 }  // namespace amd_ops

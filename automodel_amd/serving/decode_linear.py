@@ -14,7 +14,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from automodel_amd.ops.linear import inferred, squared_own
+from automodel_amd.ops.linear import gated, inferred, squared_own
 
 _PAD_TO = {5: 8, 6: 8, 7: 8, 9: 16, 10: 16, 11: 16, 12: 16, 13: 16, 14: 16, 15: 16}
 
@@ -181,6 +181,16 @@ def decode_rows(lins: list[nn.Module], x: torch.Tensor,
 
     ys = hip_ops().decode_rows(x.view(rows, K), ws, glu)
     return [y.view(*x.shape[:-1], y.shape[-1]) for y in ys]
+
+
+def glu_rows(lins: list[nn.Module], x: torch.Tensor) -> torch.Tensor | None:
+    """``silu(a) * b`` of the outputs a and b of two layers, or of the halves of one layer's, in one launch, for a prompt's
+    many rows; None where that does not apply, and nothing is done."""
+    if torch.compiler.is_compiling() or torch.is_grad_enabled():
+        return None
+    if not plain_linears(*lins) or any("forward" in lin.__dict__ for lin in lins):
+        return None
+    return gated(x, [lin.weight for lin in lins])
 
 
 class DecodeLinear(nn.Linear):

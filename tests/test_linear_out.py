@@ -114,7 +114,7 @@ def test_calls_without_gradients(T, N, K):
         assert torch.equal(L.linear(lin, x[None]), want[None])
         assert torch.equal(L.linear(lin, x, beside=True), F.linear(x, lin.weight))
         squares = project(lin, x, relu2=True)
-        if L.small(T, N, K):                       # a pass of its own, over rounded results
+        if not L.squared_own(T, N, K):             # a pass of its own, over rounded results
             assert torch.equal(squares, F.relu(want.float()).square().bfloat16())
         else:
             close(squares, (x.double() @ lin.weight.double().t()).relu().square(), K)
