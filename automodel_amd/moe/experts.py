@@ -115,8 +115,7 @@ class _Experts(torch.autograd.Function):
         ops, plan = hip_ops(), (offs, tile_map, n_tiles, bm)
         gate, up, down = gate.contiguous(), up.contiguous(), down.contiguous()
         rows = ops.permute_rows(x.contiguous(), pos)
-        g, u = ops.grouped_gemm_nt(rows, gate, *plan), ops.grouped_gemm_nt(rows, up, *plan)
-        h = ops.swiglu_fwd(g, u)
+        g, u, h = ops.grouped_glu(rows, gate, up, *plan)
         y = ops.grouped_gemm_nt(h, down, *plan)
         ctx.inner = x.shape[1] >= 2 * gate.shape[1]
         ctx.save_for_backward(rows, g, u, gate, up, down, order, src, pos, perm_probs, offs, tile_map, n_tiles,

@@ -114,6 +114,8 @@ TORCH_LIBRARY(amd_ops, m) {
   m.impl("build_group_plan", &amd_ops::build_group_plan);
   m.def("grouped_gemm_nt(Tensor x, Tensor w, Tensor offs, Tensor tile_map, Tensor? n_tiles=None, int bm=128) -> Tensor");
   m.impl("grouped_gemm_nt", &amd_ops::grouped_gemm_nt);
+  m.def("grouped_glu(Tensor x, Tensor w, Tensor up, Tensor offs, Tensor tile_map, Tensor? n_tiles=None, int bm=128) -> (Tensor, Tensor, Tensor)");
+  m.impl("grouped_glu", &amd_ops::grouped_glu);
   m.def("grouped_gemm_nn(Tensor g, Tensor w, Tensor offs, Tensor tile_map, Tensor? n_tiles=None, int bm=128) -> Tensor");
   m.impl("grouped_gemm_nn", &amd_ops::grouped_gemm_nn);
   m.def("grouped_gemm_cap(int mode, int M, int E, int N, int K) -> int");

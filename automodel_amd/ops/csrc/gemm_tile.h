@@ -104,10 +104,27 @@ __device__ __forceinline__ void load_lds(unsigned lds, int to, unsigned off, con
                :: "s"(lds + to), "v"(off), "s"(rsrc) : "memory", "m0");
 }
 
+// the same from off + more on, which takes a register for the moment only
+__device__ __forceinline__ void load_lds(unsigned lds, int to, unsigned off, unsigned more, const char* base, unsigned num) {
+  const unsigned long p = (unsigned long)base;
+  const i32x4_t rsrc{(int)(unsigned)p, (int)(unsigned)(p >> 32), (int)num, 0x00027000};
+  unsigned at;
+  asm volatile("s_mov_b32 m0, %1\n\tv_add_u32 %0, %3, %2\n\tbuffer_load_dwordx4 %0, %4, 0 offen lds"
+               : "=&v"(at) : "s"(lds + to), "v"(off), "s"(more), "s"(rsrc) : "memory", "m0");
+}
+
 // max(x, 0)^2; NaN stays
 __device__ __forceinline__ float relu2(float x) {
   const float y = x < 0.f ? 0.f : x;
   return y * y;
+}
+
+// silu(a) b as swiglu.hip has it, to the bit but for quotients below 2^-126: one step of Newton's method instead of a
+// division of ten instructions (its quotient is the rounded one but for divisors of 24 ones)
+__device__ __forceinline__ float rounded_glu(__bf16 one, __bf16 other) {
+  const float a = (float)one, d = 1.f + __expf(-a), r = __builtin_amdgcn_rcpf(d);
+  const float sigmoid = d > 3.4e38f ? 0.f : fmaf(fmaf(-d, r, 1.f), r, r);
+  return a * sigmoid * (float)other;
 }
 
 // the lane, formed anew: what follows from it is not kept in registers over the whole kernel
@@ -119,14 +136,25 @@ __device__ __forceinline__ int lane_here() {
 
 // What is multiplied: pointers to the tile's first row and column and the sum's first element.
 struct Tile {
-  const bf16 *r, *c;
-  const bf16* up;              // GLU: the second matrix of columns
-  const bf16 *r2, *c2;         // a second pair, added to the sum, or null
-  int rank, rank_c;            // EXTRA: how long a row of r2 is, a multiple of 32, and of c2, one of 8: zeros behind it
-  int rows, cols;              // of the output, from the tile's first on
-  int sum;                     // a multiple of 64 unless both operands are COLS
-  bf16* out;
-  float* part;                 // PARTS: where the tile's sums go instead
+  const bf16 *r = nullptr, *c = nullptr;
+  const bf16* up = nullptr;    // GLU: the second matrix of columns
+  bf16 *one = nullptr, *other = nullptr;       // KEEP: where its sums go
+  const bf16 *r2 = nullptr, *c2 = nullptr;     // a second pair, added to the sum, or null
+  int rank = 0, rank_c = 0;    // EXTRA: how long a row of r2 is, a multiple of 32, and of c2, one of 8: zeros behind it
+  int rows = 0, cols = 0;      // of the output, from the tile's first on
+  int sum = 0;                 // a multiple of 64 unless both operands are COLS
+  bf16* out = nullptr;
+  float* part = nullptr;       // PARTS: where the tile's sums go instead
+
+  // Member by member: a copy of the whole went through memory, and the wait for it was one for all loads under way (of
+  // groups 4% of the time).
+  __device__ __forceinline__ Tile() {}
+  __device__ __forceinline__ Tile(const Tile& t) { *this = t; }
+  __device__ __forceinline__ Tile& operator=(const Tile& t) {
+    r = t.r, c = t.c, up = t.up, one = t.one, other = t.other, r2 = t.r2, c2 = t.c2, rank = t.rank, rank_c = t.rank_c;
+    rows = t.rows, cols = t.cols, sum = t.sum, out = t.out, part = t.part;
+    return *this;
+  }
 };
 
 // 16 rows how often a wave has, in a tile with so many rows left
@@ -139,11 +167,13 @@ struct Shape {
 
 // SHORT: the sum may end within what is loaded. TWO: 16 rows of one matrix, 16 of the other, 128 of each; the first two
 // waves load the one's, the others the other's.
-template <bool COLS, bool SHORT, bool TWO = false>
+// FEW: one register for the loads' addresses, which are equally far apart, instead of N.
+template <bool COLS, bool SHORT, bool TWO = false, bool FEW = false>
 struct Operand {
+  static_assert(!COLS || !FEW);
   static constexpr int N = COLS ? 4 : 8;       // loads of a wave: for a step, or for a pair
   static constexpr int W = COLS ? 8 : 2;
-  unsigned off[N];             // a lane's part of the loads' addresses
+  unsigned off[FEW ? 1 : N];   // a lane's part of the loads' addresses
   unsigned win[W];             // and of the reads', in the pair of buffers at hand
   const char* base;
   unsigned ld, num;            // bytes: from row to row, and from base on that may be read
@@ -154,7 +184,7 @@ struct Operand {
     const int lane = threadIdx.x & 63;
     ld = ld_;
 #pragma unroll
-    for (int h = 0; h < N; ++h) {
+    for (int h = 0; h < (FEW ? 1 : N); ++h) {
       if constexpr (COLS) {
         const int row = 8 * h + 2 * wid + (lane >> 5);
         off[h] = row * ld + ((lane & 31) ^ (place(row) << 1)) * 16;
@@ -163,6 +193,11 @@ struct Operand {
         off[h] = from * ld + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
       }
     }
+  }
+  // load h, to `to` + `at`
+  __device__ __forceinline__ void load(unsigned to, int at, int h) const {
+    if constexpr (FEW) load_lds(to, at, off[0], h * (TWO ? 16 : 32) * ld, base, num);
+    else load_lds(to, at, off[h], base, num);
   }
   // The loads go on with another tile, `edge` rows or columns of the output wide. What lies outside of it or of
   // the sum is not read: rows beyond are zeros, and so are those of the summed index. (Columns beyond are the
@@ -240,11 +275,13 @@ struct Operand {
 // PARTS: tiles of sums that are added up later, 32 bits in the order of the accumulators.
 // RELU2: the results are max(sum, 0)^2.
 // GLU: the columns are 16 of one matrix and 16 of another, in turn, so that a lane has the sums of both for its column;
-// the results, half as many, are silu(one) other.
+// the results, half as many, are silu(one) other. KEEP: both sums are written too, and silu is of what is
+// written.
 // EXTRA: the second pair is [rows][rank] and [columns][rank_c], short rows that are loaded as fragments behind the
 // sum. They come from the L2, and with them the wave waits for the next tile's loads (8192 rows, a sum of 4096,
 // 4096 columns: 192 us without, 190 with it).
-template <bool RC, bool CC, class Tiles, bool SHORT = RC && CC, bool PARTS = false, bool EXTRA = false, bool RELU2 = false, bool GLU = false>
+template <bool RC, bool CC, class Tiles, bool SHORT = RC && CC, bool PARTS = false, bool EXTRA = false, bool RELU2 = false, bool GLU = false,
+          bool KEEP = false>
 struct Run {
   static constexpr bool TN = RC && CC, NN = !RC && CC, NT = !CC;
   Tiles& tiles;
@@ -252,8 +289,8 @@ struct Run {
   const Shape shape;
   unsigned lds, cur, oth;      // buffers' addresses: of the pair at hand, of the other
   int by, wid;
-  Operand<RC, SHORT> R;
-  Operand<CC, SHORT, GLU> C;
+  Operand<RC, SHORT, false, KEEP> R;   // (KEEP: with a register for each load others went to memory in every step)
+  Operand<CC, SHORT, GLU, KEEP> C;
 
   __device__ __forceinline__ Run(Tiles& t, const Shape& sh, char* s) : tiles(t), smem(s), shape(sh) {
     wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -281,12 +318,12 @@ struct Run {
   }
   __device__ __forceinline__ void rows(unsigned to, int at) {
 #pragma unroll
-    for (int h = 0; h < decltype(R)::N; ++h) load_lds(to, at + h * 4096, R.off[h], R.base, R.num);
+    for (int h = 0; h < decltype(R)::N; ++h) R.load(to, at + h * 4096, h);
     R.seek();
   }
   __device__ __forceinline__ void cols(unsigned to, int at) {
 #pragma unroll
-    for (int h = 0; h < decltype(C)::N; ++h) load_lds(to, HALF + at + h * 4096, C.off[h], C.base, C.num);
+    for (int h = 0; h < decltype(C)::N; ++h) C.load(to, HALF + at + h * 4096, h);
     C.seek();
   }
 
@@ -331,7 +368,7 @@ struct Run {
       constexpr bool FIRST = decltype(first_)::value;
       constexpr int DENSE = READS > 3 * S / 8 ? READS : 3 * S / 8;
       constexpr int MID = DENSE + 4, OVER = 2 * S - MID;       // NT: slots of a pair that loads are spread over
-      constexpr int LATER = (NT ? ((S + S / 2 - MID) * 16 + OVER - 1) / OVER : NN && P == 1 ? 8 : 16) + (FIRST ? (GLU ? 8 : 16) : 0);
+      constexpr int LATER = (NT ? ((S + S / 2 - MID) * 16 + OVER - 1) / OVER : NN && P == 1 ? 8 : 16) + (FIRST ? (GLU && !KEEP ? 8 : 16) : 0);
       // slots of the reads
       constexpr int FROM = NT && P == 1 ? S / 2 : 0, TO = TN || NN || P == 1 ? S : DENSE;
       if constexpr (!NT) {
@@ -361,8 +398,8 @@ struct Run {
           if constexpr (P * S + m >= MID)
             fa::spread<P * S + m - MID, OVER, 16>([&](auto l_) __attribute__((always_inline)) {
               constexpr int l = decltype(l_)::value / 2, odd = decltype(l_)::value % 2;
-              if constexpr (odd) load_lds(cur, l * 4096, R.off[l], R.base, R.num);
-              else load_lds(cur, HALF + l * 4096, C.off[l], C.base, C.num);
+              if constexpr (odd) R.load(cur, l * 4096, l);
+              else C.load(cur, HALF + l * 4096, l);
               if constexpr (l == 7 && odd) R.seek();
               if constexpr (l == 7 && !odd) C.seek();
             });
@@ -490,29 +527,34 @@ struct Run {
     asm volatile("" ::: "memory");
   }
 
-  // The same of silu(acc[i][2 j]) acc[i][2 j + 1], 64 columns a wave: 2 NR stores.
+  // The same of silu(acc[i][2 j]) acc[i][2 j + 1], 64 columns a wave: 2 NR stores. KEEP: of the sums too, 6 NR.
   template <int NR>
   __device__ __forceinline__ void store_glu(const f32x4_t (&acc)[NR][8], const Tile& t) {
     const int lane = lane_here(), i16 = lane & 15, g = lane >> 4;
     char* mine = smem + STAGE + wid * 4096;
     const int c0 = (wid & 1) * 64, chunks = min(t.cols - c0, 64) / 8, r0 = (wid >> 1) * (NR * 16);
-    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(t.out, 0, 0xffffff00, 0x00027000);
-    auto put = [&](auto i_) __attribute__((always_inline)) {
+    constexpr int W = KEEP ? 3 : 1;              // what is written of each row
+    const auto rsrc = [&](int what) __attribute__((always_inline)) {
+      return __builtin_amdgcn_make_buffer_rsrc(what == 0 ? t.out : what == 1 ? t.one : t.other, 0, 0xffffff00, 0x00027000);
+    };
+    auto put = [&](auto s_) __attribute__((always_inline)) {
+      constexpr int i = decltype(s_)::value / W, what = decltype(s_)::value % W;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         bf16x4_t w;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float a = acc[decltype(i_)::value][2 * j][r];
-          w[r] = (__bf16)(a * __builtin_amdgcn_rcpf(1.f + __expf(-a)) * acc[decltype(i_)::value][2 * j + 1][r]);
+          const float a = acc[i][2 * j][r], b = acc[i][2 * j + 1][r];
+          if constexpr (KEEP) w[r] = (__bf16)(what == 0 ? rounded_glu((__bf16)a, (__bf16)b) : what == 1 ? a : b);
+          else w[r] = (__bf16)(a * __builtin_amdgcn_rcpf(1.f + __expf(-a)) * b);
         }
         *reinterpret_cast<bf16x4_t*>(mine + i16 * 128 + (((2 * j + (g >> 1)) ^ (i16 >> 1)) << 4) + (g & 1) * 8) = w;
       }
       asm volatile("" ::: "memory");
     };
     put(std::integral_constant<int, 0>{});
-    fa::unrolled<NR>([&](auto i_) __attribute__((always_inline)) {
-      constexpr int i = decltype(i_)::value;
+    fa::unrolled<NR * W>([&](auto s_) __attribute__((always_inline)) {
+      constexpr int s = decltype(s_)::value, i = s / W;
       u32x4_t v[2];
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
@@ -520,12 +562,12 @@ struct Run {
         v[k] = *reinterpret_cast<const u32x4_t*>(mine + row * 128 + (((lane & 7) ^ (row >> 1)) << 4));
       }
       asm volatile("" ::: "memory");
-      if constexpr (i + 1 < NR) put(std::integral_constant<int, i + 1>{});
+      if constexpr (s + 1 < NR * W) put(std::integral_constant<int, s + 1>{});
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const int row = r0 + i * 16 + 8 * k + (lane >> 3);
         const unsigned o = row * shape.out + (c0 + (lane & 7) * 8) * 2;
-        __builtin_amdgcn_raw_buffer_store_b128(v[k], rsrc, row < t.rows && (lane & 7) < chunks ? o : 0xfffffff0u, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(v[k], rsrc(s % W), row < t.rows && (lane & 7) < chunks ? o : 0xfffffff0u, 0, 0);
       }
     });
     asm volatile("" ::: "memory");
@@ -549,7 +591,8 @@ struct Run {
     fa::barrier();
     for (;;) {
       const int next = tiles.next();
-      const Tile u = next < 0 ? t : tiles.get(next);     // (behind the last one nothing is made of the loads)
+      Tile u = t;              // (behind the last one nothing is made of the loads)
+      if (next >= 0) u = tiles.get(next);
       switch (rows16(t.rows)) {
         case 8: tile<8>(t, u); break;
         case 7: tile<7>(t, u); break;

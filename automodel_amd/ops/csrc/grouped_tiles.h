@@ -18,13 +18,14 @@ namespace amd_ops {
 struct GroupedArgs {
   const bf16 *r, *c;                   // operands of the output's rows and columns
   const bf16 *r2, *c2;                 // nn: a second pair, added to the sum
-  bf16* out;
+  const bf16* up;                      // GLU: like c
+  bf16 *out, *one, *other;             // one, other: GLU's sums
   const int *tile_map, *offs, *n_tiles;
   int n_mtiles, M, N, K, E;            // tile_map's capacity; rows; w is [E, N, K]
   int cap;                             // rows of a tile at most
 };
 
-enum Mode { NT, NN, TN };
+enum Mode { NT, NN, TN, GLU };         // GLU: nt of two weights, silu of the one times the other
 
 constexpr int MAX_GROUPS = 512, MAX_OWN = 513, BINS = 256;
 
@@ -79,7 +80,7 @@ struct GroupedTiles {
 
   __device__ __forceinline__ GroupedTiles(const GroupedArgs& a_, char* smem)
       : a(a_), s(*reinterpret_cast<Shared*>(smem + gt::SMEM)),
-        nc(((MODE == NT ? a.N : a.K) + gt::TILE - 1) / gt::TILE), nr((a.N + gt::TILE - 1) / gt::TILE) {}
+        nc(((MODE == NT ? a.N : MODE == GLU ? 2 * a.N : a.K) + gt::TILE - 1) / gt::TILE), nr((a.N + gt::TILE - 1) / gt::TILE) {}
 
   __device__ __forceinline__ int parts(int n) const { return MODE == TN ? nr : (n + a.cap - 1) / a.cap; }
   // 1 to LEVELS: how long a group's tiles take. nt, nn: their rows in 32, 4 at least (equal parts rounded up: from
@@ -101,7 +102,7 @@ struct GroupedTiles {
   // in quarters of a step's MFMAs of 32 rows: 128 cycles; a tile has some 6000 besides
   __device__ __forceinline__ int cost(int level, int most) const {
     if constexpr (MODE == TN) return (max(most, 64) + 31) / 32 * 8 / LEVELS * level + 48;
-    else return ((MODE == NT ? a.K : a.N) + 31) / 32 * (a.r2 ? 2 : 1) * level + 48;
+    else return ((MODE == NT || MODE == GLU ? a.K : a.N) + 31) / 32 * (a.r2 ? 2 : 1) * level + 48;
   }
 
   // sorts the groups, and the first tile
@@ -229,11 +230,12 @@ struct GroupedTiles {
   }
 
   __device__ __forceinline__ gt::Tile get(int id) const {
-    const int j = id / nc, c0 = (id - j * nc) * gt::TILE, i = MODE == TN ? j / nr : group_of(j);
+    int c0 = id % nc * gt::TILE;
+    const int j = id / nc, i = MODE == TN ? j / nr : group_of(j);
     const int e = __builtin_amdgcn_readfirstlane(s.group[i].e), row = __builtin_amdgcn_readfirstlane(s.group[i].row);
     const int n = __builtin_amdgcn_readfirstlane(s.group[i].n);
     const int at = j - __builtin_amdgcn_readfirstlane(s.group[i].start);
-    gt::Tile t{};
+    gt::Tile t;
     if constexpr (MODE == TN) {
       const int r0 = at * gt::TILE;
       t.rows = a.N - r0;
@@ -243,8 +245,10 @@ struct GroupedTiles {
       t.c = a.c + (long)row * a.K + c0;
       t.out = a.out + ((long)e * a.N + r0) * a.K + c0;
     } else {
-      const int h = 32 * level(n, 0), r0 = row + at * h, sum = MODE == NT ? a.K : a.N, cols = MODE == NT ? a.N : a.K;
-      const long w = (long)e * a.N * a.K + (MODE == NT ? (long)c0 * a.K : c0);
+      constexpr bool ROWS = MODE == NT || MODE == GLU;
+      const int h = 32 * level(n, 0), r0 = row + at * h, sum = ROWS ? a.K : a.N, cols = ROWS ? a.N : a.K;
+      if (MODE == GLU) c0 /= 2;
+      const long w = (long)e * a.N * a.K + (ROWS ? (long)c0 * a.K : c0);
       t.rows = min(n - at * h, h);
       t.cols = cols - c0;
       t.sum = sum;
@@ -255,6 +259,11 @@ struct GroupedTiles {
         t.c2 = a.c2 + w;
       }
       t.out = a.out + (long)r0 * cols + c0;
+      if (MODE == GLU) {
+        t.up = a.up + w;
+        t.one = a.one + (long)r0 * cols + c0;
+        t.other = a.other + (long)r0 * cols + c0;
+      }
     }
     return t;
   }

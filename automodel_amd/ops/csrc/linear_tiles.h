@@ -56,7 +56,7 @@ struct Tiles {
     const int s = u / (nr * nc), from = s * a.per;
     int r0, c0;
     place(u - s * nr * nc, nr, nc, a.height, r0, c0);
-    gt::Tile t{};
+    gt::Tile t;
     t.rows = min(a.rows - r0, a.height);
     t.cols = a.cols - c0;
     t.sum = min(a.sum - from, a.per);

@@ -186,6 +186,9 @@ bool small_takes(int64_t T, int64_t N, int64_t K);
 std::tuple<int64_t, int64_t> small_cut(int64_t rows, int64_t cols, int64_t sum);
 at::Tensor linear_small(const at::Tensor& x, const at::Tensor& w);
 at::Tensor linear_y(const at::Tensor& x, const at::Tensor& w, bool relu2);
+std::tuple<at::Tensor, at::Tensor, at::Tensor> grouped_glu(const at::Tensor& x, const at::Tensor& w, const at::Tensor& up,
+                                                           const at::Tensor& offs, const at::Tensor& tile_map,
+                                                           const std::optional<at::Tensor>& n_tiles, int64_t bm);
 at::Tensor linear_glu(const at::Tensor& x, const at::Tensor& w, const at::Tensor& up);
 std::vector<int64_t> linear_y_cut(int64_t T, int64_t N, int64_t K);
 at::Tensor linear_dw(const at::Tensor& g, const at::Tensor& x);
