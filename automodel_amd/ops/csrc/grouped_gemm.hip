@@ -24,7 +24,8 @@
 // grouped_gemm_kernel; nn and tn: four waves of 128 x 128 from 512 rows on) -> by grouped_tile_kernel: 65536
 // rows, 128 experts, 768 x 2048: 253 / 265 / 270 -> 230 / 227 / 230 us; 2048 x 768: 276 / 232 / 271 -> 252 /
 // 210 / 242 us; 19200 rows, 64 experts, 1408 x 2048: 166 / 175 / 197 -> 149 / 129 / 169 us; 16384 rows, 32
-// experts, 512 x 1024 (128-row tiles): 32 / 36 / 24 -> 30 / 32 / 24. The products alone are 137 us of the first
+// experts, 512 x 1024 (128-row tiles): 32 / 36 / 24 -> 30 / 32 / 24. Since its loads are spread
+// evenly (gemm_tile.h) nt of the first takes 220, of the second 235. The products alone are 137 us of the first
 // at the 1.5 PFLOP/s that the card holds (its clock falls to 1.2 to 1.9 GHz), its operands and results 150 us
 // at 5 TB/s.
 

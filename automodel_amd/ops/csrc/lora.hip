@@ -7,6 +7,9 @@
 // 8192 rows: 4096 -> 6144: 60 us, -> 28672: 272, 4096 -> 4096: 38, 14336 -> 4096: 88 (reading x and
 // y and writing out at 4.8 TB/s: 56, 210, 42, 77).
 //
+// Where the base layer is a plain frozen one in training, its own tiles have the second product behind their sums instead
+// (linear_grad.hip: lora_linear), and only t is formed here.
+//
 // Shapes: x [M, H] bf16, A [r, H], B [O, r], H % 64 == 0, O % 64 == 0; r 32 or 64, or a multiple of 8 below,
 // which the kernels fill up with zeros.
 // Below: the segmented kernel for several adapters in one batch (serving).
