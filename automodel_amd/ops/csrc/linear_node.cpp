@@ -3,7 +3,11 @@
 // these are the faster ones, else the library's.
 
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/forward_grad.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/ATen.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 
 #include "ops_api.h"
 
@@ -28,8 +32,15 @@ bool plain(const at::Tensor& t) {
          reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 
+// Whether something besides autograd follows the operations: a dispatch mode (maybe around the backward alone), a
+// transform, forward-mode derivatives, a trace. It sees into torch's operations but not into the kernels.
+bool followed() {
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::autograd::ForwardADLevel::try_get_by_idx(0) ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || torch::jit::tracer::isTracing();
+}
+
 bool takes(const at::Tensor& a, const at::Tensor& b, int64_t T, int64_t N, int64_t K, int64_t most) {
-  return small_takes(T, N, K) && T * N * K < most && plain(a) && plain(b) && a.device() == b.device();
+  return !followed() && small_takes(T, N, K) && T * N * K < most && plain(a) && plain(b) && a.device() == b.device();
 }
 
 at::Tensor forward_of(const at::Tensor& x, const at::Tensor& w) {

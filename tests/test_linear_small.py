@@ -162,6 +162,28 @@ def test_what_stays_the_module():
 
 @gpu
 @cuda
+def test_a_mode_around_the_backward_alone():
+    """It sees the products, as it does those of the module's own call."""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    T, N, K = 64, 128, 256
+    torch.manual_seed(0)
+    lin = nn.Linear(K, N, bias=False, device="cuda", dtype=torch.bfloat16)
+    x, g = rand(T, K).requires_grad_(), rand(T, N)
+    y = L.linear(lin, x)
+    assert "SmallLinear" in y.grad_fn.name()
+    with FlopCounterMode(display=False) as count:
+        dx, dw = _grads(y, (x, lin.weight), g)
+    assert count.get_total_flops() == 4 * T * N * K
+    close(dx, g.double() @ lin.weight.double(), N)
+    close(dw, g.double().t() @ x.double(), T)
+    with torch.autograd.forward_ad.dual_level(), FlopCounterMode(display=False) as count:
+        _grads(y, (lin.weight,), g)
+    assert count.get_total_flops() == 2 * T * N * K
+
+
+@gpu
+@cuda
 @pytest.mark.parametrize("kept", ["hooks", "cpu", "checkpoint", "reentrant"])
 def test_what_is_kept_for_the_backward(kept):
     from torch.utils.checkpoint import checkpoint
