@@ -250,6 +250,12 @@ class SharedExpert(nn.Module):
                           beside)
 
 
+def _takes_beside(shared: nn.Module) -> bool:
+    """Whether its call can be told: the forward is SharedExpert's, also that of a class made from it (by sharding, for
+    one), and none in its place on the instance."""
+    return type(shared).forward is SharedExpert.forward and "forward" not in shared.__dict__
+
+
 _SHARED_STREAMS: dict = {}
 
 
@@ -301,8 +307,8 @@ class MoE(nn.Module):
             ss = _shared_stream(xf.device)
             ss.wait_stream(torch.cuda.current_stream())
             with torch.cuda.stream(ss):
-                own = type(self.shared_experts) is SharedExpert
-                shared = self.shared_experts(xf, beside=True) if own else self.shared_experts(xf)
+                told = {"beside": True} if _takes_beside(self.shared_experts) else {}
+                shared = self.shared_experts(xf, **told)
                 if getattr(self, "shared_expert_gate", None) is not None:
                     shared = torch.sigmoid(self.shared_expert_gate(xf)) * shared
             y = self.experts(xf, probs, indices, **known)
