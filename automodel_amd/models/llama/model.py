@@ -411,6 +411,12 @@ class LlamaModel(nn.Module):
         self.register_buffer("rope_cos", cos, persistent=False)
         self.register_buffer("rope_sin", sin, persistent=False)
 
+    @property
+    def positions(self) -> int | None:
+        """How many positions there are; None where no layer looks at them."""
+        nope = self.cfg.no_rope_layers
+        return self.rope_cos.shape[0] if nope is None or any(nope) else None
+
     def forward(self, input_ids: torch.Tensor, position_ids: torch.Tensor | None = None) -> torch.Tensor:
         begun = None
         if position_ids is not None and active_kv_cache() is not None:

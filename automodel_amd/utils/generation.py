@@ -104,7 +104,8 @@ class DecodeSession:
 
     @torch.no_grad()
     def decode(self, handles: list[int], tokens: torch.Tensor) -> torch.Tensor:
-        """tokens [n], the next one of each handle -> logits [n, vocab]."""
+        """tokens [n], the next one of each handle -> logits [n, vocab]. (A token that the model does not have is not looked
+        for: it is on the device. Its logits are NaN.)"""
         cache = self.cache
         with kv_cache_context(cache):
             cache.begin_forward()
@@ -115,6 +116,7 @@ class DecodeSession:
                 return logits
             if handles != self.live:
                 raise ValueError("a dense K/V cache moves its whole batch on")
+            self.check_position(cache.pos)
             if cache.pos < len(self.places):
                 pos = self.places[cache.pos:cache.pos + 1].unsqueeze(0)
             else:
@@ -122,6 +124,12 @@ class DecodeSession:
             logits = self.model(tokens.reshape(-1, 1), position_ids=pos)[:, -1]
             cache.advance(1)
             return logits
+
+    def check_position(self, last: int) -> None:
+        """Refuses positions behind the model's last one, which the host knows; a step would have NaN in their place."""
+        n = getattr(getattr(self.model, "model", None), "positions", None)
+        if n is not None and last >= n:
+            raise IndexError(f"position {last} of a model that has {n}")
 
     def release(self, handles: list[int]) -> None:
         """Give back what finished sequences hold."""
@@ -178,6 +186,8 @@ def generate_graphed(
     dev = input_ids.device
     use_hip_graph = (dev.type == "cuda") if use_hip_graph is None else use_hip_graph
     session = DecodeSession(model, B, T + max_new_tokens, static=True)
+    if max_new_tokens > 1:
+        session.check_position(T + max_new_tokens - 2)      # the last step's
     handles, logits = session.prefill(input_ids.tolist())
     out = torch.empty(B, max_new_tokens, dtype=input_ids.dtype, device=dev)
     with kv_cache_context(session.cache):
