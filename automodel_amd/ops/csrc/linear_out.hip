@@ -1,8 +1,8 @@
 // Launches of y = x w^T by the tiles of gemm_tile.h (linear_grad.hip has the rest). The library's tiles of 256 x 256
 // are as fast where they fill the chip's rounds and the sum is short, and leave CUs idle otherwise: here tiles and sums
 // are cut as the gradients' are. us, library -> here, bf16 of unit variance, the weights not in a cache:
-//   511 x 14336 -> 4096 92 -> 67 (256 rows, 8 parts), 1001 x 21504 -> 4096 240 -> 150, 3003 x 2048 -> 2816 43 -> 34,
-//   6001 x 4096 -> 4096 156 -> 143, 24000 x 4096 -> 14336 1977 -> 1913; 8192 x 4096 -> 28672 1264 and 1282.
+//   1001 x 14336 -> 4096 136 -> 113 (256 rows, 4 parts), 1001 x 21504 -> 4096 240 -> 155, 3003 x 2048 -> 2816 43 -> 37,
+//   4096 x 4096 -> 6144 167 -> 161, 6001 x 4096 -> 4096 161 -> 151; 8192 x 4096 -> 6144 278 and 288, which stays the library's.
 // The squared ReLU of a feed-forward layer's inner results is formed on the way out (6600 x 4096 -> 21504: a pass of 92 us
 // less, of some 800). So is the gate's product with the other half of a gated one (linear_glu): the tiles' columns are 16
 // of either weight in turn, and a lane has both sums. Against two products by the faster of library and kernel and a pass

@@ -93,8 +93,9 @@ __global__ __launch_bounds__(gt::THREADS, 1) void linear_tile_kernel(const Args 
 // us that tiles of `height` rows and sums in `parts` take. A pair of steps of a tile of 32 n rows takes a + b
 // n, a little more where all CUs are at work (the card's power); fitted to 114 shapes of either gradient and 5
 // heights (1, 2, 3, 4, 6 and 8 parts for two of them): off by 7% (rms), and the choice by it by 0.5% from the
-// best one. x w^T: fitted to the three or four best by it of 1917 shapes of 100 to 24000 rows; off by 10%, the choice
-// by 1.3%.
+// best one. x w^T: fitted to three or four cuts of 1917 shapes of 100 to 24000 rows; over 3752 others, with all heights and the
+// four to six likeliest ways to cut their sums, off by 13%. Where output_own (ops/linear.py) takes the product the choice is off
+// by 0.7% in the mean, by 5% and more for one shape in 20, by 22% at most (633 x 14336 -> 3000 78 us, by 256 rows and 6 parts 64).
 inline float predicted(Form form, long rows, long cols, long sum, int height, int parts) {
   struct Fit {
     float start, a, b, a_all, b_all, tile, add, add_mb;

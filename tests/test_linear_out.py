@@ -90,6 +90,8 @@ def test_rule():
     # whole rounds of the library's tiles; few tiles; few rows
     for sizes in ((8192, 28672, 4096), (8192, 4096, 14336), (511, 4096, 4096), (255, 32768, 4096)):
         assert not L.output_own(*sizes)
+    # few rows, where the weights' reads are the bound; a long sum in parts is another matter
+    assert not L.output_own(384, 18432, 4096) and L.output_own(400, 18432, 4096) and L.output_own(384, 18432, 8192)
     # forms that the kernel refuses
     for sizes in ((3003, 2816, 2080), (3003, 2812, 2048), (65536, 4096, 64), (1 << 23, 4096, 128), (3000, 1 << 23, 128)):
         assert not L.output_own(*sizes)
