@@ -163,9 +163,9 @@ at::Tensor linear_glu(const at::Tensor& x, const at::Tensor& w, const at::Tensor
 
 // x w^T + scale (x A^T) B^T, A [r, K], B [N, r], r a multiple of 8 up to 64: B's product behind the sums, one rounding. ->
 // {it, (x A^T)^T [r rounded up to 32, T to 64] with zeros behind both, which lora_grads reads}. Against the product by
-// the faster of kernel and library and lora_forward's pass over it: 1840 shapes of 100 to 8200 rows 0.88 of their time in
-// the mean, 0.82 from 2^31 products on; 8192 rows, 4096 -> 28672 1547 -> 1344 us, 4096 -> 6144 349 -> 301, 14336 -> 4096
-// 734 -> 700. 200 shapes are above 1.02, up to 1.2, of some 25 us, where the host is the bound and has a launch less.
+// the faster of kernel and library and lora_forward's pass over it, us: 8192 rows, 4096 -> 28672 1522 -> 1316, 4096 -> 6144
+// 338 -> 294, 14336 -> 4096 717 -> 679. Few tiles lose by it, as their sums are cut in parts or not at all, and so
+// do few rows of wide layers (ops/linear.py: adapted_own has the rule and what it was fitted to).
 std::tuple<at::Tensor, at::Tensor> lora_linear(const at::Tensor& x, const at::Tensor& w, const at::Tensor& A,
                                                const at::Tensor& B, double scale) {
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && A.dim() == 2 && B.dim() == 2 && x.size(1) == w.size(1),

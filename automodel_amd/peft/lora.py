@@ -24,6 +24,7 @@ from automodel_amd.ops.linear import (
     _ordinary,
     _plain,
     _unseen,
+    adapted_own,
     input_grad_takes,
     linear,
     product,
@@ -102,12 +103,12 @@ class _FusedLoRAFn(torch.autograd.Function):
 
 
 class _LoRALinear(torch.autograd.Function):
-    """x w^T + (x @ A^T) @ B^T * scale, w frozen: one product, and so is the gradient of x."""
+    """x w^T + (x @ A^T) @ B^T * scale, w frozen: one product where ``as_one``, and so is the gradient of x."""
 
     @staticmethod
-    def forward(ctx, x2, w, wa, wb, scale):
+    def forward(ctx, x2, w, wa, wb, scale, as_one=True):
         sizes = (x2.shape[0], *w.shape)
-        if (x2.shape[0] > 0 and max(sizes) < MAX_SIZE and w.shape[1] >= 128 and not followed()
+        if (as_one and x2.shape[0] > 0 and max(sizes) < MAX_SIZE and w.shape[1] >= 128 and not followed()
                 and _ordinary(x2, w, wa, wb) and _plain(x2, w, wa, wb)):
             from automodel_amd.ops._backend import hip_ops
 
@@ -128,7 +129,7 @@ class _LoRALinear(torch.autograd.Function):
             dx = hip_ops().linear_dx_extra(g, w, dt, a_t)
         else:
             dx = g @ w + _of_rank(dt, wa) @ wa
-        return dx, None, da, db, None
+        return dx, None, da, db, None, None
 
 
 class LinearLoRA(nn.Module):
@@ -190,7 +191,8 @@ class LinearLoRA(nn.Module):
                  and (x.numel() // x.shape[-1]) % 8 == 0)
         if fused and wb.dtype == wa.dtype and torch.is_grad_enabled() and input_grad_takes(self.base, x):
             x2 = x.reshape(-1, x.shape[-1]).contiguous()
-            y2 = _LoRALinear.apply(x2, self.base.weight, wa, wb, self.scale)
+            w = self.base.weight
+            y2 = _LoRALinear.apply(x2, w, wa, wb, self.scale, adapted_own(x2.shape[0], *w.shape))
             return y2.view(*x.shape[:-1], wb.shape[0])
         y = linear(self.base, x)
         if fused and y.dtype == torch.bfloat16:

@@ -108,3 +108,35 @@ def test_function(monkeypatch, rank):
         if twice:
             got, want = (torch.autograd.grad(sum((v * v).sum() for v in vs), wrt) for vs in (got, want))
             torch.testing.assert_close(got, want)
+
+
+def test_which_layers_are_one_product():
+    assert lora.adapted_own(8192, 28672, 4096) and lora.adapted_own(408, 6144, 4096) and lora.adapted_own(1000, 2048, 1024)
+    # few rows; few tiles; a weight's reads; half of the chip
+    for sizes in ((96, 6144, 4096), (168, 2048, 2048), (200, 1024, 4096), (128, 28672, 4096), (384, 10240, 2560)):
+        assert not lora.adapted_own(*sizes)
+    for sizes in ((1 << 23, 64, 128), (8192, 4096, 64)):                   # the kernel refuses these
+        assert not lora.adapted_own(*sizes)
+
+
+class Two(Kernels):
+    """Those of a layer whose product and adapter are two."""
+
+    def lora_linear(self, *_):
+        raise AssertionError
+
+    def lora_forward(self, y, x, a, b, scale):
+        t = x @ a.t()
+        return y + scale * t @ b.t(), torch.nn.functional.pad(t.t(), (0, -x.shape[0] % 64, 0, -a.shape[0] % 32))
+
+
+def test_two_products(monkeypatch):
+    monkeypatch.setattr(_backend, "hip_ops", Two)
+    monkeypatch.setattr(lora, "_plain", lambda *ts: True)
+    torch.manual_seed(0)
+    x, w, a, b = (torch.randn(s, dtype=torch.float64) for s in ((10, 192), (64, 192), (8, 192), (64, 8)))
+    g, wrt = torch.randn(10, 64, dtype=torch.float64), [v.requires_grad_() for v in (x, a, b)]
+    own = lora._LoRALinear.apply(x, w, a, b, 0.5, False)
+    ref = x @ w.t() + 0.5 * (x @ a.t()) @ b.t()
+    torch.testing.assert_close(own, ref)
+    torch.testing.assert_close(torch.autograd.grad(own, wrt, g), torch.autograd.grad(ref, wrt, g))
