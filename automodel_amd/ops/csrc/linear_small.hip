@@ -8,7 +8,8 @@
 // call one of the library's and 4 for one of these. A workgroup is 2 x 2 waves on a tile of 64 x 64 or, where there
 // are many tiles, 128 x 128; steps of 64 of the summed index come straight to LDS, the operands as they are (read by
 // rows, or by columns with the transposing reads: flash_tile.h). Two steps are under way (128: one, two workgroups to a
-// CU). Where few tiles have long sums these are cut into parts, kept in 32 bits and added up in their order.
+// CU). Where few tiles have long sums these are cut into parts, kept in 32 bits and added up in their order. x w^T of few
+// rows is another kernel's.
 //
 // us, library -> here, captured, so that neither waits for the host: nt 256 x 256 x 256 11.7 -> 3.5, 256 x 1024 x 256
 // 4.3 -> 3.5, 1000 x 1536 x 2048 13.1 -> 14; nn 256 x 512 x 256 18.8 -> 4.4, 500 x 1536 x 2048 11.3 -> 9, 1000 x 3584 x
@@ -33,6 +34,10 @@ using namespace fa;
 
 constexpr int STEP = 64, WAVES = 4;    // of the summed index; 2 x 2 waves a workgroup
 constexpr unsigned NOWHERE = 0xfffffff0u, REACH = 0xffffff00u;
+// Up to so many rows x w^T is gemv.hip's, which reads the weights once: 0.65 of the library's time in the mean, captured,
+// above 1.05 for one shape in a hundred; the tiles here 0.96 and two in five, up to 1.67. From 17 to 32 rows 0.92 and 0.93,
+// then 1.3 and more against 0.85 (2901 shapes of 1 to 64 rows, 256 to 32768 columns and sums).
+constexpr int64_t FEW = 16;
 
 struct Args {
   const bf16 *r, *c;
@@ -268,6 +273,10 @@ bool small_takes(int64_t T, int64_t N, int64_t K) {
 at::Tensor small_nt(const at::Tensor& x, const at::Tensor& w) {
   check(x, w, "small_nt");
   TORCH_CHECK(x.size(1) == w.size(1) && small_takes(x.size(0), w.size(0), w.size(1)), "small_nt: x [T, K], w [N, K], N%8 == 0, K%8 == 0");
+  if (x.size(0) <= FEW) {
+    const c10::DeviceGuard guard(x.device());
+    return gemm_skinny_bf16(x, w, false, false, 0);
+  }
   return product<false, false>(x, w, x.size(0), w.size(0), w.size(1));
 }
 at::Tensor small_nn(const at::Tensor& g, const at::Tensor& w) {

@@ -38,6 +38,24 @@ def test_products(T, N, K):
     close(ops.small_tn(g, x), g.double().t() @ x.double(), T)
 
 
+# both sides of the line between the kernels of few rows and of tiles; whole and broken steps of either
+@gpu
+@cuda
+@pytest.mark.parametrize("T", [2, 15, 16, 17])
+@pytest.mark.parametrize("N,K", [(8, 4104), (72, 136), (1000, 512), (1536, 64)])
+def test_few_rows(T, N, K):
+    from automodel_amd.ops._backend import hip_ops
+
+    torch.manual_seed(T)
+
+    def within(*shape):                  # nothing beyond an operand is read into a result
+        whole = torch.full((shape[0] * shape[1] + 4096,), float("inf"), device="cuda", dtype=torch.bfloat16)
+        whole[: shape[0] * shape[1]] = torch.randn(shape[0] * shape[1], device="cuda")
+        return whole[: shape[0] * shape[1]].view(shape)
+    x, w = within(T, K), within(N, K)
+    close(hip_ops().small_nt(x, w), x.double() @ w.double().t(), K)
+
+
 @gpu
 @cuda
 def test_edges_of_the_operands():
