@@ -105,8 +105,9 @@ class _Experts(torch.autograd.Function):
     Where ``inner``, the backward does without the experts' outputs. With dh the gradient of an unweighted row's activation
     h, a choice's weight has the gradient dh h, a sum over the inner width, and the weighted row p h is the operand of
     the last weight's gradient (csrc/swiglu.hip). That moves two rows of the hidden width less and one of the inner
-    width more: 0.96 to 1.0 of the time with hidden widths of twice the inner and more, 0.98 to 1.03 below (8000 and 3000
-    tokens, 8 to 128 experts)."""
+    width more: with hidden widths of twice the inner and more 0.96 to 1.06 of the time of forward and backward, 0.99 in the
+    mean, below 0.94 to 1.04 and 1.00 (826 layers of 500 to 8200 tokens, 8 to 128 experts:
+    profiles/sweep_experts_backward.csv)."""
 
     @staticmethod
     def forward(ctx, x, probs, gate, up, down, order, src, pos, perm_probs, probs32, offs, tile_map, n_tiles, bm):

@@ -372,7 +372,7 @@ at::Tensor grouped_gemm_nt(const at::Tensor& x, const at::Tensor& w,
 // {x w^T, x up^T, silu(the one) the other} of the groups. By the tiles of gemm_tile.h x is read once for both and the
 // activation is no pass of its own. The tiles are nt's of twice the columns, and so is the
 // rule. us, two products and swiglu -> here: 65536 rows, 128 experts, 768 x 2048 494 -> 430; 18018 rows, 64, 1408 x 2048
-// 323 -> 276; 291 shapes (4 to 128 groups of 60 to 2000 rows, 384 to 2048 columns, sums of 512 to 4096) 0.81 of the time
+// 323 -> 276; 291 shapes (4 to 128 groups of 60 to 2000 rows, 384 to 2048 columns, sums of 512 to 4096) 0.82 of the time
 // in the mean, 4 of them above 1.02, 1.16 at most.
 std::tuple<at::Tensor, at::Tensor, at::Tensor> grouped_glu(const at::Tensor& x, const at::Tensor& w, const at::Tensor& up,
                                                            const at::Tensor& offs, const at::Tensor& tile_map,
