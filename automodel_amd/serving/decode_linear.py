@@ -40,7 +40,7 @@ def _gemv_eligible(x: torch.Tensor, w: torch.Tensor) -> bool:
         return False
     rows = x.numel() // x.shape[-1]
     # measured on MI355X (profiles/README.md): the wave-per-row GEMV beats
-    # hipBLASLt up to ~4 rows; above that the library's m-tiled path wins
+    # hipBLASLt up to ~4 rows; above that `inferred` chooses
     return rows <= 4 and x.shape[-1] % 512 == 0
 
 
